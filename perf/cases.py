@@ -332,7 +332,7 @@ def _exact_features(case, s):
     zero = total(p.mu, c == 0) + total(p.mx, c == 0)
     fk = p.female[0]
     fo, fi = count(fk // (n + 1)), count(fk % (n + 1))
-    f = np.stack([np.log1p(od), np.log1p(idg), np.log1p(wsum), carried / (wsum + 1), zero / np.maximum(od + idg, 1),
+    f = np.stack([np.log1p(od), np.log1p(idg), np.log1p(wsum), carried / (wsum + 1), zero / (od + idg + 1),
                   np.log1p(fo[pi]), np.log1p(fi[pi]), np.log1p(carried)], axis=1)
     f[0] = 0
     return f
