@@ -351,7 +351,10 @@ extern "C" int bm_anneal_verify(bm_anneal* a, int64_t* mismatches) {
     for (int64_t c = 0; c < a->n_chains; c++) {
         BmDevGraph g = a->graphs[h[c].inst];
         g.pi = a->d_pool + h[c].pi_off;
-        AHIP(a, bm_launch_score(g, bm_ctx_launch(a->ctxs[h[c].inst], BM_KERNEL_SCORE), a->d_scores + c, a->stream));
+        const bm_ctx* ctx = a->ctxs[h[c].inst];
+        int64_t n_out = 0;
+        const int4* chunks = bm_ctx_chunks(ctx, nullptr, &n_out);
+        AHIP(a, bm_launch_score(g, chunks, n_out, a->d_scores + c, bm_ctx_num_cus(ctx), a->stream));
     }
     std::vector<int64_t> s((size_t)a->n_chains);
     AHIP(a, hipMemcpyAsync(s.data(), a->d_scores, sizeof(int64_t) * (size_t)a->n_chains, hipMemcpyDeviceToHost,

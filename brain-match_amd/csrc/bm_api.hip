@@ -46,9 +46,15 @@ struct bm_ctx {
     int2* d_f_out;
     int64_t* d_f_in_ptr;
     int2* d_f_in;
+    uint64_t* d_rt_desc[4]; /* row tables (bm_rowtab.h): female out, female in, male out, male in */
+    uint4* d_rt_tab[4];
+    int32_t packed;         /* row tables hold 4-byte slots */
+    int4* d_chunks;         /* male edge chunks (BM_EDGE_CHUNK), out-lists first */
+    int64_t n_chunks, n_out_chunks;
+    int64_t* d_diag;        /* n+1: per-vertex contributions, rewritten by every evaluation that uses them */
     int32_t compact;
     int32_t row_layout;     /* BM_ROWS_P19 when female weights are in 0..8191, else BM_ROWS_P15 (compact graphs) */
-    int32_t* d_pi;
+    int32_t* d_pi;          /* matching, then its inverse (n+1 each) */
     int64_t* d_small;       /* 16 int64 of scratch for scores / flags */
     int32_t* d_reorder;     /* n ints for the changed-first enumerations */
     BmLaunch tune[BM_KERNEL_COUNT];
@@ -166,6 +172,12 @@ static BmDevGraph devgraph(const bm_ctx* c) {
     g.f_in_ptr = c->d_f_in_ptr;
     g.f_in = c->d_f_in;
     g.pi = c->d_pi;
+    g.inv = c->pi_distinct ? c->d_pi + c->n + 1 : nullptr;
+    g.f_out_t = BmRowTab{c->d_rt_desc[0], c->d_rt_tab[0]};
+    g.f_in_t = BmRowTab{c->d_rt_desc[1], c->d_rt_tab[1]};
+    g.m_out_t = BmRowTab{c->d_rt_desc[2], c->d_rt_tab[2]};
+    g.m_in_t = BmRowTab{c->d_rt_desc[3], c->d_rt_tab[3]};
+    g.packed = c->packed;
     g.compact = c->compact;
     return g;
 }
@@ -246,6 +258,12 @@ static void free_ctx(bm_ctx* c) {
     (void)hipFree(c->d_f_in_ptr);
     (void)hipFree(c->d_f_in);
     (void)hipFree(c->d_pi);
+    for (int i = 0; i < 4; i++) {
+        (void)hipFree(c->d_rt_desc[i]);
+        (void)hipFree(c->d_rt_tab[i]);
+    }
+    (void)hipFree(c->d_chunks);
+    (void)hipFree(c->d_diag);
     (void)hipFree(c->d_small);
     (void)hipFree(c->d_reorder);
     if (c->pending) {
@@ -390,6 +408,51 @@ extern "C" void bm_destroy(bm_ctx* ctx) {
     free_ctx(ctx);
 }
 
+/* Row tables of one adjacency: descriptors from the row lengths (at most half
+ * of a row's slots are used; bucket 0 stays empty for the empty rows),
+ * entries inserted on the device. */
+static int build_rowtab(bm_ctx* c, int i, const int64_t* h_ptr, const int64_t* d_ptr, const int2* d_adj) {
+    const int32_t n = c->n;
+    const int64_t per = c->packed ? 4 : 2;
+    std::vector<uint64_t> desc((size_t)n + 1, 0);
+    uint64_t at = 1;
+    for (int32_t r = 0; r <= n; r++) {
+        const int64_t deg = h_ptr[r + 1] - h_ptr[r];
+        if (deg <= 0) continue;
+        uint32_t lb = 0;
+        while ((per << lb) < 2 * deg) lb++;
+        desc[(size_t)r] = (at << 6) | lb;
+        at += (uint64_t)1 << lb;
+    }
+    int rc = dalloc(c, &c->d_rt_desc[i], (size_t)n + 1);
+    if (rc == BM_OK) rc = dalloc(c, &c->d_rt_tab[i], (size_t)at);
+    if (rc == BM_OK) rc = h2d(c, c->d_rt_desc[i], desc.data(), desc.size());
+    if (rc != BM_OK) return rc;
+    HIPCHK(c, hipMemsetAsync(c->d_rt_tab[i], 0, (size_t)at * sizeof(uint4), c->stream));
+    HIPCHK(c, bm_launch_rowtab_fill(c->packed, d_ptr, d_adj, n, c->d_rt_desc[i], c->d_rt_tab[i], c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));   /* desc goes out of scope */
+    return BM_OK;
+}
+
+/* The male lists in chunks of at most BM_EDGE_CHUNK entries, out-lists first. */
+static int build_chunks(bm_ctx* c) {
+    std::vector<int4> ch;
+    for (int in = 0; in < 2; in++) {
+        const int64_t* p = in ? c->male.in.ptr : c->male.out.ptr;
+        for (int32_t r = 1; r <= c->n; r++)
+            for (int64_t t = 0, deg = p[r + 1] - p[r]; t < deg; t += BM_EDGE_CHUNK)
+                ch.push_back(make_int4(r, in, (int32_t)t, (int32_t)(deg - t < BM_EDGE_CHUNK ? deg - t : BM_EDGE_CHUNK)));
+        if (!in) c->n_out_chunks = (int64_t)ch.size();
+    }
+    c->n_chunks = (int64_t)ch.size();
+    int rc = dalloc(c, &c->d_chunks, ch.size());
+    if (rc == BM_OK) rc = dalloc(c, &c->d_diag, (size_t)c->n + 1);
+    if (rc == BM_OK) rc = h2d(c, c->d_chunks, ch.data(), ch.size());
+    if (rc != BM_OK) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return BM_OK;
+}
+
 /* Launch shape of the scan kernels for a batch of k candidates.  Unless the
  * caller set one (bm_set_tuning), a batch too small to fill the device's wave
  * slots (k < 32,768: at most four candidates per slot) runs in 4-wave blocks
@@ -524,7 +587,7 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_out, (size_t)fg.m);
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_in_ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_in, (size_t)fg.m);
-    if (rc == BM_OK) rc = dalloc(c, &c->d_pi, (size_t)n + 1);
+    if (rc == BM_OK) rc = dalloc(c, &c->d_pi, 2 * ((size_t)n + 1));
     if (rc == BM_OK) rc = dalloc(c, &c->d_small, 16);
     if (rc == BM_OK) rc = dalloc(c, &c->d_reorder, (size_t)n);
     if (rc == BM_OK) rc = h2d(c, c->d_m_out_ptr, mg.out.ptr, (size_t)n + 2);
@@ -539,8 +602,14 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = h2d(c, c->d_f_out, fg.out.adj, (size_t)fg.m);
     if (rc == BM_OK) rc = h2d(c, c->d_f_in_ptr, fg.in.ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = h2d(c, c->d_f_in, fg.in.adj, (size_t)fg.m);
+    c->packed = c->compact && c->male_nonneg;
+    if (rc == BM_OK) rc = build_rowtab(c, 0, fg.out.ptr, c->d_f_out_ptr, c->d_f_out);
+    if (rc == BM_OK) rc = build_rowtab(c, 1, fg.in.ptr, c->d_f_in_ptr, c->d_f_in);
+    if (rc == BM_OK) rc = build_rowtab(c, 2, mg.out.ptr, c->d_m_out_ptr, c->d_m_out);
+    if (rc == BM_OK) rc = build_rowtab(c, 3, mg.in.ptr, c->d_m_in_ptr, c->d_m_in);
+    if (rc == BM_OK) rc = build_chunks(c);
     c->pi_distinct = 1;   /* all unmatched */
-    if (rc == BM_OK && hipMemsetAsync(c->d_pi, 0, ((size_t)n + 1) * sizeof(int32_t), c->stream) != hipSuccess)
+    if (rc == BM_OK && hipMemsetAsync(c->d_pi, 0, 2 * ((size_t)n + 1) * sizeof(int32_t), c->stream) != hipSuccess)
         rc = fail(c, BM_ERR_HIP, "hipMemsetAsync failed");
     if (rc == BM_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, BM_ERR_HIP, "hipStreamSynchronize failed");
     bm_rowhash_free(&ho);
@@ -575,22 +644,22 @@ extern "C" int bm_set_mapping(bm_ctx* c, const int32_t* pi) {
     for (int32_t i = 1; i <= c->n; i++)
         if (pi[i] < 0 || pi[i] > c->n)
             return fail(c, BM_ERR_ARG, "bm_set_mapping: pi[%d] = %d outside 0..%d", i, pi[i], c->n);
-    {
-        std::vector<uint8_t> seen((size_t)c->n + 1, 0);
-        c->pi_distinct = 1;
-        for (int32_t i = 1; i <= c->n && c->pi_distinct; i++) {
-            if (pi[i] != 0 && seen[pi[i]]) c->pi_distinct = 0;
-            seen[pi[i]] = 1;
-        }
+    /* the matching and its inverse in one upload (entries 0 are 0) */
+    const size_t len = (size_t)c->n + 1;
+    std::vector<int32_t> both(2 * len, 0);
+    c->pi_distinct = 1;
+    for (int32_t i = 1; i <= c->n; i++) {
+        const int32_t f = pi[i];
+        both[(size_t)i] = f;
+        if (f == 0) continue;
+        if (both[len + (size_t)f] != 0) c->pi_distinct = 0;
+        both[len + (size_t)f] = i;
     }
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipMemcpyAsync(c->d_pi + 1, pi + 1, (size_t)c->n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-    if (c->gain_on) {
-        int rc = gain_rebuild(c);
-        if (rc != BM_OK) return rc;
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return BM_OK;
+    HIPCHK(c, hipMemcpyAsync(c->d_pi, both.data(), 2 * len * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+    const int rc = c->gain_on ? gain_rebuild(c) : BM_OK;
+    HIPCHK(c, hipStreamSynchronize(c->stream));   /* on failure too: `both` is being read */
+    return rc;
 }
 
 extern "C" int bm_get_mapping(bm_ctx* c, int32_t* pi) {
@@ -608,7 +677,7 @@ extern "C" int bm_score(bm_ctx* c, int64_t* score) {
     HIPCHK(c, hipMemsetAsync(c->d_small, 0, sizeof(int64_t), c->stream));
     KTiming t;
     timing_begin(c, BM_KERNEL_SCORE, &t);
-    HIPCHK(c, bm_launch_score(devgraph(c), c->tune[BM_KERNEL_SCORE], c->d_small, c->stream));
+    HIPCHK(c, bm_launch_score(devgraph(c), c->d_chunks, c->n_out_chunks, c->d_small, c->num_cus, c->stream));
     timing_end(c, &t);
     HIPCHK(c, hipMemcpyAsync(score, c->d_small, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1167,7 +1236,7 @@ static int accept_impl(bm_batch* b, int64_t max_accept, int32_t* accepted, int64
         int rc = gain_moves_cap(c, 2 * (b->k > 0 ? b->k : 1));
         if (rc != BM_OK) return rc;
     }
-    HIPCHK(c, bm_launch_accept(devgraph(c), c->d_pi, (const int2*)b->d_cand, b->d_delta, b->k, max_accept,
+    HIPCHK(c, bm_launch_accept(devgraph(c), c->d_pi, c->d_pi + c->n + 1, (const int2*)b->d_cand, b->d_delta, b->k, max_accept,
                                b->d_acc_scratch, b->acc_scratch_bytes, b->d_acc_idx, b->d_out,
                                c->gain_on ? c->d_moves : nullptr, c->stream));
     if (c->gain_on && b->k > 0) {
@@ -1278,7 +1347,7 @@ extern "C" int bm_apply_swap(bm_ctx* c, int32_t u, int32_t v) {
         if (rc != BM_OK) return rc;
         HIPCHK(c, bm_launch_moves_from_swap(c->d_pi, u, v, c->d_moves, c->d_nmoves, c->stream));
     }
-    HIPCHK(c, bm_launch_apply_swap(c->d_pi, u, v, c->stream));
+    HIPCHK(c, bm_launch_apply_swap(c->d_pi, c->d_pi + c->n + 1, u, v, c->stream));
     if (c->gain_on) {
         const int32_t xs[2] = {u, v};
         return gain_patch(c, c->d_nmoves, 2, gt_patch_pays(c, xs, 2));
@@ -1368,7 +1437,7 @@ extern "C" int bm_apply_perm3(bm_ctx* c, int32_t a, int32_t b, int32_t d, int32_
         if (rc != BM_OK) return rc;
         HIPCHK(c, bm_launch_moves_from_perm3(c->d_pi, a, b, d, p, c->d_moves, c->d_nmoves, c->stream));
     }
-    HIPCHK(c, bm_launch_apply_perm3(c->d_pi, a, b, d, p, c->stream));
+    HIPCHK(c, bm_launch_apply_perm3(c->d_pi, c->d_pi + c->n + 1, a, b, d, p, c->stream));
     if (c->gain_on) {
         const int32_t xs[3] = {a, b, d};
         return gain_patch(c, c->d_nmoves, 3, gt_patch_pays(c, xs, 3));
@@ -1736,6 +1805,11 @@ void bm_batch_mark_pairs(bm_batch* b, int64_t k) {
 int bm_ctx_device(const bm_ctx* c) { return c->device; }
 int bm_ctx_num_cus(const bm_ctx* c) { return c->num_cus; }
 hipStream_t bm_ctx_stream(const bm_ctx* c) { return c->stream; }
+const int4* bm_ctx_chunks(const bm_ctx* c, int64_t* n_chunks, int64_t* n_out) {
+    if (n_chunks) *n_chunks = c->n_chunks;
+    if (n_out) *n_out = c->n_out_chunks;
+    return c->d_chunks;
+}
 BmLaunch bm_ctx_launch(const bm_ctx* c, int kernel) { return c->tune[kernel]; }
 
 extern "C" int bm_ctx_fail(bm_ctx* c, int code, const char* msg) { return fail(c, code, "%s", msg); }

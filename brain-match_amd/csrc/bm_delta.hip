@@ -29,6 +29,7 @@
 #include "bm_device.h"
 #include "bm_devutil.h"
 #include "bm_rng.h"
+#include "bm_rowtab.h"
 
 using namespace bmd;
 
@@ -654,44 +655,131 @@ __global__ void __launch_bounds__(512) k_rot3(BmDevGraph g, int4* __restrict__ c
 }
 
 /* ------------------------------------------------------------------ */
-/* Full score                                                          */
+/* Sums over the male lists: full score, current contributions, features */
 /* ------------------------------------------------------------------ */
 
-template <bool COMPACT>
-__global__ void __launch_bounds__(512) k_score(BmDevGraph g, int64_t* __restrict__ acc_out, uint32_t cap) {
-    typedef typename Slot<COMPACT>::T S;
-    extern __shared__ uint4 smem[];
+enum { kSumScore = 0, kSumDiag = 1, kSumFeature = 2 };
+constexpr int kStageBuckets = 256;   /* largest row table staged per wave: 4 KB */
+
+/* One wave per chunk of at most BM_EDGE_CHUNK entries of one vertex's male
+ * list (the chunks depend only on the male graph), so a hub's lists spread
+ * over many waves: every entry's contribution under the matching is a lookup
+ * in the female row of the vertex's image.  Four entries per lane, each level
+ * of their loads issued together.  A row table of at most 4 KB is first
+ * copied to the wave's LDS slice: the 216 lookups of an average in-list hit
+ * 2 KB of table, but with 32 waves' tables competing for a 32 KB L1 most of
+ * them would each fetch a 128-byte line from L2 (both lists of the 4M-edge
+ * pair: 78 us without the copy, 58 us with it).  What remains is the gather of
+ * pi and the hubs' tables, which no LDS slice holds.  n = 18,524, 4M edges:
+ * score 47 us (one wave per vertex, building its table first: 350-800 us, the
+ * longest out-list set the time), features 58 us (8-byte linear-probing
+ * tables, one dependent load per lane: 132 us).
+ *   SCORE:   out-lists only, everything into out[0];
+ *   DIAG:    out[x] += the contributions of x's out-edges and of its other
+ *            in-edges (a self-loop counts once);
+ *   FEATURE: out + 4 x += {contributions, weights, entries contributing 0}. */
+template <bool PACKED, int MODE>
+__global__ void __launch_bounds__(256) k_edge_sums(BmDevGraph g, const int4* __restrict__ chunks, int64_t nchunks,
+                                                   int64_t* __restrict__ out) {
+    constexpr int U = BM_EDGE_CHUNK / BM_WAVE;
+    __shared__ uint4 s_tab[4][kStageBuckets];
+    __shared__ int64_t s_part[4];
     const int lane = threadIdx.x & (BM_WAVE - 1);
-    const int wave = threadIdx.x / BM_WAVE;
-    const int wpb = blockDim.x / BM_WAVE;
-    S* lds = reinterpret_cast<S*>(smem) + (size_t)wave * cap;
-    const int64_t nw = (int64_t)gridDim.x * wpb;
-    int64_t acc = 0;
-    for (int64_t uu = (int64_t)blockIdx.x * wpb + wave + 1; uu <= g.n; uu += nw) {
-        const int32_t u = (int32_t)uu;
-        const int64_t b = uni64(g.m_out_ptr[u]), e = uni64(g.m_out_ptr[u + 1]);
-        if (b == e) continue;
-        Tab t[1] = {make_tab(g.f_out_desc, g.f_out_tab, g.f_out_ptr, uni(g.pi[u]))};
-        if (t[0].re - t[0].rb < 4 * (e - b) + 64) place<1>(t, cap); /* build only when probes pay for it */
-        build<COMPACT, 1>(lds, t, g.f_out, lane);
-        for (int64_t base = b; base < e; base += (int64_t)BM_WAVE * kU) {
-            int2 ed[kU];
+    const int wave = uni(threadIdx.x / BM_WAVE);
+    uint4* S = s_tab[wave];
+    const int64_t nw = (int64_t)gridDim.x * 4;
+    int64_t total = 0;
+    for (int64_t ci = (int64_t)blockIdx.x * 4 + wave; ci < nchunks; ci += nw) {
+        const int4 ch = chunks[ci];
+        const int32_t x = uni(ch.x);
+        const bool in = uni(ch.y) != 0;
+        const int32_t cnt = uni(ch.w);
+        const int2* __restrict__ adj = (in ? g.m_in + g.m_in_ptr[x] : g.m_out + g.m_out_ptr[x]) + uni(ch.z);
+        int2 e[U];
 #pragma unroll
-            for (int j = 0; j < kU; j++) {
-                const int64_t i = base + lane + (int64_t)BM_WAVE * j;
-                ed[j] = i < e ? g.m_out[i] : make_int2(0, 0);
+        for (int j = 0; j < U; j++) {
+            const int32_t i = lane + BM_WAVE * j;
+            e[j] = i < cnt ? adj[i] : make_int2(0, 0);
+        }
+        const BmRowTab t = in ? g.f_in_t : g.f_out_t;
+        const uint64_t d = (uint64_t)uni64((int64_t)t.desc[uni(g.pi[x])]);
+        const uint4* __restrict__ T = t.tab + (d >> 6);
+        const uint32_t lb = (uint32_t)(d & 63u), mask = (1u << lb) - 1u;
+        int32_t key[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) key[j] = g.pi[e[j].x];
+        /* a copy costs one 16-byte load per bucket, a lookup about one and a half */
+        const bool staged = (mask + 1u) <= (uint32_t)kStageBuckets && (int32_t)mask < 2 * cnt;
+        if (staged) {
+            wave_sync();
+            for (uint32_t q = lane; q <= mask; q += BM_WAVE) S[q] = T[q];
+            wave_sync();
+        }
+        uint32_t b[U], pend = 0;
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            if (e[j].x == 0 || (MODE != kSumScore && in && e[j].x == x)) key[j] = 0;
+            b[j] = row_home(key[j], lb);
+            pend |= (key[j] != 0 ? 1u : 0u) << j;
+        }
+        int64_t sum = 0, ws = 0, hit = 0, used = 0;
+        while (pend) {
+            uint4 y[U];
+#pragma unroll
+            for (int j = 0; j < U; j++)
+                if ((pend >> j) & 1u) y[j] = staged ? S[b[j]] : T[b[j]];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                if (!((pend >> j) & 1u)) continue;
+                int32_t w;
+                if (row_bucket<PACKED>(y[j], key[j], w)) {
+                    const int32_t c = contrib(e[j].y, w);
+                    sum += c;
+                    if (MODE == kSumFeature) hit += c != 0;
+                    pend &= ~(1u << j);
+                } else {
+                    b[j] = (b[j] + 1u) & mask;
+                }
             }
-            int32_t gx[kU];
+        }
+        if (MODE == kSumScore) {
+            total += sum;
+            continue;
+        }
+        if (MODE == kSumFeature) {
 #pragma unroll
-            for (int j = 0; j < kU; j++) gx[j] = g.pi[ed[j].x];
-            int32_t r[kU];
-            look_many<COMPACT, kU>(lds, t[0], gx, r);
-#pragma unroll
-            for (int j = 0; j < kU; j++) acc += contrib(ed[j].y, r[j]);
+            for (int j = 0; j < U; j++)
+                if (e[j].x != 0 && !(in && e[j].x == x)) {
+                    ws += e[j].y;
+                    used++;
+                }
+        }
+        sum = wave_sum64(sum);
+        if (MODE == kSumDiag) {
+            if (lane == 0 && sum != 0)
+                atomicAdd(reinterpret_cast<unsigned long long*>(&out[x]), (unsigned long long)sum);
+        } else {
+            ws = wave_sum64(ws);
+            const int64_t miss = wave_sum64(used - hit);
+            if (lane < 3)
+                atomicAdd(reinterpret_cast<unsigned long long*>(&out[4 * (int64_t)x + lane]),
+                          (unsigned long long)(lane == 0 ? sum : (lane == 1 ? ws : miss)));
         }
     }
-    acc = wave_sum64(acc);
-    if (lane == 0 && acc != 0) atomicAdd(reinterpret_cast<unsigned long long*>(acc_out), (unsigned long long)acc);
+    if (MODE == kSumScore) {
+        total = wave_sum64(total);
+        if (lane == 0) s_part[wave] = total;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int64_t all = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+            if (all != 0) atomicAdd(reinterpret_cast<unsigned long long*>(out), (unsigned long long)all);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_zero64(int64_t* __restrict__ p, int64_t count) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) p[i] = 0;
 }
 
 /* ------------------------------------------------------------------ */
@@ -968,18 +1056,30 @@ hipError_t bm_launch_anneal(const BmDevGraph* insts, int compact, BmChain* chain
     return hipGetLastError();
 }
 
-hipError_t bm_launch_score(const BmDevGraph& g, const BmLaunch& L, int64_t* acc, hipStream_t s) {
-    dim3 grid, block;
-    size_t lds;
-    hipError_t e;
-    if (g.compact) {
-        e = launch_delta(k_score<true>, L, g.n, 4, s, &grid, &block, &lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_score<true>, grid, block, lds, s, g, acc, (uint32_t)L.lds_slots);
-    } else {
-        e = launch_delta(k_score<false>, L, g.n, 8, s, &grid, &block, &lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_score<false>, grid, block, lds, s, g, acc, (uint32_t)L.lds_slots);
-    }
+template <int MODE>
+static hipError_t launch_edge_sums(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* out,
+                                   int32_t num_cus, hipStream_t s) {
+    if (nchunks <= 0) return hipSuccess;
+    int64_t blocks = (nchunks + 3) / 4;
+    const int64_t cap = (int64_t)(num_cus > 0 ? num_cus : 256) * 8;
+    if (blocks > cap) blocks = cap;
+    auto kern = g.packed ? k_edge_sums<true, MODE> : k_edge_sums<false, MODE>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, g, chunks, nchunks, out);
     return hipGetLastError();
+}
+
+hipError_t bm_launch_score(const BmDevGraph& g, const int4* chunks, int64_t n_out_chunks, int64_t* acc,
+                           int32_t num_cus, hipStream_t s) {
+    return launch_edge_sums<kSumScore>(g, chunks, n_out_chunks, acc, num_cus, s);
+}
+
+hipError_t bm_launch_diag(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* diag, int32_t num_cus,
+                          hipStream_t s) {
+    hipLaunchKernelGGL(k_zero64, dim3((unsigned)((g.n + 256) / 256)), dim3(256), 0, s, diag, (int64_t)g.n + 1);
+    return launch_edge_sums<kSumDiag>(g, chunks, nchunks, diag, num_cus, s);
+}
+
+hipError_t bm_launch_feature_sums(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* acc,
+                                  int32_t num_cus, hipStream_t s) {
+    return launch_edge_sums<kSumFeature>(g, chunks, nchunks, acc, num_cus, s);
 }

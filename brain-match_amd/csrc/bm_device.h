@@ -9,6 +9,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+/* Row tables of one adjacency (bm_rowtab.h): descriptor per row 0..n and the
+ * 16-byte buckets they point into. */
+struct BmRowTab {
+    const uint64_t* desc;
+    const uint4* tab;
+};
+
 /* Graph and matching as seen by the kernels (passed by value). */
 struct BmDevGraph {
     int32_t n;
@@ -25,8 +32,22 @@ struct BmDevGraph {
     const int64_t* f_in_ptr;    /* female CSC, n+2 */
     const int2* f_in;           /* {src, w} */
     const int32_t* pi;          /* matching, n+1 */
+    const int32_t* inv;         /* inverse matching (female -> male, 0 = none), n+1; NULL when two males share a female */
+    BmRowTab f_out_t, f_in_t, m_out_t, m_in_t;
+    int32_t packed;             /* 1: row tables hold 4-byte slots (compact, and male weights >= 0) */
     int32_t compact;            /* 1: LDS slots are (key << 15) | w (n < 2^17, weights 0..32767) */
 };
+
+/* Inserts the rows (ptr, adj) into the zeroed row tables described by desc. */
+hipError_t bm_launch_rowtab_fill(int packed, const int64_t* ptr, const int2* adj, int32_t n, const uint64_t* desc,
+                                 uint4* tab, hipStream_t s);
+/* Chunks {row, in (1) or out (0), first, count} of at most BM_EDGE_CHUNK
+ * entries covering the male lists, all out-lists first. */
+#define BM_EDGE_CHUNK 256
+/* diag[v] = the score of v's incident male edges under the matching: its
+ * out-edges (self-loop included) and its other in-edges, rows 0..n. */
+hipError_t bm_launch_diag(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* diag, int32_t num_cus,
+                          hipStream_t s);
 
 /* Bytes per LDS table slot for this graph (4 compact, 8 otherwise). */
 size_t bm_slot_bytes(const BmDevGraph& g);
@@ -184,7 +205,13 @@ hipError_t bm_launch_gen_umajor(int32_t n, uint64_t seed, const int64_t* off, in
 hipError_t bm_launch_gen_amajor(int32_t n, uint64_t seed, const int64_t* off, int64_t k, int4* cand, hipStream_t s);
 hipError_t bm_launch_rot3(const BmDevGraph& g, const BmLaunch& L, const int4* cand, int64_t k,
                           int64_t* best, uint8_t* perm, int4* cand_out_perm, hipStream_t s);
-hipError_t bm_launch_score(const BmDevGraph& g, const BmLaunch& L, int64_t* acc, hipStream_t s);
+/* Adds the score of the matching g.pi to *acc (chunks: the out-list ones). */
+hipError_t bm_launch_score(const BmDevGraph& g, const int4* chunks, int64_t n_out_chunks, int64_t* acc,
+                           int32_t num_cus, hipStream_t s);
+/* acc[4 x + 0..2] += {contributions, weights, entries contributing 0} of
+ * vertex x's male edges (a self-loop once). */
+hipError_t bm_launch_feature_sums(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* acc,
+                                  int32_t num_cus, hipStream_t s);
 
 /* Annealing chains (k_anneal in bm_delta.hip): per-chain state in device memory. */
 struct BmChain {
@@ -251,7 +278,7 @@ hipError_t bm_launch_pick(const int64_t* d, int64_t k, int32_t kind, int64_t ran
 
 /* Disjoint acceptance.  Scratch sizes come from bm_accept_scratch_bytes. */
 size_t bm_accept_scratch_bytes(int64_t k);
-hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, const int2* cand, const int64_t* d,
+hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, int32_t* inv_rw, const int2* cand, const int64_t* d,
                             int64_t k, int64_t max_accept, void* scratch, size_t scratch_bytes,
                             int64_t* out_acc_idx /* k */, int64_t* out_meta /* [n_acc, gain, n_moves] */,
                             int4* out_moves /* 2k {x, old, new, 0}, may be NULL */, hipStream_t s);
@@ -278,10 +305,8 @@ struct BmMlpDev {
     void* W2Tf;
 };
 int32_t bm_mlp_param_count(void);
-/* Per-vertex features from edge chunks {x, out (1) or in (0), first, count}
- * of the male lists (at most bm_feature_chunk_edges() edges each); acc
- * holds (n+1) x 32 zeroed bytes of accumulators and is left zeroed. */
-int32_t bm_feature_chunk_edges(void);
+/* Per-vertex features from the male edge chunks; acc holds (n+1) x 32 zeroed
+ * bytes of accumulators and is left zeroed. */
 hipError_t bm_launch_vertex_features(const BmDevGraph& g, const int4* chunks, int64_t nchunks, void* acc, float* vf,
                                      int32_t num_cus, hipStream_t s);
 hipError_t bm_launch_mlp_pack(const BmMlpDev& d, hipStream_t s);
@@ -315,6 +340,8 @@ int bm_ctx_device(const bm_ctx* c);
 int bm_ctx_num_cus(const bm_ctx* c);
 hipStream_t bm_ctx_stream(const bm_ctx* c);
 BmLaunch bm_ctx_launch(const bm_ctx* c, int kernel);
+/* The context's male edge chunks (BM_EDGE_CHUNK); the first *n_out are the out-lists'. */
+const int4* bm_ctx_chunks(const bm_ctx* c, int64_t* n_chunks, int64_t* n_out);
 int bm_ctx_set_error(bm_ctx* c, int code, const char* msg);
 struct bm_batch;
 int2* bm_batch_pairs_dev(bm_batch* b);
@@ -332,7 +359,9 @@ int bm_batch_has_pair_deltas(const bm_batch* b);
 /* The batch now holds k device-generated pairs (not yet evaluated). */
 void bm_batch_mark_pairs(bm_batch* b, int64_t k);
 
-hipError_t bm_launch_apply_swap(int32_t* pi, int32_t u, int32_t v, hipStream_t s);
-hipError_t bm_launch_apply_perm3(int32_t* pi, int32_t a, int32_t b, int32_t c, int32_t p, hipStream_t s);
+/* Moves on the matching and its inverse (inv: see BmDevGraph; always an n+1
+ * array here, its contents unused while images are shared). */
+hipError_t bm_launch_apply_swap(int32_t* pi, int32_t* inv, int32_t u, int32_t v, hipStream_t s);
+hipError_t bm_launch_apply_perm3(int32_t* pi, int32_t* inv, int32_t a, int32_t b, int32_t c, int32_t p, hipStream_t s);
 
 #endif

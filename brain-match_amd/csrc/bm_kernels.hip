@@ -7,6 +7,7 @@
 #include "bm_device.h"
 #include "bm_devutil.h"
 #include "bm_rng.h"
+#include "bm_rowtab.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -309,6 +310,7 @@ constexpr int kAccThreads = 1024;
 /* Sequential greedy in priority order, one block.  lock[] is a bitmap of
  * vertices in the closed neighbourhood of accepted swaps (LDS, n+1 bits). */
 __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int32_t* __restrict__ pi,
+                                                               int32_t* __restrict__ inv,
                                                                const int2* __restrict__ cand,
                                                                const int64_t* __restrict__ d,
                                                                const int64_t* __restrict__ order, int64_t npos,
@@ -387,22 +389,29 @@ __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int
         }
         pi[p.x] = fv;
         pi[p.y] = fu;
+        if (fv) inv[fv] = p.x;
+        if (fu) inv[fu] = p.y;
     }
     if (t == 0) { meta[0] = nacc; meta[1] = s_gain; meta[2] = 2 * nacc; }
 }
 
-__global__ void k_apply_swap(int32_t* pi, int32_t u, int32_t v) {
-    const int32_t t = pi[u];
-    pi[u] = pi[v];
-    pi[v] = t;
+__global__ void k_apply_swap(int32_t* pi, int32_t* inv, int32_t u, int32_t v) {
+    const int32_t fu = pi[u], fv = pi[v];
+    pi[u] = fv;
+    pi[v] = fu;
+    if (fv) inv[fv] = u;
+    if (fu) inv[fu] = v;
 }
 
 /* apply_permutation (src/graph-re-alignment-gpu-3-swap.cu:925-956). */
-__global__ void k_apply_perm3(int32_t* pi, int32_t a, int32_t b, int32_t c, int32_t p) {
-    const int32_t f[3] = {pi[a], pi[b], pi[c]};
-    pi[a] = f[perm_of(p, 0)];
-    pi[b] = f[perm_of(p, 1)];
-    pi[c] = f[perm_of(p, 2)];
+__global__ void k_apply_perm3(int32_t* pi, int32_t* inv, int32_t a, int32_t b, int32_t c, int32_t p) {
+    const int32_t f[3] = {pi[a], pi[b], pi[c]}, v[3] = {a, b, c};
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int32_t x = f[perm_of(p, i)];
+        pi[v[i]] = x;
+        if (x) inv[x] = v[i];
+    }
 }
 
 /* ---- u-major uniform stream (bm_umajor_first / bm_umajor_partner) ---- */
@@ -483,6 +492,32 @@ __global__ void k_gen_amajor(int32_t n, uint64_t seed, const int64_t* __restrict
     }
 }
 
+/* One block per row: every entry takes the first empty slot from its home
+ * bucket on (compare-and-swap; keys are unique in a row).  Within a bucket
+ * slots fill in order, which the lookups rely on. */
+template <bool PACKED>
+__global__ void __launch_bounds__(256) k_rowtab_fill(const int64_t* __restrict__ ptr, const int2* __restrict__ adj,
+                                                     const uint64_t* __restrict__ desc, uint4* __restrict__ tab) {
+    const int32_t row = blockIdx.x;
+    const int64_t b = ptr[row], e = ptr[row + 1];
+    const uint64_t d = desc[row];
+    const uint32_t lb = (uint32_t)(d & 63u);
+    const uint32_t per = RowSlots<PACKED>::kPerBucket, smask = (per << lb) - 1u;
+    for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
+        const int2 x = adj[i];
+        uint32_t s = row_home(x.x, lb) * per;
+        if (PACKED) {
+            uint32_t* T = reinterpret_cast<uint32_t*>(tab + (d >> 6));
+            const uint32_t v = ((uint32_t)x.x << 15) | (uint32_t)x.y;
+            while (atomicCAS(&T[s], 0u, v) != 0u) s = (s + 1u) & smask;
+        } else {
+            unsigned long long* T = reinterpret_cast<unsigned long long*>(tab + (d >> 6));
+            const unsigned long long v = ((unsigned long long)(uint32_t)x.y << 32) | (uint32_t)x.x;
+            while (atomicCAS(&T[s], 0ull, v) != 0ull) s = (s + 1u) & smask;
+        }
+    }
+}
+
 int grid_for(int64_t work, int threads) {
     int64_t b = (work + threads - 1) / threads;
     if (b < 1) b = 1;
@@ -498,6 +533,13 @@ int grid_for(int64_t work, int threads) {
 
 static hipError_t set_lds(const void* fn, size_t bytes) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+hipError_t bm_launch_rowtab_fill(int packed, const int64_t* ptr, const int2* adj, int32_t n, const uint64_t* desc,
+                                 uint4* tab, hipStream_t s) {
+    auto k = packed ? k_rowtab_fill<true> : k_rowtab_fill<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)n + 1u), dim3(256), 0, s, ptr, adj, desc, tab);
+    return hipGetLastError();
 }
 
 hipError_t bm_launch_gen_pairs(int32_t n, uint64_t seed, int64_t k, int2* cand, hipStream_t s) {
@@ -571,7 +613,7 @@ size_t bm_accept_scratch_bytes(int64_t k) {
     return (size_t)k * 4 * sizeof(int64_t) + 256 + cub_temp_bytes(k) + 256;
 }
 
-hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, const int2* cand, const int64_t* d, int64_t k,
+hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, int32_t* inv_rw, const int2* cand, const int64_t* d, int64_t k,
                             int64_t max_accept, void* scratch, size_t scratch_bytes, int64_t* out_acc_idx,
                             int64_t* out_meta, int4* out_moves, hipStream_t s) {
     if (k <= 0) {
@@ -612,18 +654,18 @@ hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, const int2* can
     e = set_lds((const void*)k_accept_greedy, lds);
     if (e != hipSuccess) return e;
     if (max_accept <= 0) max_accept = INT64_MAX;
-    hipLaunchKernelGGL(k_accept_greedy, dim3(1), dim3(kAccThreads), lds, s, g, pi_rw, cand, d, sidx, npos,
+    hipLaunchKernelGGL(k_accept_greedy, dim3(1), dim3(kAccThreads), lds, s, g, pi_rw, inv_rw, cand, d, sidx, npos,
                        max_accept, out_acc_idx, out_meta, out_moves);
     return hipGetLastError();
 }
 
-hipError_t bm_launch_apply_swap(int32_t* pi, int32_t u, int32_t v, hipStream_t s) {
-    hipLaunchKernelGGL(k_apply_swap, dim3(1), dim3(1), 0, s, pi, u, v);
+hipError_t bm_launch_apply_swap(int32_t* pi, int32_t* inv, int32_t u, int32_t v, hipStream_t s) {
+    hipLaunchKernelGGL(k_apply_swap, dim3(1), dim3(1), 0, s, pi, inv, u, v);
     return hipGetLastError();
 }
 
-hipError_t bm_launch_apply_perm3(int32_t* pi, int32_t a, int32_t b, int32_t c, int32_t p, hipStream_t s) {
-    hipLaunchKernelGGL(k_apply_perm3, dim3(1), dim3(1), 0, s, pi, a, b, c, p);
+hipError_t bm_launch_apply_perm3(int32_t* pi, int32_t* inv, int32_t a, int32_t b, int32_t c, int32_t p, hipStream_t s) {
+    hipLaunchKernelGGL(k_apply_perm3, dim3(1), dim3(1), 0, s, pi, inv, a, b, c, p);
     return hipGetLastError();
 }
 

@@ -75,67 +75,9 @@ __device__ __forceinline__ v4f mfma32(v8s a, v8s b, v4f c) {
                                                     0);
 }
 
-/* w_F(a, b) through a row hash table (descriptor (offset << 6) | bits). */
-__device__ __forceinline__ int32_t row_w(const uint64_t* __restrict__ desc, const int2* __restrict__ tab, int32_t row,
-                                         int32_t key) {
-    if (row == 0 || key == 0) return BM_ABSENT;
-    const uint64_t d = desc[row];
-    const uint32_t bits = (uint32_t)(d & 63u);
-    if (!bits) return BM_ABSENT;
-    const int2* T = tab + (d >> 6);
-    const uint32_t mask = (1u << bits) - 1u;
-    uint32_t s = slot_hash(key, bits);
-    for (;;) {
-        const int2 e = T[s];
-        if (e.x == 0) return BM_ABSENT;
-        if (e.x == key) return e.y;
-        s = (s + 1u) & mask;
-    }
-}
-
-/* Per-vertex features in two passes.  k_feature_chunks: one wave per chunk
- * {x, direction, first, count} of at most kFeatChunk edges of one of x's male
- * lists (the chunks depend only on the male graph), so a hub's lists spread
- * over many waves; each edge's contribution under pi (a probe of the female
- * row of pi(x)) is summed with its weight and whether it is 0, and the wave
- * adds the sums to x's accumulators {L, weight sum, zero count} (a self-loop
- * counts once, with the out-edges).  k_feature_finish: one thread per vertex
- * turns the exact integer sums into the 8 floats and clears the
- * accumulators. */
-__global__ void __launch_bounds__(256) k_feature_chunks(BmDevGraph g, const int4* __restrict__ chunks, int64_t nchunks,
-                                                        longlong4* __restrict__ acc) {
-    const int lane = threadIdx.x & (BM_WAVE - 1);
-    const int64_t nw = (int64_t)gridDim.x * (blockDim.x / BM_WAVE);
-    for (int64_t ci = (int64_t)blockIdx.x * (blockDim.x / BM_WAVE) + threadIdx.x / BM_WAVE; ci < nchunks; ci += nw) {
-        const int4 ch = chunks[ci];
-        const int32_t x = uni(ch.x);
-        const int out = uni(ch.y);
-        const int32_t fx = uni(g.pi[x]);
-        const int64_t base = (out ? g.m_out_ptr[x] : g.m_in_ptr[x]) + uni(ch.z);
-        const int2* adj = out ? g.m_out : g.m_in;
-        const uint64_t* desc = out ? g.f_out_desc : g.f_in_desc;
-        const int2* tab = out ? g.f_out_tab : g.f_in_tab;
-        int64_t L = 0, ws = 0, miss = 0;
-        for (int32_t i = lane; i < ch.w; i += BM_WAVE) {
-            const int2 ed = adj[base + i];
-            if (!out && ed.x == x) continue;   /* a self-loop counted once, with the out-edges */
-            const int32_t fy = ed.x == x ? fx : g.pi[ed.x];
-            const int32_t c = contrib(ed.y, row_w(desc, tab, fx, fy));
-            L += c;
-            ws += ed.y;
-            miss += c == 0;
-        }
-        L = wave_sum64(L);
-        ws = wave_sum64(ws);
-        miss = wave_sum64(miss);
-        if (lane == 0) {
-            atomicAdd(reinterpret_cast<unsigned long long*>(&acc[x].x), (unsigned long long)L);
-            atomicAdd(reinterpret_cast<unsigned long long*>(&acc[x].y), (unsigned long long)ws);
-            atomicAdd(reinterpret_cast<unsigned long long*>(&acc[x].z), (unsigned long long)miss);
-        }
-    }
-}
-
+/* Second half of the per-vertex features: one thread per vertex turns the
+ * exact integer sums of its edges (bm_launch_feature_sums: contributions,
+ * weights, entries contributing 0) into the 8 floats and clears them. */
 __global__ void k_feature_finish(BmDevGraph g, longlong4* __restrict__ acc, float4* __restrict__ vf) {
     for (int32_t x = blockIdx.x * blockDim.x + threadIdx.x; x <= g.n; x += gridDim.x * blockDim.x) {
         if (x == 0) {
@@ -840,16 +782,10 @@ MlpDev mlpdev(const BmMlpDev& d) {
 
 int32_t bm_mlp_param_count(void) { return kParams; }
 
-int32_t bm_feature_chunk_edges(void) { return 256; }
-
 hipError_t bm_launch_vertex_features(const BmDevGraph& g, const int4* chunks, int64_t nchunks, void* acc, float* vf,
                                      int32_t num_cus, hipStream_t s) {
-    const int64_t cap = (int64_t)(num_cus > 0 ? num_cus : 256) * 16;
-    int64_t blocks = (nchunks + 3) / 4;
-    if (blocks > cap) blocks = cap;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_feature_chunks, dim3((unsigned)blocks), dim3(256), 0, s, g, chunks, nchunks,
-                       static_cast<longlong4*>(acc));
+    const hipError_t e = bm_launch_feature_sums(g, chunks, nchunks, static_cast<int64_t*>(acc), num_cus, s);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_feature_finish, dim3(grid_of((int64_t)g.n + 1, 256)), dim3(256), 0, s, g,
                        static_cast<longlong4*>(acc), reinterpret_cast<float4*>(vf));
     return hipGetLastError();
