@@ -23,7 +23,7 @@
 
 /* Device scratch of bm_batch_gen_learned_noalloc: the pool's scores, the
  * select state and the selected keys for pools of up to BM_NOALLOC_POOL pairs
- * (bm_mlp_select_bytes(BM_NOALLOC_POOL) = 4,325,928 bytes fit).  Each device
+ * (bm_mlp_select_bytes(BM_NOALLOC_POOL) = 4,293,376 bytes fit).  Each device
  * holds its own copy for the life of the process; host code uses the address
  * hipGetSymbolAddress returns for the device (g_scratch_dev), never the
  * array's name.  Every call on a device shares that device's copy. */
@@ -57,7 +57,9 @@ struct bm_mlp {
     float* d_vf;
     void* d_feat_acc;       /* (n+1) x 32 bytes of feature accumulators, zero between passes */
     int features_ready;
-    float* d_loss;
+    float* d_loss;          /* summed squared error of the batch in hand, 0 between batches */
+    float* d_trace;         /* that of every step since the last read-back */
+    int64_t trace_cap;
     float* d_target;
     int64_t target_cap;
     void* d_act;
@@ -122,6 +124,7 @@ extern "C" void bm_mlp_destroy(bm_mlp* m) {
     (void)hipFree(m->d_vf);
     (void)hipFree(m->d_feat_acc);
     (void)hipFree(m->d_loss);
+    (void)hipFree(m->d_trace);
     (void)hipFree(m->d_target);
     (void)hipFree(m->d_act);
     (void)hipFree(m->d_pairs);
@@ -203,6 +206,8 @@ extern "C" int bm_mlp_create(bm_ctx* ctx, uint64_t seed, bm_mlp** out) {
     alloc(&m->d.W2Tf, 128 * 128 * 2);
     alloc((void**)&m->d_vf, ((size_t)m->n + 1) * 8 * sizeof(float));
     alloc((void**)&m->d_loss, sizeof(float));
+    if (rc == BM_OK && hipMemset(m->d_loss, 0, sizeof(float)) != hipSuccess)
+        rc = bm_ctx_set_error(ctx, BM_ERR_HIP, "bm_mlp_create: hipMemset failed");
     alloc(&m->d_feat_acc, ((size_t)m->n + 1) * 32);
     if (rc == BM_OK && hipMemset(m->d_feat_acc, 0, ((size_t)m->n + 1) * 32) != hipSuccess)
         rc = bm_ctx_set_error(ctx, BM_ERR_HIP, "bm_mlp_create: hipMemset failed");
@@ -262,14 +267,14 @@ extern "C" int bm_mlp_score_pairs(bm_mlp* m, const int32_t* uv, int64_t k, float
     return BM_OK;
 }
 
-/* Gradient of one batch into m->d.grad (which the caller has cleared); the
- * squared error into *d_loss (cleared here). */
-static int batch_gradient(bm_mlp* m, const int2* list, uint64_t seed, int64_t k, const float* d_target) {
+/* Gradient of one batch into m->d.grad and its squared error into *d_loss
+ * (both 0 before), from targets or, with d_target NULL, exact deltas. */
+static int batch_gradient(bm_mlp* m, const int2* list, uint64_t seed, int64_t k, const float* d_target,
+                          const int64_t* d_delta) {
     int rc = grow_bytes(m, &m->d_act, &m->act_bytes, bm_mlp_train_bytes(k));
     if (rc != BM_OK) return rc;
-    MHIP(m, hipMemsetAsync(m->d_loss, 0, sizeof(float), m->stream));
-    MHIP(m, bm_launch_mlp_gradient(m->d, m->d_vf, list, seed, m->n, k, d_target, m->d_act, m->d_loss, m->num_cus,
-                                   m->stream));
+    MHIP(m, bm_launch_mlp_gradient(m->d, m->d_vf, list, seed, m->n, k, d_target, d_delta, m->d_act, m->d_loss,
+                                   m->num_cus, m->stream));
     return BM_OK;
 }
 
@@ -283,13 +288,13 @@ extern "C" int bm_mlp_gradient(bm_mlp* m, const int32_t* uv, const float* target
     if (rc != BM_OK) return rc;
     MHIP(m, hipMemcpyAsync(m->d_target, target, (size_t)k * sizeof(float), hipMemcpyHostToDevice, m->stream));
     const size_t np = (size_t)bm_mlp_param_count();
-    MHIP(m, hipMemsetAsync(m->d.grad, 0, np * sizeof(float), m->stream));
-    rc = batch_gradient(m, m->d_pairs, 0, k, m->d_target);
+    rc = batch_gradient(m, m->d_pairs, 0, k, m->d_target, nullptr);
     if (rc != BM_OK) return rc;
     float se = 0.f;
     MHIP(m, hipMemcpyAsync(grad, m->d.grad, np * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MHIP(m, hipMemcpyAsync(&se, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MHIP(m, hipMemsetAsync(m->d.grad, 0, np * sizeof(float), m->stream));
+    MHIP(m, hipMemsetAsync(m->d_loss, 0, sizeof(float), m->stream));
     MHIP(m, hipStreamSynchronize(m->stream));
     if (mse) *mse = se / (float)k;
     return BM_OK;
@@ -309,24 +314,22 @@ extern "C" int bm_mlp_train(bm_mlp* m, uint64_t seed, int64_t steps, int32_t bat
         if (rc != BM_OK) return rc;
         m->train_cap = batch;
     }
-    int rc = grow(m, &m->d_target, &m->target_cap, batch);
+    int rc = grow(m, &m->d_trace, &m->trace_cap, steps);
     if (rc != BM_OK) return rc;
     for (int64_t s = 0; s < steps; s++) {
         const uint64_t sd = bm_rand_at(seed, (uint64_t)s);
         /* exact deltas of the batch from the context's own evaluator */
         rc = bm_batch_eval_swaps_uniform(m->train_batch, sd, batch);
         if (rc != BM_OK) return rc;
-        MHIP(m, bm_launch_mlp_targets(bm_batch_deltas_dev(m->train_batch), batch, m->d_target, m->stream));
-        rc = batch_gradient(m, nullptr, sd, batch, m->d_target);
+        rc = batch_gradient(m, nullptr, sd, batch, nullptr, bm_batch_deltas_dev(m->train_batch));
         if (rc != BM_OK) return rc;
         m->adam_step++;
-        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->stream));
-        if (mse_trace) {
-            float se = 0.f;
-            MHIP(m, hipMemcpyAsync(&se, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
-            MHIP(m, hipStreamSynchronize(m->stream));
-            mse_trace[s] = se / (float)batch;
-        }
+        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_loss, m->d_trace + s, m->stream));
+    }
+    if (mse_trace && steps > 0) {
+        MHIP(m, hipMemcpyAsync(mse_trace, m->d_trace, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+        MHIP(m, hipStreamSynchronize(m->stream));
+        for (int64_t s = 0; s < steps; s++) mse_trace[s] /= (float)batch;
     }
     MHIP(m, hipStreamSynchronize(m->stream));
     return BM_OK;
@@ -369,16 +372,14 @@ extern "C" int bm_mlp_train_batch(bm_mlp* m, bm_batch* b, float lr, float* mse) 
     const int64_t k = bm_batch_size(b);
     if (k < 1) return BM_OK;
     MHIP(m, hipSetDevice(m->device));
-    int rc = grow(m, &m->d_target, &m->target_cap, k);
-    if (rc != BM_OK) return rc;
-    MHIP(m, bm_launch_mlp_targets(bm_batch_deltas_dev(b), k, m->d_target, m->stream));
-    rc = batch_gradient(m, bm_batch_pairs_dev(b), 0, k, m->d_target);
+    int rc = grow(m, &m->d_trace, &m->trace_cap, 1);
+    if (rc == BM_OK) rc = batch_gradient(m, bm_batch_pairs_dev(b), 0, k, nullptr, bm_batch_deltas_dev(b));
     if (rc != BM_OK) return rc;
     m->adam_step++;
-    MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->stream));
+    MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_loss, m->d_trace, m->stream));
     if (mse) {
         float se = 0.f;
-        MHIP(m, hipMemcpyAsync(&se, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
+        MHIP(m, hipMemcpyAsync(&se, m->d_trace, sizeof(float), hipMemcpyDeviceToHost, m->stream));
         MHIP(m, hipStreamSynchronize(m->stream));
         *mse = se / (float)k;
     }

@@ -140,6 +140,7 @@ __device__ __forceinline__ int2 pair_at(const PairSrc& ps, int64_t p) {
     return make_int2(u, v);
 }
 
+constexpr int kHistBins = 4096;   /* first 12 bits of the order-preserving score bits */
 constexpr int kFwdThreads = 256;
 constexpr int kFwdWaves = kFwdThreads / BM_WAVE;
 constexpr int kHPad = kH + 8;   /* padded bf16 row of a staged 16 x 128 tile (272 bytes: 16-byte reads hit distinct banks) */
@@ -151,7 +152,8 @@ struct FwdShared {
     short Ht[kFwdWaves][16][kHPad];
 };
 
-__device__ __forceinline__ void stage_weights(FwdShared& S, const MlpDev& M) {
+template <typename Shared>
+__device__ __forceinline__ void stage_weights(Shared& S, const MlpDev& M) {
     for (int q = threadIdx.x; q < kT * 64; q += blockDim.x) S.W1[q] = M.W1f[q];
     for (int q = threadIdx.x; q < kS * kT * 64; q += blockDim.x) S.W2[q] = M.W2f[q];
     for (int q = threadIdx.x; q < kH; q += blockDim.x) {
@@ -201,60 +203,126 @@ __device__ __forceinline__ void load_tile32(const short (*Ht)[kHPad], v8s* a, in
     for (int s = 0; s < kS; s++) a[s] = *reinterpret_cast<const v8s*>(&Ht[lane % 16][32 * s + 8 * (lane / 16)]);
 }
 
-/* Forward: scores of k pairs (one wave per 16-pair tile), in the transposed
- * form: z1^T = W1^T x^T (A = W1^T fragments, B = the input fragment) leaves
- * lane l with hidden units 16 t + 4 (l / 16) .. +3 of pair l % 16, stored to
- * the pair's LDS row in one 8-byte write per t; z2^T = W2^T h1^T takes h1^T
- * fragments as 16-byte reads of those rows; the output layer sums the lane's
- * 32 hidden units, then over the four lanes of the pair. */
-__global__ void __launch_bounds__(kFwdThreads) k_mlp_forward(const float4* __restrict__ vf, PairSrc ps, int64_t k,
-                                                             MlpDev M, float* __restrict__ score) {
+/* Forward: scores of k pairs, in the transposed form: z1^T = W1^T x^T (A =
+ * W1^T fragments, B = the input fragment) leaves lane l with hidden units
+ * 16 t + 4 (l / 16) .. +3 of pair l % 16, stored to the pair's LDS row in one
+ * 8-byte write per t; z2^T = W2^T h1^T takes h1^T fragments as 16-byte reads
+ * of those rows; the output layer sums the lane's 32 hidden units, then over
+ * the four lanes of the pair.
+ *
+ * A tile is 640 MFMA cycles but reads 36 KB of weights and 1.5 KB of biases
+ * from LDS (290 cycles of the CU's one LDS port per wave, so four SIMDs wait
+ * for it), so a wave takes kFwdTiles tiles with each weight read, and one
+ * block of 16 waves per CU shares one copy of the weights (four waves per
+ * SIMD; with 4-wave blocks the 54 KB per block left two).  The next tiles'
+ * features load while this one's products run.  2^20 pairs: 104 -> 58 us
+ * (three or four tiles per weight read spill). */
+constexpr int kScoreThreads = 1024, kScoreWaves = kScoreThreads / BM_WAVE, kFwdTiles = 2;
+
+struct ScoreShared {
+    v4s W1[kT * 64];
+    v8s W2[kS * kT * 64];
+    float b1[kH], b2[kH], w3[kH];
+    short Ht[kScoreWaves][16][kHPad];
+};
+
+template <bool HIST>
+__global__ void __launch_bounds__(kScoreThreads) k_mlp_forward(const float4* __restrict__ vf, PairSrc ps, int64_t k,
+                                                               MlpDev M, float* __restrict__ score,
+                                                               uint32_t* __restrict__ hist) {
     extern __shared__ uint4 smem[];
-    FwdShared& S = *reinterpret_cast<FwdShared*>(smem);
+    ScoreShared& S = *reinterpret_cast<ScoreShared*>(smem);
+    uint32_t* h0 = reinterpret_cast<uint32_t*>(&S + 1);   /* HIST: first digit of the ranking select */
+    if (HIST)
+        for (int i = threadIdx.x; i < kHistBins; i += blockDim.x) h0[i] = 0;
     stage_weights(S, M);
     __syncthreads();
     const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE;
     const int q = lane / 16;
     short(*Ht)[kHPad] = S.Ht[wave];
     const float b3 = M.b3[0];
-    const int64_t tiles = (k + 15) / 16;
-    for (int64_t tile = (int64_t)blockIdx.x * kFwdWaves + wave; tile < tiles; tile += (int64_t)gridDim.x * kFwdWaves) {
-        const int64_t p = tile * 16 + (lane % 16);
-        const bool valid = p < k;
-        const int2 uv = valid ? pair_at(ps, p) : make_int2(0, 0);
-        const v4s xb = input_frag(vf, uv, valid, lane);
+    const int64_t groups = (k + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
+    const int64_t step = (int64_t)gridDim.x * kScoreWaves;
+    int64_t gr = (int64_t)blockIdx.x * kScoreWaves + wave;
+    v4s xn[kFwdTiles];
 #pragma unroll
-        for (int t = 0; t < kT; t++) {
-            v4f acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma(S.W1[t * 64 + lane], xb, acc);
-            v4s h;
+    for (int z = 0; z < kFwdTiles; z++) {
+        const int64_t p = (gr * kFwdTiles + z) * 16 + (lane % 16);
+        xn[z] = input_frag(vf, p < k ? pair_at(ps, p) : make_int2(0, 0), p < k, lane);
+    }
+    for (; gr < groups; gr += step) {
+        v4s xb[kFwdTiles];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float z = acc[j] + S.b1[16 * t + 4 * q + j];
-                h[j] = bf16_of(z > 0.f ? z : 0.f);
-            }
-            *reinterpret_cast<v4s*>(&Ht[lane % 16][16 * t + 4 * q]) = h;
+        for (int z = 0; z < kFwdTiles; z++) {
+            xb[z] = xn[z];
+            const int64_t p = ((gr + step) * kFwdTiles + z) * 16 + (lane % 16);
+            xn[z] = input_frag(vf, p < k ? pair_at(ps, p) : make_int2(0, 0), p < k, lane);
         }
-        wave_sync();
-        v8s hb[kS];
-        load_tile32(Ht, hb, lane);
-        float part = 0.f;
+        v8s hb[kFwdTiles][kS];
 #pragma unroll
+        for (int z = 0; z < kFwdTiles; z++) {
+#pragma unroll 4
+            for (int t = 0; t < kT; t++) {
+                v4f acc = {0.f, 0.f, 0.f, 0.f};
+                acc = mfma(S.W1[t * 64 + lane], xb[z], acc);
+                const float4 b1 = *reinterpret_cast<const float4*>(&S.b1[16 * t + 4 * q]);
+                const float bb[4] = {b1.x, b1.y, b1.z, b1.w};
+                v4s h;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float y = acc[j] + bb[j];
+                    h[j] = bf16_of(y > 0.f ? y : 0.f);
+                }
+                *reinterpret_cast<v4s*>(&Ht[lane % 16][16 * t + 4 * q]) = h;
+            }
+            wave_sync();
+            load_tile32(Ht, hb[z], lane);
+            wave_sync();
+        }
+        float part[kFwdTiles];
+#pragma unroll
+        for (int z = 0; z < kFwdTiles; z++) part[z] = 0.f;
+#pragma unroll 2   /* fully unrolled, the weight reads move up and spill */
         for (int t = 0; t < kT; t++) {
-            v4f acc = {0.f, 0.f, 0.f, 0.f};
+            v4f acc[kFwdTiles];
 #pragma unroll
-            for (int s2 = 0; s2 < kS; s2++) acc = mfma32(S.W2[(s2 * kT + t) * 64 + lane], hb[s2], acc);
+            for (int z = 0; z < kFwdTiles; z++) acc[z] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int u = 16 * t + 4 * q + j;
-                const float h2 = acc[j] + S.b2[u];
-                part += (h2 > 0.f ? h2 : 0.f) * S.w3[u];
+            for (int s2 = 0; s2 < kS; s2++) {
+                const v8s w = S.W2[(s2 * kT + t) * 64 + lane];
+#pragma unroll
+                for (int z = 0; z < kFwdTiles; z++) acc[z] = mfma32(w, hb[z][s2], acc[z]);
+            }
+            const float4 b2 = *reinterpret_cast<const float4*>(&S.b2[16 * t + 4 * q]);
+            const float4 w3 = *reinterpret_cast<const float4*>(&S.w3[16 * t + 4 * q]);
+            const float bb[4] = {b2.x, b2.y, b2.z, b2.w}, ww[4] = {w3.x, w3.y, w3.z, w3.w};
+#pragma unroll
+            for (int z = 0; z < kFwdTiles; z++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float h2 = acc[z][j] + bb[j];
+                    part[z] += (h2 > 0.f ? h2 : 0.f) * ww[j];
+                }
+        }
+#pragma unroll
+        for (int z = 0; z < kFwdTiles; z++) {
+            part[z] += __shfl_xor(part[z], 16, BM_WAVE);
+            part[z] += __shfl_xor(part[z], 32, BM_WAVE);
+            const int64_t p = (gr * kFwdTiles + z) * 16 + (lane % 16);
+            if (lane < 16 && p < k) {
+                const float y = part[z] + b3;
+                score[p] = y;
+                if (HIST) {
+                    const uint32_t u = __float_as_uint(y);
+                    atomicAdd(&h0[((u & 0x80000000u) ? ~u : (u | 0x80000000u)) >> 20], 1u);
+                }
             }
         }
-        part += __shfl_xor(part, 16, BM_WAVE);
-        part += __shfl_xor(part, 32, BM_WAVE);
-        if (lane < 16 && valid) score[p] = part + b3;
-        wave_sync();
+    }
+    if (HIST) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < kHistBins; i += blockDim.x)
+            if (h0[i]) atomicAdd(&hist[i], h0[i]);
     }
 }
 
@@ -490,38 +558,30 @@ __device__ __forceinline__ uint64_t rank_key(float x, int64_t p) {
     return ((uint64_t)u << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)p);
 }
 
-constexpr int kSelBits = 11, kSelBins = 1 << kSelBits, kSelThreads = 256, kSelPasses = 6;
+constexpr int kSelBits = 12, kSelBins = 1 << kSelBits, kSelThreads = 256;
+static_assert(kSelBins == kHistBins, "the scoring kernel fills the first digit's histogram");
 constexpr int kSelPer = 16;          /* consecutive keys per lane, loaded before any is used */
-constexpr int kSelCopies = 8;        /* copies of the global histogram (block b adds to copy b % 8) */
-constexpr int kSortMax = 8192;       /* largest top sorted in one block */
+constexpr int kSortMax = 8192;       /* largest top, and most keys ranked */
 
+/* 2^20 scores, 4,096 wanted: 27 us with the clearing (six 11-bit passes handed
+ * from block to block, a compaction and a one-block bitonic sort: 125 us).
+ * The select takes two 12-bit digits: the first histogram comes out of the
+ * scoring kernel, the second out of one pass over the scores; then every key
+ * at or above the 24-bit threshold is written out and ranked by counting.
+ * Those are the `top` and the few others that share the threshold's 24 bits.
+ * Only when so many keys share them that the written set would pass kSortMax
+ * (scores equal to 2^-15: a network with dead units) does k_select_rest fix
+ * further digits. */
 struct SelState {
-    uint64_t prefix;      /* key bits fixed so far (the bits of the current digit and below are 0) */
-    uint64_t fixed;       /* mask of the fixed bits */
-    int64_t remaining;    /* rank (1-based) of the wanted key within the keys sharing the prefix */
-    uint32_t done;        /* blocks of the current pass that have merged their histogram */
-    uint32_t count;       /* keys written by the compaction */
-    uint32_t settled;     /* 1: the keys >= prefix under the mask are exactly the top */
-    uint32_t pad;
-    uint32_t hist[kSelCopies][kSelBins];
+    uint32_t count;       /* keys written */
+    uint32_t pad[63];
+    uint32_t hist[2][kSelBins];
 };
 
-__device__ __forceinline__ void sel_digit(int pass, int* shift, int* width) {
-    *width = pass < kSelPasses - 1 ? kSelBits : 64 - kSelBits * (kSelPasses - 1);
-    *shift = 64 - kSelBits * (pass + 1);
-    if (*shift < 0) *shift = 0;
-}
-
-__global__ void k_select_init(SelState* st, int64_t top) {
-    if (threadIdx.x == 0) {
-        st->prefix = 0;
-        st->fixed = 0;
-        st->remaining = top;
-        st->done = 0;
-        st->count = 0;
-        st->settled = 0;
-    }
-    for (int i = threadIdx.x; i < kSelCopies * kSelBins; i += blockDim.x) (&st->hist[0][0])[i] = 0;
+__global__ void __launch_bounds__(256) k_select_init(SelState* st) {
+    uint32_t* p = reinterpret_cast<uint32_t*>(st);
+    const int words = (int)(sizeof(SelState) / sizeof(uint32_t));
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
 /* Adds 1 to bin b of the LDS histogram for every lane with `valid`: lanes
@@ -537,169 +597,126 @@ __device__ __forceinline__ void wave_hist_add(uint32_t* h, bool valid, uint32_t 
     if (valid && b != lb) atomicAdd(&h[b], 1u);
 }
 
-/* One digit of the select: every block histograms the digit of the keys that
- * share the prefix (LDS counters, merged into one of kSelCopies global
- * copies with atomics); the last block to finish sums the copies, finds the
- * digit holding the wanted rank (suffix sums from the top bin), extends the
- * prefix and clears the histograms.  When the wanted rank is the last key of
- * its digit's bin, every key of that bin and above belongs to the top: the
- * select is settled and the remaining passes do nothing. */
-__global__ void __launch_bounds__(kSelThreads) k_select_pass(const float* __restrict__ sc, int64_t P,
-                                                             SelState* st, int pass) {
-    __shared__ uint32_t h[kSelBins];
-    __shared__ uint32_t part[kSelThreads];
-    __shared__ int last;
-    if (st->settled) return;
-    int shift, width;
-    sel_digit(pass, &shift, &width);
-    const int bins = 1 << width;
-    const int top = shift + width;
-    const uint64_t fixed = top >= 64 ? 0ull : (~0ull << top);
-    const uint64_t prefix = st->prefix;
-    const int lane = threadIdx.x & (BM_WAVE - 1);
-    for (int i = threadIdx.x; i < bins; i += blockDim.x) h[i] = 0;
+/* Digit holding the rank-th largest key (1-based) of a histogram, *rank
+ * reduced to the rank inside that digit and *inside its count; all NT threads
+ * get the result.  A thread's bins stay in registers, its wave sums them by
+ * shuffles, and two barriers cover the waves. */
+struct DigitShared {
+    uint32_t wave[16];
+    uint32_t d, r, in;
+};
+template <int NT>
+__device__ __forceinline__ uint32_t find_digit(const uint32_t* h, uint32_t* rank, uint32_t* inside, DigitShared& S) {
+    constexpr int kPer = kSelBins / NT, kWaves = NT / BM_WAVE;
+    const int t = threadIdx.x, lane = t & (BM_WAVE - 1), wave = t / BM_WAVE;
+    uint32_t c[kPer], mine = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; j += 4) {
+        const uint4 q = *reinterpret_cast<const uint4*>(&h[t * kPer + j]);
+        c[j] = q.x;
+        c[j + 1] = q.y;
+        c[j + 2] = q.z;
+        c[j + 3] = q.w;
+        mine += q.x + q.y + q.z + q.w;
+    }
+    uint32_t suffix = mine;   /* keys in this lane's and the higher lanes' bins */
+#pragma unroll
+    for (int o = 1; o < BM_WAVE; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_down((int)suffix, o, BM_WAVE);
+        if (lane + o < BM_WAVE) suffix += y;
+    }
+    __syncthreads();          /* the previous call's results have been read */
+    if (lane == 0) S.wave[wave] = suffix;
     __syncthreads();
-    /* a wave takes 64 kSelPer consecutive keys, kSelPer per lane, loaded
-     * before any is used; every lane of a wave runs the same iterations (the
-     * ballots need them all) */
+    for (int w = wave + 1; w < kWaves; w++) suffix += S.wave[w];
+    const uint32_t above = suffix - mine;
+    if (above < *rank && *rank <= suffix) {
+        uint32_t r = *rank - above;
+        int d = -1;
+        uint32_t in = 0;
+#pragma unroll
+        for (int j = kPer - 1; j >= 0; j--)
+            if (d < 0) {
+                if (r <= c[j]) {
+                    d = j;
+                    in = c[j];
+                } else {
+                    r -= c[j];
+                }
+            }
+        S.d = (uint32_t)(t * kPer + d);
+        S.r = r;
+        S.in = in;
+    }
+    __syncthreads();
+    *rank = S.r;
+    *inside = S.in;
+    return S.d;
+}
+
+/* kSelPer consecutive scores per lane from p0 on (0 past the end). */
+__device__ __forceinline__ void load_scores(const float* __restrict__ sc, int64_t p0, int64_t P, float* v) {
+    if (p0 + kSelPer <= P) {
+#pragma unroll
+        for (int j = 0; j < kSelPer; j += 4) {
+            const float4 f = *reinterpret_cast<const float4*>(&sc[p0 + j]);
+            v[j] = f.x;
+            v[j + 1] = f.y;
+            v[j + 2] = f.z;
+            v[j + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kSelPer; j++) v[j] = p0 + j < P ? sc[p0 + j] : 0.f;
+    }
+}
+
+/* Second digit: every block finds the first digit from the finished first
+ * histogram itself (16 KB from L2, about 2 us, against a last-block hand-over
+ * and its fence in every pass), then histograms the second digit of the keys
+ * that share it. */
+__global__ void __launch_bounds__(kSelThreads) k_select_second(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                               uint32_t top) {
+    __shared__ alignas(16) uint32_t h[kSelBins];
+    __shared__ DigitShared S;
+    const int lane = threadIdx.x & (BM_WAVE - 1);
+    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x) h[i] = 0;
+    uint32_t r = top, in;
+    const uint32_t d0 = find_digit<kSelThreads>(st->hist[0], &r, &in, S);
+    /* every lane of a wave runs the same iterations (the ballots need them all) */
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / BM_WAVE) * BM_WAVE * kSelPer;
     for (int64_t w0 = ((int64_t)blockIdx.x * (blockDim.x / BM_WAVE) + threadIdx.x / BM_WAVE) * BM_WAVE * kSelPer;
          w0 < P; w0 += wstride) {
         const int64_t p0 = w0 + (int64_t)lane * kSelPer;
         float v[kSelPer];
-        if (p0 + kSelPer <= P) {
-#pragma unroll
-            for (int j = 0; j < kSelPer; j += 4) {
-                const float4 f = *reinterpret_cast<const float4*>(&sc[p0 + j]);
-                v[j] = f.x;
-                v[j + 1] = f.y;
-                v[j + 2] = f.z;
-                v[j + 3] = f.w;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < kSelPer; j++) v[j] = p0 + j < P ? sc[p0 + j] : 0.f;
-        }
+        load_scores(sc, p0, P, v);
 #pragma unroll
         for (int j = 0; j < kSelPer; j++) {
-            const uint64_t k = rank_key(v[j], p0 + j);
-            const bool valid = p0 + j < P && (k & fixed) == prefix;
-            wave_hist_add(h, valid, (uint32_t)(k >> shift) & (uint32_t)(bins - 1), lane);
+            const uint32_t u = (uint32_t)(rank_key(v[j], p0 + j) >> 32);
+            wave_hist_add(h, p0 + j < P && (u >> 20) == d0, (u >> 8) & (kSelBins - 1), lane);
         }
     }
     __syncthreads();
-    uint32_t* gh = st->hist[blockIdx.x % kSelCopies];
-    for (int i = threadIdx.x; i < bins; i += blockDim.x)
-        if (h[i]) atomicAdd(&gh[i], h[i]);
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(&st->done, 1u) == gridDim.x - 1;
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    /* every thread reads the rank before the barriers below; one thread rewrites it */
-    const int64_t rem = st->remaining;
-    /* thread t owns bins [t * per, (t + 1) * per) (per = 8 or 2); the
-     * device-scope fence above makes the other blocks' counts visible to
-     * plain loads, all issued before any is summed */
-    const int per = bins / kSelThreads;
-    const int t = threadIdx.x;
-    uint32_t mine = 0;
-    if (per == 8) {
-        uint4 a[kSelCopies][2];
-#pragma unroll
-        for (int cp = 0; cp < kSelCopies; cp++) {
-            a[cp][0] = *reinterpret_cast<const uint4*>(&st->hist[cp][t * 8]);
-            a[cp][1] = *reinterpret_cast<const uint4*>(&st->hist[cp][t * 8 + 4]);
-        }
-        uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int cp = 0; cp < kSelCopies; cp++) {
-            c[0] += a[cp][0].x;
-            c[1] += a[cp][0].y;
-            c[2] += a[cp][0].z;
-            c[3] += a[cp][0].w;
-            c[4] += a[cp][1].x;
-            c[5] += a[cp][1].y;
-            c[6] += a[cp][1].z;
-            c[7] += a[cp][1].w;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            h[t * 8 + j] = c[j];
-            mine += c[j];
-        }
-    } else {
-        for (int j = 0; j < per; j++) {
-            uint32_t c = 0;
-            for (int cp = 0; cp < kSelCopies; cp++) c += st->hist[cp][t * per + j];
-            h[t * per + j] = c;
-            mine += c;
-        }
-    }
-    part[t] = mine;
-    __syncthreads();
-    for (int o = 1; o < kSelThreads; o <<= 1) {
-        const uint32_t add = t + o < kSelThreads ? part[t + o] : 0u;
-        __syncthreads();
-        part[t] += add;
-        __syncthreads();
-    }
-    /* part[t] = keys in bins >= t * per; the digit lies with the thread where
-     * part[t + 1] < remaining <= part[t] */
-    const uint32_t above = t + 1 < kSelThreads ? part[t + 1] : 0u;
-    if ((int64_t)above < rem && rem <= (int64_t)part[t]) {
-        int64_t r = rem - above;
-        int d = t * per + per - 1;
-        for (; d > t * per; d--) {
-            if (r <= (int64_t)h[d]) break;
-            r -= h[d];
-        }
-        st->prefix = prefix | ((uint64_t)d << shift);
-        st->fixed = top - width >= 64 ? ~0ull : (~0ull << (top - width));
-        st->remaining = r;
-        st->settled = r == (int64_t)h[d];
-    }
-    if (t == 0) st->done = 0;
-    for (int cp = 0; cp < kSelCopies; cp++)
-        for (int i = 4 * t; i < bins; i += 4 * blockDim.x) *reinterpret_cast<uint4*>(&st->hist[cp][i]) = make_uint4(0, 0, 0, 0);
+    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x)
+        if (h[i]) atomicAdd(&st->hist[1][i], h[i]);
 }
 
-/* Keys at or above the selected prefix under its mask (exactly `top` of
- * them; the bound only guards the buffer).  Each wave ballots its lanes'
- * keys, the block scans its waves' counts in LDS, and one global atomic per
- * block reserves the block's slots. */
-__global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __restrict__ sc, int64_t P, SelState* st,
-                                                                uint64_t* __restrict__ out, uint32_t top) {
-    __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
-    __shared__ uint32_t base;
-    const uint64_t kstar = st->prefix, fixed = st->fixed;
-    const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE;
-    const int64_t bstride = (int64_t)gridDim.x * blockDim.x * kSelPer;
-    for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x * kSelPer; b0 < P; b0 += bstride) {
+/* Keys >= thr appended to out (at most kSortMax) by one block's share of the
+ * pool: each wave counts its lanes' keys, the block scans its waves' counts,
+ * and one global atomic per block and round reserves the slots. */
+__device__ __forceinline__ void append_keys(const float* __restrict__ sc, int64_t P, uint64_t thr, uint32_t* count,
+                                            uint64_t* __restrict__ out, uint32_t* wcount, uint32_t* base, int64_t block,
+                                            int64_t blocks) {
+    const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE, nw = blockDim.x / BM_WAVE;
+    for (int64_t b0 = block * blockDim.x * kSelPer; b0 < P; b0 += blocks * blockDim.x * kSelPer) {
         const int64_t p0 = b0 + ((int64_t)wave * BM_WAVE + lane) * kSelPer;
         float v[kSelPer];
-        if (p0 + kSelPer <= P) {
-#pragma unroll
-            for (int j = 0; j < kSelPer; j += 4) {
-                const float4 f = *reinterpret_cast<const float4*>(&sc[p0 + j]);
-                v[j] = f.x;
-                v[j + 1] = f.y;
-                v[j + 2] = f.z;
-                v[j + 3] = f.w;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < kSelPer; j++) v[j] = p0 + j < P ? sc[p0 + j] : 0.f;
-        }
+        load_scores(sc, p0, P, v);
         uint32_t inmask = 0;   /* bit j: this lane's key j is in */
 #pragma unroll
-        for (int j = 0; j < kSelPer; j++) {
-            const uint64_t k = rank_key(v[j], p0 + j);
-            if (p0 + j < P && (k & fixed) >= kstar) inmask |= 1u << j;
-        }
-        uint32_t mine = (uint32_t)__popc(inmask);
-        /* exclusive prefix of the lanes' counts within the wave */
+        for (int j = 0; j < kSelPer; j++)
+            if (p0 + j < P && rank_key(v[j], p0 + j) >= thr) inmask |= 1u << j;
+        const uint32_t mine = (uint32_t)__popc(inmask);
         uint32_t incl = mine;
 #pragma unroll
         for (int o = 1; o < BM_WAVE; o <<= 1) {
@@ -710,52 +727,122 @@ __global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __r
         __syncthreads();
         if (threadIdx.x == 0) {
             uint32_t tot = 0;
-            for (int w = 0; w < kSelThreads / BM_WAVE; w++) {
+            for (int w = 0; w < nw; w++) {
                 const uint32_t c = wcount[w];
                 wcount[w] = tot;
                 tot += c;
             }
-            base = tot ? atomicAdd(&st->count, tot) : 0u;
+            *base = tot ? atomicAdd(count, tot) : 0u;
         }
         __syncthreads();
-        uint32_t at = base + wcount[wave] + incl - mine;
+        uint32_t at = *base + wcount[wave] + incl - mine;
 #pragma unroll
         for (int j = 0; j < kSelPer; j++)
             if (inmask & (1u << j)) {
-                if (at < top) out[at] = rank_key(v[j], p0 + j);
+                if (at < (uint32_t)kSortMax) out[at] = rank_key(v[j], p0 + j);
                 at++;
             }
         __syncthreads();
     }
 }
 
-/* One block: the `top` selected keys in descending order (bitonic sort in
- * LDS, padded with zero keys to a power of two), then their stream pairs. */
-__global__ void __launch_bounds__(1024) k_select_sort(const uint64_t* __restrict__ keys, int32_t top, int32_t padded,
-                                                      uint64_t seed, int32_t n, int2* __restrict__ out) {
-    extern __shared__ uint64_t sk[];
-    for (int i = threadIdx.x; i < padded; i += blockDim.x) sk[i] = i < top ? keys[i] : 0ull;
-    __syncthreads();
-    for (int size = 2; size <= padded; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = threadIdx.x; i < padded / 2; i += blockDim.x) {
-                const int lo = 2 * i - (i & (stride - 1));
-                const int hi = lo + stride;
-                const bool desc = (lo & size) == 0;
-                const uint64_t a = sk[lo], b = sk[hi];
-                if ((a < b) == desc) {
-                    sk[lo] = b;
-                    sk[hi] = a;
-                }
+/* Threshold of the two digits; returns whether the keys at or above it fit
+ * kSortMax. */
+template <int NT>
+__device__ __forceinline__ bool select_threshold(const SelState* st, uint32_t top, uint64_t* thr, DigitShared& S) {
+    uint32_t r = top, in;
+    const uint32_t d0 = find_digit<NT>(st->hist[0], &r, &in, S);
+    const uint32_t d1 = find_digit<NT>(st->hist[1], &r, &in, S);
+    *thr = ((uint64_t)((d0 << 20) | (d1 << 8))) << 32;
+    return (top - r) + in <= (uint32_t)kSortMax;
+}
+
+__global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                                uint64_t* __restrict__ out, uint32_t top) {
+    __shared__ DigitShared S;
+    __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
+    __shared__ uint32_t base;
+    uint64_t thr;
+    if (!select_threshold<kSelThreads>(st, top, &thr, S)) return;
+    append_keys(sc, P, thr, &st->count, out, wcount, &base, blockIdx.x, gridDim.x);
+}
+
+/* One block: nothing when the two digits settled the select; otherwise the
+ * remaining 40 bits of the threshold, digit by digit, and the keys. */
+__global__ void __launch_bounds__(1024) k_select_rest(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                      uint64_t* __restrict__ out, uint32_t top) {
+    __shared__ alignas(16) uint32_t h[kSelBins];
+    __shared__ DigitShared S;
+    __shared__ uint32_t wcount[1024 / BM_WAVE];
+    __shared__ uint32_t base;
+    uint32_t r = top, in;
+    const uint32_t d0 = find_digit<1024>(st->hist[0], &r, &in, S);
+    const uint32_t d1 = find_digit<1024>(st->hist[1], &r, &in, S);
+    uint64_t thr = ((uint64_t)((d0 << 20) | (d1 << 8))) << 32;
+    if ((top - r) + in <= (uint32_t)kSortMax) return;
+    const int lane = threadIdx.x & (BM_WAVE - 1);
+    for (int shift = 28; shift >= 0; shift = shift == 4 ? 0 : (shift == 0 ? -1 : shift - 12)) {
+        const int width = shift == 0 ? 4 : 12;
+        const uint64_t fixed = ~0ull << (shift + width);
+        __syncthreads();
+        for (int i = threadIdx.x; i < kSelBins; i += blockDim.x) h[i] = 0;
+        __syncthreads();
+        for (int64_t w0 = (int64_t)(threadIdx.x / BM_WAVE) * BM_WAVE * kSelPer; w0 < P;
+             w0 += (int64_t)blockDim.x * kSelPer) {
+            const int64_t p0 = w0 + (int64_t)lane * kSelPer;
+            float v[kSelPer];
+            load_scores(sc, p0, P, v);
+#pragma unroll
+            for (int j = 0; j < kSelPer; j++) {
+                const uint64_t k = rank_key(v[j], p0 + j);
+                wave_hist_add(h, p0 + j < P && (k & fixed) == thr, (uint32_t)(k >> shift) & ((1u << width) - 1u), lane);
             }
-            __syncthreads();
         }
+        __syncthreads();
+        const uint32_t d = find_digit<1024>(h, &r, &in, S);
+        thr |= (uint64_t)d << shift;
+        if ((top - r) + in <= (uint32_t)kSortMax) break;
     }
-    for (int i = threadIdx.x; i < top; i += blockDim.x) {
-        const uint32_t p = 0xFFFFFFFFu - (uint32_t)sk[i];
+    append_keys(sc, P, thr, &st->count, out, wcount, &base, 0, 1);
+}
+
+/* The written keys ranked by counting: a key's place in descending order is
+ * the number of larger ones (keys are distinct).  Every block holds all keys
+ * in LDS and ranks kRankKeys of them, 16 lanes per key counting a sixteenth
+ * each; the `top` first places get their stream pairs. */
+constexpr int kRankLanes = 16, kRankKeys = kSelThreads / kRankLanes;
+
+__global__ void __launch_bounds__(kSelThreads) k_select_rank(const uint64_t* __restrict__ keys, const SelState* st,
+                                                             uint32_t top, uint64_t seed, int32_t n,
+                                                             int2* __restrict__ out) {
+    extern __shared__ ulonglong2 sk[];
+    const uint32_t cnt = st->count < (uint32_t)kSortMax ? st->count : (uint32_t)kSortMax;
+    if ((uint32_t)blockIdx.x * kRankKeys >= cnt) return;
+    uint64_t* s = reinterpret_cast<uint64_t*>(sk);
+    /* every lane counts the same whole number of 16-byte words; key 0 is below every key */
+    const uint32_t words = (cnt + 2 * kRankLanes - 1) / (2 * kRankLanes) * kRankLanes;
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) {
+        ulonglong2 x;
+        x.x = 2 * i < cnt ? keys[2 * i] : 0ull;
+        x.y = 2 * i + 1 < cnt ? keys[2 * i + 1] : 0ull;
+        sk[i] = x;
+    }
+    __syncthreads();
+    const uint32_t i = blockIdx.x * kRankKeys + threadIdx.x / kRankLanes, part = threadIdx.x % kRankLanes;
+    const uint64_t me = i < cnt ? s[i] : 0ull;
+    uint32_t rank = 0;
+#pragma unroll 8
+    for (uint32_t q = part; q < words; q += kRankLanes) {
+        const ulonglong2 x = sk[q];
+        rank += (x.x > me ? 1u : 0u) + (x.y > me ? 1u : 0u);
+    }
+#pragma unroll
+    for (int o = 1; o < kRankLanes; o <<= 1) rank += (uint32_t)__shfl_xor((int)rank, o, BM_WAVE);
+    if (part == 0 && i < cnt && rank < top) {
+        const uint32_t p = 0xFFFFFFFFu - (uint32_t)me;
         int32_t u, v;
         bm_uniform_pair(seed, (uint64_t)p, n, &u, &v);
-        out[i] = make_int2(u, v);
+        out[rank] = make_int2(u, v);
     }
 }
 
@@ -801,20 +888,27 @@ hipError_t bm_launch_mlp_pack(const BmMlpDev& d, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <bool HIST>
+static hipError_t launch_forward(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
+                                 int64_t k, float* score, uint32_t* hist, int32_t num_cus, hipStream_t s) {
+    PairSrc ps{list, seed, n};
+    const int64_t groups = (k + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
+    int64_t blocks = (groups + kScoreWaves - 1) / kScoreWaves;
+    const int64_t cap = num_cus > 0 ? num_cus : 256;
+    if (blocks > cap) blocks = cap;
+    const size_t lds = sizeof(ScoreShared) + (HIST ? kHistBins * sizeof(uint32_t) : 0);
+    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_forward<HIST>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_mlp_forward<HIST>, dim3((unsigned)blocks), dim3(kScoreThreads), lds, s,
+                       reinterpret_cast<const float4*>(vf), ps, k, mlpdev(d), score, hist);
+    return hipGetLastError();
+}
+
 hipError_t bm_launch_mlp_forward(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
                                  int64_t k, float* score, int32_t num_cus, hipStream_t s) {
     if (k <= 0) return hipSuccess;
-    PairSrc ps{list, seed, n};
-    const int64_t tiles = (k + 15) / 16;
-    int64_t blocks = (tiles + kFwdWaves - 1) / kFwdWaves;
-    const int64_t cap = (int64_t)(num_cus > 0 ? num_cus : 256) * 4;
-    if (blocks > cap) blocks = cap;
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_forward, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)sizeof(FwdShared));
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)blocks), dim3(kFwdThreads), sizeof(FwdShared), s,
-                       reinterpret_cast<const float4*>(vf), ps, k, mlpdev(d), score);
-    return hipGetLastError();
+    return launch_forward<false>(d, vf, list, seed, n, k, score, nullptr, num_cus, s);
 }
 
 size_t bm_mlp_train_bytes(int64_t k) { return (size_t)((k + 31) / 32 * 32) * (kF + 3 * kH) * sizeof(short); }
@@ -868,36 +962,34 @@ size_t bm_mlp_select_bytes(int64_t pool) {
 
 int64_t bm_mlp_select_max_top(void) { return kSortMax; }
 
-/* Scores of the pool's pairs, radix select of the `top` largest keys and a
- * one-block sort of them into pairs; scratch holds the scores, the select
- * state and the selected keys (bm_mlp_select_bytes(pool)), and the state's
- * counters and histograms are cleared by k_select_init, so the call
- * allocates nothing and needs no memset. */
+/* Scores of the pool's pairs with the first digit's histogram, the second
+ * digit, the keys at or above the threshold and their ranking; scratch holds
+ * the scores, the select state and the selected keys
+ * (bm_mlp_select_bytes(pool)), and the state is cleared by k_select_init, so
+ * the call allocates nothing and needs no memset. */
 hipError_t bm_launch_mlp_rank_select(const BmMlpDev& d, const float* vf, uint64_t seed, int32_t n, int64_t pool,
                                      int64_t top, void* scratch, size_t scratch_bytes, int2* out, int32_t num_cus,
                                      hipStream_t s) {
     if (pool <= 0 || top <= 0) return hipSuccess;
-    if (top > kSortMax || pool >= (1LL << 32) || scratch_bytes < bm_mlp_select_bytes(pool)) return hipErrorInvalidValue;
+    if (top > kSortMax || top > pool || pool >= (1LL << 32) || scratch_bytes < bm_mlp_select_bytes(pool))
+        return hipErrorInvalidValue;
     float* sc = static_cast<float*>(scratch);
-    hipError_t e = bm_launch_mlp_forward(d, vf, nullptr, seed, n, pool, sc, num_cus, s);
-    if (e != hipSuccess) return e;
     char* q = reinterpret_cast<char*>(sc + pool);
     q += (256 - (reinterpret_cast<uintptr_t>(q) & 255)) & 255;
     SelState* st = reinterpret_cast<SelState*>(q);
     uint64_t* keys = reinterpret_cast<uint64_t*>(st + 1);
-    const int blocks = grid_of(pool, kSelThreads * kSelPer, (int64_t)(num_cus > 0 ? num_cus : 256) * 4);
-    hipLaunchKernelGGL(k_select_init, dim3(1), dim3(256), 0, s, st, top);
-    for (int pass = 0; pass < kSelPasses; pass++)
-        hipLaunchKernelGGL(k_select_pass, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, pass);
-    hipLaunchKernelGGL(k_select_compact, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top);
-    int padded = 1;
-    while (padded < top) padded <<= 1;
-    if (padded < 2) padded = 2;
-    e = hipFuncSetAttribute((const void*)k_select_sort, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)((size_t)padded * sizeof(uint64_t)));
+    hipLaunchKernelGGL(k_select_init, dim3(8), dim3(256), 0, s, st);
+    hipError_t e = launch_forward<true>(d, vf, nullptr, seed, n, pool, sc, st->hist[0], num_cus, s);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_select_sort, dim3(1), dim3(1024), (size_t)padded * sizeof(uint64_t), s, keys, (int32_t)top,
-                       padded, seed, n, out);
+    const int blocks = grid_of(pool, kSelThreads * kSelPer, (int64_t)(num_cus > 0 ? num_cus : 256) * 4);
+    hipLaunchKernelGGL(k_select_second, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top);
+    hipLaunchKernelGGL(k_select_compact, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top);
+    hipLaunchKernelGGL(k_select_rest, dim3(1), dim3(1024), 0, s, sc, pool, st, keys, (uint32_t)top);
+    const size_t lds = kSortMax * sizeof(uint64_t);
+    e = hipFuncSetAttribute((const void*)k_select_rank, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_select_rank, dim3(kSortMax / kRankKeys), dim3(kSelThreads), lds, s, keys, st, (uint32_t)top,
+                       seed, n, out);
     return hipGetLastError();
 }
 
