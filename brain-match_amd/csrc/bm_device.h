@@ -313,16 +313,18 @@ hipError_t bm_launch_mlp_pack(const BmMlpDev& d, hipStream_t s);
 /* Scores of k pairs (list, or uniform stream `seed` when list is NULL). */
 hipError_t bm_launch_mlp_forward(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
                                  int64_t k, float* score, int32_t num_cus, hipStream_t s);
-/* Gradient of the mean squared error over k pairs, added into d.grad; the
- * summed squared error is added into *loss.  Targets are `target`, or, with
- * target NULL, sign(x) log(1 + |x|) of the exact deltas x = delta[0..k).  act:
- * bm_mlp_train_bytes(k). */
+/* Gradient of the mean squared error over k pairs, left as partial sums in
+ * act (bm_mlp_train_bytes(k)).  Targets are `target`, or, with target NULL,
+ * sign(x) log(1 + |x|) of the exact deltas x = delta[0..k). */
 size_t bm_mlp_train_bytes(int64_t k);
 hipError_t bm_launch_mlp_gradient(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
-                                  int64_t k, const float* target, const int64_t* delta, void* act, float* loss,
-                                  int32_t num_cus, hipStream_t s);
-/* One Adam step from d.grad, which it clears, with *loss moved to *loss_out. */
-hipError_t bm_launch_mlp_adam(const BmMlpDev& d, float lr, int64_t step, float* loss, float* loss_out, hipStream_t s);
+                                  int64_t k, const float* target, const int64_t* delta, void* act, int32_t num_cus,
+                                  hipStream_t s);
+/* The partials of a batch of k pairs as a gradient in d.grad and the summed
+ * squared error in *loss, or as one Adam step. */
+hipError_t bm_launch_mlp_reduce(const BmMlpDev& d, void* act, int64_t k, float* loss, int32_t num_cus, hipStream_t s);
+hipError_t bm_launch_mlp_adam(const BmMlpDev& d, float lr, int64_t step, void* act, int64_t k, float* loss,
+                              int32_t num_cus, hipStream_t s);
 /* Top `top` of `pool` uniform-stream pairs by score, as a pair list. */
 size_t bm_mlp_rank_scratch(int64_t pool);
 /* Scratch bytes of the select-only ranking of a pool (bm_launch_mlp_rank_select)

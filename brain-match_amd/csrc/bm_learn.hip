@@ -57,8 +57,7 @@ struct bm_mlp {
     float* d_vf;
     void* d_feat_acc;       /* (n+1) x 32 bytes of feature accumulators, zero between passes */
     int features_ready;
-    float* d_loss;          /* summed squared error of the batch in hand, 0 between batches */
-    float* d_trace;         /* that of every step since the last read-back */
+    float* d_trace;         /* summed squared error of the steps of one call */
     int64_t trace_cap;
     float* d_target;
     int64_t target_cap;
@@ -123,7 +122,6 @@ extern "C" void bm_mlp_destroy(bm_mlp* m) {
     (void)hipFree(m->d.W2Tf);
     (void)hipFree(m->d_vf);
     (void)hipFree(m->d_feat_acc);
-    (void)hipFree(m->d_loss);
     (void)hipFree(m->d_trace);
     (void)hipFree(m->d_target);
     (void)hipFree(m->d_act);
@@ -160,7 +158,6 @@ extern "C" int bm_mlp_set_params(bm_mlp* m, const float* p) {
     MHIP(m, hipSetDevice(m->device));
     const size_t np = (size_t)bm_mlp_param_count();
     MHIP(m, hipMemcpyAsync(m->d.params, p, np * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    MHIP(m, hipMemsetAsync(m->d.grad, 0, np * sizeof(float), m->stream));
     MHIP(m, hipMemsetAsync(m->d.adam_m, 0, np * sizeof(float), m->stream));
     MHIP(m, hipMemsetAsync(m->d.adam_v, 0, np * sizeof(float), m->stream));
     MHIP(m, bm_launch_mlp_pack(m->d, m->stream));
@@ -205,9 +202,6 @@ extern "C" int bm_mlp_create(bm_ctx* ctx, uint64_t seed, bm_mlp** out) {
     alloc(&m->d.W2f, 128 * 128 * 2);
     alloc(&m->d.W2Tf, 128 * 128 * 2);
     alloc((void**)&m->d_vf, ((size_t)m->n + 1) * 8 * sizeof(float));
-    alloc((void**)&m->d_loss, sizeof(float));
-    if (rc == BM_OK && hipMemset(m->d_loss, 0, sizeof(float)) != hipSuccess)
-        rc = bm_ctx_set_error(ctx, BM_ERR_HIP, "bm_mlp_create: hipMemset failed");
     alloc(&m->d_feat_acc, ((size_t)m->n + 1) * 32);
     if (rc == BM_OK && hipMemset(m->d_feat_acc, 0, ((size_t)m->n + 1) * 32) != hipSuccess)
         rc = bm_ctx_set_error(ctx, BM_ERR_HIP, "bm_mlp_create: hipMemset failed");
@@ -267,14 +261,14 @@ extern "C" int bm_mlp_score_pairs(bm_mlp* m, const int32_t* uv, int64_t k, float
     return BM_OK;
 }
 
-/* Gradient of one batch into m->d.grad and its squared error into *d_loss
- * (both 0 before), from targets or, with d_target NULL, exact deltas. */
+/* Partial sums of one batch's gradient into m->d_act, from targets or, with
+ * d_target NULL, exact deltas. */
 static int batch_gradient(bm_mlp* m, const int2* list, uint64_t seed, int64_t k, const float* d_target,
                           const int64_t* d_delta) {
     int rc = grow_bytes(m, &m->d_act, &m->act_bytes, bm_mlp_train_bytes(k));
     if (rc != BM_OK) return rc;
-    MHIP(m, bm_launch_mlp_gradient(m->d, m->d_vf, list, seed, m->n, k, d_target, d_delta, m->d_act, m->d_loss,
-                                   m->num_cus, m->stream));
+    MHIP(m, bm_launch_mlp_gradient(m->d, m->d_vf, list, seed, m->n, k, d_target, d_delta, m->d_act, m->num_cus,
+                                   m->stream));
     return BM_OK;
 }
 
@@ -289,12 +283,12 @@ extern "C" int bm_mlp_gradient(bm_mlp* m, const int32_t* uv, const float* target
     MHIP(m, hipMemcpyAsync(m->d_target, target, (size_t)k * sizeof(float), hipMemcpyHostToDevice, m->stream));
     const size_t np = (size_t)bm_mlp_param_count();
     rc = batch_gradient(m, m->d_pairs, 0, k, m->d_target, nullptr);
+    if (rc == BM_OK) rc = grow(m, &m->d_trace, &m->trace_cap, 1);
     if (rc != BM_OK) return rc;
+    MHIP(m, bm_launch_mlp_reduce(m->d, m->d_act, k, m->d_trace, m->num_cus, m->stream));
     float se = 0.f;
     MHIP(m, hipMemcpyAsync(grad, m->d.grad, np * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    MHIP(m, hipMemcpyAsync(&se, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    MHIP(m, hipMemsetAsync(m->d.grad, 0, np * sizeof(float), m->stream));
-    MHIP(m, hipMemsetAsync(m->d_loss, 0, sizeof(float), m->stream));
+    MHIP(m, hipMemcpyAsync(&se, m->d_trace, sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MHIP(m, hipStreamSynchronize(m->stream));
     if (mse) *mse = se / (float)k;
     return BM_OK;
@@ -324,7 +318,7 @@ extern "C" int bm_mlp_train(bm_mlp* m, uint64_t seed, int64_t steps, int32_t bat
         rc = batch_gradient(m, nullptr, sd, batch, nullptr, bm_batch_deltas_dev(m->train_batch));
         if (rc != BM_OK) return rc;
         m->adam_step++;
-        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_loss, m->d_trace + s, m->stream));
+        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_act, batch, m->d_trace + s, m->num_cus, m->stream));
     }
     if (mse_trace && steps > 0) {
         MHIP(m, hipMemcpyAsync(mse_trace, m->d_trace, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, m->stream));
@@ -376,7 +370,7 @@ extern "C" int bm_mlp_train_batch(bm_mlp* m, bm_batch* b, float lr, float* mse) 
     if (rc == BM_OK) rc = batch_gradient(m, bm_batch_pairs_dev(b), 0, k, nullptr, bm_batch_deltas_dev(b));
     if (rc != BM_OK) return rc;
     m->adam_step++;
-    MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_loss, m->d_trace, m->stream));
+    MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_act, k, m->d_trace, m->num_cus, m->stream));
     if (mse) {
         float se = 0.f;
         MHIP(m, hipMemcpyAsync(&se, m->d_trace, sizeof(float), hipMemcpyDeviceToHost, m->stream));

@@ -62,6 +62,9 @@ constexpr int kF = 16;     /* features per pair */
 constexpr int kH = 128;    /* hidden width */
 constexpr int kT = kH / 16;   /* 16-wide tiles per hidden layer */
 constexpr int kS = kH / 32;   /* 32-deep k-steps over a hidden layer */
+/* parameter layout */
+constexpr int kOffW1 = 0, kOffB1 = kF * kH, kOffW2 = kOffB1 + kH, kOffB2 = kOffW2 + kH * kH, kOffW3 = kOffB2 + kH,
+              kOffB3 = kOffW3 + kH, kParams = kOffB3 + 1;
 
 /* bfloat16 bits of x, rounded to nearest even (v_cvt_pk_bf16_f32). */
 __device__ __forceinline__ short bf16_of(float x) { return __builtin_bit_cast(short, (__bf16)x); }
@@ -99,21 +102,34 @@ __global__ void k_feature_finish(BmDevGraph g, longlong4* __restrict__ acc, floa
     }
 }
 
-/* Weights in fragment order with k-steps of KB rows (16 or 32):
- * frag[((s * (NN / 16) + t) * 64 + l) * (KB / 4) + i] = M[KB s + (KB / 4) (l / 16) + i][16 t + l % 16]
- * for the KK x NN matrix M = W (K x N, row-major) or, with transpose, W^T. */
-__global__ void k_mlp_pack(const float* __restrict__ W, int K, int N, int transpose, int KB, short* __restrict__ frag) {
-    const int KK = transpose ? N : K, NN = transpose ? K : N;   /* shape of the packed matrix */
-    const int per = KB / 4;
-    const int total = (KK / KB) * (NN / 16) * 64;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += gridDim.x * blockDim.x) {
-        const int l = q & 63, f = q >> 6;
-        const int s = f / (NN / 16), t = f % (NN / 16);
-        for (int i = 0; i < per; i++) {
-            const int r = KB * s + per * (l / 16) + i, c = 16 * t + (l % 16);
-            frag[(size_t)q * per + i] = bf16_of(transpose ? W[c * N + r] : W[r * N + c]);
-        }
+/* Weights in fragment order with k-steps of KB rows (16 or 32), for a KK x NN
+ * matrix M:
+ * frag[((s * (NN / 16) + t) * 64 + l) * (KB / 4) + i] = M[KB s + (KB / 4) (l / 16) + i][16 t + l % 16].
+ * Place of element (r, c) there. */
+template <int KB>
+__device__ __forceinline__ int frag_at(int r, int c, int NN) {
+    constexpr int per = KB / 4;
+    const int s = r / KB, rr = r % KB;
+    return ((s * (NN / 16) + c / 16) * 64 + 16 * (rr / per) + c % 16) * per + rr % per;
+}
+
+/* The bf16 copies of parameter i with value x: W1 once, W2 as itself and
+ * transposed; biases and w3 stay fp32. */
+__device__ __forceinline__ void pack_param(short* __restrict__ W1f, short* __restrict__ W2f, short* __restrict__ W2Tf,
+                                           int i, float x) {
+    if (i < kF * kH) {
+        W1f[frag_at<16>(i / kH, i % kH, kH)] = bf16_of(x);
+    } else if (i >= kOffW2 && i < kOffW2 + kH * kH) {
+        const int r = (i - kOffW2) / kH, c = (i - kOffW2) % kH;
+        W2f[frag_at<32>(r, c, kH)] = bf16_of(x);
+        W2Tf[frag_at<32>(c, r, kH)] = bf16_of(x);
     }
+}
+
+__global__ void k_mlp_pack(const float* __restrict__ p, short* __restrict__ W1f, short* __restrict__ W2f,
+                           short* __restrict__ W2Tf) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kParams; i += gridDim.x * blockDim.x)
+        pack_param(W1f, W2f, W2Tf, i, p[i]);
 }
 
 struct MlpDev {
@@ -141,16 +157,7 @@ __device__ __forceinline__ int2 pair_at(const PairSrc& ps, int64_t p) {
 }
 
 constexpr int kHistBins = 4096;   /* first 12 bits of the order-preserving score bits */
-constexpr int kFwdThreads = 256;
-constexpr int kFwdWaves = kFwdThreads / BM_WAVE;
 constexpr int kHPad = kH + 8;   /* padded bf16 row of a staged 16 x 128 tile (272 bytes: 16-byte reads hit distinct banks) */
-
-struct FwdShared {
-    v4s W1[kT * 64];
-    v8s W2[kS * kT * 64];
-    float b1[kH], b2[kH], w3[kH];
-    short Ht[kFwdWaves][16][kHPad];
-};
 
 template <typename Shared>
 __device__ __forceinline__ void stage_weights(Shared& S, const MlpDev& M) {
@@ -181,7 +188,8 @@ __device__ __forceinline__ v4s input_frag(const float4* __restrict__ vf, int2 uv
 /* Layer 1 for one tile in the pair-major form (training): z1 (D layout:
  * lane l has pairs 4 (l / 16) + j of hidden unit 16 t + l % 16, kept for the
  * backward mask) and h1 into the wave's LDS tile. */
-__device__ __forceinline__ void layer1(const FwdShared& S, short (*Ht)[kHPad], v4s xa, v4f* z1, int lane) {
+template <typename Shared>
+__device__ __forceinline__ void layer1(const Shared& S, short (*Ht)[kHPad], v4s xa, v4f* z1, int lane) {
 #pragma unroll
     for (int t = 0; t < kT; t++) {
         v4f acc = {0.f, 0.f, 0.f, 0.f};
@@ -326,51 +334,80 @@ __global__ void __launch_bounds__(kScoreThreads) k_mlp_forward(const float4* __r
     }
 }
 
+/* Regression target of an exact int64 delta: sign(d) log(1 + |d|). */
+__device__ __forceinline__ float delta_target(int64_t d) {
+    const double x = (double)d;
+    return (float)(x < 0 ? -log1p(-x) : log1p(x));
+}
+
 /* Training pass over a batch of B pairs (B a multiple of 32): forward, loss,
  * and the backward through the activations.  Stores bf(x)^T (16 x B), h1^T,
- * g1^T and g2^T (128 x B) for the weight-gradient products and accumulates
- * the bias gradients, dw3 and the summed squared error with atomics. */
+ * g1^T and g2^T (128 x B) for the weight-gradient products.  The bias
+ * gradients, dw3 and the summed squared error stay in registers over all of a
+ * wave's tiles, are summed per block in LDS and written as one partial per
+ * block, which k_mlp_adam / k_mlp_reduce add up in a fixed order.  Added to
+ * the gradient per 16-pair tile they were 1.6M device-wide atomics per 65,536
+ * pairs, which run at about 1.3e10 a second here: 221 us, now 31 us.  Eight
+ * waves per block share the weights (two per SIMD). */
 struct TrainBuf {
     short* XT;      /* 16 x B */
     short* H1T;     /* 128 x B */
     short* G1T;     /* 128 x B */
     short* G2T;     /* 128 x B */
-    float* grad;    /* gradient in the parameter layout */
-    float* loss;    /* summed squared error */
+    float* wpart;   /* slices x kWParams: weight gradients (dW1 then dW2) of each slice */
+    float* bpart;   /* kBParams x blocks: db1, db2, dw3, db3 and the summed squared error of each block */
+    const float* target;    /* one of the two */
+    const int64_t* delta;   /* targets are delta_target of these */
     int64_t B;
+    int64_t ld;     /* row stride of the four */
 };
 
-constexpr int kOffW1 = 0, kOffB1 = kF * kH, kOffW2 = kOffB1 + kH, kOffB2 = kOffW2 + kH * kH, kOffW3 = kOffB2 + kH,
-              kOffB3 = kOffW3 + kH, kParams = kOffB3 + 1;
+/* W1 and W2 in the partials; the other parameters in bpart's order, then the loss. */
+constexpr int kWParams = kF * kH + kH * kH, kBParams = 3 * kH + 2;
+
+constexpr int kTrainThreads = 512, kTrainWaves = kTrainThreads / BM_WAVE;
 
 struct TrainShared {
-    FwdShared f;
+    v4s W1[kT * 64];
+    v8s W2[kS * kT * 64];
+    float b1[kH], b2[kH], w3[kH];
     v8s W2T[kS * kT * 64];
+    float part[kTrainWaves][kBParams];
+    short Ht[kTrainWaves][16][kHPad];
 };
 
-__global__ void __launch_bounds__(kFwdThreads) k_mlp_train_act(const float4* __restrict__ vf, PairSrc ps, int64_t k,
-                                                               const float* __restrict__ target, MlpDev M, TrainBuf T) {
+__global__ void __launch_bounds__(kTrainThreads) k_mlp_train_act(const float4* __restrict__ vf, PairSrc ps, int64_t k,
+                                                                 MlpDev M, TrainBuf T) {
     extern __shared__ uint4 smem[];
     TrainShared& S = *reinterpret_cast<TrainShared*>(smem);
-    stage_weights(S.f, M);
+    stage_weights(S, M);
     for (int q = threadIdx.x; q < kS * kT * 64; q += blockDim.x) S.W2T[q] = M.W2Tf[q];
     __syncthreads();
     const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE;
-    short(*Ht)[kHPad] = S.f.Ht[wave];
+    short(*Ht)[kHPad] = S.Ht[wave];
     const float b3 = M.b3[0];
     const float inv = 2.f / (float)k;
-    const int64_t B = T.B;
-    const int64_t tiles = B / 16;
-    for (int64_t tile = (int64_t)blockIdx.x * kFwdWaves + wave; tile < tiles; tile += (int64_t)gridDim.x * kFwdWaves) {
+    const int64_t ld = T.ld;
+    const int64_t tiles = T.B / 16;
+    float ab1[kT], ab2[kT], aw3[kT], ab3 = 0.f, ase = 0.f;
+#pragma unroll
+    for (int t = 0; t < kT; t++) ab1[t] = ab2[t] = aw3[t] = 0.f;
+    for (int64_t tile = (int64_t)blockIdx.x * kTrainWaves + wave; tile < tiles; tile += (int64_t)gridDim.x * kTrainWaves) {
         const int64_t base = tile * 16;
         const int64_t p = base + (lane % 16);
         const bool valid = p < k;
         const int2 uv = valid ? pair_at(ps, p) : make_int2(0, 0);
         const v4s xa = input_frag(vf, uv, valid, lane);
+        float tg[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) T.XT[(int64_t)(4 * (lane / 16) + i) * B + p] = xa[i];
+        for (int j = 0; j < 4; j++) {
+            const int64_t q = base + 4 * (lane / 16) + j;
+            tg[j] = q >= k ? 0.f : (T.delta ? delta_target(T.delta[q]) : T.target[q]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) T.XT[(int64_t)(4 * (lane / 16) + i) * ld + p] = xa[i];
         v4f z1[kT];
-        layer1(S.f, Ht, xa, z1, lane);
+        layer1(S, Ht, xa, z1, lane);
         wave_sync();
         v8s a[kS];
         load_tile32(Ht, a, lane);
@@ -381,7 +418,7 @@ __global__ void __launch_bounds__(kFwdThreads) k_mlp_train_act(const float4* __r
             v4s h;
 #pragma unroll
             for (int j = 0; j < 4; j++) h[j] = Ht[4 * (lane / 16) + j][col];
-            *reinterpret_cast<v4s*>(&T.H1T[(int64_t)col * B + base + 4 * (lane / 16)]) = h;
+            *reinterpret_cast<v4s*>(&T.H1T[(int64_t)col * ld + base + 4 * (lane / 16)]) = h;
         }
         v4f z2[kT];
         float part[4] = {0.f, 0.f, 0.f, 0.f};
@@ -389,12 +426,12 @@ __global__ void __launch_bounds__(kFwdThreads) k_mlp_train_act(const float4* __r
         for (int t = 0; t < kT; t++) {
             v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < kS; s++) acc = mfma32(a[s], S.f.W2[(s * kT + t) * 64 + lane], acc);
+            for (int s = 0; s < kS; s++) acc = mfma32(a[s], S.W2[(s * kT + t) * 64 + lane], acc);
             const int col = 16 * t + (lane % 16);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                acc[j] += S.f.b2[col];
-                part[j] += (acc[j] > 0.f ? acc[j] : 0.f) * S.f.w3[col];
+                acc[j] += S.b2[col];
+                part[j] += (acc[j] > 0.f ? acc[j] : 0.f) * S.w3[col];
             }
             z2[t] = acc;
         }
@@ -403,48 +440,34 @@ __global__ void __launch_bounds__(kFwdThreads) k_mlp_train_act(const float4* __r
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) part[j] += __shfl_xor(part[j], o, BM_WAVE);
         /* dy for this lane's four rows (every lane of a 16-lane group has the sums) */
-        float dy[4], se = 0.f;
+        float dy[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int64_t q = base + 4 * (lane / 16) + j;
-            const bool ok = q < k;
+            const bool ok = base + 4 * (lane / 16) + j < k;
             const float y = part[j] + b3;
-            const float r = ok ? y - target[q] : 0.f;
+            const float r = ok ? y - tg[j] : 0.f;
             dy[j] = r * inv;
-            se += r * r;
+            if ((lane % 16) == 0) {
+                ase += r * r;
+                ab3 += dy[j];
+            }
         }
-        if ((lane % 16) == 0) atomicAdd(T.loss, se);
         /* g2 = bf(dy w3 [z2 > 0]); dw3 += h2 dy; db2 += dy w3 [z2 > 0] */
         wave_sync();
 #pragma unroll
         for (int t = 0; t < kT; t++) {
             const int col = 16 * t + (lane % 16);
-            float gsum = 0.f, wsum = 0.f;
             v4s gv;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float h = z2[t][j] > 0.f ? z2[t][j] : 0.f;
-                const float g = z2[t][j] > 0.f ? dy[j] * S.f.w3[col] : 0.f;
-                gsum += g;
-                wsum += h * dy[j];
+                const float g = z2[t][j] > 0.f ? dy[j] * S.w3[col] : 0.f;
+                ab2[t] += g;
+                aw3[t] += h * dy[j];
                 gv[j] = bf16_of(g);
                 Ht[4 * (lane / 16) + j][col] = gv[j];
             }
-            *reinterpret_cast<v4s*>(&T.G2T[(int64_t)col * B + base + 4 * (lane / 16)]) = gv;
-            gsum += __shfl_xor(gsum, 16, BM_WAVE);
-            gsum += __shfl_xor(gsum, 32, BM_WAVE);
-            wsum += __shfl_xor(wsum, 16, BM_WAVE);
-            wsum += __shfl_xor(wsum, 32, BM_WAVE);
-            if (lane < 16) {
-                atomicAdd(&T.grad[kOffB2 + col], gsum);
-                atomicAdd(&T.grad[kOffW3 + col], wsum);
-            }
-        }
-        {
-            float d = dy[0] + dy[1] + dy[2] + dy[3];
-            d += __shfl_xor(d, 16, BM_WAVE);
-            d += __shfl_xor(d, 32, BM_WAVE);
-            if (lane == 0) atomicAdd(&T.grad[kOffB3], d);
+            *reinterpret_cast<v4s*>(&T.G2T[(int64_t)col * ld + base + 4 * (lane / 16)]) = gv;
         }
         wave_sync();
         /* g1 = bf((g2 @ W2^T) [z1 > 0]) */
@@ -456,79 +479,179 @@ __global__ void __launch_bounds__(kFwdThreads) k_mlp_train_act(const float4* __r
 #pragma unroll
             for (int s = 0; s < kS; s++) acc = mfma32(ga[s], S.W2T[(s * kT + t) * 64 + lane], acc);
             const int col = 16 * t + (lane % 16);
-            float gsum = 0.f;
             v4s gv;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float g = z1[t][j] > 0.f ? acc[j] : 0.f;
-                gsum += g;
+                ab1[t] += g;
                 gv[j] = bf16_of(g);
             }
-            *reinterpret_cast<v4s*>(&T.G1T[(int64_t)col * B + base + 4 * (lane / 16)]) = gv;
-            gsum += __shfl_xor(gsum, 16, BM_WAVE);
-            gsum += __shfl_xor(gsum, 32, BM_WAVE);
-            if (lane < 16) atomicAdd(&T.grad[kOffB1 + col], gsum);
+            *reinterpret_cast<v4s*>(&T.G1T[(int64_t)col * ld + base + 4 * (lane / 16)]) = gv;
         }
         wave_sync();
+    }
+#pragma unroll
+    for (int t = 0; t < kT; t++) {
+        float x[3] = {ab1[t], ab2[t], aw3[t]};
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            x[j] += __shfl_xor(x[j], 16, BM_WAVE);
+            x[j] += __shfl_xor(x[j], 32, BM_WAVE);
+        }
+        if (lane < 16) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) S.part[wave][j * kH + 16 * t + lane] = x[j];
+        }
+    }
+    ab3 += __shfl_xor(ab3, 16, BM_WAVE);
+    ab3 += __shfl_xor(ab3, 32, BM_WAVE);
+    ase += __shfl_xor(ase, 16, BM_WAVE);
+    ase += __shfl_xor(ase, 32, BM_WAVE);
+    if (lane == 0) {
+        S.part[wave][3 * kH] = ab3;
+        S.part[wave][3 * kH + 1] = ase;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < kBParams; q += blockDim.x) {
+        float sum = 0.f;
+        for (int w = 0; w < kTrainWaves; w++) sum += S.part[w][q];
+        T.bpart[(int64_t)q * gridDim.x + blockIdx.x] = sum;
     }
 }
 
 /* Weight gradients: dW1 = bf(x)^T g1 (16 x 128), dW2 = h1^T g2 (128 x 128),
- * 32 batch entries per MFMA.  Work item = (output tile, slice of the batch);
- * one wave each, summed into the gradient with atomics. */
-constexpr int kWgTiles = 1 * kT + kT * kT;
+ * 32 batch entries per MFMA.  Work item = (block of output tiles, slice of
+ * the batch), one 4-wave block each: its waves take a quarter of the slice,
+ * each accumulating the whole 32 x 64 (dW2) or 16 x 64 (dW1) block, so an
+ * operand fragment loaded from L2 serves two or four products; they sum in
+ * LDS, in wave order, and write the slice's partial.  One tile per wave and
+ * atomics into the gradient took 44 us per 65,536 pairs, bound by the
+ * 590,000 atomics; now WGUS us. */
+constexpr int kWgRows = 2, kWgCols = 4;
+constexpr int kWgItems = kT / kWgCols + (kT / kWgRows) * (kT / kWgCols);
 
 __global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBuf T, int32_t slices) {
-    const int lane = threadIdx.x & (BM_WAVE - 1);
-    const int64_t items = (int64_t)kWgTiles * slices;
-    const int64_t B = T.B;
-    const int64_t steps = B / 32;
-    for (int64_t it = (int64_t)blockIdx.x * (blockDim.x / BM_WAVE) + threadIdx.x / BM_WAVE; it < items;
-         it += (int64_t)gridDim.x * (blockDim.x / BM_WAVE)) {
-        const int tile = (int)(it % kWgTiles), slice = (int)(it / kWgTiles);
-        const bool first = tile < kT;                     /* dW1 tiles, else dW2 */
-        const int mt = first ? 0 : (tile - kT) / kT, nt = first ? tile : (tile - kT) % kT;
-        const short* AT = first ? T.XT : T.H1T;           /* rows = input features / neurons */
-        const short* BT = first ? T.G1T : T.G2T;          /* rows = output neurons */
-        const int64_t s0 = steps * slice / slices, s1 = steps * (slice + 1) / slices;
-        v4f acc = {0.f, 0.f, 0.f, 0.f};
-        const int64_t arow = (int64_t)(16 * mt + lane % 16) * B, brow = (int64_t)(16 * nt + lane % 16) * B;
-        for (int64_t s = s0; s < s1; s++) {
-            const int64_t kk = 32 * s + 8 * (lane / 16);
-            const v8s a = *reinterpret_cast<const v8s*>(&AT[arow + kk]);
-            const v8s b = *reinterpret_cast<const v8s*>(&BT[brow + kk]);
-            acc = mfma32(a, b, acc);
-        }
-        const int off = first ? kOffW1 : kOffW2;
+    __shared__ float s_sum[4][kWgRows * kWgCols][256];
+    const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE;
+    const int64_t ld = T.ld;
+    const int64_t steps = T.B / 32;
+    const int item = (int)(blockIdx.x % kWgItems), slice = (int)(blockIdx.x / kWgItems);
+    const bool first = item < kT / kWgCols;           /* dW1, else dW2 */
+    const int it2 = item - kT / kWgCols;
+    const int mt = first ? 0 : it2 / (kT / kWgCols) * kWgRows, nt = (first ? item : it2 % (kT / kWgCols)) * kWgCols;
+    const int rows = first ? 1 : kWgRows;
+    const short* AT = first ? T.XT : T.H1T;           /* rows = input features / neurons */
+    const short* BT = first ? T.G1T : T.G2T;          /* rows = output neurons */
+    const int64_t parts = 4 * (int64_t)slices, part = 4 * (int64_t)slice + wave;
+    const int64_t s0 = steps * part / parts, s1 = steps * (part + 1) / parts;
+    v4f acc[kWgRows][kWgCols];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = 16 * mt + 4 * (lane / 16) + j, c = 16 * nt + lane % 16;
-            atomicAdd(&T.grad[off + r * kH + c], acc[j]);
-        }
+    for (int r = 0; r < kWgRows; r++)
+#pragma unroll
+        for (int c = 0; c < kWgCols; c++) acc[r][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    const short* ap = AT + (int64_t)(16 * mt + lane % 16) * ld + 8 * (lane / 16);
+    const short* bp = BT + (int64_t)(16 * nt + lane % 16) * ld + 8 * (lane / 16);
+    v8s an[kWgRows], bn[kWgCols];   /* the next step's fragments load while this one's products run */
+    const auto load = [&](int64_t s) {
+#pragma unroll
+        for (int r = 0; r < kWgRows; r++) an[r] = *reinterpret_cast<const v8s*>(ap + (r < rows ? 16 * r * ld : 0) + 32 * s);
+#pragma unroll
+        for (int c = 0; c < kWgCols; c++) bn[c] = *reinterpret_cast<const v8s*>(bp + 16 * c * ld + 32 * s);
+    };
+    if (s0 < s1) load(s0);
+    for (int64_t s = s0; s < s1; s++) {
+        v8s a[kWgRows], b[kWgCols];
+#pragma unroll
+        for (int r = 0; r < kWgRows; r++) a[r] = an[r];
+#pragma unroll
+        for (int c = 0; c < kWgCols; c++) b[c] = bn[c];
+        if (s + 1 < s1) load(s + 1);
+#pragma unroll
+        for (int r = 0; r < kWgRows; r++)
+#pragma unroll
+            for (int c = 0; c < kWgCols; c++) acc[r][c] = mfma32(a[r], b[c], acc[r][c]);
+    }
+#pragma unroll
+    for (int r = 0; r < kWgRows; r++)
+#pragma unroll
+        for (int c = 0; c < kWgCols; c++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                s_sum[wave][r * kWgCols + c][64 * j + lane] = acc[r][c][j];
+    __syncthreads();
+    float* out = T.wpart + (int64_t)slice * kWParams + (first ? 0 : kF * kH);
+    for (int i = threadIdx.x; i < rows * kWgCols * 256; i += 256) {
+        const int tile = i / 256, j = (i % 256) / 64, l = i % 64;
+        const int r = 16 * (mt + tile / kWgCols) + 4 * (l / 16) + j, c = 16 * (nt + tile % kWgCols) + l % 16;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) sum += s_sum[w][tile][64 * j + l];
+        out[r * kH + c] = sum;
     }
 }
 
-/* Adam on the fp32 master parameters; clears the gradient. */
-__global__ void k_mlp_adam(float* __restrict__ p, float* __restrict__ g, float* __restrict__ m, float* __restrict__ v,
-                           int32_t count, float lr, float b1c, float b2c) {
+/* Partials of one batch's gradient. */
+struct GradParts {
+    const float* w;
+    const float* b;
+    int32_t slices, blocks;
+};
+
+constexpr int kGradThreads = 256;
+/* blocks summing W1 and W2 (a thread per parameter over the slices), then one
+ * wave per other parameter (and the loss) over the blocks */
+constexpr int kGradWBlocks = kWParams / kGradThreads, kGradBBlocks = (kBParams + 3) / 4;
+
+/* The gradient value of this thread's parameter and its index (-1: none;
+ * kParams: the summed squared error), every slice and block added in order. */
+__device__ __forceinline__ float grad_sum(const GradParts& P, int* param) {
+    *param = -1;
+    if ((int)blockIdx.x < kGradWBlocks) {
+        const int i = blockIdx.x * kGradThreads + threadIdx.x;
+        float sum = 0.f;
+#pragma unroll 8
+        for (int q = 0; q < P.slices; q++) sum += P.w[(int64_t)q * kWParams + i];
+        *param = i < kF * kH ? kOffW1 + i : kOffW2 + (i - kF * kH);
+        return sum;
+    }
+    const int q = ((int)blockIdx.x - kGradWBlocks) * 4 + threadIdx.x / BM_WAVE, lane = threadIdx.x & (BM_WAVE - 1);
+    if (q >= kBParams) return 0.f;
+    float sum = 0.f;
+    for (int i = lane; i < P.blocks; i += BM_WAVE) sum += P.b[(int64_t)q * P.blocks + i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, BM_WAVE);
+    if (lane == 0)
+        *param = q < kH ? kOffB1 + q
+                        : (q < 2 * kH ? kOffB2 + q - kH : (q < 3 * kH ? kOffW3 + q - 2 * kH : (q == 3 * kH ? kOffB3 : kParams)));
+    return sum;
+}
+
+/* The whole gradient and the loss of a batch. */
+__global__ void __launch_bounds__(kGradThreads) k_mlp_reduce(GradParts P, float* __restrict__ g, float* loss) {
+    int i;
+    const float x = grad_sum(P, &i);
+    if (i == kParams) *loss = x;
+    else if (i >= 0) g[i] = x;
+}
+
+/* Adam on the fp32 master parameters and their bf16 copies, from the batch's
+ * partials; the summed squared error goes to *loss. */
+__global__ void __launch_bounds__(kGradThreads) k_mlp_adam(GradParts P, float* __restrict__ p, float* __restrict__ m,
+                                                           float* __restrict__ v, float lr, float b1c, float b2c,
+                                                           short* __restrict__ W1f, short* __restrict__ W2f,
+                                                           short* __restrict__ W2Tf, float* loss) {
     const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-    for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-        const float gi = g[i];
-        const float mi = beta1 * m[i] + (1.f - beta1) * gi;
-        const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        p[i] -= lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
-        g[i] = 0.f;
-    }
-}
-
-/* Regression target t = sign(d) log(1 + |d|) of exact int64 deltas. */
-__global__ void k_mlp_targets(const int64_t* __restrict__ d, int64_t k, float* __restrict__ t) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < k; i += (int64_t)gridDim.x * blockDim.x) {
-        const double x = (double)d[i];
-        t[i] = (float)(x < 0 ? -log1p(-x) : log1p(x));
-    }
+    int i;
+    const float gi = grad_sum(P, &i);
+    if (i == kParams) *loss = gi;
+    if (i < 0 || i >= kParams) return;
+    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
+    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float x = p[i] - lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
+    p[i] = x;
+    pack_param(W1f, W2f, W2Tf, i, x);
 }
 
 __global__ void k_iota(int32_t* __restrict__ p, int64_t k) {
@@ -879,12 +1002,8 @@ hipError_t bm_launch_vertex_features(const BmDevGraph& g, const int4* chunks, in
 }
 
 hipError_t bm_launch_mlp_pack(const BmMlpDev& d, hipStream_t s) {
-    hipLaunchKernelGGL(k_mlp_pack, dim3(2), dim3(256), 0, s, d.params + kOffW1, kF, kH, 0, 16,
-                       static_cast<short*>(d.W1f));
-    hipLaunchKernelGGL(k_mlp_pack, dim3(8), dim3(256), 0, s, d.params + kOffW2, kH, kH, 0, 32,
-                       static_cast<short*>(d.W2f));
-    hipLaunchKernelGGL(k_mlp_pack, dim3(8), dim3(256), 0, s, d.params + kOffW2, kH, kH, 1, 32,
-                       static_cast<short*>(d.W2Tf));
+    hipLaunchKernelGGL(k_mlp_pack, dim3(grid_of(kParams, 256)), dim3(256), 0, s, d.params, static_cast<short*>(d.W1f),
+                       static_cast<short*>(d.W2f), static_cast<short*>(d.W2Tf));
     return hipGetLastError();
 }
 
@@ -911,48 +1030,78 @@ hipError_t bm_launch_mlp_forward(const BmMlpDev& d, const float* vf, const int2*
     return launch_forward<false>(d, vf, list, seed, n, k, score, nullptr, num_cus, s);
 }
 
-size_t bm_mlp_train_bytes(int64_t k) { return (size_t)((k + 31) / 32 * 32) * (kF + 3 * kH) * sizeof(short); }
+/* Scratch of one batch: the four activation arrays, then the partials.  The
+ * rows are padded by 64 entries, so that the 16 rows a fragment reads do not
+ * start a multiple of 4 KB apart. */
+constexpr int kMaxSlices = 32, kMaxTrainBlocks = 1024;
+static int64_t train_stride(int64_t k) { return (k + 31) / 32 * 32 + 64; }
+
+size_t bm_mlp_train_bytes(int64_t k) {
+    return (size_t)train_stride(k) * (kF + 3 * kH) * sizeof(short) +
+           ((size_t)kMaxSlices * kWParams + (size_t)kBParams * kMaxTrainBlocks) * sizeof(float);
+}
+
+static int train_blocks(int64_t B, int32_t num_cus) {
+    int64_t blocks = (B / 16 + kTrainWaves - 1) / kTrainWaves;
+    int64_t cap = num_cus > 0 ? num_cus : 256;
+    if (cap > kMaxTrainBlocks) cap = kMaxTrainBlocks;
+    return (int)(blocks < cap ? blocks : cap);
+}
+
+/* a wave takes at least four 32-pair steps; 32 slices give 320 blocks */
+static int train_slices(int64_t B) {
+    const int64_t s = B / 32 / 16;
+    return (int)(s < 1 ? 1 : (s > kMaxSlices ? kMaxSlices : s));
+}
+
+static GradParts grad_parts(void* act, int64_t k, int32_t num_cus) {
+    const int64_t B = (k + 31) / 32 * 32;
+    GradParts P;
+    P.w = reinterpret_cast<const float*>(reinterpret_cast<const short*>(act) + (size_t)train_stride(k) * (kF + 3 * kH));
+    P.b = P.w + (size_t)kMaxSlices * kWParams;
+    P.slices = train_slices(B);
+    P.blocks = train_blocks(B, num_cus);
+    return P;
+}
 
 hipError_t bm_launch_mlp_gradient(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
-                                  int64_t k, const float* target, void* act, float* loss, int32_t num_cus,
+                                  int64_t k, const float* target, const int64_t* delta, void* act, int32_t num_cus,
                                   hipStream_t s) {
     if (k <= 0) return hipSuccess;
+    const GradParts P = grad_parts(act, k, num_cus);
     TrainBuf T;
     T.B = (k + 31) / 32 * 32;
+    T.ld = train_stride(k);
     T.XT = reinterpret_cast<short*>(act);
-    T.H1T = T.XT + (size_t)kF * T.B;
-    T.G1T = T.H1T + (size_t)kH * T.B;
-    T.G2T = T.G1T + (size_t)kH * T.B;
-    T.grad = d.grad;
-    T.loss = loss;
+    T.H1T = T.XT + (size_t)kF * T.ld;
+    T.G1T = T.H1T + (size_t)kH * T.ld;
+    T.G2T = T.G1T + (size_t)kH * T.ld;
+    T.wpart = const_cast<float*>(P.w);
+    T.bpart = const_cast<float*>(P.b);
+    T.target = target;
+    T.delta = delta;
     PairSrc ps{list, seed, n};
-    const int64_t tiles = T.B / 16;
-    int64_t blocks = (tiles + kFwdWaves - 1) / kFwdWaves;
-    const int64_t cap = (int64_t)(num_cus > 0 ? num_cus : 256) * 2;
-    if (blocks > cap) blocks = cap;
     hipError_t e = hipFuncSetAttribute((const void*)k_mlp_train_act, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)sizeof(TrainShared));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_train_act, dim3((unsigned)blocks), dim3(kFwdThreads), sizeof(TrainShared), s,
-                       reinterpret_cast<const float4*>(vf), ps, k, target, mlpdev(d), T);
-    int32_t slices = (int32_t)(tiles / 128);
-    if (slices < 1) slices = 1;
-    if (slices > 64) slices = 64;
-    const int64_t items = (int64_t)kWgTiles * slices;
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3((unsigned)grid_of(items, 4)), dim3(256), 0, s, T, slices);
+    hipLaunchKernelGGL(k_mlp_train_act, dim3((unsigned)P.blocks), dim3(kTrainThreads), sizeof(TrainShared), s,
+                       reinterpret_cast<const float4*>(vf), ps, k, mlpdev(d), T);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3((unsigned)(kWgItems * P.slices)), dim3(256), 0, s, T, P.slices);
     return hipGetLastError();
 }
 
-hipError_t bm_launch_mlp_adam(const BmMlpDev& d, float lr, int64_t step, hipStream_t s) {
-    const float b1c = 1.f - powf(0.9f, (float)step), b2c = 1.f - powf(0.999f, (float)step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3(grid_of(kParams, 256)), dim3(256), 0, s, d.params, d.grad, d.adam_m,
-                       d.adam_v, kParams, lr, b1c, b2c);
-    return bm_launch_mlp_pack(d, s);
+hipError_t bm_launch_mlp_reduce(const BmMlpDev& d, void* act, int64_t k, float* loss, int32_t num_cus, hipStream_t s) {
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(kGradWBlocks + kGradBBlocks), dim3(kGradThreads), 0, s,
+                       grad_parts(act, k, num_cus), d.grad, loss);
+    return hipGetLastError();
 }
 
-hipError_t bm_launch_mlp_targets(const int64_t* delta, int64_t k, float* t, hipStream_t s) {
-    if (k <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_mlp_targets, dim3(grid_of(k, 256)), dim3(256), 0, s, delta, k, t);
+hipError_t bm_launch_mlp_adam(const BmMlpDev& d, float lr, int64_t step, void* act, int64_t k, float* loss,
+                              int32_t num_cus, hipStream_t s) {
+    const float b1c = 1.f - powf(0.9f, (float)step), b2c = 1.f - powf(0.999f, (float)step);
+    hipLaunchKernelGGL(k_mlp_adam, dim3(kGradWBlocks + kGradBBlocks), dim3(kGradThreads), 0, s,
+                       grad_parts(act, k, num_cus), d.params, d.adam_m, d.adam_v, lr, b1c, b2c,
+                       static_cast<short*>(d.W1f), static_cast<short*>(d.W2f), static_cast<short*>(d.W2Tf), loss);
     return hipGetLastError();
 }
 
