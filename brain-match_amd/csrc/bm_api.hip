@@ -56,6 +56,7 @@ struct bm_ctx {
     int32_t row_layout;     /* BM_ROWS_P19 when female weights are in 0..8191, else BM_ROWS_P15 (compact graphs) */
     int32_t* d_pi;          /* matching, then its inverse (n+1 each) */
     int64_t* d_small;       /* 16 int64 of scratch for scores / flags */
+    int64_t* h_pin;         /* 16 pinned int64 that kernels write results to (read after a stream sync) */
     int32_t* d_reorder;     /* n ints for the changed-first enumerations */
     BmLaunch tune[BM_KERNEL_COUNT];
     int32_t user_tuned[BM_KERNEL_COUNT];   /* bm_set_tuning was called: no batch-size choice */
@@ -265,6 +266,7 @@ static void free_ctx(bm_ctx* c) {
     (void)hipFree(c->d_chunks);
     (void)hipFree(c->d_diag);
     (void)hipFree(c->d_small);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
     (void)hipFree(c->d_reorder);
     if (c->pending) {
         for (KTiming& t : *c->pending) {
@@ -602,6 +604,8 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = h2d(c, c->d_f_out, fg.out.adj, (size_t)fg.m);
     if (rc == BM_OK) rc = h2d(c, c->d_f_in_ptr, fg.in.ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = h2d(c, c->d_f_in, fg.in.adj, (size_t)fg.m);
+    if (rc == BM_OK && hipHostMalloc((void**)&c->h_pin, 16 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
+        rc = fail(c, BM_ERR_NOMEM, "hipHostMalloc failed");
     c->packed = c->compact && c->male_nonneg;
     if (rc == BM_OK) rc = build_rowtab(c, 0, fg.out.ptr, c->d_f_out_ptr, c->d_f_out);
     if (rc == BM_OK) rc = build_rowtab(c, 1, fg.in.ptr, c->d_f_in_ptr, c->d_f_in);
@@ -1237,15 +1241,14 @@ static int accept_impl(bm_batch* b, int64_t max_accept, int32_t* accepted, int64
         if (rc != BM_OK) return rc;
     }
     HIPCHK(c, bm_launch_accept(devgraph(c), c->d_pi, c->d_pi + c->n + 1, (const int2*)b->d_cand, b->d_delta, b->k, max_accept,
-                               b->d_acc_scratch, b->acc_scratch_bytes, b->d_acc_idx, b->d_out,
+                               b->d_acc_scratch, b->acc_scratch_bytes, b->d_acc_idx, b->d_out, c->h_pin,
                                c->gain_on ? c->d_moves : nullptr, c->stream));
     if (c->gain_on && b->k > 0) {
         int rc = gain_patch(c, b->d_out + 2, 2 * b->k, false);
         if (rc != BM_OK) return rc;
     }
-    int64_t meta[2];
-    HIPCHK(c, hipMemcpyAsync(meta, b->d_out, sizeof meta, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const int64_t meta[2] = {c->h_pin[0], c->h_pin[1]};
     if (accepted && meta[0] > 0) {
         std::vector<int64_t> idx((size_t)meta[0]);
         HIPCHK(c, hipMemcpy(idx.data(), b->d_acc_idx, (size_t)meta[0] * sizeof(int64_t), hipMemcpyDeviceToHost));

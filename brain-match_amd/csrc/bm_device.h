@@ -281,7 +281,7 @@ size_t bm_accept_scratch_bytes(int64_t k);
 hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, int32_t* inv_rw, const int2* cand, const int64_t* d,
                             int64_t k, int64_t max_accept, void* scratch, size_t scratch_bytes,
                             int64_t* out_acc_idx /* k */, int64_t* out_meta /* [n_acc, gain, n_moves] */,
-                            int4* out_moves /* 2k {x, old, new, 0}, may be NULL */, hipStream_t s);
+                            int64_t* host_meta /* pinned, [n_acc, gain] */, int4* out_moves /* 2k {x, old, new, 0}, may be NULL */, hipStream_t s);
 
 /* 2-hop proposals (bm_twohop.hip).  K > 0: pairs[a*K + j] for anchor a
  * (anchors[a], or drawn from `seed` when anchors is NULL); K == 0: the whole

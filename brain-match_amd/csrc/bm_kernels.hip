@@ -305,76 +305,184 @@ __global__ void k_gather_keys(const int64_t* __restrict__ d, const int64_t* __re
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) keys[i] = d[idx[i]];
 }
 
-constexpr int kAccThreads = 1024;
+/* Order of a small batch's positive candidates: (delta desc, index asc), by
+ * counting.  Every block holds all k deltas in LDS; 16 lanes per candidate
+ * count the ones before it.  One launch and no host round trip, where
+ * compaction, gather and radix sort take seven launches with the count read
+ * back in between (4,096 candidates: 8 us against 30 us of kernels and the gaps). */
+constexpr int kOrderMax = 8192, kOrderThreads = 256, kOrderLanes = 16, kOrderKeys = kOrderThreads / kOrderLanes;
+
+__global__ void __launch_bounds__(kOrderThreads) k_accept_order(const int64_t* __restrict__ d, int32_t k,
+                                                                int64_t* __restrict__ order,
+                                                                int64_t* __restrict__ npos) {
+    extern __shared__ longlong2 sd[];
+    const int32_t words = (k + 2 * kOrderLanes - 1) / (2 * kOrderLanes) * kOrderLanes;
+    int32_t pos = 0;
+    const longlong2* dv = reinterpret_cast<const longlong2*>(d);
+    for (int32_t b = 0; b < words; b += 8 * kOrderThreads) {   /* eight loads in flight */
+        longlong2 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int32_t i = b + j * kOrderThreads + threadIdx.x;
+            x[j] = make_longlong2(0, 0);
+            if (2 * i + 1 < k) x[j] = dv[i];
+            else if (2 * i < k) x[j].x = d[2 * i];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int32_t i = b + j * kOrderThreads + threadIdx.x;
+            if (i < words) sd[i] = x[j];
+            pos += (x[j].x > 0) + (x[j].y > 0);
+        }
+    }
+    __shared__ int32_t s_pos;
+    if (threadIdx.x == 0) s_pos = 0;
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        if (pos) atomicAdd(&s_pos, pos);
+        __syncthreads();
+        if (threadIdx.x == 0) *npos = s_pos;
+    }
+    const int32_t i = blockIdx.x * kOrderKeys + threadIdx.x / kOrderLanes, part = threadIdx.x % kOrderLanes;
+    const int64_t me = i < k ? reinterpret_cast<const int64_t*>(sd)[i] : 0;
+    if (!__ballot(me > 0)) return;
+    int32_t rank = 0;
+#pragma unroll 8
+    for (int32_t q = part; q < words; q += kOrderLanes) {
+        const longlong2 x = sd[q];   /* an equal delta counts when its index is smaller */
+        rank += x.x > (2 * q < i ? me - 1 : me) ? 1 : 0;
+        rank += x.y > (2 * q + 1 < i ? me - 1 : me) ? 1 : 0;
+    }
+#pragma unroll
+    for (int o = 1; o < kOrderLanes; o <<= 1) rank += __shfl_xor(rank, o, BM_WAVE);
+    if (part == 0 && me > 0) order[rank] = i;
+}
+
+constexpr int kAccThreads = 1024, kAccWaves = kAccThreads / BM_WAVE;
+constexpr int kAccBatch = 16;   /* free candidates decided together */
 
 /* Sequential greedy in priority order, one block.  lock[] is a bitmap of
- * vertices in the closed neighbourhood of accepted swaps (LDS, n+1 bits). */
+ * vertices in the closed neighbourhood of accepted swaps (LDS, n+1 bits).
+ * The candidates are taken 1,024 at a time, one per thread.  A round takes
+ * the first 16 of them whose endpoints are unlocked; whether one's acceptance
+ * would lock another follows from row-table lookups among their endpoints
+ * (120 pairs x 8 lookups, one per thread), one thread decides the 16 in
+ * order, and each wave locks the neighbourhoods of one accepted swap.  That is
+ * the decision of the one-at-a-time loop: a later candidate of the 16 is
+ * rejected exactly when an earlier accepted one locks an endpoint.  One
+ * candidate per round (five barriers and a list walk each) took 150 us, this
+ * 55 us, for
+ * the 50 swaps of an early climb round at n = 18,524. */
+template <bool PACKED>
 __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int32_t* __restrict__ pi,
                                                                int32_t* __restrict__ inv,
                                                                const int2* __restrict__ cand,
                                                                const int64_t* __restrict__ d,
-                                                               const int64_t* __restrict__ order, int64_t npos,
-                                                               int64_t max_accept, int64_t* __restrict__ acc_idx,
-                                                               int64_t* __restrict__ meta, int4* __restrict__ moves) {
+                                                               const int64_t* __restrict__ order,
+                                                               const int64_t* __restrict__ npos_at, int64_t max_accept,
+                                                               int64_t* __restrict__ acc_idx,
+                                                               int64_t* __restrict__ meta, int64_t* __restrict__ host,
+                                                               int4* __restrict__ moves) {
     extern __shared__ uint32_t lock[];
-    __shared__ int s_first;
-    __shared__ int32_t s_u, s_v;
+    __shared__ int32_t s_cnt[kAccWaves];
+    __shared__ int2 s_end[kAccBatch];        /* endpoints of the round's candidates */
+    __shared__ int64_t s_ci[kAccBatch], s_d[kAccBatch];
+    __shared__ uint32_t s_conf[kAccBatch];   /* earlier candidates of the round that would lock it */
+    __shared__ uint32_t s_acc;               /* accepted candidates of the round */
+    __shared__ int32_t s_last;               /* thread of the round's last candidate */
     __shared__ int64_t s_nacc, s_gain;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & (BM_WAVE - 1), wave = t / BM_WAVE;
+    const int64_t npos = *npos_at;
     const int words = (g.n + 32) / 32;
     for (int i = t; i < words; i += kAccThreads) lock[i] = 0;
     if (t == 0) { s_nacc = 0; s_gain = 0; }
+    /* this thread's lookup in a round: candidates qi < qj, endpoints and direction */
+    int qi = -1, qj = -1;
+    if (t < kAccBatch * (kAccBatch - 1) / 2 * 8) {
+        const int pr = t >> 3;
+        qj = 1;
+        while (qj * (qj + 1) / 2 <= pr) qj++;
+        qi = pr - qj * (qj - 1) / 2;
+    }
     __syncthreads();
     for (int64_t base = 0; base < npos; base += kAccThreads) {
-        if (s_nacc >= max_accept) break;
         const int64_t i = base + t;
         const bool valid = i < npos;
-        int64_t ci = -1;
+        int64_t ci = -1, di = 0;
         int32_t u = 0, v = 0;
         if (valid) {
             ci = order[i];
             const int2 p = cand[ci];
+            di = d[ci];
             u = p.x;
             v = p.y;
         }
         int start = 0;
         for (;;) {
-            if (t == 0) s_first = kAccThreads;
-            __syncthreads();
+            if (s_nacc >= max_accept) break;
             const bool free_ = valid && t >= start && u != v && !((lock[u >> 5] >> (u & 31)) & 1u) &&
                                !((lock[v >> 5] >> (v & 31)) & 1u);
-            if (free_) atomicMin(&s_first, t);
+            const uint64_t m = __ballot(free_);
+            if (lane == 0) s_cnt[wave] = __popcll(m);
+            if (t < kAccBatch) s_conf[t] = 0;
             __syncthreads();
-            const int first = s_first;
-            if (first >= kAccThreads) break;
-            if (t == first) {
-                acc_idx[s_nacc] = ci;
-                s_nacc += 1;
-                s_gain += d[ci];
-                s_u = u;
-                s_v = v;
+            int before = 0, total = 0;
+#pragma unroll
+            for (int w = 0; w < kAccWaves; w++) {
+                const int c = s_cnt[w];
+                before += w < wave ? c : 0;
+                total += c;
+            }
+            if (total == 0) break;
+            const int q = before + __popcll(m & ((1ull << lane) - 1ull));
+            if (free_ && q < kAccBatch) {
+                s_end[q] = make_int2(u, v);
+                s_ci[q] = ci;
+                s_d[q] = di;
+                if (q == kAccBatch - 1 || q == total - 1) s_last = t;
             }
             __syncthreads();
-            const int32_t au = s_u, av = s_v;
+            const int cnt = total < kAccBatch ? total : kAccBatch;
+            if (qj >= 0 && qj < cnt) {
+                const int2 a = s_end[qi], b = s_end[qj];
+                const int32_t x = (t & 1) ? a.y : a.x, y = (t & 2) ? b.y : b.x;
+                const int32_t row = (t & 4) ? y : x, key = (t & 4) ? x : y;
+                if (x == y || row_find<PACKED>(g.m_out_t.tab, g.m_out_t.desc[row], key) != BM_ABSENT)
+                    atomicOr(&s_conf[qj], 1u << qi);
+            }
+            __syncthreads();
             if (t == 0) {
-                atomicOr(&lock[au >> 5], 1u << (au & 31));
-                atomicOr(&lock[av >> 5], 1u << (av & 31));
-            }
-            const int32_t ends[2] = {au, av};
-            for (int q = 0; q < 2; q++) {
-                const int32_t x = ends[q];
-                for (int64_t e = g.m_out_ptr[x] + t; e < g.m_out_ptr[x + 1]; e += kAccThreads) {
-                    const int32_t y = g.m_out[e].x;
-                    atomicOr(&lock[y >> 5], 1u << (y & 31));
-                }
-                for (int64_t e = g.m_in_ptr[x] + t; e < g.m_in_ptr[x + 1]; e += kAccThreads) {
-                    const int32_t y = g.m_in[e].x;
-                    atomicOr(&lock[y >> 5], 1u << (y & 31));
-                }
+                uint32_t acc = 0;
+                int64_t nacc = s_nacc, gain = s_gain;
+                for (int z = 0; z < cnt && nacc < max_accept; z++)
+                    if (!(s_conf[z] & acc)) {
+                        acc |= 1u << z;
+                        acc_idx[nacc++] = s_ci[z];
+                        gain += s_d[z];
+                    }
+                s_acc = acc;
+                s_nacc = nacc;
+                s_gain = gain;
             }
             __syncthreads();
-            start = first + 1;
-            if (s_nacc >= max_accept) break;
+            static_assert(kAccBatch == kAccWaves, "one wave per candidate of a round");
+            if ((s_acc >> wave) & 1u) {
+                const int2 e = s_end[wave];
+#pragma unroll
+                for (int z = 0; z < 4; z++) {
+                    const int32_t x = (z & 1) ? e.y : e.x;
+                    const int64_t* ptr = (z & 2) ? g.m_in_ptr : g.m_out_ptr;
+                    const int2* adj = (z & 2) ? g.m_in : g.m_out;
+                    const int64_t b0 = ptr[x], b1 = ptr[x + 1];
+                    for (int64_t o = b0 + lane; o < b1; o += BM_WAVE) {
+                        const int32_t y = adj[o].x;
+                        atomicOr(&lock[y >> 5], 1u << (y & 31));
+                    }
+                    if (z < 2 && lane == 0) atomicOr(&lock[x >> 5], 1u << (x & 31));
+                }
+            }
+            start = s_last + 1;
+            __syncthreads();
         }
         __syncthreads();
     }
@@ -392,7 +500,10 @@ __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int
         if (fv) inv[fv] = p.x;
         if (fu) inv[fu] = p.y;
     }
-    if (t == 0) { meta[0] = nacc; meta[1] = s_gain; meta[2] = 2 * nacc; }
+    if (t == 0) {
+        meta[0] = nacc; meta[1] = s_gain; meta[2] = 2 * nacc;
+        host[0] = nacc; host[1] = s_gain;
+    }
 }
 
 __global__ void k_apply_swap(int32_t* pi, int32_t* inv, int32_t u, int32_t v) {
@@ -613,49 +724,60 @@ size_t bm_accept_scratch_bytes(int64_t k) {
     return (size_t)k * 4 * sizeof(int64_t) + 256 + cub_temp_bytes(k) + 256;
 }
 
-hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, int32_t* inv_rw, const int2* cand, const int64_t* d, int64_t k,
-                            int64_t max_accept, void* scratch, size_t scratch_bytes, int64_t* out_acc_idx,
-                            int64_t* out_meta, int4* out_moves, hipStream_t s) {
-    if (k <= 0) {
-        hipError_t e = hipMemsetAsync(out_meta, 0, 3 * sizeof(int64_t), s);
-        return e;
-    }
+hipError_t bm_launch_accept(const BmDevGraph& g, int32_t* pi_rw, int32_t* inv_rw, const int2* cand, const int64_t* d,
+                            int64_t k, int64_t max_accept, void* scratch, size_t scratch_bytes, int64_t* out_acc_idx,
+                            int64_t* out_meta, int64_t* host_meta, int4* out_moves, hipStream_t s) {
     char* p = (char*)scratch;
     int64_t* idx = (int64_t*)p;
     int64_t* keys = idx + k;
     int64_t* skeys = keys + k;
     int64_t* sidx = skeys + k;
     int64_t* cnt = sidx + k;
-    char* temp = (char*)(cnt) + 256;
-    size_t temp_bytes = scratch_bytes - ((size_t)(temp - p));
-    hipcub::CountingInputIterator<int64_t> it(0);
-    PosDelta pred{d};
-    size_t tb = temp_bytes;
-    hipError_t e = hipcub::DeviceSelect::If(temp, tb, it, idx, cnt, (int)k, pred, s);
-    if (e != hipSuccess) return e;
-    int64_t npos = 0;
-    e = hipMemcpyAsync(&npos, cnt, sizeof(int64_t), hipMemcpyDeviceToHost, s);
-    if (e != hipSuccess) return e;
-    e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    if (npos > 0) {
-        size_t need = 0;
-        e = hipcub::DeviceRadixSort::SortPairsDescending(nullptr, need, (const int64_t*)nullptr, (int64_t*)nullptr,
-                                                         (const int64_t*)nullptr, (int64_t*)nullptr, (int)npos, 0,
-                                                         64, s);
+    hipError_t e;
+    if (k <= kOrderMax) {
+        const size_t lds = (size_t)((k + 2 * kOrderLanes - 1) / (2 * kOrderLanes) * kOrderLanes) * sizeof(longlong2);
+        if (lds > 48 * 1024) {
+            e = set_lds((const void*)k_accept_order, lds);
+            if (e != hipSuccess) return e;
+        }
+        int64_t blocks = (k + kOrderKeys - 1) / kOrderKeys;
+        if (blocks < 1) blocks = 1;
+        hipLaunchKernelGGL(k_accept_order, dim3((unsigned)blocks), dim3(kOrderThreads), lds, s, d, (int32_t)k, sidx, cnt);
+    } else {
+        char* temp = (char*)(cnt) + 256;
+        const size_t temp_bytes = scratch_bytes - ((size_t)(temp - p));
+        hipcub::CountingInputIterator<int64_t> it(0);
+        PosDelta pred{d};
+        size_t tb = temp_bytes;
+        e = hipcub::DeviceSelect::If(temp, tb, it, idx, cnt, (int)k, pred, s);
         if (e != hipSuccess) return e;
-        if (need > temp_bytes) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_gather_keys, dim3(grid_for(npos, 256)), dim3(256), 0, s, d, idx, npos, keys);
-        tb = temp_bytes;
-        e = hipcub::DeviceRadixSort::SortPairsDescending(temp, tb, keys, skeys, idx, sidx, (int)npos, 0, 64, s);
+        int64_t npos = 0;
+        e = hipMemcpyAsync(&npos, cnt, sizeof(int64_t), hipMemcpyDeviceToHost, s);
         if (e != hipSuccess) return e;
+        e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+        if (npos > 0) {
+            size_t need = 0;
+            e = hipcub::DeviceRadixSort::SortPairsDescending(nullptr, need, (const int64_t*)nullptr, (int64_t*)nullptr,
+                                                             (const int64_t*)nullptr, (int64_t*)nullptr, (int)npos, 0,
+                                                             64, s);
+            if (e != hipSuccess) return e;
+            if (need > temp_bytes) return hipErrorInvalidValue;
+            hipLaunchKernelGGL(k_gather_keys, dim3(grid_for(npos, 256)), dim3(256), 0, s, d, idx, npos, keys);
+            tb = temp_bytes;
+            e = hipcub::DeviceRadixSort::SortPairsDescending(temp, tb, keys, skeys, idx, sidx, (int)npos, 0, 64, s);
+            if (e != hipSuccess) return e;
+        }
     }
     const size_t lds = (size_t)((g.n + 32) / 32) * sizeof(uint32_t);
-    e = set_lds((const void*)k_accept_greedy, lds);
-    if (e != hipSuccess) return e;
+    auto greedy = g.packed ? k_accept_greedy<true> : k_accept_greedy<false>;
+    if (lds > 48 * 1024) {
+        e = set_lds((const void*)greedy, lds);
+        if (e != hipSuccess) return e;
+    }
     if (max_accept <= 0) max_accept = INT64_MAX;
-    hipLaunchKernelGGL(k_accept_greedy, dim3(1), dim3(kAccThreads), lds, s, g, pi_rw, inv_rw, cand, d, sidx, npos,
-                       max_accept, out_acc_idx, out_meta, out_moves);
+    hipLaunchKernelGGL(greedy, dim3(1), dim3(kAccThreads), lds, s, g, pi_rw, inv_rw, cand, d, sidx, cnt, max_accept,
+                       out_acc_idx, out_meta, host_meta, out_moves);
     return hipGetLastError();
 }
 
