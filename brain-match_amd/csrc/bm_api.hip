@@ -455,12 +455,30 @@ static int build_chunks(bm_ctx* c) {
     return BM_OK;
 }
 
+/* The per-vertex contributions for a batch of k candidates, or NULL.  One
+ * pass over the male lists is 2m lookups and two launches, and saves every
+ * candidate the walk of its two vertices' own lists, 4m/n lookups on average;
+ * the launches are worth about 6e5 lookups.  4M edges, n = 18,524: from
+ * 10,000 candidates on (12,000: 211 us without the pass; 13,000: 167 us with
+ * it); 40,000 edges, n = 2,000: from 8,500 (16,384: 54 us without, 28 us
+ * with; 4,096: 20 us either way). */
+static int scan_diag(bm_ctx* c, int64_t k, const int64_t** diag) {
+    *diag = nullptr;
+    const double m = (double)c->male.m;
+    if ((double)k * (4.0 * m / c->n) < 2.0 * m + 6e5) return BM_OK;
+    HIPCHK(c, bm_launch_diag(devgraph(c), c->d_chunks, c->n_chunks, c->d_diag, c->num_cus, c->stream));
+    *diag = c->d_diag;
+    return BM_OK;
+}
+
 /* Launch shape of the scan kernels for a batch of k candidates.  Unless the
  * caller set one (bm_set_tuning), a batch too small to fill the device's wave
- * slots (k < 32,768: at most four candidates per slot) runs in 4-wave blocks
- * with 8 list entries per lane -- there the slowest candidate's latency sets
- * the time (a climb round of 4,096 pairs: 1.0 vs 1.15 ms) -- and a larger
- * one in the default throughput shape. */
+ * slots (k < 32,768: at most four candidates per slot) is bound by its longest
+ * lists, so the swap kernel gives each candidate the four waves of a block
+ * (n = 18,524: 4,096 pairs 111 us against 255 us with one wave each, 32,768
+ * pairs 314 against 353 us, 65,536 pairs 527 against 476 us), the 3-vertex
+ * kernel 4-wave blocks with more list entries per lane; a larger one runs in
+ * the default throughput shape. */
 static BmLaunch scan_launch(const bm_ctx* c, int kernel, int64_t k);
 
 static void default_tuning(bm_ctx* c) {
@@ -469,12 +487,12 @@ static void default_tuning(bm_ctx* c) {
     const int s = c->compact ? 1280 : 640;
     /* swap and 3-vertex kernels: the shape for large batches (see
      * scan_launch for small ones) -- 8-wave blocks, 2 list entries per lane:
-     * occupancy over per-lane depth, 7.1e7 vs 4.9e7 pairs/s (4-wave blocks, 8
-     * entries) at n = 18,524; 148.8 vs 156.1 ms per 2^22 triples */
-    c->tune[BM_KERNEL_SWAP] = BmLaunch{8, s, 8, cus, 2};
-    c->tune[BM_KERNEL_ROT3] = BmLaunch{8, 2 * s, 8, cus, 2};
-    c->tune[BM_KERNEL_SCORE] = BmLaunch{4, s, 8, cus, 8};
-    c->tune[BM_KERNEL_GAIN_BUILD] = BmLaunch{4, s, 8, cus, 4};   /* only unroll is used */
+     * occupancy over per-lane depth (2^20 pairs at n = 18,524: 4.5 against
+     * 4.8 ms with 4 entries; 2^22 triples 148.8 against 156.1 ms) */
+    c->tune[BM_KERNEL_SWAP] = BmLaunch{8, s, 8, cus, 2, 0};
+    c->tune[BM_KERNEL_ROT3] = BmLaunch{8, 2 * s, 8, cus, 2, 0};
+    c->tune[BM_KERNEL_SCORE] = BmLaunch{4, s, 8, cus, 8, 0};
+    c->tune[BM_KERNEL_GAIN_BUILD] = BmLaunch{4, s, 8, cus, 4, 0};   /* only unroll is used */
     for (int i = 0; i < BM_KERNEL_COUNT; i++) {
         c->group_lanes[i] = 64;
         c->user_tuned[i] = 0;
@@ -488,6 +506,7 @@ static BmLaunch scan_launch(const bm_ctx* c, int kernel, int64_t k) {
     L.lds_slots = c->compact ? 1280 : 640;
     L.blocks_per_cu = 8;
     L.unroll = kernel == BM_KERNEL_ROT3 ? 4 : 8;
+    L.coop = kernel == BM_KERNEL_SWAP;
     return L;
 }
 
@@ -952,8 +971,14 @@ extern "C" int bm_batch_eval_swaps(bm_batch* b) {
                                       b->d_delta, pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_SWAP, &t);
+        const int64_t* diag = nullptr;
+        const int rc = scan_diag(c, b->k, &diag);
+        if (rc != BM_OK) {
+            timing_end(c, &t);
+            return rc;
+        }
         HIPCHK(c, bm_launch_swap(devgraph(c), scan_launch(c, BM_KERNEL_SWAP, b->k), BM_CAND_LIST, (const int2*)b->d_cand, nullptr, 0, b->k,
-                                 b->d_delta, c->stream));
+                                 b->d_delta, diag, c->stream));
     }
     timing_end(c, &t);
     b->evaluated = 1;
@@ -978,8 +1003,14 @@ extern "C" int bm_batch_eval_swaps_uniform(bm_batch* b, uint64_t seed, int64_t k
                                       pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_SWAP, &t);
+        const int64_t* diag = nullptr;
+        const int rc = scan_diag(c, k, &diag);
+        if (rc != BM_OK) {
+            timing_end(c, &t);
+            return rc;
+        }
         HIPCHK(c, bm_launch_swap(devgraph(c), scan_launch(c, BM_KERNEL_SWAP, k), BM_CAND_UNIFORM, nullptr, nullptr, seed, k, b->d_delta,
-                                 c->stream));
+                                 diag, c->stream));
     }
     timing_end(c, &t);
     b->k = k;
@@ -1071,8 +1102,13 @@ extern "C" int bm_batch_eval_swaps_umajor(bm_batch* b, uint64_t seed, int64_t k)
         }
     } else {
         timing_begin(c, BM_KERNEL_SWAP, &t);
+        const int64_t* diag = nullptr;
+        if ((rc = scan_diag(c, k, &diag)) != BM_OK) {
+            timing_end(c, &t);
+            return rc;
+        }
         HIPCHK(c, bm_launch_swap(devgraph(c), scan_launch(c, BM_KERNEL_SWAP, k), BM_CAND_UMAJOR, nullptr, c->d_um_off, seed, k,
-                                 b->d_delta, c->stream));
+                                 b->d_delta, diag, c->stream));
     }
     timing_end(c, &t);
     b->k = k;
@@ -1779,7 +1815,7 @@ extern "C" int bm_set_tuning(bm_ctx* c, int32_t kernel, const bm_tuning* t) {
     } else if (t->unroll != 2 && t->unroll != 4 && t->unroll != 8) {
         return fail(c, BM_ERR_ARG, "bm_set_tuning: unroll must be 2, 4 or 8");
     }
-    c->tune[kernel] = BmLaunch{w, t->lds_slots, t->blocks_per_cu, cus, t->unroll};
+    c->tune[kernel] = BmLaunch{w, t->lds_slots, t->blocks_per_cu, cus, t->unroll, 0};
     c->group_lanes[kernel] = t->group_lanes;
     c->user_tuned[kernel] = 1;
     return BM_OK;

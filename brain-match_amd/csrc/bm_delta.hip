@@ -456,18 +456,160 @@ __device__ __forceinline__ int64_t swap_delta_wave(const BmDevGraph& g, int32_t 
     return wave_sum64(acc);
 }
 
-template <int MODE, bool COMPACT, int U>
-__global__ void __launch_bounds__(512) k_swap(BmDevGraph g, const int2* __restrict__ cand,
-                                             const int64_t* __restrict__ off, uint64_t seed, int64_t k,
-                                             int64_t* __restrict__ delta, uint32_t cap) {
-    typedef typename Slot<COMPACT>::T S;
-    extern __shared__ uint4 smem[];
+/* ---- list intersections -------------------------------------------- */
+
+/* One term of a delta: the edges of one list of a male vertex x (out or in)
+ * that land on edges of the matching row of a female f.  The wave walks the
+ * shorter of the two (the male list, mapped by pi, or the female row, mapped
+ * by the inverse matching) and looks each mapped id up in the other's row
+ * table, so a hub placed on an ordinary female costs the female's degree. */
+struct alignas(16) ScanList {
+    const int2* rows;    /* entries walked */
+    const uint4* tab;    /* buckets of the row probed */
+    uint32_t meta;       /* log2 buckets | kSideF | kIn | kNew */
+    int32_t start;       /* first position in the wave's index space */
+    int32_t pad[2];
+};
+constexpr uint32_t kSideF = 64u, kIn = 128u, kNew = 256u;
+
+/* List of (male x, female f, direction) into t; returns its length. */
+__device__ __forceinline__ int32_t scan_list(const BmDevGraph& g, int32_t x, int32_t f, bool in, ScanList& t) {
+    const int64_t* mp = in ? g.m_in_ptr : g.m_out_ptr;
+    const int64_t* fp = in ? g.f_in_ptr : g.f_out_ptr;
+    const int64_t m0 = mp[x], m1 = mp[x + 1], a0 = fp[f], a1 = fp[f + 1];
+    const uint64_t md = (in ? g.m_in_t.desc : g.m_out_t.desc)[x];
+    const uint64_t fd = (in ? g.f_in_t.desc : g.f_out_t.desc)[f];
+    const int32_t dm = (int32_t)(m1 - m0), df = (int32_t)(a1 - a0);
+    const bool side = g.inv != nullptr && df < dm;
+    const uint64_t d = side ? md : fd;
+    t.rows = side ? (in ? g.f_in : g.f_out) + a0 : (in ? g.m_in : g.m_out) + m0;
+    t.tab = (side ? (in ? g.m_in_t.tab : g.m_out_t.tab) : (in ? g.f_in_t.tab : g.f_out_t.tab)) + (d >> 6);
+    t.meta = (uint32_t)(d & 63u) | (side ? kSideF : 0u) | (in ? kIn : 0u);
+    return side ? df : (df == 0 ? 0 : dm);
+}
+
+/* Sum of contributions new - old of the lists of a swap (u on f2, v on f1:
+ * new; with NT = 4 also u on f1, v on f2: old), the lane's share of wave wv
+ * of W.  An out-list prices an edge to u or v at that endpoint's image in
+ * the matching it belongs to (which makes u <-> v edges and self-loops
+ * exact); an in-list leaves edges from u or v out (counted by the out-list).
+ * Positions in 32 bits: 8 lists of at most n entries each. */
+template <bool PACKED, int NT, int U, int W>
+__device__ __forceinline__ typename std::conditional<PACKED, int32_t, int64_t>::type
+swap_lists(const BmDevGraph& g, int32_t u, int32_t v, int32_t f1, int32_t f2, ScanList* __restrict__ L, int lane,
+           int wv) {
+    typedef typename std::conditional<PACKED, int32_t, int64_t>::type Acc;
+    constexpr int NL = 2 * NT;
+    int32_t len = 0;
+    ScanList t;
+    t.pad[0] = t.pad[1] = 0;
+    if (lane < NL) {
+        const int q = lane >> 1;
+        const bool onu = (q & 1) == 0;
+        len = scan_list(g, onu ? u : v, (q == 0 || q == 3) ? f2 : f1, lane & 1, t);
+        if (q < 2) t.meta |= kNew;
+    }
+    int32_t incl = len;
+#pragma unroll
+    for (int o = 1; o < NL; o <<= 1) {
+        const int32_t y = __shfl_up(incl, o, BM_WAVE);
+        if (lane >= o) incl += y;
+    }
+    t.start = incl - len;
+    wave_sync();
+    if (lane < NL) L[lane] = t;
+    wave_sync();
+    int32_t st[NL];
+#pragma unroll
+    for (int q = 1; q < NL; q++) st[q] = __builtin_amdgcn_readlane(t.start, q);
+    const int32_t total = __builtin_amdgcn_readlane(incl, NL - 1);
+    const int32_t* __restrict__ pi = g.pi;
+    const int32_t* __restrict__ inv = g.inv;
+    Acc acc = 0;
+    for (int32_t base = wv * BM_WAVE * U; base < total; base += W * BM_WAVE * U) {
+        const uint4* T[U];
+        uint32_t meta[U];
+        int2 e[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int32_t i = base + BM_WAVE * j + lane;
+            int q = 0;
+#pragma unroll
+            for (int z = 1; z < NL; z++) q += i >= st[z] ? 1 : 0;
+            const ScanList l = L[q];
+            T[j] = l.tab;
+            meta[j] = l.meta;
+            e[j] = i < total ? l.rows[i - l.start] : make_int2(0, 0);
+        }
+        int32_t key[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) key[j] = ((meta[j] & kSideF) ? inv : pi)[e[j].x];
+        uint32_t b[U];
+        uint32_t pend = 0;
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const bool side = meta[j] & kSideF;
+            const int32_t id = e[j].x;
+            const bool ha = id == (side ? f1 : u), hb = id == (side ? f2 : v);
+            if (ha || hb) {
+                if (meta[j] & kIn) key[j] = 0;
+                else if (meta[j] & kNew) key[j] = side ? (ha ? v : u) : (ha ? f2 : f1);
+            }
+            if (id == 0) key[j] = 0;
+            b[j] = row_home(key[j], meta[j] & 63u);
+            pend |= (key[j] != 0 ? 1u : 0u) << j;
+        }
+        while (pend) {
+            uint4 x[U];
+#pragma unroll
+            for (int j = 0; j < U; j++)
+                if ((pend >> j) & 1u) x[j] = T[j][b[j]];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                if (!((pend >> j) & 1u)) continue;
+                int32_t w;
+                if (row_bucket<PACKED>(x[j], key[j], w)) {
+                    const int32_t c = contrib(e[j].y, w);
+                    acc += (meta[j] & kNew) ? (Acc)c : -(Acc)c;
+                    pend &= ~(1u << j);
+                } else {
+                    b[j] = (b[j] + 1u) & ((1u << (meta[j] & 63u)) - 1u);
+                }
+            }
+        }
+    }
+    return acc;
+}
+
+/* Exact swap deltas.  What bounds it is the lookups: each is a 16-byte gather
+ * (and a 4-byte gather of the matching), about 2e11 a second, so the shorter
+ * side of every term is walked and the current terms are shared where a batch
+ * is large enough.  At n = 18,524 with 4M edges a pair takes 555 lookups with
+ * diag (1,322 without) and no hub pair more than 21,000; scanning both
+ * vertices' lists against LDS copies of the four female rows took 1,728
+ * lookups and 860 inserts, and up to 74,000 for a hub pair, which set the time
+ * of small batches (4,096 pairs: 1,263 us, now 111; 65,536: 1,457, now 476;
+ * 2^20: 12 ms, now 4.5).
+ * W = 1: one wave per candidate, any number of waves per
+ * block; W = 4: the four waves of a block share a candidate (batches too
+ * small to fill the device, where the longest list sets the time).  DIAG:
+ * the current contributions of u and v come from diag (k_diag), so only the
+ * lists of the new images are walked; their edges u <-> v, counted by both,
+ * are looked up. */
+template <int MODE, bool PACKED, int U, int W, bool DIAG>
+__global__ void __launch_bounds__(W == 1 ? 512 : 64 * W) k_swap(BmDevGraph g, const int2* __restrict__ cand,
+                                                                const int64_t* __restrict__ off, uint64_t seed,
+                                                                int64_t k, int64_t* __restrict__ delta,
+                                                                const int64_t* __restrict__ diag) {
+    constexpr int NT = DIAG ? 2 : 4;
+    __shared__ ScanList s_lists[8][2 * NT];
+    __shared__ int64_t s_part[2][W];
     const int lane = threadIdx.x & (BM_WAVE - 1);
-    const int wave = threadIdx.x / BM_WAVE;
-    const int wpb = blockDim.x / BM_WAVE;
-    S* lds = reinterpret_cast<S*>(smem) + (size_t)wave * cap;
+    const int wave = uni(threadIdx.x / BM_WAVE);
+    const int wpb = W == 1 ? (int)(blockDim.x / BM_WAVE) : 1;
     const int64_t nw = (int64_t)gridDim.x * wpb;
-    for (int64_t c = (int64_t)blockIdx.x * wpb + wave; c < k; c += nw) {
+    int par = 0;
+    for (int64_t c = (int64_t)blockIdx.x * wpb + (W == 1 ? wave : 0); c < k; c += nw) {
         int32_t u, v;
         if (MODE == BM_CAND_LIST) {
             const int2 p = cand[c];
@@ -482,12 +624,34 @@ __global__ void __launch_bounds__(512) k_swap(BmDevGraph g, const int2* __restri
         u = uni(u);
         v = uni(v);
         if (u == v) {
-            if (lane == 0) delta[c] = 0;
+            if (threadIdx.x % (BM_WAVE * W) == 0) delta[c] = 0;
             continue;
         }
         const int32_t f1 = uni(g.pi[u]), f2 = uni(g.pi[v]);
-        const int64_t acc = swap_delta_wave<COMPACT, U>(g, u, v, f1, f2, lds, cap, lane);
-        if (lane == 0) delta[c] = acc;
+        int64_t acc = (int64_t)swap_lists<PACKED, NT, U, W>(g, u, v, f1, f2, s_lists[wave], lane, W == 1 ? 0 : wave);
+        if (DIAG && (W == 1 || wave == 0)) {
+            if (lane < 2) {   /* edge u -> v (lane 0), v -> u (lane 1) at its current images */
+                const int32_t a = lane ? v : u, b = lane ? u : v, fa = lane ? f2 : f1, fb = lane ? f1 : f2;
+                acc -= diag[a];
+                const int32_t w = row_find<PACKED>(g.m_out_t.tab, g.m_out_t.desc[a], b);
+                if (w != BM_ABSENT) acc += contrib(w, row_find<PACKED>(g.f_out_t.tab, g.f_out_t.desc[fa], fb));
+            }
+        }
+        acc = wave_sum64(acc);
+        if (W == 1) {
+            if (lane == 0) delta[c] = acc;
+        } else {
+            /* two buffers: thread 0 has read one before the barrier after which it is written again */
+            if (lane == 0) s_part[par][wave] = acc;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                int64_t sum = 0;
+#pragma unroll
+                for (int q = 0; q < W; q++) sum += s_part[par][q];
+                delta[c] = sum;
+            }
+            par ^= 1;
+        }
     }
 }
 
@@ -967,30 +1131,47 @@ hipError_t launch_delta(K kernel, const BmLaunch& L, int64_t work, size_t slot_b
 
 size_t bm_slot_bytes(const BmDevGraph& g) { return g.compact ? 4 : 8; }
 
-hipError_t bm_launch_swap(const BmDevGraph& g, const BmLaunch& L, int mode, const int2* cand, const int64_t* off,
-                          uint64_t seed, int64_t k, int64_t* delta, hipStream_t s) {
-    if (k <= 0) return hipSuccess;
-    dim3 grid, block;
-    size_t lds;
-    hipError_t e;
-#define BM_SWAP_CASE(M, C, U)                                                                           \
-    e = launch_delta(k_swap<M, C, U>, L, k, C ? 4 : 8, s, &grid, &block, &lds);                         \
-    if (e != hipSuccess) return e;                                                                      \
-    hipLaunchKernelGGL((k_swap<M, C, U>), grid, block, lds, s, g, cand, off, seed, k, delta, (uint32_t)L.lds_slots);
-#define BM_SWAP_U(M, C)                             \
-    if (L.unroll == 4) { BM_SWAP_CASE(M, C, 4) }     \
-    else if (L.unroll == 2) { BM_SWAP_CASE(M, C, 2) } \
-    else { BM_SWAP_CASE(M, C, 8) }
-    if (mode == BM_CAND_LIST) {
-        if (g.compact) { BM_SWAP_U(BM_CAND_LIST, true) } else { BM_SWAP_U(BM_CAND_LIST, false) }
-    } else if (mode == BM_CAND_UMAJOR) {
-        if (g.compact) { BM_SWAP_U(BM_CAND_UMAJOR, true) } else { BM_SWAP_U(BM_CAND_UMAJOR, false) }
-    } else {
-        if (g.compact) { BM_SWAP_U(BM_CAND_UNIFORM, true) } else { BM_SWAP_U(BM_CAND_UNIFORM, false) }
-    }
-#undef BM_SWAP_U
-#undef BM_SWAP_CASE
+template <int M, bool P, int U, int W, bool D>
+static hipError_t launch_swap_one(const BmDevGraph& g, const BmLaunch& L, const int2* cand, const int64_t* off,
+                                  uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag, hipStream_t s) {
+    const int waves = W == 1 ? L.waves_per_block : W;
+    int occ = 0;
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)k_swap<M, P, U, W, D>, waves * BM_WAVE, 0);
+    if (e != hipSuccess) return e;
+    int per_cu = L.blocks_per_cu < occ ? L.blocks_per_cu : occ;
+    if (per_cu < 1) per_cu = 1;
+    const int64_t need = W == 1 ? (k + waves - 1) / waves : k;
+    const int64_t cap = (int64_t)per_cu * (L.num_cus > 0 ? L.num_cus : 256);
+    const int64_t blocks = need < cap ? need : cap;
+    hipLaunchKernelGGL((k_swap<M, P, U, W, D>), dim3((unsigned)blocks), dim3(waves * BM_WAVE), 0, s, g, cand, off, seed,
+                       k, delta, diag);
     return hipGetLastError();
+}
+
+template <int M, bool P, bool D>
+static hipError_t launch_swap_u(const BmDevGraph& g, const BmLaunch& L, const int2* cand, const int64_t* off,
+                                uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag, hipStream_t s) {
+    if (L.coop) return launch_swap_one<M, P, 4, 4, D>(g, L, cand, off, seed, k, delta, diag, s);
+    if (L.unroll == 2) return launch_swap_one<M, P, 2, 1, D>(g, L, cand, off, seed, k, delta, diag, s);
+    return launch_swap_one<M, P, 4, 1, D>(g, L, cand, off, seed, k, delta, diag, s);
+}
+
+template <int M>
+static hipError_t launch_swap_mode(const BmDevGraph& g, const BmLaunch& L, const int2* cand, const int64_t* off,
+                                   uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag, hipStream_t s) {
+    if (g.packed)
+        return diag ? launch_swap_u<M, true, true>(g, L, cand, off, seed, k, delta, diag, s)
+                    : launch_swap_u<M, true, false>(g, L, cand, off, seed, k, delta, diag, s);
+    return diag ? launch_swap_u<M, false, true>(g, L, cand, off, seed, k, delta, diag, s)
+                : launch_swap_u<M, false, false>(g, L, cand, off, seed, k, delta, diag, s);
+}
+
+hipError_t bm_launch_swap(const BmDevGraph& g, const BmLaunch& L, int mode, const int2* cand, const int64_t* off,
+                          uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag, hipStream_t s) {
+    if (k <= 0) return hipSuccess;
+    if (mode == BM_CAND_LIST) return launch_swap_mode<BM_CAND_LIST>(g, L, cand, off, seed, k, delta, diag, s);
+    if (mode == BM_CAND_UMAJOR) return launch_swap_mode<BM_CAND_UMAJOR>(g, L, cand, off, seed, k, delta, diag, s);
+    return launch_swap_mode<BM_CAND_UNIFORM>(g, L, cand, off, seed, k, delta, diag, s);
 }
 
 template <bool C, int U3>

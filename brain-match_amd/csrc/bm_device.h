@@ -187,13 +187,17 @@ struct BmLaunch {
     int32_t blocks_per_cu;     /* persistent grid: blocks per CU (capped by occupancy) */
     int32_t num_cus;
     int32_t unroll;            /* list entries per lane in flight (2, 4 or 8) */
+    int32_t coop;              /* swap kernel: 1 = the four waves of a block share a candidate */
 };
 
 /* Candidate sources. */
 enum BmCandMode { BM_CAND_LIST = 0, BM_CAND_UNIFORM = 1, BM_CAND_UMAJOR = 2 };
 
+/* Swap deltas; diag (bm_launch_diag of the current matching) or NULL, when
+ * every candidate sums its two vertices' current contributions itself. */
 hipError_t bm_launch_swap(const BmDevGraph& g, const BmLaunch& L, int mode, const int2* cand,
-                          const int64_t* off, uint64_t seed, int64_t k, int64_t* delta, hipStream_t s);
+                          const int64_t* off, uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag,
+                          hipStream_t s);
 
 /* u-major stream (bm_umajor_first / bm_umajor_partner): counts (n+1 int32)
  * and offsets off[0..n+1] (int64) of k draws; pairs written as a list. */

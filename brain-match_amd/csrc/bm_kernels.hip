@@ -367,12 +367,11 @@ constexpr int kAccBatch = 16;   /* free candidates decided together */
  * the first 16 of them whose endpoints are unlocked; whether one's acceptance
  * would lock another follows from row-table lookups among their endpoints
  * (120 pairs x 8 lookups, one per thread), one thread decides the 16 in
- * order, and each wave locks the neighbourhoods of one accepted swap.  That is
+ * order, and the waves lock the accepted swaps' neighbourhoods.  That is
  * the decision of the one-at-a-time loop: a later candidate of the 16 is
  * rejected exactly when an earlier accepted one locks an endpoint.  One
- * candidate per round (five barriers and a list walk each) took 150 us, this
- * 55 us, for
- * the 50 swaps of an early climb round at n = 18,524. */
+ * candidate per round (five barriers and a list walk each) took 150 us for
+ * the 50 swaps of an early climb round at n = 18,524, this 55 us with one wave per list. */
 template <bool PACKED>
 __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int32_t* __restrict__ pi,
                                                                int32_t* __restrict__ inv,
@@ -443,6 +442,15 @@ __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int
             }
             __syncthreads();
             const int cnt = total < kAccBatch ? total : kAccBatch;
+            /* lane l of every wave: list l % 4 (u out, v out, u in, v in) of candidate l / 4 */
+            int64_t l0 = 0, l1 = 0;
+            int32_t end = 0;
+            if ((lane >> 2) < cnt) {
+                end = (lane & 1) ? s_end[lane >> 2].y : s_end[lane >> 2].x;
+                const int64_t* ptr = (lane & 2) ? g.m_in_ptr : g.m_out_ptr;
+                l0 = ptr[end];
+                l1 = ptr[end + 1];
+            }
             if (qj >= 0 && qj < cnt) {
                 const int2 a = s_end[qi], b = s_end[qj];
                 const int32_t x = (t & 1) ? a.y : a.x, y = (t & 2) ? b.y : b.x;
@@ -465,21 +473,30 @@ __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int
                 s_gain = gain;
             }
             __syncthreads();
-            static_assert(kAccBatch == kAccWaves, "one wave per candidate of a round");
-            if ((s_acc >> wave) & 1u) {
-                const int2 e = s_end[wave];
+            /* lock the accepted swaps' neighbourhoods: their lists in units of
+             * 256 entries, taken by the waves in turn, so that a hub's list
+             * does not hang on one wave */
+            const bool on = (s_acc >> (lane >> 2)) & 1u;
+            if (on && lane % 4 < 2 && wave == 0) atomicOr(&lock[end >> 5], 1u << (end & 31));
+            const int32_t units = on ? (int32_t)((l1 - l0 + 255) / 256) : 0;
+            int32_t incl = units;
 #pragma unroll
-                for (int z = 0; z < 4; z++) {
-                    const int32_t x = (z & 1) ? e.y : e.x;
-                    const int64_t* ptr = (z & 2) ? g.m_in_ptr : g.m_out_ptr;
-                    const int2* adj = (z & 2) ? g.m_in : g.m_out;
-                    const int64_t b0 = ptr[x], b1 = ptr[x + 1];
-                    for (int64_t o = b0 + lane; o < b1; o += BM_WAVE) {
-                        const int32_t y = adj[o].x;
-                        atomicOr(&lock[y >> 5], 1u << (y & 31));
-                    }
-                    if (z < 2 && lane == 0) atomicOr(&lock[x >> 5], 1u << (x & 31));
-                }
+            for (int o = 1; o < BM_WAVE; o <<= 1) {
+                const int32_t y = __shfl_up(incl, o, BM_WAVE);
+                if (lane >= o) incl += y;
+            }
+            const int32_t all = __builtin_amdgcn_readlane(incl, BM_WAVE - 1);
+            for (int32_t unit = wave; unit < all; unit += kAccWaves) {
+                const int l = __popcll(__ballot(incl <= unit));
+                const int64_t first = __shfl(l0, l, BM_WAVE), last = __shfl(l1, l, BM_WAVE);
+                const int64_t o = first + (int64_t)(unit - __shfl(incl - units, l, BM_WAVE)) * 256 + lane;
+                const int2* adj = (l & 2) ? g.m_in : g.m_out;
+                int32_t y[4];
+#pragma unroll
+                for (int z = 0; z < 4; z++) y[z] = o + BM_WAVE * z < last ? adj[o + BM_WAVE * z].x : 0;
+#pragma unroll
+                for (int z = 0; z < 4; z++)
+                    if (y[z]) atomicOr(&lock[y[z] >> 5], 1u << (y[z] & 31));
             }
             start = s_last + 1;
             __syncthreads();
