@@ -6,8 +6,9 @@
  *           copied);
  *   chains  one BmChain per chain (running score, best score, step and
  *           acceptance counters, stream seed, offset of its matchings);
- *   pool    per chain the current matching and the best-so-far copy,
- *           2 * (n_i + 1) int32 each, chains of one instance contiguous;
+ *   pool    per chain the current matching, the best-so-far copy and the
+ *           current matching's inverse, 3 * (n_i + 1) int32 in all, chains of
+ *           one instance contiguous;
  *   traj    chains x traj_cap int64 score samples, one per launch;
  *   props   one BmProposalPool per instance, pointing at that instance's
  *           proposal pairs (a device buffer owned here, grown on demand).
@@ -30,6 +31,10 @@
 
 extern "C" const char* bm_global_error(void);
 
+/* Chains that leave wave slots idle (256 CUs x 16 waves) are bound by the
+ * latency of a step, so each gets the four waves of a block. */
+static constexpr int64_t kCoopChains = 1024;
+
 struct bm_anneal {
     int device;
     hipStream_t stream;
@@ -40,7 +45,8 @@ struct bm_anneal {
     std::vector<BmDevGraph> graphs;   /* host copies of the instance graphs */
     std::vector<int64_t> pi_off;      /* per chain */
     std::vector<BmChain> h_init;      /* chain states at creation (for bm_anneal_reset) */
-    int32_t* d_init;                  /* each instance's initial matching, concatenated */
+    int32_t* d_init;                  /* each instance's initial matching and its inverse, concatenated */
+    int64_t* d_init_off;              /* n_inst */
     std::vector<int64_t> init_off;    /* per instance offset into d_init */
     BmDevGraph* d_insts;
     BmChain* d_chains;
@@ -54,8 +60,8 @@ struct bm_anneal {
     BmAnnealSched sc;
     BmLaunch L;
     int compact;
+    int packed;
     dim3 grid, block;
-    size_t lds;
     hipGraph_t graph;
     hipGraphExec_t exec;
     int64_t graph_steps;
@@ -99,6 +105,7 @@ static void free_anneal(bm_anneal* a) {
     (void)hipFree(a->d_traj);
     (void)hipFree(a->d_scores);
     (void)hipFree(a->d_init);
+    (void)hipFree(a->d_init_off);
     (void)hipFree(a->d_props);
     for (int2* p : a->prop_buf) (void)hipFree(p);
     if (a->stream) (void)hipStreamDestroy(a->stream);
@@ -164,15 +171,16 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
         }
     }
 
-    a->compact = 1;
+    a->compact = a->packed = 1;
     for (int32_t i = 0; i < n_inst; i++) {
         a->graphs.push_back(bm_ctx_devgraph(ctxs[i]));
         a->compact &= a->graphs.back().compact ? 1 : 0;
+        a->packed &= a->graphs.back().packed ? 1 : 0;
     }
-    /* launch shape: the swap kernel's tuning of the first context, the LDS
-     * slice kept at the same byte size when the slot format widens */
+    /* launch shape: the swap kernel's tuning of the first context */
     a->L = bm_ctx_launch(ctxs[0], BM_KERNEL_SWAP);
     if (!a->compact && a->graphs[0].compact) a->L.lds_slots /= 2;
+    a->L.coop = a->n_chains <= kCoopChains;
 
     int64_t pool = 0;
     a->pi_off.resize((size_t)a->n_chains);
@@ -190,18 +198,21 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
             ch.seed = bm_rand_at(p->seed, (uint64_t)c);
             ch.inst = i;
             ch.at_best = 1;
-            pool += 2 * len;
+            pool += 3 * len;
         }
     }
     int64_t init_len = 0;
     for (int32_t i = 0; i < n_inst; i++) {
         a->init_off.push_back(init_len);
-        init_len += (int64_t)a->graphs[i].n + 1;
+        init_len += 2 * ((int64_t)a->graphs[i].n + 1);
     }
     ACHK(hipMalloc((void**)&a->d_init, sizeof(int32_t) * (size_t)init_len));
     for (int32_t i = 0; i < n_inst; i++)
-        ACHK(hipMemcpyAsync(a->d_init + a->init_off[i], a->graphs[i].pi, sizeof(int32_t) * ((size_t)a->graphs[i].n + 1),
-                            hipMemcpyDeviceToDevice, a->stream));
+        ACHK(hipMemcpyAsync(a->d_init + a->init_off[i], a->graphs[i].pi,
+                            2 * sizeof(int32_t) * ((size_t)a->graphs[i].n + 1), hipMemcpyDeviceToDevice, a->stream));
+    ACHK(hipMalloc((void**)&a->d_init_off, sizeof(int64_t) * (size_t)n_inst));
+    ACHK(hipMemcpyAsync(a->d_init_off, a->init_off.data(), sizeof(int64_t) * (size_t)n_inst, hipMemcpyHostToDevice,
+                        a->stream));
     a->h_init = h;
     ACHK(hipMalloc((void**)&a->d_insts, sizeof(BmDevGraph) * (size_t)n_inst));
     ACHK(hipMalloc((void**)&a->d_chains, sizeof(BmChain) * (size_t)a->n_chains));
@@ -218,22 +229,14 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
                         a->stream));
     ACHK(hipMemcpyAsync(a->d_chains, h.data(), sizeof(BmChain) * (size_t)a->n_chains, hipMemcpyHostToDevice,
                         a->stream));
-    for (int32_t i = 0; i < n_inst; i++) {
-        const size_t bytes = sizeof(int32_t) * ((size_t)a->graphs[i].n + 1);
-        for (int64_t j = 0; j < a->per_inst; j++) {
-            const int64_t off = a->pi_off[(size_t)i * a->per_inst + j];
-            ACHK(hipMemcpyAsync(a->d_pool + off, a->graphs[i].pi, bytes, hipMemcpyDeviceToDevice, a->stream));
-            ACHK(hipMemcpyAsync(a->d_pool + off + a->graphs[i].n + 1, a->graphs[i].pi, bytes, hipMemcpyDeviceToDevice,
-                                a->stream));
-        }
-    }
+    ACHK(bm_launch_anneal_reset(a->d_insts, a->d_chains, a->n_chains, a->d_init, a->d_init_off, a->d_pool, a->stream));
     a->sc.beta0 = 1.0 / p->t0;
     a->sc.lam = -log(p->decay);
     a->sc.p_rot3 = (uint64_t)llround(p->p_rot3 * 4294967296.0);
     a->sc.traj_cap = p->traj_cap;
     a->sc.pad = 0;
     a->sc.p_pool = (uint64_t)llround(p->p_pool * 4294967296.0);
-    ACHK(bm_anneal_grid(a->compact, a->sc.p_rot3 != 0, a->L, a->n_chains, &a->grid, &a->block, &a->lds));
+    ACHK(bm_anneal_grid(a->packed, a->sc.p_rot3 != 0, a->L, a->n_chains, &a->grid, &a->block));
     ACHK(hipStreamSynchronize(a->stream));
 #undef ACHK
     *out = a;
@@ -250,8 +253,8 @@ extern "C" int bm_anneal_run(bm_anneal* a, int64_t steps, int32_t launches) {
         a->exec = nullptr;
         a->graph = nullptr;
         AHIP(a, hipStreamBeginCapture(a->stream, hipStreamCaptureModeThreadLocal));
-        hipError_t le = bm_launch_anneal(a->d_insts, a->compact, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
-                                         a->d_traj, a->d_props, a->L, a->grid, a->block, a->lds, a->stream);
+        hipError_t le = bm_launch_anneal(a->d_insts, a->packed, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
+                                         a->d_traj, a->d_props, a->L, a->grid, a->block, a->stream);
         hipGraph_t g = nullptr;
         hipError_t ce = hipStreamEndCapture(a->stream, &g);
         if (le != hipSuccess || ce != hipSuccess) {
@@ -350,7 +353,7 @@ extern "C" int bm_anneal_verify(bm_anneal* a, int64_t* mismatches) {
     AHIP(a, hipMemsetAsync(a->d_scores, 0, sizeof(int64_t) * (size_t)a->n_chains, a->stream));
     for (int64_t c = 0; c < a->n_chains; c++) {
         BmDevGraph g = a->graphs[h[c].inst];
-        g.pi = a->d_pool + h[c].pi_off;
+        g.pi = a->d_pool + h[c].pi_off;   /* (a score takes no inverse) */
         const bm_ctx* ctx = a->ctxs[h[c].inst];
         int64_t n_out = 0;
         const int4* chunks = bm_ctx_chunks(ctx, nullptr, &n_out);
@@ -486,14 +489,7 @@ static int reset_chains(bm_anneal* a) {
     AHIP(a, hipSetDevice(a->device));
     AHIP(a, hipMemcpyAsync(a->d_chains, a->h_init.data(), sizeof(BmChain) * (size_t)a->n_chains, hipMemcpyHostToDevice,
                            a->stream));
-    for (int64_t c = 0; c < a->n_chains; c++) {
-        const int32_t i = a->h_init[c].inst;
-        const size_t len = (size_t)a->graphs[i].n + 1;
-        AHIP(a, hipMemcpyAsync(a->d_pool + a->pi_off[c], a->d_init + a->init_off[i], len * sizeof(int32_t),
-                               hipMemcpyDeviceToDevice, a->stream));
-        AHIP(a, hipMemcpyAsync(a->d_pool + a->pi_off[c] + len, a->d_init + a->init_off[i], len * sizeof(int32_t),
-                               hipMemcpyDeviceToDevice, a->stream));
-    }
+    AHIP(a, bm_launch_anneal_reset(a->d_insts, a->d_chains, a->n_chains, a->d_init, a->d_init_off, a->d_pool, a->stream));
     AHIP(a, hipStreamSynchronize(a->stream));
     a->launches = 0;
     a->total_ms = 0;
@@ -530,13 +526,11 @@ extern "C" int bm_anneal_set_tuning(bm_anneal* a, const bm_tuning* t) {
     L.blocks_per_cu = t->blocks_per_cu;
     L.unroll = t->unroll;
     dim3 grid, block;
-    size_t lds;
     AHIP(a, hipSetDevice(a->device));
-    AHIP(a, bm_anneal_grid(a->compact, a->sc.p_rot3 != 0, L, a->n_chains, &grid, &block, &lds));
+    AHIP(a, bm_anneal_grid(a->packed, a->sc.p_rot3 != 0, L, a->n_chains, &grid, &block));
     a->L = L;
     a->grid = grid;
     a->block = block;
-    a->lds = lds;
     if (a->exec) (void)hipGraphExecDestroy(a->exec);
     if (a->graph) (void)hipGraphDestroy(a->graph);
     a->exec = nullptr;
@@ -579,8 +573,8 @@ extern "C" int bm_anneal_autotune(bm_anneal* a, int64_t steps, bm_tuning* best, 
                 if ((rc = reset_chains(a)) != BM_OK) break;
                 hipError_t e = hipEventRecord(e0, a->stream);
                 if (e == hipSuccess)
-                    e = bm_launch_anneal(a->d_insts, a->compact, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
-                                         nullptr, a->d_props, a->L, a->grid, a->block, a->lds, a->stream);
+                    e = bm_launch_anneal(a->d_insts, a->packed, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
+                                         nullptr, a->d_props, a->L, a->grid, a->block, a->stream);
                 if (e == hipSuccess) e = hipEventRecord(e1, a->stream);
                 if (e == hipSuccess) e = hipEventSynchronize(e1);
                 float ms = 0.f;

@@ -506,7 +506,7 @@ static BmLaunch scan_launch(const bm_ctx* c, int kernel, int64_t k) {
     L.lds_slots = c->compact ? 1280 : 640;
     L.blocks_per_cu = 8;
     L.unroll = kernel == BM_KERNEL_ROT3 ? 4 : 8;
-    L.coop = kernel == BM_KERNEL_SWAP;
+    L.coop = 1;
     return L;
 }
 

@@ -49,9 +49,6 @@ hipError_t bm_launch_rowtab_fill(int packed, const int64_t* ptr, const int2* adj
 hipError_t bm_launch_diag(const BmDevGraph& g, const int4* chunks, int64_t nchunks, int64_t* diag, int32_t num_cus,
                           hipStream_t s);
 
-/* Bytes per LDS table slot for this graph (4 compact, 8 otherwise). */
-size_t bm_slot_bytes(const BmDevGraph& g);
-
 /* Placement-gain table (bm_gain.hip). */
 struct BmGain {
     int32_t* G;                 /* (n+1) x stride int32, row-major; row 0 / column 0 zero */
@@ -183,11 +180,11 @@ hipError_t bm_launch_moves_from_perm3(const int32_t* pi_before, int32_t a, int32
 
 struct BmLaunch {
     int32_t waves_per_block;   /* 1, 2, 4 or 8 */
-    int32_t lds_slots;         /* table slots per wave (8 bytes each) */
+    int32_t lds_slots;         /* accepted and reported; no kernel builds LDS tables */
     int32_t blocks_per_cu;     /* persistent grid: blocks per CU (capped by occupancy) */
     int32_t num_cus;
     int32_t unroll;            /* list entries per lane in flight (2, 4 or 8) */
-    int32_t coop;              /* swap kernel: 1 = the four waves of a block share a candidate */
+    int32_t coop;              /* 1 = the four waves of a block share a candidate or chain */
 };
 
 /* Candidate sources. */
@@ -251,13 +248,19 @@ struct BmAnnealSched {
     uint64_t p_pool;    /* probability that a move is drawn from the proposal pool, units of 2^-32 */
 };
 
-/* Persistent grid for n_chains chains (one wave each); computed once. */
-hipError_t bm_anneal_grid(int compact, int rot, const BmLaunch& L, int64_t n_chains, dim3* grid, dim3* block, size_t* lds);
-/* Advances every chain by `steps` steps.  insts: device array of graphs. */
-hipError_t bm_launch_anneal(const BmDevGraph* insts, int compact, BmChain* chains, int64_t n_chains,
-                            int32_t* pool, int64_t steps, const BmAnnealSched& sc, int64_t* traj,
-                            const BmProposalPool* proposals, const BmLaunch& L, dim3 grid, dim3 block, size_t lds,
-                            hipStream_t s);
+/* Persistent grid for n_chains chains; computed once.  packed: every
+ * instance's row tables are packed (otherwise each chain follows its own). */
+hipError_t bm_anneal_grid(int packed, int rot, const BmLaunch& L, int64_t n_chains, dim3* grid, dim3* block);
+/* Advances every chain by `steps` steps.  insts: device array of graphs;
+ * pool: per chain the current matching, the best copy and the current
+ * matching's inverse, n_i + 1 each. */
+hipError_t bm_launch_anneal(const BmDevGraph* insts, int packed, BmChain* chains, int64_t n_chains, int32_t* pool,
+                            int64_t steps, const BmAnnealSched& sc, int64_t* traj, const BmProposalPool* proposals,
+                            const BmLaunch& L, dim3 grid, dim3 block, hipStream_t s);
+/* Every chain's matchings back to its instance's initial one: init +
+ * init_off[inst] holds that matching and its inverse. */
+hipError_t bm_launch_anneal_reset(const BmDevGraph* insts, const BmChain* chains, int64_t n_chains,
+                                  const int32_t* init, const int64_t* init_off, int32_t* pool, hipStream_t s);
 
 hipError_t bm_launch_gen_pairs(int32_t n, uint64_t seed, int64_t k, int2* cand, hipStream_t s);
 hipError_t bm_launch_gen_triples(int32_t n, uint64_t seed, int64_t k, int4* cand, hipStream_t s);

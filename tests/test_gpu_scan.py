@@ -77,3 +77,45 @@ def test_smallest_graphs(bm, orc, n):
     with bm.Context(n, male, female) as ctx:
         ctx.set_mapping(pi)
         assert np.array_equal(ctx.swap_deltas(uv), orc.Oracle(n, male, female).swap_deltas(pi, uv))
+
+
+@pytest.mark.parametrize("kind", ["plain", "quirky", "negative_male", "wide_weights", "shared_images", "empty_rows"])
+@pytest.mark.parametrize("k", [1, 200, 33000])
+def test_triples_every_form(bm, orc, kind, k):
+    n, male, female, pi = _variant(bm, kind)
+    o = orc.Oracle(n, male, female)
+    rng = np.random.default_rng(4)
+    abc = np.stack([rng.permutation(np.arange(1, n + 1))[:3] for _ in range(k)]).astype(np.int32)
+    want_b, want_p = o.rot3_many(pi, abc)
+    with bm.Context(n, male, female) as ctx:
+        ctx.set_mapping(pi)
+        best, perm = ctx.rot3_deltas(abc)
+        assert np.array_equal(best, want_b) and np.array_equal(perm.astype(np.int32), want_p)
+
+
+@pytest.mark.parametrize("per_instance", [3, 1400])
+def test_chains_over_mixed_instances(bm, orc, per_instance):
+    """Instances with packed and with wide row tables, with and without an
+    inverse matching, in one launch: four waves per chain and (many chains)
+    one; every chain's recount agrees and one of each instance replays."""
+    parts = [_variant(bm, k) for k in ("plain", "wide_weights", "shared_images")]
+    ctxs = []
+    for n, male, female, pi in parts:
+        c = bm.Context(n, male, female)
+        c.set_mapping(pi)
+        ctxs.append(c)
+    with bm.Anneal(ctxs, chains_per_instance=per_instance, seed=6, t0=20.0, decay=0.999, p_rot3=0.3) as ann:
+        for _ in range(2):          # the second time after a reset
+            ann.run(40, 2)
+            assert ann.verify() == 0
+            st = ann.state()
+            beta0, lam, p3 = ann.schedule()
+            for i, (n, male, female, pi) in enumerate(parts):
+                c = i * per_instance + per_instance // 2
+                o = orc.Oracle(n, male, female)
+                got, _, rs = orc.anneal_chain(o, pi, o.score(pi), orc.chain_seed(6, c), 0, 80, beta0, lam, p3)
+                assert rs[0] == st["score"][c] and rs[1] == st["best"][c]
+                assert np.array_equal(got, ann.mapping(c))
+            ann.reset()
+    for c in ctxs:
+        c.close()
