@@ -51,6 +51,11 @@ struct bm_ctx {
     int32_t packed;         /* row tables hold 4-byte slots */
     int4* d_chunks;         /* male edge chunks (BM_EDGE_CHUNK), out-lists first */
     int64_t n_chunks, n_out_chunks;
+    int32_t rows_fit;       /* every placement-row sum fits int32 */
+    double row_adds;        /* additions of an average placement row: sum of squared female degrees / n */
+    int32_t* d_place;       /* placement rows of one group of changed vertices (bm_changed.hip) */
+    int64_t place_cap;      /* int32 */
+    int64_t* d_cross;       /* 2 (n+1): the third section's terms */
     int64_t* d_diag;        /* n+1: per-vertex contributions, rewritten by every evaluation that uses them */
     int32_t compact;
     int32_t row_layout;     /* BM_ROWS_P19 when female weights are in 0..8191, else BM_ROWS_P15 (compact graphs) */
@@ -123,6 +128,9 @@ struct bm_batch {
     int kind;               /* 0 empty, 1 pairs, 2 triples */
     int generated;          /* candidates came from a device generator */
     int evaluated;
+    int32_t enum_c;         /* the list is the changed-first enumeration of this many vertices (0: it is not) */
+    int32_t* d_changed;     /* those vertices, ascending */
+    int32_t changed_cap;
     void* d_cand;           /* cap * 16 bytes (int2 pairs or int4 triples) */
     int64_t* d_delta;
     uint8_t* d_perm;
@@ -265,6 +273,8 @@ static void free_ctx(bm_ctx* c) {
     }
     (void)hipFree(c->d_chunks);
     (void)hipFree(c->d_diag);
+    (void)hipFree(c->d_place);
+    (void)hipFree(c->d_cross);
     (void)hipFree(c->d_small);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
     (void)hipFree(c->d_reorder);
@@ -408,6 +418,23 @@ extern "C" void bm_destroy(bm_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     free_ctx(ctx);
+}
+
+/* The first vertex u whose placement sums could leave int32 (|G(u, f)| <= sum
+ * over u's edges of max(|w|, max |w_F|)), or 0. */
+static int32_t gain_overflow(const bm_ctx* c) {
+    for (int32_t u = 1; u <= c->n; u++) {
+        int64_t bound = 0;
+        for (int pass = 0; pass < 2; pass++) {
+            const bm_csr_host& L = pass ? c->male.in : c->male.out;
+            for (int64_t e = L.ptr[u]; e < L.ptr[u + 1]; e++) {
+                const int64_t w = L.adj[e].y < 0 ? -(int64_t)L.adj[e].y : L.adj[e].y;
+                bound += w > c->max_abs_fw ? w : c->max_abs_fw;
+            }
+        }
+        if (bound > INT32_MAX) return u;
+    }
+    return 0;
 }
 
 /* Row tables of one adjacency: descriptors from the row lengths (at most half
@@ -631,6 +658,13 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = build_rowtab(c, 2, mg.out.ptr, c->d_m_out_ptr, c->d_m_out);
     if (rc == BM_OK) rc = build_rowtab(c, 3, mg.in.ptr, c->d_m_in_ptr, c->d_m_in);
     if (rc == BM_OK) rc = build_chunks(c);
+    if (rc == BM_OK) rc = dalloc(c, &c->d_m_self, (size_t)n + 1);
+    if (rc == BM_OK) rc = dalloc(c, &c->d_f_self, (size_t)n + 1);
+    if (rc == BM_OK) rc = h2d(c, c->d_m_self, c->h_m_self, (size_t)n + 1);
+    if (rc == BM_OK) rc = h2d(c, c->d_f_self, c->h_f_self, (size_t)n + 1);
+    c->rows_fit = gain_overflow(c) == 0;
+    for (int32_t r = 1; r <= n; r++)
+        c->row_adds += ((double)c->f_out_deg[r] * c->f_out_deg[r] + (double)c->f_in_deg[r] * c->f_in_deg[r]) / n;
     c->pi_distinct = 1;   /* all unmatched */
     if (rc == BM_OK && hipMemsetAsync(c->d_pi, 0, 2 * ((size_t)n + 1) * sizeof(int32_t), c->stream) != hipSuccess)
         rc = fail(c, BM_ERR_HIP, "hipMemsetAsync failed");
@@ -724,6 +758,7 @@ extern "C" void bm_batch_destroy(bm_batch* b) {
     (void)hipFree(b->d_out);
     (void)hipFree(b->d_acc_scratch);
     (void)hipFree(b->d_acc_idx);
+    (void)hipFree(b->d_changed);
     free(b);
 }
 
@@ -767,6 +802,7 @@ extern "C" int bm_batch_set_pairs(bm_batch* b, const int32_t* uv, int64_t k) {
     b->kind = 1;
     b->generated = 0;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -789,6 +825,7 @@ extern "C" int bm_batch_set_triples(bm_batch* b, const int32_t* abc, int64_t k) 
     b->kind = 2;
     b->generated = 0;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -802,6 +839,7 @@ extern "C" int bm_batch_gen_pairs(bm_batch* b, uint64_t seed, int64_t k) {
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -816,6 +854,7 @@ extern "C" int bm_batch_gen_triples(bm_batch* b, uint64_t seed, int64_t k) {
     b->kind = 2;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -840,6 +879,25 @@ static int build_reorder(bm_ctx* c, const int32_t* changed, int32_t cnum, std::v
     return BM_OK;
 }
 
+/* The changed vertices of an enumeration (the head of d_reorder) kept with
+ * the batch: d_reorder belongs to the context's next enumeration. */
+static int keep_changed(bm_batch* b, int32_t cnum) {
+    bm_ctx* c = b->ctx;
+    if (b->changed_cap < cnum) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        (void)hipFree(b->d_changed);
+        b->d_changed = nullptr;
+        b->changed_cap = 0;
+        int rc = dalloc(c, &b->d_changed, (size_t)cnum);
+        if (rc != BM_OK) return rc;
+        b->changed_cap = cnum;
+    }
+    if (cnum > 0)
+        HIPCHK(c, hipMemcpyAsync(b->d_changed, c->d_reorder, (size_t)cnum * sizeof(int32_t), hipMemcpyDeviceToDevice,
+                                 c->stream));
+    return BM_OK;
+}
+
 extern "C" int bm_batch_gen_changed_pairs(bm_batch* b, const int32_t* changed, int32_t cnum) {
     if (!b) return BM_ERR_ARG;
     bm_ctx* c = b->ctx;
@@ -851,11 +909,13 @@ extern "C" int bm_batch_gen_changed_pairs(bm_batch* b, const int32_t* changed, i
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipMemcpyAsync(c->d_reorder, re.data(), re.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, bm_launch_gen_changed_pairs(c->n, cnum, c->d_reorder, P, (int2*)b->d_cand, c->stream));
+    if ((rc = keep_changed(b, cnum)) != BM_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));  /* re goes out of scope */
     b->k = P;
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = cnum;
     return BM_OK;
 }
 
@@ -912,6 +972,7 @@ extern "C" int bm_batch_gen_twohop(bm_batch* b, const int32_t* anchors, int32_t 
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -930,11 +991,13 @@ extern "C" int bm_batch_gen_changed_triples(bm_batch* b, const int32_t* changed,
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipMemcpyAsync(c->d_reorder, re.data(), re.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, bm_launch_gen_changed_triples(c->n, cnum, c->d_reorder, T, (int4*)b->d_cand, c->stream));
+    if ((rc = keep_changed(b, cnum)) != BM_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     b->k = T;
     b->kind = 2;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = cnum;
     return BM_OK;
 }
 
@@ -951,6 +1014,78 @@ static const int4* pair_pis(bm_ctx* c, int64_t k, int* rc) {
         return nullptr;
     }
     return c->d_pis;
+}
+
+/* Whether an enumeration of k candidates over cnum changed vertices goes by
+ * placement rows: 2 cnum rows of row_adds additions (about 8e11 a second) and
+ * the sums over all vertices, against 2.6 m (pairs) or 2.8 m lookups (per
+ * 18,523 triples 52M) a changed vertex at about 2e11 a second; the extra
+ * launches are worth 5e6 lookups.  `lookups` is what the candidates would take
+ * one by one. */
+static bool by_place_rows(const bm_ctx* c, int32_t cnum, double lookups) {
+    if (cnum < 1 || !c->pi_distinct || !c->rows_fit || c->n < 3) return false;
+    if (bm_place_lds(bm_gain_stride(c->n)) > 160 * 1024) return false;
+    return lookups > 0.5 * (double)cnum * c->row_adds + 5e6;
+}
+
+/* Placement rows of changed vertices [i0, i0 + ng) of the batch. */
+static int place_group(bm_batch* b, int32_t i0, int32_t ng, BmPlace* p) {
+    bm_ctx* c = b->ctx;
+    const int64_t stride = bm_gain_stride(c->n);
+    const int64_t need = 2 * (int64_t)ng * bm_place_splits(ng) * stride;
+    if (c->place_cap < need) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        (void)hipFree(c->d_place);
+        c->d_place = nullptr;
+        c->place_cap = 0;
+        int rc = dalloc(c, &c->d_place, (size_t)need);
+        if (rc != BM_OK) return rc;
+        c->place_cap = need;
+    }
+    p->rows = c->d_place;
+    p->changed = b->d_changed + i0;
+    p->ng = ng;
+    p->stride = stride;
+    p->diag = c->d_diag;
+    p->m_self = c->d_m_self;
+    p->f_self = c->d_f_self;
+    HIPCHK(c, bm_launch_place_rows(devgraph(c), p->changed, ng, stride, c->d_place, c->stream));
+    return BM_OK;
+}
+
+static int eval_changed_pairs(bm_batch* b) {
+    bm_ctx* c = b->ctx;
+    const int64_t cnum = b->enum_c, cc = cnum * (cnum - 1) / 2, nu = c->n - cnum;
+    HIPCHK(c, bm_launch_diag(devgraph(c), c->d_chunks, c->n_chunks, c->d_diag, c->num_cus, c->stream));
+    for (int64_t i0 = 0; i0 < cnum; i0 += BM_PLACE_GROUP) {
+        const int64_t ng = cnum - i0 < BM_PLACE_GROUP ? cnum - i0 : BM_PLACE_GROUP, i1 = i0 + ng;
+        BmPlace p;
+        int rc = place_group(b, (int32_t)i0, (int32_t)ng, &p);
+        if (rc != BM_OK) return rc;
+        /* pairs with a first vertex in the group: rows i0..i1-1 of the triangle, then of the rectangle */
+        const int64_t a0 = i0 * (2 * cnum - i0 - 1) / 2, a1 = i1 < cnum ? i1 * (2 * cnum - i1 - 1) / 2 : cc;
+        HIPCHK(c, bm_launch_changed_pairs(devgraph(c), p, (const int2*)b->d_cand, a0, a1 - a0, cc + i0 * nu, ng * nu,
+                                          b->d_delta, c->stream));
+    }
+    return BM_OK;
+}
+
+static int eval_changed_triples(bm_batch* b) {
+    bm_ctx* c = b->ctx;
+    const int64_t cc = b->enum_c, nn = c->n;
+    const int64_t s2 = cc * (cc - 1) * (cc - 2) / 6 + cc * (cc - 1) / 2 * (nn - cc);
+    const int64_t rest = nn - cc - 1;
+    if (!c->d_cross) {
+        int rc = dalloc(c, &c->d_cross, 2 * ((size_t)c->n + 1));
+        if (rc != BM_OK) return rc;
+    }
+    HIPCHK(c, bm_launch_diag(devgraph(c), c->d_chunks, c->n_chunks, c->d_diag, c->num_cus, c->stream));
+    BmPlace p;
+    int rc = place_group(b, 0, b->enum_c, &p);
+    if (rc != BM_OK) return rc;
+    HIPCHK(c, bm_launch_changed_triples(devgraph(c), p, (int4*)b->d_cand, b->k, s2, rest, c->d_cross, b->d_delta,
+                                        b->d_perm, c->stream));
+    return BM_OK;
 }
 
 extern "C" int bm_batch_eval_swaps(bm_batch* b) {
@@ -971,6 +1106,12 @@ extern "C" int bm_batch_eval_swaps(bm_batch* b) {
                                       b->d_delta, pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_SWAP, &t);
+        if (by_place_rows(c, b->enum_c, (double)b->k * 2.6 * c->male.m / c->n)) {
+            const int rc = eval_changed_pairs(b);
+            timing_end(c, &t);
+            if (rc == BM_OK) b->evaluated = 1;
+            return rc;
+        }
         const int64_t* diag = nullptr;
         const int rc = scan_diag(c, b->k, &diag);
         if (rc != BM_OK) {
@@ -1017,6 +1158,7 @@ extern "C" int bm_batch_eval_swaps_uniform(bm_batch* b, uint64_t seed, int64_t k
     b->kind = 3; /* deltas only: candidates implicit in (seed, index) */
     b->generated = 1;
     b->evaluated = 1;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -1066,6 +1208,7 @@ extern "C" int bm_batch_gen_umajor(bm_batch* b, uint64_t seed, int64_t k) {
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -1115,6 +1258,7 @@ extern "C" int bm_batch_eval_swaps_umajor(bm_batch* b, uint64_t seed, int64_t k)
     b->kind = 3; /* deltas only: candidates implicit in (seed, index) */
     b->generated = 1;
     b->evaluated = 1;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -1136,6 +1280,12 @@ extern "C" int bm_batch_eval_rot3(bm_batch* b) {
                                       (int4*)b->d_cand, pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_ROT3, &t);
+        if (b->enum_c <= BM_PLACE_GROUP && by_place_rows(c, b->enum_c, (double)b->k * 13.0 * c->male.m / c->n)) {
+            const int rc = eval_changed_triples(b);
+            timing_end(c, &t);
+            if (rc == BM_OK) b->evaluated = 1;
+            return rc;
+        }
         HIPCHK(c, bm_launch_rot3(devgraph(c), scan_launch(c, BM_KERNEL_ROT3, b->k), (const int4*)b->d_cand, b->k, b->d_delta,
                                  b->d_perm, (int4*)b->d_cand, c->stream));
     }
@@ -1157,6 +1307,7 @@ extern "C" int bm_batch_gen_amajor(bm_batch* b, uint64_t seed, int64_t k) {
     b->kind = 2;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -1201,6 +1352,7 @@ extern "C" int bm_batch_eval_rot3_amajor(bm_batch* b, uint64_t seed, int64_t k) 
     b->kind = 4; /* best deltas and permutations only: triples implicit in (seed, index) */
     b->generated = 1;
     b->evaluated = 1;
+    b->enum_c = 0;
     return BM_OK;
 }
 
@@ -1517,20 +1669,10 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
         return BM_OK;
     }
     if (c->gain_on) return BM_OK;
-    /* every table entry must fit int32: |G(u,f)| <= sum over u's edges of max(|w|, max|w_F|) */
     const bm_graph_host& mg = c->male;
-    for (int32_t u = 1; u <= c->n; u++) {
-        int64_t bound = 0;
-        for (int pass = 0; pass < 2; pass++) {
-            const bm_csr_host& L = pass ? mg.in : mg.out;
-            for (int64_t e = L.ptr[u]; e < L.ptr[u + 1]; e++) {
-                const int64_t w = L.adj[e].y < 0 ? -(int64_t)L.adj[e].y : L.adj[e].y;
-                bound += w > c->max_abs_fw ? w : c->max_abs_fw;
-            }
-        }
-        if (bound > INT32_MAX)
-            return fail(c, BM_ERR_ARG, "bm_gain_enable: vertex %d's incident weights can exceed int32 in the table", u);
-    }
+    if (!c->rows_fit)
+        return fail(c, BM_ERR_ARG, "bm_gain_enable: vertex %d's incident weights can exceed int32 in the table",
+                    gain_overflow(c));
     const size_t bytes = (size_t)bm_gain_table_bytes(c->n);
     size_t free_b = 0, total_b = 0;
     HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
@@ -1543,13 +1685,9 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
         if (bm_rowhash_build(&mg.out, &hm) != BM_OK) return fail(c, BM_ERR_NOMEM, "bm_gain_enable: out of host memory");
         int rc = dalloc(c, &c->d_m_out_desc, (size_t)c->n + 1);
         if (rc == BM_OK) rc = dalloc(c, &c->d_m_out_tab, (size_t)(hm.slots ? hm.slots : 2));
-        if (rc == BM_OK) rc = dalloc(c, &c->d_m_self, (size_t)c->n + 1);
-        if (rc == BM_OK) rc = dalloc(c, &c->d_f_self, (size_t)c->n + 1);
         if (rc == BM_OK) rc = dalloc(c, &c->d_nmoves, 1);
         if (rc == BM_OK) rc = h2d(c, c->d_m_out_desc, hm.desc, (size_t)c->n + 1);
         if (rc == BM_OK) rc = h2d(c, c->d_m_out_tab, hm.tab, (size_t)hm.slots);
-        if (rc == BM_OK) rc = h2d(c, c->d_m_self, c->h_m_self, (size_t)c->n + 1);
-        if (rc == BM_OK) rc = h2d(c, c->d_f_self, c->h_f_self, (size_t)c->n + 1);
         if (rc == BM_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, BM_ERR_HIP, "sync failed");
         bm_rowhash_free(&hm);
         if (rc != BM_OK) return rc;
@@ -1840,6 +1978,7 @@ void bm_batch_mark_pairs(bm_batch* b, int64_t k) {
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
+    b->enum_c = 0;
 }
 int bm_ctx_device(const bm_ctx* c) { return c->device; }
 int bm_ctx_num_cus(const bm_ctx* c) { return c->num_cus; }

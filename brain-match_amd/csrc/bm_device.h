@@ -196,6 +196,32 @@ hipError_t bm_launch_swap(const BmDevGraph& g, const BmLaunch& L, int mode, cons
                           const int64_t* off, uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag,
                           hipStream_t s);
 
+/* Changed-first enumerations from placement rows (bm_changed.hip).  Needs the
+ * inverse matching, every row sum within int32, and bm_place_lds(stride) bytes
+ * of LDS (stride: n + 1 rounded up to 32). */
+#define BM_PLACE_ROWS 2048      /* partial rows of a group, at most */
+#define BM_PLACE_GROUP 128      /* changed vertices of a group, at most */
+size_t bm_place_lds(int64_t stride);
+int32_t bm_place_splits(int32_t ng);
+struct BmPlace {
+    const int32_t* rows;        /* 2 ng x bm_place_splits(ng) x stride, filled by bm_launch_place_rows */
+    const int32_t* changed;     /* the group's ng vertices, ascending */
+    int32_t ng;
+    int64_t stride;
+    const int64_t* diag;        /* bm_launch_diag of the matching */
+    const int32_t* m_self;
+    const int32_t* f_self;
+};
+hipError_t bm_launch_place_rows(const BmDevGraph& g, const int32_t* changed, int32_t ng, int64_t stride, int32_t* rows,
+                                hipStream_t s);
+/* Deltas of the pairs at [a0, a0 + la) and [b0, b0 + lb) of the list. */
+hipError_t bm_launch_changed_pairs(const BmDevGraph& g, const BmPlace& p, const int2* cand, int64_t a0, int64_t la,
+                                   int64_t b0, int64_t lb, int64_t* delta, hipStream_t s);
+/* The whole triple enumeration; its third section starts at s2 and holds
+ * `rest` triples per changed vertex; cross: 2 rest int64 of scratch. */
+hipError_t bm_launch_changed_triples(const BmDevGraph& g, const BmPlace& p, int4* cand, int64_t k, int64_t s2,
+                                     int64_t rest, int64_t* cross, int64_t* best, uint8_t* perm, hipStream_t s);
+
 /* u-major stream (bm_umajor_first / bm_umajor_partner): counts (n+1 int32)
  * and offsets off[0..n+1] (int64) of k draws; pairs written as a list. */
 hipError_t bm_launch_umajor_offsets(int32_t n, uint64_t seed, int64_t k, int32_t* counts, int64_t* off,

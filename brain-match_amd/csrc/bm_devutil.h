@@ -79,6 +79,41 @@ __device__ __forceinline__ T sel3(int j, const T& a, const T& b, const T& c) {
     return j == 0 ? a : (j == 1 ? b : c);
 }
 
+/* Best of the five permutations of a triple from its nine gains Gv[i][j] =
+ * G(vtx_i, f_j), the male self-loops s and female self-loops fs of f_0..f_2
+ * (BM_ABSENT when missing), the male weights w[i][j] of edges inside the
+ * triple and the female weights F[x][y] = w_F(f_x, f_y) (needed only where a
+ * male edge exists).  An edge i -> j is corrected exactly: under permutation
+ * p it contributes c(w, F(f_pi, f_pj)) where the gains counted
+ * c(w, F(f_pi, f_j)) and c(w, F(f_i, f_pj)) and the old score
+ * c(w, F(f_i, f_j)); all of these are among the nine F[x][y].  bd = the
+ * largest positive delta (0 if none), bp its permutation (first p on ties). */
+__device__ __forceinline__ void rot3_from_gains(const int64_t (*Gv)[3], const int32_t (*w)[3], const int32_t (*F)[3],
+                                                const int32_t* s, const int32_t* fs, int64_t& bd, int& bp) {
+    bd = 0;
+    bp = 0;
+#pragma unroll
+    for (int p = 1; p <= 5; p++) {
+        int64_t d = 0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int pi = perm_of(p, i);
+            d += sel3(pi, Gv[i][0], Gv[i][1], Gv[i][2]) - Gv[i][i];
+            if (s[i] != BM_ABSENT) d += contrib(s[i], fs[pi]) - (int64_t)contrib(s[i], fs[i]);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                if (i == j) continue;
+                const int pj = perm_of(p, j);
+                const int32_t x = w[i][j];
+                if (x != BM_ABSENT)
+                    d += (int64_t)contrib(x, F[pi][pj]) - contrib(x, F[pi][j]) - contrib(x, F[i][pj]) +
+                         contrib(x, F[i][j]);
+            }
+        }
+        if (d > bd) { bd = d; bp = p; }
+    }
+}
+
 }  // namespace bmd
 
 #endif
