@@ -52,6 +52,9 @@ struct bm_ctx {
     int4* d_chunks;         /* male edge chunks (BM_EDGE_CHUNK), out-lists first */
     int64_t n_chunks, n_out_chunks;
     int32_t rows_fit;       /* every placement-row sum fits int32 */
+    int32_t rows_small;     /* ... and is at most 2^28 */
+    int32_t max_mw;         /* largest male weight */
+    int32_t pi_full;        /* every male is matched, none to a shared female (moves keep this) */
     double row_adds;        /* additions of an average placement row: sum of squared female degrees / n */
     int32_t* d_place;       /* placement rows of one group of changed vertices (bm_changed.hip) */
     int64_t place_cap;      /* int32 */
@@ -420,9 +423,9 @@ extern "C" void bm_destroy(bm_ctx* ctx) {
     free_ctx(ctx);
 }
 
-/* The first vertex u whose placement sums could leave int32 (|G(u, f)| <= sum
+/* The first vertex u whose placement sums could exceed limit (|G(u, f)| <= sum
  * over u's edges of max(|w|, max |w_F|)), or 0. */
-static int32_t gain_overflow(const bm_ctx* c) {
+static int32_t gain_overflow(const bm_ctx* c, int64_t limit) {
     for (int32_t u = 1; u <= c->n; u++) {
         int64_t bound = 0;
         for (int pass = 0; pass < 2; pass++) {
@@ -432,7 +435,7 @@ static int32_t gain_overflow(const bm_ctx* c) {
                 bound += w > c->max_abs_fw ? w : c->max_abs_fw;
             }
         }
-        if (bound > INT32_MAX) return u;
+        if (bound > limit) return u;
     }
     return 0;
 }
@@ -590,7 +593,10 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
         if (c->male.out.adj[e].y < -32767 || c->male.out.adj[e].y > 32767) c->compact = 0;
     c->male_nonneg = 1;
     for (int64_t e = 0; e < c->male.m; e++)
+    {
         if (c->male.out.adj[e].y < 0) c->male_nonneg = 0;
+        if (c->male.out.adj[e].y > c->max_mw) c->max_mw = c->male.out.adj[e].y;
+    }
     for (int32_t r = 1; r <= n; r++) {
         c->f_out_deg[r] = (int32_t)(fg.out.ptr[r + 1] - fg.out.ptr[r]);
         c->f_in_deg[r] = (int32_t)(fg.in.ptr[r + 1] - fg.in.ptr[r]);
@@ -662,7 +668,8 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_self, (size_t)n + 1);
     if (rc == BM_OK) rc = h2d(c, c->d_m_self, c->h_m_self, (size_t)n + 1);
     if (rc == BM_OK) rc = h2d(c, c->d_f_self, c->h_f_self, (size_t)n + 1);
-    c->rows_fit = gain_overflow(c) == 0;
+    c->rows_fit = gain_overflow(c, INT32_MAX) == 0;
+    c->rows_small = gain_overflow(c, 1 << 28) == 0;
     for (int32_t r = 1; r <= n; r++)
         c->row_adds += ((double)c->f_out_deg[r] * c->f_out_deg[r] + (double)c->f_in_deg[r] * c->f_in_deg[r]) / n;
     c->pi_distinct = 1;   /* all unmatched */
@@ -704,14 +711,18 @@ extern "C" int bm_set_mapping(bm_ctx* c, const int32_t* pi) {
     /* the matching and its inverse in one upload (entries 0 are 0) */
     const size_t len = (size_t)c->n + 1;
     std::vector<int32_t> both(2 * len, 0);
-    c->pi_distinct = 1;
+    c->pi_distinct = c->pi_full = 1;
     for (int32_t i = 1; i <= c->n; i++) {
         const int32_t f = pi[i];
         both[(size_t)i] = f;
-        if (f == 0) continue;
+        if (f == 0) {
+            c->pi_full = 0;
+            continue;
+        }
         if (both[len + (size_t)f] != 0) c->pi_distinct = 0;
         both[len + (size_t)f] = i;
     }
+    if (!c->pi_distinct) c->pi_full = 0;
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipMemcpyAsync(c->d_pi, both.data(), 2 * len * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     const int rc = c->gain_on ? gain_rebuild(c) : BM_OK;
@@ -1555,18 +1566,27 @@ extern "C" int bm_best_swap(bm_ctx* c, int64_t* delta, int32_t* u, int32_t* v) {
     if (!c || !delta || !u || !v) return fail(c, BM_ERR_ARG, "bm_best_swap: null argument");
     if (!c->gain_on) return fail(c, BM_ERR_ARG, "bm_best_swap: needs the placement-gain table (bm_gain_enable)");
     HIPCHK(c, hipSetDevice(c->device));
-    int rc = gain_transposed(c);
+    /* the table alone while every male has an image of its own; otherwise by
+     * first vertex, with the transposed copy */
+    const bool tiles = c->pi_full && c->packed && c->rows_small && c->d_m_adj;
+    int rc = tiles ? BM_OK : gain_transposed(c);
+    if (rc == BM_OK && !c->d_pis) rc = dalloc(c, &c->d_pis, (size_t)c->n + 1);
+    if (rc == BM_OK && !c->d_best) rc = dalloc(c, &c->d_best, (size_t)kBestSwapParts + 1);
     if (rc != BM_OK) return rc;
-    if (!c->d_best && (rc = dalloc(c, &c->d_best, (size_t)kBestSwapParts + 1)) != BM_OK) return rc;
+    int4* out = reinterpret_cast<int4*>(c->h_pin);
     KTiming t;
     timing_begin(c, BM_KERNEL_GAIN_SWAP, &t);
     HIPCHK(c, bm_launch_gain_pis(devgraph(c), devgain(c), c->d_pis, c->stream));
-    HIPCHK(c, bm_launch_gain_best_swap(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_best + 1, kBestSwapParts,
-                                       c->d_best, c->num_cus, c->stream));
+    if (tiles)
+        HIPCHK(c, bm_launch_gain_best_tiles(devgraph(c), devgain(c), c->d_pis, c->d_chunks, c->n_out_chunks, c->max_mw,
+                                            reinterpret_cast<int32_t*>(c->d_best), c->d_best + 1, kBestSwapParts, out,
+                                            c->num_cus, c->stream));
+    else
+        HIPCHK(c, bm_launch_gain_best_swap(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_best + 1, kBestSwapParts,
+                                           out, c->num_cus, c->stream));
     timing_end(c, &t);
-    int4 h;
-    HIPCHK(c, hipMemcpyAsync(&h, c->d_best, sizeof h, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const int4 h = *out;
     if (h.z == INT32_MAX) {   /* n < 2: no pair */
         *delta = 0;
         *u = *v = 0;
@@ -1672,7 +1692,7 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
     const bm_graph_host& mg = c->male;
     if (!c->rows_fit)
         return fail(c, BM_ERR_ARG, "bm_gain_enable: vertex %d's incident weights can exceed int32 in the table",
-                    gain_overflow(c));
+                    gain_overflow(c, INT32_MAX));
     const size_t bytes = (size_t)bm_gain_table_bytes(c->n);
     size_t free_b = 0, total_b = 0;
     HIPCHK(c, hipMemGetInfo(&free_b, &total_b));

@@ -166,6 +166,12 @@ hipError_t bm_launch_gain_swap_umajor(const BmDevGraph& g, const BmGain& G, cons
 constexpr int32_t kBestSwapParts = 2048;
 hipError_t bm_launch_gain_best_swap(const BmDevGraph& g, const BmGain& G, const int32_t* GT, const int4* pis,
                                     int4* part, int32_t max_parts, int4* out, int32_t num_cus, hipStream_t s);
+/* The same from the table alone (no transposed copy), while every male is
+ * matched, no female is shared (g.inv), male weights are in 0..max_w, |G| <=
+ * 2^28 and G.m_adj is kept; chunks: the male out-lists'. */
+hipError_t bm_launch_gain_best_tiles(const BmDevGraph& g, const BmGain& G, const int4* pis, const int4* chunks,
+                                     int64_t n_out_chunks, int32_t max_w, int32_t* thr, int4* part, int32_t max_parts,
+                                     int4* out, int32_t num_cus, hipStream_t s);
 /* Best partner of each u in u0 .. u0 + count - 1 over v = u+1..n: out[i] =
  * {delta lo, delta hi, u0 + i, v} (ties to the smaller v; delta INT64_MIN and
  * v INT32_MAX for u = n). */

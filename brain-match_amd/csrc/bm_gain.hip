@@ -40,6 +40,7 @@
 #include "bm_device.h"
 #include "bm_devutil.h"
 #include "bm_rng.h"
+#include "bm_rowtab.h"
 
 using namespace bmd;
 
@@ -989,7 +990,7 @@ __global__ void __launch_bounds__(kBestThreads) k_gain_best_partners(BmDevGraph 
 }
 
 __global__ void __launch_bounds__(kBestThreads) k_best_swap_final(const int4* __restrict__ part, int32_t nparts,
-                                                                  int4* __restrict__ out) {
+                                                                  int4* __restrict__ out /* pinned */) {
     int64_t bd = INT64_MIN;
     int32_t bu = INT32_MAX, bv = INT32_MAX;
     for (int32_t i = threadIdx.x; i < nparts; i += kBestThreads) {
@@ -1000,6 +1001,173 @@ __global__ void __launch_bounds__(kBestThreads) k_best_swap_final(const int4* __
     best_block_reduce(bd, bu, bv);
     if (threadIdx.x == 0)
         out[0] = make_int4((int32_t)(uint32_t)(uint64_t)bd, (int32_t)(uint32_t)((uint64_t)bd >> 32), bu, bv);
+}
+
+/* ---- best swap from the table alone --------------------------------- */
+
+/* While every male is matched and no female is shared, number the vertices by
+ * their images: with H(f, f') = G(inv(f), f') the rows of H are whole rows of
+ * the table in another order, and the pair {inv(f), inv(f')} has
+ *   H(f, f') + H(f', f) - diagonals (+ self-loops, + the u <-> v correction).
+ * So the table is read once, as 64 x 64 tiles of H against their mirror tiles
+ * transposed through LDS, and needs no transposed copy to be kept, patched or
+ * rebuilt: its 1.37 GB at n = 18,524 are what bounds the search (299 us, 4.6
+ * TB/s, and 146 us for 4M edges; by first vertex with a transposed copy 3.15
+ * ms and 0.54 ms for the copy).  The
+ * correction of adjacent pairs is left out here: a pair that would be the best
+ * so far is looked up in the adjacency bitmap and dropped if adjacent (rare,
+ * since all blocks share the best value found), and k_best_edges goes through
+ * the male edges.  Sums are 32-bit: |G| <= 2^28 (the caller checks). */
+constexpr int kTile = 64, kTilePad = kTile + 1;
+constexpr int32_t kNoVertex = 1 << 29;   /* "diagonal" of a row or column outside 1..n (vertex 0): rarely near the best */
+
+struct BestPair {
+    int32_t d, u, v;
+};
+__device__ __forceinline__ bool pair_before(const BestPair& a, const BestPair& b) {
+    return a.d > b.d || (a.d == b.d && (a.u < b.u || (a.u == b.u && a.v < b.v)));
+}
+
+__device__ __forceinline__ void best_to_part(const BestPair& b, int4* part) {
+    int64_t d = b.u == INT32_MAX ? INT64_MIN : (int64_t)b.d;
+    int32_t u = b.u, v = b.v;
+    best_block_reduce(d, u, v);
+    if (threadIdx.x == 0)
+        *part = make_int4((int32_t)(uint32_t)(uint64_t)d, (int32_t)(uint32_t)((uint64_t)d >> 32), u, v);
+}
+
+__global__ void k_best_init(int32_t* thr) { *thr = INT32_MIN; }
+
+__global__ void __launch_bounds__(kBestThreads) k_best_tiles(BmDevGraph g, BmGain G, const int4* __restrict__ pis,
+                                                             int32_t tiles, int32_t* __restrict__ thr,
+                                                             int4* __restrict__ part) {
+    __shared__ int32_t s_t[kTile * kTilePad];
+    __shared__ int4 s_i[kTile], s_j[kTile];   /* {vertex, diagonal, male self-loop, female self-loop} by image */
+    __shared__ int32_t s_thr;
+    static_assert(kBestThreads == 256, "16 entries of each tile per thread");
+    const int t = threadIdx.x, c4 = 4 * (t % 16), r0 = t / 16;
+    const int64_t total = (int64_t)tiles * (tiles + 1) / 2;
+    BestPair best = {INT32_MIN, INT32_MAX, INT32_MAX};
+    for (int64_t p = blockIdx.x; p < total; p += gridDim.x) {
+        /* p -> (I <= J), row I of the triangle after I tiles of row I - 1, ... */
+        const double b = 2.0 * tiles + 1.0;
+        int64_t I = (int64_t)((b - sqrt(b * b - 8.0 * (double)p)) * 0.5);
+        while (I > 0 && I * (2 * (int64_t)tiles - I + 1) / 2 > p) I--;
+        while ((I + 1) * (2 * (int64_t)tiles - I) / 2 <= p) I++;
+        const int64_t J = I + (p - I * (2 * (int64_t)tiles - I + 1) / 2);
+        __syncthreads();   /* the previous tile has been read */
+        if (t < 2 * kTile) {
+            const int64_t f = (t < kTile ? I : J) * kTile + t % kTile;
+            int4 e = make_int4(0, kNoVertex, BM_ABSENT, BM_ABSENT);
+            if (f >= 1 && f <= g.n) {
+                const int32_t x = g.inv[f];
+                e = pis[x];
+                e.x = x;
+            }
+            (t < kTile ? s_i : s_j)[t % kTile] = e;
+        }
+        if (t == 0) s_thr = *reinterpret_cast<volatile int32_t*>(thr);
+        __syncthreads();
+        int4 a[4], m[4];   /* rows of tile (I, J) and of its mirror (J, I) */
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            a[k] = *reinterpret_cast<const int4*>(&G.G[(int64_t)s_i[r0 + 16 * k].x * G.stride + J * kTile + c4]);
+            m[k] = *reinterpret_cast<const int4*>(&G.G[(int64_t)s_j[r0 + 16 * k].x * G.stride + I * kTile + c4]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            int32_t* q = &s_t[(r0 + 16 * k) * kTilePad + c4];
+            q[0] = m[k].x;
+            q[1] = m[k].y;
+            q[2] = m[k].z;
+            q[3] = m[k].w;
+        }
+        __syncthreads();
+        int32_t lim = s_thr;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = r0 + 16 * k;
+            const int4 pi = s_i[i];
+            const int32_t h[4] = {a[k].x, a[k].y, a[k].z, a[k].w};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int j = c4 + q;
+                const int4 pj = s_j[j];
+                int32_t d = h[q] + s_t[j * kTilePad + i] - pi.y - pj.y;
+                if (pi.z != BM_ABSENT) d += contrib(pi.z, pj.w) - contrib(pi.z, pi.w);
+                if (pj.z != BM_ABSENT) d += contrib(pj.z, pi.w) - contrib(pj.z, pj.w);
+                if (d >= lim && pi.x != 0 && pj.x != 0 && (I != J || i < j)) {
+                    const int32_t u = pi.x < pj.x ? pi.x : pj.x, v = pi.x < pj.x ? pj.x : pi.x;
+                    const BestPair c = {d, u, v};
+                    if (pair_before(c, best) && !male_maybe(G, u, v)) {
+                        best = c;
+                        lim = d;
+                    }
+                }
+            }
+        }
+        if (lim > s_thr) atomicMax(&s_thr, lim);
+        __syncthreads();
+        if (t == 0 && s_thr > *reinterpret_cast<volatile int32_t*>(thr)) atomicMax(thr, s_thr);
+    }
+    best_to_part(best, &part[blockIdx.x]);
+}
+
+/* The best adjacent pair: one wave per chunk of an out-list, four edges u -> v
+ * per lane.  A pair is put right only where it could still reach the best: the
+ * correction of an edge of weight w is at most 2 w (weights are not negative
+ * here), and v -> u is looked up only then. */
+template <bool PACKED>
+__global__ void __launch_bounds__(kBestThreads) k_best_edges(BmDevGraph g, BmGain G, const int4* __restrict__ pis,
+                                                             const int4* __restrict__ chunks, int64_t nchunks,
+                                                             int32_t max_w, const int32_t* __restrict__ thr,
+                                                             int4* __restrict__ part) {
+    constexpr int U = BM_EDGE_CHUNK / BM_WAVE;
+    const int lane = threadIdx.x & (BM_WAVE - 1);
+    const int64_t nw = (int64_t)gridDim.x * (kBestThreads / BM_WAVE);
+    BestPair best = {INT32_MIN, INT32_MAX, INT32_MAX};
+    const int32_t lim = *thr;
+    for (int64_t ci = (int64_t)blockIdx.x * (kBestThreads / BM_WAVE) + uni(threadIdx.x / BM_WAVE); ci < nchunks; ci += nw) {
+        const int4 ch = chunks[ci];
+        const int32_t u = uni(ch.x), cnt = uni(ch.w);
+        const int2* adj = g.m_out + g.m_out_ptr[u] + uni(ch.z);
+        const int4 pu = pis[u];
+        int2 e[U];
+        int4 pv[U];
+        int32_t gu[U], gv[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int32_t i = lane + BM_WAVE * j;
+            e[j] = i < cnt ? adj[i] : make_int2(0, 0);
+            if (e[j].x == u) e[j].x = 0;   /* a self-loop */
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) pv[j] = pis[e[j].x];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            gu[j] = G.G[(int64_t)u * G.stride + pv[j].x];
+            gv[j] = G.G[(int64_t)e[j].x * G.stride + pu.x];
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int32_t v = e[j].x;
+            if (v == 0) continue;
+            int32_t d = gu[j] + gv[j] - pu.y - pv[j].y;
+            if (pu.z != BM_ABSENT) d += contrib(pu.z, pv[j].w) - contrib(pu.z, pu.w);
+            if (pv[j].z != BM_ABSENT) d += contrib(pv[j].z, pu.w) - contrib(pv[j].z, pv[j].w);
+            const int32_t uv = e[j].y;
+            if ((int64_t)d + 2 * uv + 2 * max_w < lim) continue;
+            const int32_t vu = row_find<PACKED>(g.m_in_t.tab, g.m_in_t.desc[u], v);
+            const int32_t F12 = row_find<PACKED>(g.f_out_t.tab, g.f_out_t.desc[pu.x], pv[j].x);
+            const int32_t F21 = row_find<PACKED>(g.f_in_t.tab, g.f_in_t.desc[pu.x], pv[j].x);
+            const int32_t F11 = pu.w, F22 = pv[j].w;
+            d += contrib(uv, F21) - contrib(uv, F22) - contrib(uv, F11) + contrib(uv, F12);
+            if (vu != BM_ABSENT) d += contrib(vu, F12) - contrib(vu, F11) - contrib(vu, F22) + contrib(vu, F21);
+            const BestPair c = {d, u < v ? u : v, u < v ? v : u};
+            if (pair_before(c, best)) best = c;
+        }
+    }
+    best_to_part(best, &part[blockIdx.x]);
 }
 
 /* Transposed table: GT(f, u) = G(u, f) for f < nrows, with GT(f, u) = 0 in
@@ -1740,6 +1908,27 @@ hipError_t bm_launch_gain_best_swap(const BmDevGraph& g, const BmGain& G, const 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_best_swap_final, dim3(1), dim3(kBestThreads), 0, s, part, (int32_t)blocks, out);
+    return hipGetLastError();
+}
+
+hipError_t bm_launch_gain_best_tiles(const BmDevGraph& g, const BmGain& G, const int4* pis, const int4* chunks,
+                                     int64_t n_out_chunks, int32_t max_w, int32_t* thr, int4* part, int32_t max_parts,
+                                     int4* out, int32_t num_cus, hipStream_t s) {
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    const int32_t tiles = (g.n + kTile) / kTile;   /* images 0..n */
+    int64_t tb = (int64_t)tiles * (tiles + 1) / 2, eb = (n_out_chunks + 3) / 4;
+    if (tb > 6 * cus) tb = 6 * cus;
+    if (tb > max_parts / 2) tb = max_parts / 2;
+    if (eb > 6 * cus) eb = 6 * cus;
+    if (eb > max_parts / 2) eb = max_parts / 2;
+    hipLaunchKernelGGL(k_best_init, dim3(1), dim3(1), 0, s, thr);
+    hipLaunchKernelGGL(k_best_tiles, dim3((unsigned)tb), dim3(kBestThreads), 0, s, g, G, pis, tiles, thr, part);
+    if (eb > 0) {
+        auto kern = g.packed ? k_best_edges<true> : k_best_edges<false>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)eb), dim3(kBestThreads), 0, s, g, G, pis, chunks, n_out_chunks, max_w, thr,
+                           part + tb);
+    }
+    hipLaunchKernelGGL(k_best_swap_final, dim3(1), dim3(kBestThreads), 0, s, part, (int32_t)(tb + eb), out);
     return hipGetLastError();
 }
 
