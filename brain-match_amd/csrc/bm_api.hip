@@ -86,8 +86,8 @@ struct bm_ctx {
     int32_t* d_f_self;
     int4* d_moves;
     int64_t moves_cap;
-    int64_t* d_patch_plan;  /* 4 moves_cap + 1 work-item offsets of a table patch */
     int64_t* d_nmoves;
+    int32_t* d_patch_rows;  /* rows touched by a table patch (bm_gain_update_rows) */
     int64_t gain_version;   /* bumped by every build and patch of the table */
     /* u-major evaluation (bm_batch_eval_swaps_umajor) */
     int32_t* d_um_counts;   /* n+1 */
@@ -295,8 +295,8 @@ static void free_ctx(bm_ctx* c) {
     (void)hipFree(c->d_m_self);
     (void)hipFree(c->d_f_self);
     (void)hipFree(c->d_moves);
-    (void)hipFree(c->d_patch_plan);
     (void)hipFree(c->d_nmoves);
+    (void)hipFree(c->d_patch_rows);
     (void)hipFree(c->d_um_counts);
     (void)hipFree(c->d_um_off);
     (void)hipFree(c->d_GT);
@@ -371,12 +371,9 @@ static int gain_moves_cap(bm_ctx* c, int64_t need) {
     if (c->moves_cap >= need) return BM_OK;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     (void)hipFree(c->d_moves);
-    (void)hipFree(c->d_patch_plan);
     c->d_moves = nullptr;
-    c->d_patch_plan = nullptr;
     c->moves_cap = 0;
     HIPCHK(c, hipMalloc((void**)&c->d_moves, (size_t)need * sizeof(int4)));
-    HIPCHK(c, hipMalloc((void**)&c->d_patch_plan, (size_t)(4 * need + 1) * sizeof(int64_t)));
     c->moves_cap = need;
     return BM_OK;
 }
@@ -388,7 +385,7 @@ static int64_t male_degree(const bm_ctx* c, int32_t x) {
 
 /* Whether a patch of moves of the vertices xs (k of them) should also patch
  * the transposed copy: its additions land in as many rows as the moved
- * vertices have male edges, one 4-byte atomic per row and female entry, so it
+ * vertices have male edges, one 4-byte add per row and female entry, so it
  * pays against a 0.54 ms transpose (n = 18,524) only for moves of vertices of
  * ordinary degree (together at most 8x the mean); hub moves leave the copy to
  * be rebuilt. */
@@ -409,7 +406,7 @@ static int gain_patch(bm_ctx* c, const int64_t* d_count, int64_t max_moves, bool
      * the caller found that cheaper (gt_patch_pays) */
     const bool gt = gt_allowed && c->d_GT && c->gt_version == c->gain_version;
     HIPCHK(c, bm_launch_gain_update(devgraph(c), devgain(c), gt ? c->d_GT : nullptr, c->d_moves, d_count, max_moves,
-                                    c->d_patch_plan, c->num_cus, c->stream));
+                                    c->d_patch_rows, c->num_cus, c->stream));
     timing_end(c, &t);
     c->gain_version++;
     if (gt) c->gt_version = c->gain_version;
@@ -1706,6 +1703,7 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
         int rc = dalloc(c, &c->d_m_out_desc, (size_t)c->n + 1);
         if (rc == BM_OK) rc = dalloc(c, &c->d_m_out_tab, (size_t)(hm.slots ? hm.slots : 2));
         if (rc == BM_OK) rc = dalloc(c, &c->d_nmoves, 1);
+        if (rc == BM_OK) rc = dalloc(c, &c->d_patch_rows, (size_t)bm_gain_update_rows(c->n));
         if (rc == BM_OK) rc = h2d(c, c->d_m_out_desc, hm.desc, (size_t)c->n + 1);
         if (rc == BM_OK) rc = h2d(c, c->d_m_out_tab, hm.tab, (size_t)hm.slots);
         if (rc == BM_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, BM_ERR_HIP, "sync failed");

@@ -128,11 +128,12 @@ hipError_t bm_launch_row_bounds(const int64_t* ptr, const int2* rows, int32_t n,
 /* Table build: per column chunk, the work list (k_gain_edge_desc) then the
  * rows.  G.edesc must hold 2 x male edges + 1 entries. */
 hipError_t bm_launch_gain_build(const BmDevGraph& g, const BmGain& G, int32_t num_cus, hipStream_t s);
-/* Table patch after moves (moves[0..*count), *count <= max_moves); plan
- * holds 4 max_moves + 1 int64 of scratch for the work-item offsets; GT (may
- * be NULL) is a transposed copy patched alongside. */
+/* Table patch after moves (moves[0..*count), *count <= max_moves); rows is
+ * scratch of bm_gain_update_rows(n) int32 for the rows touched; GT (may be
+ * NULL) is a transposed copy patched alongside. */
+int64_t bm_gain_update_rows(int32_t n);
 hipError_t bm_launch_gain_update(const BmDevGraph& g, const BmGain& G, int32_t* GT, const int4* moves, const int64_t* count,
-                                 int64_t max_moves, int64_t* plan, int32_t num_cus, hipStream_t s);
+                                 int64_t max_moves, int32_t* rows, int32_t num_cus, hipStream_t s);
 /* Per-pair table lookups; with pis (the per-vertex words, refreshed) the
  * diagonal entries and self-loops come from them. */
 hipError_t bm_launch_gain_swap(const BmDevGraph& g, const BmGain& G, int mode, const int2* cand, const int64_t* off,
@@ -307,7 +308,8 @@ hipError_t bm_launch_gen_changed_triples(int32_t n, int32_t c, const int32_t* re
 hipError_t bm_launch_check_pairs(int32_t n, const int2* cand, int64_t k, int32_t* bad, hipStream_t s);
 hipError_t bm_launch_check_triples(int32_t n, const int4* cand, int64_t k, int32_t* bad, hipStream_t s);
 
-/* Reductions over int64 deltas.  part must hold bm_stats_parts(k) * 6 int64. */
+/* Reductions over k > 0 int64 deltas (16-byte aligned).  part must hold
+ * bm_stats_blocks(k) * 5 int64; out6 and out may be pinned host memory. */
 int64_t bm_stats_blocks(int64_t k);
 hipError_t bm_launch_stats(const int64_t* d, int64_t k, int64_t* part, int64_t* out6, hipStream_t s);
 /* rank-th index with delta > 0 (kind 1) or == 0 (kind 0); out = -1 if none.
