@@ -1396,13 +1396,12 @@ extern "C" int bm_batch_stats(bm_batch* b, bm_stats* out) {
     bm_ctx* c = b->ctx;
     if (!b->evaluated) return fail(c, BM_ERR_STATE, "bm_batch_stats: batch not evaluated");
     HIPCHK(c, hipSetDevice(c->device));
-    int64_t h[6];
+    const int64_t* h = c->h_pin;
     if (b->k == 0) {
         out->count = 0; out->sum = 0; out->max = INT64_MIN; out->argmax = -1; out->n_pos = 0; out->n_zero = 0;
         return BM_OK;
     }
-    HIPCHK(c, bm_launch_stats(b->d_delta, b->k, b->d_part, b->d_out, c->stream));
-    HIPCHK(c, hipMemcpyAsync(h, b->d_out, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, bm_launch_stats(b->d_delta, b->k, b->d_part, c->h_pin, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     out->count = h[0]; out->sum = h[1]; out->max = h[2]; out->argmax = h[3]; out->n_pos = h[4]; out->n_zero = h[5];
     return BM_OK;
@@ -1416,9 +1415,9 @@ extern "C" int bm_batch_pick(bm_batch* b, int32_t kind, int64_t rank, int64_t* i
     *index = -1;
     if (rank < 0 || b->k == 0) return BM_OK;
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, bm_launch_pick(b->d_delta, b->k, kind, rank, b->d_part, b->d_out, c->stream));
-    HIPCHK(c, hipMemcpyAsync(index, b->d_out, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, bm_launch_pick(b->d_delta, b->k, kind, rank, b->d_part, c->h_pin, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    *index = c->h_pin[0];
     return BM_OK;
 }
 

@@ -133,161 +133,210 @@ __global__ void k_check_triples(int32_t n, const int4* __restrict__ cand, int64_
 /* Reductions                                                          */
 /* ------------------------------------------------------------------ */
 
+/* A batch's deltas are read once by at most kRedBlocks blocks, one chunk of a
+ * power of two each, so that the one block which combines the partial results
+ * has at most eight per thread; up to 2^25 deltas the chunk is 4,096.  What
+ * bounds both passes is the read: 16-byte loads, eight in flight per thread,
+ * and shuffles instead of an LDS tree (2^28 deltas: stats 465 + 165 us ->
+ * 378 + 12 us; the pick's count 405 us -> 342 us). */
 constexpr int kRedThreads = 256;
-constexpr int kRedChunk = 4096;   /* elements per block */
+constexpr int kRedWaves = kRedThreads / BM_WAVE;
+constexpr int64_t kRedChunk = 4096;    /* smallest chunk */
+constexpr int64_t kRedBlocks = 8192;
+constexpr int kRedLoads = 8;
+constexpr int kFinThreads = 1024;
+constexpr int kFinWaves = kFinThreads / BM_WAVE;
 
-__global__ void __launch_bounds__(kRedThreads) k_stats_part(const int64_t* __restrict__ d, int64_t k,
-                                                            int64_t* __restrict__ part) {
-    __shared__ int64_t s_sum[kRedThreads], s_max[kRedThreads], s_arg[kRedThreads], s_pos[kRedThreads],
-        s_zero[kRedThreads];
-    const int64_t base = (int64_t)blockIdx.x * kRedChunk;
-    int64_t sum = 0, mx = INT64_MIN, arg = -1, pos = 0, zero = 0;
-    for (int q = threadIdx.x; q < kRedChunk; q += kRedThreads) {
-        const int64_t i = base + q;
-        if (i >= k) break;
-        const int64_t x = d[i];
-        sum += x;
+int64_t red_chunk(int64_t k) {
+    int64_t chunk = kRedChunk;
+    while (chunk * kRedBlocks < k) chunk *= 2;
+    return chunk;
+}
+
+struct Stats {
+    int64_t sum, max, arg, pos, zero;   /* arg: first index of max, -1 none */
+};
+
+__device__ __forceinline__ void stats_join(Stats& a, const Stats& b) {
+    a.sum += b.sum;
+    a.pos += b.pos;
+    a.zero += b.zero;
+    if (b.arg >= 0 && (a.arg < 0 || b.max > a.max || (b.max == a.max && b.arg < a.arg))) {
+        a.max = b.max;
+        a.arg = b.arg;
+    }
+}
+
+/* All threads' results joined in thread 0; s: one entry per wave. */
+template <int WAVES>
+__device__ __forceinline__ Stats stats_block(Stats a, Stats* s) {
+#pragma unroll
+    for (int o = BM_WAVE / 2; o > 0; o >>= 1) {
+        const Stats b = {__shfl_down(a.sum, o), __shfl_down(a.max, o), __shfl_down(a.arg, o), __shfl_down(a.pos, o),
+                         __shfl_down(a.zero, o)};
+        stats_join(a, b);   /* lanes past the wave's end repeat their own: only lane 0 counts */
+    }
+    if ((threadIdx.x & (BM_WAVE - 1)) == 0) s[threadIdx.x / BM_WAVE] = a;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < WAVES; w++) stats_join(a, s[w]);
+    return a;
+}
+
+__device__ __forceinline__ void stats_put(const Stats& a, int64_t k, int64_t* out) {
+    out[0] = k; out[1] = a.sum; out[2] = a.max; out[3] = a.arg; out[4] = a.pos; out[5] = a.zero;
+}
+
+/* Partial results of chunk b at part[field * blocks + b]; a single chunk's
+ * are the answer. */
+__global__ void __launch_bounds__(kRedThreads) k_stats_part(const int64_t* __restrict__ d, int64_t k, int64_t chunk,
+                                                            int64_t* __restrict__ part, int64_t* __restrict__ out) {
+    __shared__ Stats s[kRedWaves];
+    const int64_t base = (int64_t)blockIdx.x * chunk;
+    const int64_t end = k - base < chunk ? k : base + chunk;
+    Stats a = {0, INT64_MIN, -1, 0, 0};
+    int32_t pos = 0, zero = 0;
+    auto take = [&](int64_t x, int64_t i) {
+        a.sum += x;
         pos += x > 0;
         zero += x == 0;
-        if (x > mx) { mx = x; arg = i; }
-    }
-    s_sum[threadIdx.x] = sum; s_max[threadIdx.x] = mx; s_arg[threadIdx.x] = arg;
-    s_pos[threadIdx.x] = pos; s_zero[threadIdx.x] = zero;
-    __syncthreads();
-    for (int o = kRedThreads / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            const int a = threadIdx.x, b = threadIdx.x + o;
-            s_sum[a] += s_sum[b];
-            s_pos[a] += s_pos[b];
-            s_zero[a] += s_zero[b];
-            if (s_max[b] > s_max[a] || (s_max[b] == s_max[a] && s_arg[b] >= 0 && (s_arg[a] < 0 || s_arg[b] < s_arg[a]))) {
-                s_max[a] = s_max[b];
-                s_arg[a] = s_arg[b];
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        int64_t* o = part + (int64_t)blockIdx.x * 5;
-        o[0] = s_sum[0]; o[1] = s_max[0]; o[2] = s_arg[0]; o[3] = s_pos[0]; o[4] = s_zero[0];
-    }
-}
-
-__global__ void __launch_bounds__(kRedThreads) k_stats_final(const int64_t* __restrict__ part, int64_t nb, int64_t k,
-                                                             int64_t* __restrict__ out) {
-    __shared__ int64_t s_sum[kRedThreads], s_max[kRedThreads], s_arg[kRedThreads], s_pos[kRedThreads],
-        s_zero[kRedThreads];
-    int64_t sum = 0, mx = INT64_MIN, arg = -1, pos = 0, zero = 0;
-    for (int64_t b = threadIdx.x; b < nb; b += kRedThreads) {
-        const int64_t* p = part + b * 5;
-        sum += p[0];
-        pos += p[3];
-        zero += p[4];
-        if (p[2] >= 0 && (p[1] > mx || (p[1] == mx && (arg < 0 || p[2] < arg)))) { mx = p[1]; arg = p[2]; }
-    }
-    s_sum[threadIdx.x] = sum; s_max[threadIdx.x] = mx; s_arg[threadIdx.x] = arg;
-    s_pos[threadIdx.x] = pos; s_zero[threadIdx.x] = zero;
-    __syncthreads();
-    for (int o = kRedThreads / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            const int a = threadIdx.x, b = threadIdx.x + o;
-            s_sum[a] += s_sum[b];
-            s_pos[a] += s_pos[b];
-            s_zero[a] += s_zero[b];
-            if (s_arg[b] >= 0 && (s_max[b] > s_max[a] || (s_max[b] == s_max[a] && (s_arg[a] < 0 || s_arg[b] < s_arg[a])))) {
-                s_max[a] = s_max[b];
-                s_arg[a] = s_arg[b];
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[0] = k; out[1] = s_sum[0]; out[2] = s_max[0]; out[3] = s_arg[0]; out[4] = s_pos[0]; out[5] = s_zero[0];
-    }
-}
-
-__global__ void __launch_bounds__(kRedThreads) k_pick_count(const int64_t* __restrict__ d, int64_t k, int32_t kind,
-                                                            int64_t* __restrict__ cnt) {
-    __shared__ int64_t s[kRedThreads];
-    const int64_t base = (int64_t)blockIdx.x * kRedChunk;
-    int64_t c = 0;
-    for (int q = threadIdx.x; q < kRedChunk; q += kRedThreads) {
-        const int64_t i = base + q;
-        if (i >= k) break;
-        const int64_t x = d[i];
-        c += kind ? (x > 0) : (x == 0);
-    }
-    s[threadIdx.x] = c;
-    __syncthreads();
-    for (int o = kRedThreads / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) cnt[blockIdx.x] = s[0];
-}
-
-/* One block: locate the chunk holding the rank-th match, then the element. */
-__global__ void __launch_bounds__(1024) k_pick_find(const int64_t* __restrict__ d, int64_t k, int32_t kind,
-                                                    const int64_t* __restrict__ cnt, int64_t nb, int64_t rank,
-                                                    int64_t* __restrict__ out) {
-    __shared__ int64_t s[1024];
-    __shared__ int64_t s_chunk, s_before;
-    const int t = threadIdx.x;
-    const int64_t per = (nb + 1023) / 1024;
-    const int64_t b0 = (int64_t)t * per, b1 = b0 + per < nb ? b0 + per : nb;
-    int64_t mine = 0;
-    for (int64_t b = b0; b < b1; b++) mine += cnt[b];
-    s[t] = mine;
-    if (t == 0) { s_chunk = -1; s_before = 0; }
-    __syncthreads();
-    /* inclusive scan (Hillis-Steele) */
-    for (int o = 1; o < 1024; o <<= 1) {
-        int64_t x = t >= o ? s[t - o] : 0;
-        __syncthreads();
-        s[t] += x;
-        __syncthreads();
-    }
-    const int64_t incl = s[t], excl = incl - mine;
-    if (rank >= excl && rank < incl) {
-        int64_t acc = excl;
-        for (int64_t b = b0; b < b1; b++) {
-            if (rank < acc + cnt[b]) { s_chunk = b; s_before = acc; break; }
-            acc += cnt[b];
+        if (x > a.max) { a.max = x; a.arg = i; }
+    };
+    int64_t i = base;
+    constexpr int64_t kStep = 2 * kRedThreads * kRedLoads;
+    for (; i + kStep <= end; i += kStep) {
+        longlong2 x[kRedLoads];
+#pragma unroll
+        for (int j = 0; j < kRedLoads; j++)
+            x[j] = reinterpret_cast<const longlong2*>(d + i)[j * kRedThreads + threadIdx.x];
+#pragma unroll
+        for (int j = 0; j < kRedLoads; j++) {
+            const int64_t at = i + 2 * (j * kRedThreads + threadIdx.x);
+            take(x[j].x, at);
+            take(x[j].y, at + 1);
         }
     }
-    __syncthreads();
-    if (s_chunk < 0) {
-        if (t == 0) out[0] = -1;
+    for (i += threadIdx.x; i < end; i += kRedThreads) take(d[i], i);
+    a.pos = pos;
+    a.zero = zero;
+    a = stats_block<kRedWaves>(a, s);
+    if (threadIdx.x) return;
+    const int64_t nb = gridDim.x;
+    if (nb == 1) {
+        stats_put(a, k, out);
         return;
     }
-    /* within the chunk: 4 elements per thread, block prefix over counts */
-    const int64_t base = s_chunk * kRedChunk;
-    int64_t local = 0;
-    int flags[4];
+    int64_t* o = part + blockIdx.x;
+    o[0] = a.sum; o[nb] = a.max; o[2 * nb] = a.arg; o[3 * nb] = a.pos; o[4 * nb] = a.zero;
+}
+
+__global__ void __launch_bounds__(kFinThreads) k_stats_final(const int64_t* __restrict__ part, int64_t nb, int64_t k,
+                                                             int64_t* __restrict__ out) {
+    __shared__ Stats s[kFinWaves];
+    Stats a = {0, INT64_MIN, -1, 0, 0};
+#pragma unroll 4
+    for (int64_t b = threadIdx.x; b < nb; b += kFinThreads) {
+        const int64_t* p = part + b;
+        stats_join(a, {p[0], p[nb], p[2 * nb], p[3 * nb], p[4 * nb]});
+    }
+    a = stats_block<kFinWaves>(a, s);
+    if (threadIdx.x == 0) stats_put(a, k, out);
+}
+
+__device__ __forceinline__ bool picked(int64_t x, int32_t kind) { return kind ? x > 0 : x == 0; }
+
+__global__ void __launch_bounds__(kRedThreads) k_pick_count(const int64_t* __restrict__ d, int64_t k, int32_t kind,
+                                                            int64_t chunk, int64_t* __restrict__ cnt) {
+    __shared__ int32_t s[kRedWaves];
+    const int64_t base = (int64_t)blockIdx.x * chunk;
+    const int64_t end = k - base < chunk ? k : base + chunk;
+    int32_t c = 0;
+    int64_t i = base;
+    constexpr int64_t kStep = 2 * kRedThreads * kRedLoads;
+    for (; i + kStep <= end; i += kStep) {
+        longlong2 x[kRedLoads];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int64_t i = base + (int64_t)t * 4 + q;
-        const int64_t x = i < k ? d[i] : -1;
-        flags[q] = i < k && (kind ? (x > 0) : (x == 0));
-        local += flags[q];
+        for (int j = 0; j < kRedLoads; j++)
+            x[j] = reinterpret_cast<const longlong2*>(d + i)[j * kRedThreads + threadIdx.x];
+#pragma unroll
+        for (int j = 0; j < kRedLoads; j++) c += picked(x[j].x, kind) + picked(x[j].y, kind);
+    }
+    for (i += threadIdx.x; i < end; i += kRedThreads) c += picked(d[i], kind);
+#pragma unroll
+    for (int o = BM_WAVE / 2; o > 0; o >>= 1) c += __shfl_down(c, o);
+    if ((threadIdx.x & (BM_WAVE - 1)) == 0) s[threadIdx.x / BM_WAVE] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t all = 0;
+        for (int w = 0; w < kRedWaves; w++) all += s[w];
+        cnt[blockIdx.x] = all;
+    }
+}
+
+/* Block scan of one value per thread: the sum before this thread's. */
+__device__ __forceinline__ int64_t fin_scan(int64_t x, int64_t* s) {
+    const int lane = threadIdx.x & (BM_WAVE - 1), wave = threadIdx.x / BM_WAVE;
+    int64_t inc = x;
+#pragma unroll
+    for (int o = 1; o < BM_WAVE; o <<= 1) {
+        const int64_t y = __shfl_up(inc, o);
+        inc += lane >= o ? y : 0;
+    }
+    __syncthreads();   /* s may still be read */
+    if (lane == BM_WAVE - 1) s[wave] = inc;
+    __syncthreads();
+    for (int w = 0; w < wave; w++) inc += s[w];
+    return inc - x;
+}
+
+/* One block: locate the chunk holding the rank-th match (a single chunk has
+ * no counts), then the wave's share of it, then the element. */
+__global__ void __launch_bounds__(kFinThreads) k_pick_find(const int64_t* __restrict__ d, int64_t k, int32_t kind,
+                                                           int64_t chunk, const int64_t* __restrict__ cnt, int64_t nb,
+                                                           int64_t rank, int64_t* __restrict__ out) {
+    __shared__ int64_t s[kFinWaves];
+    __shared__ int64_t s_chunk, s_before, s_hit;
+    const int t = threadIdx.x, lane = t & (BM_WAVE - 1), wave = t / BM_WAVE;
+    if (t == 0) {
+        s_hit = -1;
+        s_chunk = nb == 1 ? 0 : -1;
+        s_before = 0;
+    }
+    if (nb > 1) {
+        const int64_t per = (nb + kFinThreads - 1) / kFinThreads;
+        const int64_t b0 = (int64_t)t * per, b1 = b0 + per < nb ? b0 + per : nb;
+        int64_t mine = 0;
+        for (int64_t b = b0; b < b1; b++) mine += cnt[b];
+        int64_t acc = fin_scan(mine, s);
+        if (rank >= acc && rank < acc + mine)
+            for (int64_t b = b0; b < b1; b++) {
+                if (rank < acc + cnt[b]) { s_chunk = b; s_before = acc; break; }
+                acc += cnt[b];
+            }
     }
     __syncthreads();
-    s[t] = local;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        int64_t x = t >= o ? s[t - o] : 0;
-        __syncthreads();
-        s[t] += x;
-        __syncthreads();
-    }
-    int64_t r = s_before + s[t] - local;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (flags[q]) {
-            if (r == rank) out[0] = base + (int64_t)t * 4 + q;
-            r++;
+    if (s_chunk >= 0) {   /* block-uniform */
+        const int64_t share = chunk / kFinWaves;   /* a multiple of the wave */
+        const int64_t base = s_chunk * chunk + wave * share;
+        int64_t mine = 0;
+#pragma unroll 4
+        for (int64_t q = 0; q < share; q += BM_WAVE) {
+            const int64_t i = base + q + lane;
+            mine += __popcll(__ballot(i < k && picked(i < k ? d[i] : -1, kind)));
         }
+        int64_t at = s_before + fin_scan(lane == 0 ? mine : 0, s);
+        at = __shfl(at, 0);
+        if (rank >= at && rank < at + mine)
+            for (int64_t q = 0; q < share; q += BM_WAVE) {
+                const int64_t i = base + q + lane;
+                const bool hit = i < k && picked(i < k ? d[i] : -1, kind);
+                const uint64_t m = __ballot(hit);
+                if (hit && at + __popcll(m & ((1ull << lane) - 1)) == rank) s_hit = i;
+                at += __popcll(m);
+            }
+        __syncthreads();
     }
+    if (t == 0) out[0] = s_hit;
 }
 
 /* ------------------------------------------------------------------ */
@@ -708,20 +757,25 @@ hipError_t bm_launch_check_triples(int32_t n, const int4* cand, int64_t k, int32
     return hipGetLastError();
 }
 
-int64_t bm_stats_blocks(int64_t k) { return k <= 0 ? 1 : (k + kRedChunk - 1) / kRedChunk; }
+int64_t bm_stats_blocks(int64_t k) {
+    const int64_t nb = (k + kRedChunk - 1) / kRedChunk;
+    return nb < 1 ? 1 : nb < kRedBlocks ? nb : kRedBlocks;
+}
 
 hipError_t bm_launch_stats(const int64_t* d, int64_t k, int64_t* part, int64_t* out6, hipStream_t s) {
-    const int64_t nb = bm_stats_blocks(k);
-    hipLaunchKernelGGL(k_stats_part, dim3((unsigned)nb), dim3(kRedThreads), 0, s, d, k, part);
-    hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(kRedThreads), 0, s, part, nb, k, out6);
+    if (k <= 0) return hipErrorInvalidValue;
+    const int64_t chunk = red_chunk(k), nb = (k + chunk - 1) / chunk;
+    hipLaunchKernelGGL(k_stats_part, dim3((unsigned)nb), dim3(kRedThreads), 0, s, d, k, chunk, part, out6);
+    if (nb > 1) hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(kFinThreads), 0, s, part, nb, k, out6);
     return hipGetLastError();
 }
 
 hipError_t bm_launch_pick(const int64_t* d, int64_t k, int32_t kind, int64_t rank, int64_t* cnt, int64_t* out,
                           hipStream_t s) {
-    const int64_t nb = bm_stats_blocks(k);
-    hipLaunchKernelGGL(k_pick_count, dim3((unsigned)nb), dim3(kRedThreads), 0, s, d, k, kind, cnt);
-    hipLaunchKernelGGL(k_pick_find, dim3(1), dim3(1024), 0, s, d, k, kind, cnt, nb, rank, out);
+    if (k <= 0) return hipErrorInvalidValue;
+    const int64_t chunk = red_chunk(k), nb = (k + chunk - 1) / chunk;
+    if (nb > 1) hipLaunchKernelGGL(k_pick_count, dim3((unsigned)nb), dim3(kRedThreads), 0, s, d, k, kind, chunk, cnt);
+    hipLaunchKernelGGL(k_pick_find, dim3(1), dim3(kFinThreads), 0, s, d, k, kind, chunk, cnt, nb, rank, out);
     return hipGetLastError();
 }
 
