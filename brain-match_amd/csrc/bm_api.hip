@@ -54,6 +54,7 @@ struct bm_ctx {
     int32_t rows_fit;       /* every placement-row sum fits int32 */
     int32_t rows_small;     /* ... and is at most 2^28 */
     int32_t max_mw;         /* largest male weight */
+    int32_t male_loops;     /* some male vertex has a self-loop */
     int32_t pi_full;        /* every male is matched, none to a shared female (moves keep this) */
     double row_adds;        /* additions of an average placement row: sum of squared female degrees / n */
     int32_t* d_place;       /* placement rows of one group of changed vertices (bm_changed.hip) */
@@ -589,8 +590,7 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     for (int64_t e = 0; e < c->male.m && c->compact; e++)
         if (c->male.out.adj[e].y < -32767 || c->male.out.adj[e].y > 32767) c->compact = 0;
     c->male_nonneg = 1;
-    for (int64_t e = 0; e < c->male.m; e++)
-    {
+    for (int64_t e = 0; e < c->male.m; e++) {
         if (c->male.out.adj[e].y < 0) c->male_nonneg = 0;
         if (c->male.out.adj[e].y > c->max_mw) c->max_mw = c->male.out.adj[e].y;
     }
@@ -614,7 +614,10 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     for (int32_t r = 0; r <= n; r++) c->h_m_self[r] = c->h_f_self[r] = INT32_MIN;
     for (int32_t r = 1; r <= n; r++) {
         for (int64_t e = c->male.out.ptr[r]; e < c->male.out.ptr[r + 1]; e++)
-            if (c->male.out.adj[e].x == r) c->h_m_self[r] = c->male.out.adj[e].y;
+            if (c->male.out.adj[e].x == r) {
+                c->h_m_self[r] = c->male.out.adj[e].y;
+                c->male_loops = 1;
+            }
         for (int64_t e = fg.out.ptr[r]; e < fg.out.ptr[r + 1]; e++)
             if (fg.out.adj[e].x == r) c->h_f_self[r] = fg.out.adj[e].y;
     }
@@ -1016,7 +1019,7 @@ extern "C" int bm_batch_gen_changed_triples(bm_batch* b, const int32_t* changed,
 static const int4* pair_pis(bm_ctx* c, int64_t k, int* rc) {
     *rc = BM_OK;
     if (k < c->n) return nullptr;
-    if (!c->d_pis && (*rc = dalloc(c, &c->d_pis, (size_t)c->n + 1)) != BM_OK) return nullptr;
+    if (!c->d_pis && (*rc = dalloc(c, &c->d_pis, (size_t)bm_gain_pis_words(c->n))) != BM_OK) return nullptr;
     if (bm_launch_gain_pis(devgraph(c), devgain(c), c->d_pis, c->stream) != hipSuccess) {
         *rc = fail(c, BM_ERR_HIP, "refreshing the per-vertex words failed");
         return nullptr;
@@ -1189,7 +1192,7 @@ static int umajor_offsets(bm_ctx* c, uint64_t seed, int64_t k) {
 static int gain_transposed(bm_ctx* c) {
     if (c->gt_version == c->gain_version) return BM_OK;
     if (!c->d_pis) {
-        int rc = dalloc(c, &c->d_pis, (size_t)c->n + 1);
+        int rc = dalloc(c, &c->d_pis, (size_t)bm_gain_pis_words(c->n));
         if (rc != BM_OK) return rc;
     }
     if (!c->d_GT) {
@@ -1234,14 +1237,25 @@ extern "C" int bm_batch_eval_swaps_umajor(bm_batch* b, uint64_t seed, int64_t k)
          * lookups when not even the bitmaps fit */
         const bool staged = bm_gain_umajor_lds(c->n) <= 160 * 1024;
         const bool bitmaps = !staged && bm_gain_umajor_bitmap_lds(c->n) <= 160 * 1024;
+        /* one row of deltas per first vertex where 32-bit sums and the image
+         * order hold and a row serves half as many pairs as it has entries: the
+         * row costs more than the two rows staged as they are, a pair less (n =
+         * 18,524, 2^26 pairs 1.08 ms by rows as they are, 1.22 by rows of
+         * deltas; 2^28 pairs 2.00 and 1.69) */
+        const bool delta_rows = staged && c->pi_full && c->packed && c->rows_small &&
+                                k >= (int64_t)c->n * c->n / 2;
         if (staged && (rc = gain_transposed(c)) != BM_OK) return rc;
-        if (bitmaps && !c->d_pis && (rc = dalloc(c, &c->d_pis, (size_t)c->n + 1)) != BM_OK) return rc;
+        if (bitmaps && !c->d_pis && (rc = dalloc(c, &c->d_pis, (size_t)bm_gain_pis_words(c->n))) != BM_OK) return rc;
         timing_begin(c, BM_KERNEL_GAIN_SWAP, &t);
         if (staged || bitmaps) {
             /* pi and the diagonal G(v, pi(v)) are cheap: refreshed every call */
             HIPCHK(c, bm_launch_gain_pis(devgraph(c), devgain(c), c->d_pis, c->stream));
-            HIPCHK(c, bm_launch_gain_swap_umajor(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_um_off, seed,
-                                                 b->d_delta, c->num_cus, c->stream));
+            if (delta_rows)
+                HIPCHK(c, bm_launch_gain_swap_rows(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_um_off, seed,
+                                                   c->male_loops, b->d_delta, c->num_cus, c->stream));
+            else
+                HIPCHK(c, bm_launch_gain_swap_umajor(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_um_off, seed,
+                                                     b->d_delta, c->num_cus, c->stream));
         } else {
             const int4* pis = pair_pis(c, k, &rc);
             if (rc != BM_OK) {
@@ -1566,7 +1580,7 @@ extern "C" int bm_best_swap(bm_ctx* c, int64_t* delta, int32_t* u, int32_t* v) {
      * first vertex, with the transposed copy */
     const bool tiles = c->pi_full && c->packed && c->rows_small && c->d_m_adj;
     int rc = tiles ? BM_OK : gain_transposed(c);
-    if (rc == BM_OK && !c->d_pis) rc = dalloc(c, &c->d_pis, (size_t)c->n + 1);
+    if (rc == BM_OK && !c->d_pis) rc = dalloc(c, &c->d_pis, (size_t)bm_gain_pis_words(c->n));
     if (rc == BM_OK && !c->d_best) rc = dalloc(c, &c->d_best, (size_t)kBestSwapParts + 1);
     if (rc != BM_OK) return rc;
     int4* out = reinterpret_cast<int4*>(c->h_pin);

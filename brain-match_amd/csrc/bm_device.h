@@ -146,6 +146,9 @@ hipError_t bm_launch_gain_swap(const BmDevGraph& g, const BmGain& G, int mode, c
 size_t bm_gain_umajor_lds(int32_t n);
 size_t bm_gain_umajor_bitmap_lds(int32_t n);
 hipError_t bm_launch_gain_transpose(const BmGain& G, int32_t nrows, int32_t* GT, int32_t num_cus, hipStream_t s);
+/* The per-vertex words {pi(v), G(v, pi(v)), self-loops}: bm_gain_pis_words(n)
+ * int4, the diagonal alone behind them. */
+int64_t bm_gain_pis_words(int32_t n);
 hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, hipStream_t s);
 /* a-major 3-vertex lookups (best delta and permutation per stream entry);
  * needs bm_gain_rot3_amajor_lds(n) bytes of LDS.  Triples with an edge are
@@ -158,6 +161,12 @@ hipError_t bm_launch_gain_rot3_amajor(const BmDevGraph& g, const BmGain& G, cons
                                       const int64_t* off, uint64_t seed, int64_t* best, uint8_t* perm, int4* queue,
                                       int64_t queue_entries, int32_t* queue_counts, int32_t queue_regions,
                                       int32_t num_cus, hipStream_t s);
+/* u-major lookups from one LDS row of deltas per first vertex: a complete
+ * matching with distinct images, packed row tables, |G| <= 2^28, and
+ * n + 1 <= 20,480; loops = some male vertex has a self-loop. */
+hipError_t bm_launch_gain_swap_rows(const BmDevGraph& g, const BmGain& G, const int32_t* GT, const int4* pis,
+                                    const int64_t* off, uint64_t seed, int32_t loops, int64_t* delta, int32_t num_cus,
+                                    hipStream_t s);
 hipError_t bm_launch_gain_swap_umajor(const BmDevGraph& g, const BmGain& G, const int32_t* GT, const int4* pis,
                                       const int64_t* off, uint64_t seed, int64_t* delta, int32_t num_cus,
                                       hipStream_t s);

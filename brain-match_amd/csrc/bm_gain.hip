@@ -1290,14 +1290,129 @@ __global__ void __launch_bounds__(256) k_gain_transpose(const int32_t* __restric
     }
 }
 
+/* G(v, pi(v)) alone, in a row of the table's stride behind the n + 1 words. */
+__device__ __forceinline__ int32_t* pis_diag(int4* pis, int32_t n) { return reinterpret_cast<int32_t*>(pis + n + 1); }
+__device__ __forceinline__ const int32_t* pis_diag(const int4* pis, int32_t n) {
+    return reinterpret_cast<const int32_t*>(pis + n + 1);
+}
+
 /* Per vertex v: {pi(v), G(v, pi(v)), male self-loop weight of v, female
  * self-loop weight of pi(v)} (BM_ABSENT for a missing loop). */
 __global__ void k_gain_pis(BmDevGraph g, BmGain G, int4* __restrict__ pis) {
+    int32_t* diag = pis_diag(pis, g.n);
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= g.n; v += stride) {
         const int32_t f = v ? g.pi[v] : 0;
-        pis[v] = make_int4(f, v ? G.G[v * G.stride + f] : 0, v ? G.m_self[v] : BM_ABSENT,
-                           f ? G.f_self[f] : BM_ABSENT);
+        const int32_t own = v ? G.G[v * G.stride + f] : 0;
+        pis[v] = make_int4(f, own, v ? G.m_self[v] : BM_ABSENT, f ? G.f_self[f] : BM_ABSENT);
+        diag[v] = own;
+    }
+}
+
+/* u-major lookups while every male is matched and no female is shared: the
+ * block of first vertex u makes one LDS row of its deltas against every v,
+ *   S(v) = G(u, pi(v)) - G(u, pi(u)) + G(v, pi(u)) - G(v, pi(v)) + corrections,
+ * the first term scattered by images from row u, the third from row pi(u) of
+ * the transposed table, the corrections added by u's male neighbours and, if
+ * any male has one, the self-loops.  A pair is then one LDS read and the
+ * store; with two rows and bitmaps in LDS it was two reads, a 16-byte gather
+ * from cache and two bit tests, one block to a CU instead of two.  Sums are
+ * 32-bit: |G| <= 2^28 (the caller checks).
+ * 2^28 pairs at n = 18,524: 1,785 -> 1,445 us, of which the rows of deltas
+ * take about 900 (300 of them the corrections, a chain of three dependent
+ * reads per row) and the pairs the rest, near the time of their store.  The
+ * scatter is a plain store and the other terms follow as whole words: as LDS
+ * atomics they cost 120 us more; bitmaps of f1's neighbours in place of the
+ * early bucket reads 90 us more. */
+constexpr int kPrThreads = 1024;
+constexpr int kPrPairs = 8;      /* pairs per thread in flight */
+constexpr int kPrWords = 5;      /* 16-byte words per thread of a row of up to 20,480 entries */
+
+/* The correction of an edge u -> v or v -> u of weight w: its image moves
+ * between (f1, f2) and (f2, f1), and the rows count it at (f1, f1), (f2, f2). */
+__device__ __forceinline__ int32_t pair_correction(int32_t w, int32_t F12, int32_t F21, int32_t F11, int32_t F22) {
+    return contrib(w, F21) - contrib(w, F22) - contrib(w, F11) + contrib(w, F12);
+}
+
+__global__ void __launch_bounds__(kPrThreads, 8) k_gain_swap_rows(BmDevGraph g, BmGain G, const int32_t* __restrict__ GT,
+                                                                  const int4* __restrict__ pis,
+                                                                  const int64_t* __restrict__ off, uint64_t seed,
+                                                                  int32_t loops, int64_t* __restrict__ delta) {
+    extern __shared__ int4 S4[];
+    int32_t* S = reinterpret_cast<int32_t*>(S4);
+    const int32_t n = g.n, tid = threadIdx.x;
+    const int32_t s4 = (int32_t)(G.stride >> 2);
+    const int4* diag = reinterpret_cast<const int4*>(pis_diag(pis, n));
+    for (int32_t u = blockIdx.x + 1; u <= n; u += gridDim.x) {
+        const int64_t i0 = off[u], i1 = off[u + 1];
+        if (i0 == i1) continue;   /* block-uniform */
+        const int4 pu = pis[u];
+        const int32_t f1 = pu.x;
+        const int64_t ob = g.m_out_ptr[u], oc = g.m_out_ptr[u + 1] - ob;
+        const int64_t ib = g.m_in_ptr[u], ic = g.m_in_ptr[u + 1] - ib;
+        const uint64_t d12 = g.f_out_t.desc[f1], d21 = g.f_in_t.desc[f1];
+        /* u's first kPrThreads neighbours: each step of their chain (entry,
+         * words of v, first buckets) is requested ahead of the rows' */
+        auto edge = [&](int64_t e) {
+            return e < oc ? g.m_out[ob + e] : e < oc + ic ? g.m_in[ib + (e - oc)] : make_int2(0, 0);
+        };
+        const int2 ed = edge(tid);
+        const int4* gt = reinterpret_cast<const int4*>(GT + (int64_t)f1 * G.stride);
+        const int32_t* gu = G.G + (int64_t)u * G.stride;
+        __syncthreads();   /* the previous row has been read */
+#pragma unroll 6
+        for (int32_t f = 1 + tid; f <= n; f += kPrThreads) S[g.inv[f]] = gu[f] - pu.y;
+        const int4 pv = pis[ed.x];
+        int4 t[kPrWords];
+#pragma unroll
+        for (int j = 0; j < kPrWords; j++) {
+            const int32_t c = tid + kPrThreads * j;
+            t[j] = c < s4 ? gt[c] : make_int4(0, 0, 0, 0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPrWords; j++) {
+            const int32_t c = tid + kPrThreads * j;
+            if (c < s4) {
+                const int4 dg = diag[c], x = S4[c];
+                S4[c] = make_int4(x.x + t[j].x - dg.x, x.y + t[j].y - dg.y, x.z + t[j].z - dg.z, x.w + t[j].w - dg.w);
+            }
+        }
+        const uint4* T12 = g.f_out_t.tab + (d12 >> 6);
+        const uint4* T21 = g.f_in_t.tab + (d21 >> 6);
+        const uint4 b12 = T12[row_home(pv.x, (uint32_t)(d12 & 63u))], b21 = T21[row_home(pv.x, (uint32_t)(d21 & 63u))];
+        __syncthreads();
+        if (ed.x != 0 && ed.x != u) {
+            int32_t F12, F21;
+            if (!row_bucket<true>(b12, pv.x, F12)) F12 = row_find<true>(g.f_out_t.tab, d12, pv.x);
+            if (!row_bucket<true>(b21, pv.x, F21)) F21 = row_find<true>(g.f_in_t.tab, d21, pv.x);
+            atomicAdd(&S[ed.x], pair_correction(ed.y, F12, F21, pu.w, pv.w));
+        }
+        for (int64_t e = tid + kPrThreads; e < oc + ic; e += kPrThreads) {
+            const int2 ed = edge(e);
+            if (ed.x == u) continue;
+            const int4 pv = pis[ed.x];
+            const int32_t F12 = row_find<true>(g.f_out_t.tab, d12, pv.x);
+            const int32_t F21 = row_find<true>(g.f_in_t.tab, d21, pv.x);
+            atomicAdd(&S[ed.x], pair_correction(ed.y, F12, F21, pu.w, pv.w));
+        }
+        if (loops)
+            for (int32_t v = 1 + tid; v <= n; v += kPrThreads) {
+                const int4 pv = pis[v];
+                int32_t d = 0;
+                if (pu.z != BM_ABSENT) d += contrib(pu.z, pv.w) - contrib(pu.z, pu.w);
+                if (pv.z != BM_ABSENT) d += contrib(pv.z, pu.w) - contrib(pv.z, pv.w);
+                if (d) atomicAdd(&S[v], d);
+            }
+        __syncthreads();
+        for (int64_t p = i0 + tid; p < i1; p += (int64_t)kPrThreads * kPrPairs) {
+#pragma unroll
+            for (int j = 0; j < kPrPairs; j++) {
+                const int64_t i = p + (int64_t)kPrThreads * j;
+                if (i < i1)
+                    __builtin_nontemporal_store((int64_t)S[bm_umajor_partner(seed, (uint64_t)i, u, n)], &delta[i]);
+            }
+        }
     }
 }
 
@@ -1969,6 +2084,22 @@ hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, h
     int64_t blocks = ((int64_t)g.n + 256) / 256;
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(k_gain_pis, dim3((unsigned)blocks), dim3(256), 0, s, g, G, pis);
+    return hipGetLastError();
+}
+
+int64_t bm_gain_pis_words(int32_t n) { return (int64_t)n + 1 + bm_gain_stride(n) / 4; }
+
+hipError_t bm_launch_gain_swap_rows(const BmDevGraph& g, const BmGain& G, const int32_t* GT, const int4* pis,
+                                    const int64_t* off, uint64_t seed, int32_t loops, int64_t* delta, int32_t num_cus,
+                                    hipStream_t s) {
+    const size_t lds = (size_t)G.stride * sizeof(int32_t);
+    if (!GT || !g.inv || G.stride > (int64_t)4 * kPrWords * kPrThreads || lds > kLdsBytes / 2) return hipErrorInvalidValue;
+    hipError_t e = hipFuncSetAttribute((const void*)k_gain_swap_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    int64_t blocks = 2 * (int64_t)(num_cus > 0 ? num_cus : 256);
+    if (blocks > g.n) blocks = g.n;
+    hipLaunchKernelGGL(k_gain_swap_rows, dim3((unsigned)blocks), dim3(kPrThreads), lds, s, g, G, GT, pis, off, seed, loops,
+                       delta);
     return hipGetLastError();
 }
 
