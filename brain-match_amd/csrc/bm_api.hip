@@ -38,10 +38,6 @@ struct bm_ctx {
     int2* d_m_out;
     int64_t* d_m_in_ptr;
     int2* d_m_in;
-    uint64_t* d_f_out_desc;
-    int2* d_f_out_tab;
-    uint64_t* d_f_in_desc;
-    int2* d_f_in_tab;
     int64_t* d_f_out_ptr;   /* female CSR / CSC rows */
     int2* d_f_out;
     int64_t* d_f_in_ptr;
@@ -81,8 +77,6 @@ struct bm_ctx {
     int32_t* h_f_self;
     int32_t max_abs_fw;     /* largest |female weight| */
     int32_t* d_G;
-    uint64_t* d_m_out_desc;
-    int2* d_m_out_tab;
     int32_t* d_m_self;
     int32_t* d_f_self;
     int4* d_moves;
@@ -176,10 +170,6 @@ static BmDevGraph devgraph(const bm_ctx* c) {
     g.m_out = c->d_m_out;
     g.m_in_ptr = c->d_m_in_ptr;
     g.m_in = c->d_m_in;
-    g.f_out_desc = c->d_f_out_desc;
-    g.f_out_tab = c->d_f_out_tab;
-    g.f_in_desc = c->d_f_in_desc;
-    g.f_in_tab = c->d_f_in_tab;
     g.f_out_ptr = c->d_f_out_ptr;
     g.f_out = c->d_f_out;
     g.f_in_ptr = c->d_f_in_ptr;
@@ -262,10 +252,6 @@ static void free_ctx(bm_ctx* c) {
     (void)hipFree(c->d_m_out);
     (void)hipFree(c->d_m_in_ptr);
     (void)hipFree(c->d_m_in);
-    (void)hipFree(c->d_f_out_desc);
-    (void)hipFree(c->d_f_out_tab);
-    (void)hipFree(c->d_f_in_desc);
-    (void)hipFree(c->d_f_in_tab);
     (void)hipFree(c->d_f_out_ptr);
     (void)hipFree(c->d_f_out);
     (void)hipFree(c->d_f_in_ptr);
@@ -291,8 +277,6 @@ static void free_ctx(bm_ctx* c) {
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     (void)hipFree(c->d_G);
-    (void)hipFree(c->d_m_out_desc);
-    (void)hipFree(c->d_m_out_tab);
     (void)hipFree(c->d_m_self);
     (void)hipFree(c->d_f_self);
     (void)hipFree(c->d_moves);
@@ -330,8 +314,6 @@ static BmGain devgain(const bm_ctx* c) {
     BmGain G;
     G.G = c->d_G;
     G.stride = bm_gain_stride(c->n);
-    G.m_out_desc = c->d_m_out_desc;
-    G.m_out_tab = c->d_m_out_tab;
     G.m_self = c->d_m_self;
     G.f_self = c->d_f_self;
     G.f_out_p = c->d_f_out_p;
@@ -570,16 +552,10 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     c->female_m = fg.m;
     c->f_out_deg = (int32_t*)calloc((size_t)n + 1, sizeof(int32_t));
     c->f_in_deg = (int32_t*)calloc((size_t)n + 1, sizeof(int32_t));
-    bm_rowhash_host ho, hi;
-    memset(&ho, 0, sizeof ho);
-    memset(&hi, 0, sizeof hi);
-    if (!c->f_out_deg || !c->f_in_deg || bm_rowhash_build(&fg.out, &ho) != BM_OK ||
-        bm_rowhash_build(&fg.in, &hi) != BM_OK) {
+    if (!c->f_out_deg || !c->f_in_deg) {
         bm_graph_free(&fg);
-        bm_rowhash_free(&ho);
-        bm_rowhash_free(&hi);
         free_ctx(c);
-        return fail(nullptr, BM_ERR_NOMEM, "bm_create: out of host memory building female tables");
+        return fail(nullptr, BM_ERR_NOMEM, "bm_create: out of host memory");
     }
     /* Compact LDS slots need keys below 2^17 and female weights in 0..32767;
      * compact kernels also sum a lane's contributions in 32 bits, which needs
@@ -605,8 +581,6 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     c->h_m_self = (int32_t*)malloc(sizeof(int32_t) * ((size_t)n + 1));
     c->h_f_self = (int32_t*)malloc(sizeof(int32_t) * ((size_t)n + 1));
     if (!c->h_m_self || !c->h_f_self) {
-        bm_rowhash_free(&ho);
-        bm_rowhash_free(&hi);
         bm_graph_free(&fg);
         free_ctx(c);
         return fail(nullptr, BM_ERR_NOMEM, "bm_create: out of host memory");
@@ -633,10 +607,6 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = dalloc(c, &c->d_m_out, (size_t)mg.m);
     if (rc == BM_OK) rc = dalloc(c, &c->d_m_in_ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = dalloc(c, &c->d_m_in, (size_t)mg.m);
-    if (rc == BM_OK) rc = dalloc(c, &c->d_f_out_desc, (size_t)n + 1);
-    if (rc == BM_OK) rc = dalloc(c, &c->d_f_out_tab, (size_t)(ho.slots ? ho.slots : 2));
-    if (rc == BM_OK) rc = dalloc(c, &c->d_f_in_desc, (size_t)n + 1);
-    if (rc == BM_OK) rc = dalloc(c, &c->d_f_in_tab, (size_t)(hi.slots ? hi.slots : 2));
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_out_ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_out, (size_t)fg.m);
     if (rc == BM_OK) rc = dalloc(c, &c->d_f_in_ptr, (size_t)n + 2);
@@ -648,10 +618,6 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK) rc = h2d(c, c->d_m_out, mg.out.adj, (size_t)mg.m);
     if (rc == BM_OK) rc = h2d(c, c->d_m_in_ptr, mg.in.ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = h2d(c, c->d_m_in, mg.in.adj, (size_t)mg.m);
-    if (rc == BM_OK) rc = h2d(c, c->d_f_out_desc, ho.desc, (size_t)n + 1);
-    if (rc == BM_OK) rc = h2d(c, c->d_f_out_tab, ho.tab, (size_t)ho.slots);
-    if (rc == BM_OK) rc = h2d(c, c->d_f_in_desc, hi.desc, (size_t)n + 1);
-    if (rc == BM_OK) rc = h2d(c, c->d_f_in_tab, hi.tab, (size_t)hi.slots);
     if (rc == BM_OK) rc = h2d(c, c->d_f_out_ptr, fg.out.ptr, (size_t)n + 2);
     if (rc == BM_OK) rc = h2d(c, c->d_f_out, fg.out.adj, (size_t)fg.m);
     if (rc == BM_OK) rc = h2d(c, c->d_f_in_ptr, fg.in.ptr, (size_t)n + 2);
@@ -676,8 +642,6 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
     if (rc == BM_OK && hipMemsetAsync(c->d_pi, 0, 2 * ((size_t)n + 1) * sizeof(int32_t), c->stream) != hipSuccess)
         rc = fail(c, BM_ERR_HIP, "hipMemsetAsync failed");
     if (rc == BM_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, BM_ERR_HIP, "hipStreamSynchronize failed");
-    bm_rowhash_free(&ho);
-    bm_rowhash_free(&hi);
     bm_graph_free(&fg);
     if (rc != BM_OK) {
         bm_set_global_error("bm_create: %s", c->err);
@@ -1699,7 +1663,6 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
         return BM_OK;
     }
     if (c->gain_on) return BM_OK;
-    const bm_graph_host& mg = c->male;
     if (!c->rows_fit)
         return fail(c, BM_ERR_ARG, "bm_gain_enable: vertex %d's incident weights can exceed int32 in the table",
                     gain_overflow(c, INT32_MAX));
@@ -1709,18 +1672,9 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
     const size_t list_bytes = (size_t)(2 * c->male.m + 1) * sizeof(int4);
     if (bytes + list_bytes + ((size_t)1 << 30) > free_b)
         return fail(c, BM_ERR_NOMEM, "bm_gain_enable: table needs %zu bytes, %zu free on the device", bytes, free_b);
-    if (!c->d_m_out_desc) {
-        bm_rowhash_host hm;
-        memset(&hm, 0, sizeof hm);
-        if (bm_rowhash_build(&mg.out, &hm) != BM_OK) return fail(c, BM_ERR_NOMEM, "bm_gain_enable: out of host memory");
-        int rc = dalloc(c, &c->d_m_out_desc, (size_t)c->n + 1);
-        if (rc == BM_OK) rc = dalloc(c, &c->d_m_out_tab, (size_t)(hm.slots ? hm.slots : 2));
-        if (rc == BM_OK) rc = dalloc(c, &c->d_nmoves, 1);
+    if (!c->d_nmoves) {
+        int rc = dalloc(c, &c->d_nmoves, 1);
         if (rc == BM_OK) rc = dalloc(c, &c->d_patch_rows, (size_t)bm_gain_update_rows(c->n));
-        if (rc == BM_OK) rc = h2d(c, c->d_m_out_desc, hm.desc, (size_t)c->n + 1);
-        if (rc == BM_OK) rc = h2d(c, c->d_m_out_tab, hm.tab, (size_t)hm.slots);
-        if (rc == BM_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, BM_ERR_HIP, "sync failed");
-        bm_rowhash_free(&hm);
         if (rc != BM_OK) return rc;
     }
     if (c->compact && !c->d_f_out_p && c->female_m > 0) {
@@ -1819,7 +1773,7 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
     if (!c->d_echunks) {
         std::vector<int2> ch;
         for (int32_t u = 1; u <= c->n; u++) {
-            const int64_t L = (mg.out.ptr[u + 1] - mg.out.ptr[u]) + (mg.in.ptr[u + 1] - mg.in.ptr[u]);
+            const int64_t L = male_degree(c, (int32_t)u);
             for (int64_t t = 0; t < L; t += BM_DESC_CHUNK) ch.push_back(make_int2(u, (int32_t)t));
         }
         c->n_echunks = (int64_t)ch.size();

@@ -23,10 +23,6 @@ struct BmDevGraph {
     const int2* m_out;          /* {dst, w} */
     const int64_t* m_in_ptr;    /* male CSC column offsets, n+2 */
     const int2* m_in;           /* {src, w} */
-    const uint64_t* f_out_desc; /* female out-row hash table descriptors, n+1 */
-    const int2* f_out_tab;
-    const uint64_t* f_in_desc;  /* female in-row hash table descriptors, n+1 */
-    const int2* f_in_tab;
     const int64_t* f_out_ptr;   /* female CSR (sorted rows), n+2 */
     const int2* f_out;          /* {dst, w} */
     const int64_t* f_in_ptr;    /* female CSC, n+2 */
@@ -53,8 +49,6 @@ hipError_t bm_launch_diag(const BmDevGraph& g, const int4* chunks, int64_t nchun
 struct BmGain {
     int32_t* G;                 /* (n+1) x stride int32, row-major; row 0 / column 0 zero */
     int64_t stride;             /* row stride in int32: n + 1 rounded up to 32 (rows start on 128-byte lines) */
-    const uint64_t* m_out_desc; /* male out-row hash tables (adjacency tests) */
-    const int2* m_out_tab;
     const uint32_t* m_adj;      /* dense male adjacency, m_adj_words uint32 per row (n+1 rows), or NULL;
                                  * symmetric: bit max(a,b) of row min(a,b) is set when a -> b or b -> a */
     int64_t m_adj_words;

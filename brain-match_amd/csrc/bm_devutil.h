@@ -12,11 +12,6 @@
 
 namespace bmd {
 
-/* Multiplicative hash of a vertex id into 2^bits slots (bits >= 1). */
-__device__ __forceinline__ uint32_t slot_hash(int32_t key, uint32_t bits) {
-    return ((uint32_t)key * 0x9E3779B1u) >> (32u - bits);
-}
-
 /* Exact contribution of a male edge of weight w whose image is a female
  * lookup result fw: min(w, fw) when the female edge exists, else 0. */
 __device__ __forceinline__ int32_t contrib(int32_t w, int32_t fw) {

@@ -72,42 +72,34 @@ __device__ __forceinline__ bool male_maybe(const BmGain& G, int32_t a, int32_t b
     return !G.m_adj || ((adj_word(G, a, b) >> ((a < b ? b : a) & 31)) & 1u);
 }
 
-/* K hash lookups at once: key[k] in table (T[k], bits[k]) where go[k], else
- * BM_ABSENT without a load.  Every first slot is loaded before any collision
- * chain is followed, so the K lookups cost one memory latency unless a key
- * sits past its home slot. */
-template <int K>
-__device__ __forceinline__ void probe_many(const int2* const* T, const uint32_t* bits, const int32_t* key,
-                                           const bool* go, int32_t* out) {
-    int2 e[K];
+/* K row-table lookups at once: key[k] in the row of descriptor d[k] where
+ * go[k], else BM_ABSENT without a load.  Every first bucket is loaded before
+ * any later one, so the K lookups cost one memory latency unless a key sits
+ * past its home bucket. */
+template <bool PACKED, int K>
+__device__ __forceinline__ void find_many(const uint4* tab, const uint64_t* d, const int32_t* key, const bool* go,
+                                          int32_t* out) {
+    uint4 e[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        e[k] = make_int2(0, 0);
-        if (go[k] && bits[k] != 0u && key[k] != 0) e[k] = T[k][slot_hash(key[k], bits[k])];
+        e[k] = make_uint4(0u, 0u, 0u, 0u);
+        if (go[k] && key[k] != 0) e[k] = tab[(d[k] >> 6) + row_home(key[k], (uint32_t)(d[k] & 63u))];
     }
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        if (e[k].x != 0 && e[k].x != key[k]) {   /* past its home slot: walk the chain */
-            const uint32_t mask = (1u << bits[k]) - 1u;
-            uint32_t s = slot_hash(key[k], bits[k]);
-            do {
-                s = (s + 1u) & mask;
-                e[k] = T[k][s];
-            } while (e[k].x != 0 && e[k].x != key[k]);
-        }
-        out[k] = e[k].x != 0 ? e[k].y : BM_ABSENT;
-    }
+    for (int k = 0; k < K; k++)
+        if (!row_bucket<PACKED>(e[k], key[k] != 0 ? key[k] : -1, out[k])) out[k] = row_find<PACKED>(tab, d[k], key[k]);
 }
 
 /* Weights inside a triple of male vertices v[0..2] with images f[0..2]:
  * w[i][j] = w_M(v[i], v[j]) for the pairs with have[i][j] (the others are
  * known absent and cost nothing) and, when any such pair exists, the nine
  * female weights F[x][y] = w_F(f[x], f[y]) (the diagonal is the female
- * self-loops fs[x]); BM_ABSENT elsewhere.  md / fd are the hash-table
+ * self-loops fs[x]); BM_ABSENT elsewhere.  md / fd are the row-table
  * descriptors of the rows of v[i] in M and f[x] in F (loaded by the caller
- * with its other gathers), so the up to 12 probes cost one memory latency.
+ * with its other gathers), so the up to 12 lookups cost two memory latencies
+ * (six 16-byte buckets in registers at a time).
  * v[2] = f[2] = 0 serves a pair. */
-__device__ __forceinline__ void triple_weights(const BmDevGraph& g, const BmGain& G, const int32_t* v,
+__device__ __forceinline__ void triple_weights(const BmDevGraph& g, const int32_t* v,
                                                const uint64_t* md, const int32_t* f, const uint64_t* fd,
                                                const int32_t* fs, const bool (*have)[3], int32_t (*w)[3],
                                                int32_t (*F)[3]) {
@@ -121,27 +113,30 @@ __device__ __forceinline__ void triple_weights(const BmDevGraph& g, const BmGain
             if (i != j) any = any || have[i][j];
         }
     if (!any) return;
-    const int2* T[12];
-    uint32_t bits[12];
-    int32_t key[12], out[12];
-    bool go[12];
+    uint64_t mt[6], ft[6];
+    int32_t mk[6], fk[6], mw[6], fw[6];
+    bool mg[6], fg[6];
     int k = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             if (i == j) continue;
-            T[k] = G.m_out_tab + (md[i] >> 6);
-            bits[k] = (uint32_t)(md[i] & 63u);
-            key[k] = v[j];
-            go[k] = have[i][j];
-            T[k + 6] = g.f_out_tab + (fd[i] >> 6);
-            bits[k + 6] = (uint32_t)(fd[i] & 63u);
-            key[k + 6] = f[j];
-            go[k + 6] = f[i] != 0;
+            mt[k] = md[i];
+            mk[k] = v[j];
+            mg[k] = have[i][j];
+            ft[k] = fd[i];
+            fk[k] = f[j];
+            fg[k] = f[i] != 0;
             k++;
         }
-    probe_many<12>(T, bits, key, go, out);
+    if (g.packed) {   /* uniform */
+        find_many<true, 6>(g.m_out_t.tab, mt, mk, mg, mw);
+        find_many<true, 6>(g.f_out_t.tab, ft, fk, fg, fw);
+    } else {
+        find_many<false, 6>(g.m_out_t.tab, mt, mk, mg, mw);
+        find_many<false, 6>(g.f_out_t.tab, ft, fk, fg, fw);
+    }
     k = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
@@ -149,8 +144,8 @@ __device__ __forceinline__ void triple_weights(const BmDevGraph& g, const BmGain
 #pragma unroll
         for (int j = 0; j < 3; j++)
             if (i != j) {
-                w[i][j] = out[k];
-                F[i][j] = out[k + 6];
+                w[i][j] = mw[k];
+                F[i][j] = fw[k];
                 k++;
             }
     }
@@ -875,7 +870,7 @@ __global__ void __launch_bounds__(kPatchThreads) k_gain_update(BmDevGraph g, BmG
 /* Swap delta of u != v from its four table entries guf2 = G(u, f2),
  * guf1 = G(u, f1), gvf1 = G(v, f1), gvf2 = G(v, f2), with e_uv = "a male
  * edge between u and v may exist" (either direction): an edge's weight and
- * the female weights its correction needs are hash-probed only then. */
+ * the female weights its correction needs are looked up only then. */
 __device__ __forceinline__ int64_t gain_swap_delta_from(const BmDevGraph& g, const BmGain& G, int32_t u, int32_t v,
                                                         int32_t f1, int32_t f2, bool e_uv, int64_t guf2, int64_t guf1,
                                                         int64_t gvf1, int64_t gvf2, int32_t su, int32_t sv,
@@ -884,14 +879,14 @@ __device__ __forceinline__ int64_t gain_swap_delta_from(const BmDevGraph& g, con
     const int32_t fs[3] = {fs1, fs2, BM_ABSENT};
     if (e_uv) {
         /* male edges u -> v and v -> u; their corrections need the four
-         * female weights among f1 and f2 (rare: the hash-row descriptors are
+         * female weights among f1 and f2 (rare: the row descriptors are
          * loaded only here) */
         const bool have[3][3] = {{false, true, false}, {true, false, false}, {false, false, false}};
-        const uint64_t md[3] = {G.m_out_desc[u], G.m_out_desc[v], 0ull};
-        const uint64_t fd[3] = {g.f_out_desc[f1], g.f_out_desc[f2], 0ull};
+        const uint64_t md[3] = {g.m_out_t.desc[u], g.m_out_t.desc[v], 0ull};
+        const uint64_t fd[3] = {g.f_out_t.desc[f1], g.f_out_t.desc[f2], 0ull};
         const int32_t vtx[3] = {u, v, 0}, f[3] = {f1, f2, 0};
         int32_t w[3][3], F[3][3];
-        triple_weights(g, G, vtx, md, f, fd, fs, have, w, F);
+        triple_weights(g, vtx, md, f, fd, fs, have, w, F);
         const int32_t w1 = w[0][1], w2 = w[1][0];
         /* u -> v lands on f2 -> f1; v -> u on f1 -> f2 */
         if (w1 != BM_ABSENT)
@@ -1656,11 +1651,11 @@ __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4*
             uint64_t md[3], fd[3];
 #pragma unroll
             for (int i = 0; i < 3; i++) {
-                md[i] = G.m_out_desc[vtx[i]];
-                fd[i] = g.f_out_desc[f[i]];
+                md[i] = g.m_out_t.desc[vtx[i]];
+                fd[i] = g.f_out_t.desc[f[i]];
             }
             const bool have[3][3] = {{false, e01, e02}, {e01, false, e12}, {e02, e12, false}};
-            triple_weights(g, G, vtx, md, f, fd, fs, have, w, F);
+            triple_weights(g, vtx, md, f, fd, fs, have, w, F);
         }
         int64_t bd;
         int bp;
@@ -1714,7 +1709,7 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, B
         if (i0 == i1) continue;   /* block-uniform */
         const int4 pa = pis[a];
         const int32_t fa = pa.x;
-        const uint64_t mda = G.m_out_desc[a], fda = g.f_out_desc[fa];
+        const uint64_t mda = g.m_out_t.desc[a], fda = g.f_out_t.desc[fa];
         for (int32_t w = tid; w < 2 * w32; w += kUmThreads) mo[w] = 0;
         __syncthreads();
         const int64_t mob = g.m_out_ptr[a], moe = g.m_out_ptr[a + 1];
@@ -1776,9 +1771,9 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, B
                 const bool bc = (wbc >> ((b < c ? c : b) & 31)) & 1u;   /* either direction */
                 const int32_t vtx[3] = {a, b, c};
                 const bool have[3][3] = {{false, ab, ac}, {ba, false, bc}, {ca, bc, false}};
-                const uint64_t md[3] = {mda, G.m_out_desc[b], G.m_out_desc[c]};
-                const uint64_t fd[3] = {fda, g.f_out_desc[pb.x], g.f_out_desc[pc.x]};
-                triple_weights(g, G, vtx, md, f, fd, fs, have, w, F);
+                const uint64_t md[3] = {mda, g.m_out_t.desc[b], g.m_out_t.desc[c]};
+                const uint64_t fd[3] = {fda, g.f_out_t.desc[pb.x], g.f_out_t.desc[pc.x]};
+                triple_weights(g, vtx, md, f, fd, fs, have, w, F);
             }
             int64_t bd;
             int bp;
@@ -1862,10 +1857,10 @@ __global__ void __launch_bounds__(256) k_gain_rot3_edges(BmDevGraph g, BmGain G,
         const bool have[3][3] = {{false, (fl & 1) != 0, (fl & 4) != 0},
                                  {(fl & 2) != 0, false, (fl & 16) != 0},
                                  {(fl & 8) != 0, (fl & 16) != 0, false}};
-        const uint64_t md[3] = {G.m_out_desc[vtx[0]], G.m_out_desc[vtx[1]], G.m_out_desc[vtx[2]]};
-        const uint64_t fd[3] = {g.f_out_desc[f[0]], g.f_out_desc[f[1]], g.f_out_desc[f[2]]};
+        const uint64_t md[3] = {g.m_out_t.desc[vtx[0]], g.m_out_t.desc[vtx[1]], g.m_out_t.desc[vtx[2]]};
+        const uint64_t fd[3] = {g.f_out_t.desc[f[0]], g.f_out_t.desc[f[1]], g.f_out_t.desc[f[2]]};
         int32_t w[3][3], F[3][3];
-        triple_weights(g, G, vtx, md, f, fd, fs, have, w, F);
+        triple_weights(g, vtx, md, f, fd, fs, have, w, F);
         int64_t bd;
         int bp;
         rot3_from_gains(Gv, w, F, sv, fs, bd, bp);

@@ -129,61 +129,3 @@ int bm_graph_build(int32_t n, const bm_edges* e, bm_graph_host* g, const char** 
     free(cnt);
     return BM_OK;
 }
-
-void bm_rowhash_free(bm_rowhash_host* h) {
-    if (!h) return;
-    free(h->desc);
-    free(h->tab);
-    memset(h, 0, sizeof *h);
-}
-
-static uint32_t table_bits_for(int64_t deg) {
-    if (deg <= 0) return 0;
-    uint32_t bits = 1;
-    while (((int64_t)1 << bits) < 2 * deg) bits++;
-    return bits;
-}
-
-int bm_rowhash_build(const bm_csr_host* rows, bm_rowhash_host* h) {
-    memset(h, 0, sizeof *h);
-    const int32_t n = rows->n;
-    h->n = n;
-    h->desc = (uint64_t*)calloc((size_t)(n + 1), sizeof(uint64_t));
-    if (!h->desc) return BM_ERR_NOMEM;
-    int64_t total = 0;
-    for (int32_t r = 0; r <= n; r++) {
-        int64_t d = rows->ptr[r + 1] - rows->ptr[r];
-        uint32_t bits = table_bits_for(d);
-        h->desc[r] = ((uint64_t)total << 6) | bits;
-        if (bits) total += (int64_t)1 << bits;
-    }
-    h->slots = total;
-    h->tab = (bm_pair32*)calloc((size_t)(total ? total : 2), sizeof(bm_pair32));
-    if (!h->tab) { bm_rowhash_free(h); return BM_ERR_NOMEM; }
-    for (int32_t r = 0; r <= n; r++) {
-        uint32_t bits = (uint32_t)(h->desc[r] & 63u);
-        if (!bits) continue;
-        bm_pair32* t = h->tab + (h->desc[r] >> 6);
-        uint32_t mask = (1u << bits) - 1u;
-        for (int64_t p = rows->ptr[r]; p < rows->ptr[r + 1]; p++) {
-            uint32_t s = bm_slot_hash(rows->adj[p].x, bits);
-            while (t[s].x != 0) s = (s + 1u) & mask;
-            t[s] = rows->adj[p];
-        }
-    }
-    return BM_OK;
-}
-
-int bm_rowhash_get(const bm_rowhash_host* h, int32_t row, int32_t key, int32_t* w) {
-    if (row < 0 || row > h->n) return 0;
-    uint32_t bits = (uint32_t)(h->desc[row] & 63u);
-    if (!bits) return 0;
-    const bm_pair32* t = h->tab + (h->desc[row] >> 6);
-    uint32_t mask = (1u << bits) - 1u;
-    uint32_t s = bm_slot_hash(key, bits);
-    for (;;) {
-        if (t[s].x == 0) return 0;
-        if (t[s].x == key) { *w = t[s].y; return 1; }
-        s = (s + 1u) & mask;
-    }
-}
