@@ -19,8 +19,9 @@ identical deltas:
            current matching (plus its transpose for the umajor stream), then
            evaluates every pair from table entries plus an exact correction
            for adjacent pairs (default headline);
-  scan  -- each pair scans its four male lists against LDS-staged female rows
-           (one wavefront per pair).
+  scan  -- each pair's terms are intersections of male lists with female rows,
+           the shorter side looked up in the longer one's row table (one
+           wavefront per pair).
 The 3-vertex permutation kernels are timed on 2^26 uniform triples per step
 in the same run (the a-major stream: triples grouped by first vertex, same law
 as independent triples, see bm_amajor_partners in bm_rng.h) and reported

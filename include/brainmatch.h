@@ -150,8 +150,8 @@ int bm_greedy_match_device(bm_ctx* ctx, int32_t* pi);
 /* Context: graphs + matching resident in HBM                          */
 /* ------------------------------------------------------------------ */
 
-/* Builds male CSR/CSC and the per-row female hash tables, copies them to
- * device `device`, and sets pi = identity-free zero matching.  Replaces the
+/* Builds CSR/CSC of both graphs, copies them to device `device`, builds the
+ * per-row hash tables there, and sets pi = identity-free zero matching.  Replaces the
  * dense (n+1)^2 short matrices and their 1.37 GB H2D copy
  * (src/graph-re-alignment-gpu-swap.cu:1040-1062). */
 int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm_edges* female,
@@ -281,7 +281,8 @@ int bm_batch_eval_rot3(bm_batch* b);
  * same stream without materialising it.  With the gain table enabled and
  * n <= 18,975, one block per first vertex stages the two table rows it needs
  * and its adjacency bitmaps in LDS (the table's transpose is kept next to it,
- * doubling the table's memory); up to n of about 218,000 it stages only the
+ * doubling the table's memory) or, for a complete matching, small non-negative
+ * weights and at least n^2 / 2 pairs, one row of deltas; up to n of about 218,000 it stages only the
  * bitmaps and gathers both table entries (no transpose); beyond that each
  * pair is evaluated on its own. */
 int bm_batch_gen_umajor(bm_batch* b, uint64_t seed, int64_t k);
@@ -351,7 +352,9 @@ int bm_gain_row(bm_ctx* ctx, int32_t u, int32_t* row);
  * src/best-swap/score-lookup.c:246-293 (create_score_lookup) and :612-620
  * (extract_max): recomputed from the table on every call, so no entry is
  * stale and no delta is truncated to int16.  Needs the table (BM_ERR_ARG
- * otherwise) and, once, a transposed copy of it (bm_gain_table_bytes more). */
+ * otherwise); a matching that is incomplete or shares females, or weights that
+ * are negative or large, also need, once, a transposed copy of it
+ * (bm_gain_table_bytes more). */
 int bm_best_swap(bm_ctx* ctx, int64_t* delta, int32_t* u, int32_t* v);
 /* Best partner of every u in u0 .. u0 + count - 1 under the context
  * matching: delta[i] = the largest exact delta of swapping u = u0 + i with a
@@ -393,9 +396,9 @@ int bm_uniform_algo_bytes(bm_ctx* ctx, uint64_t seed, int64_t k, int64_t* bytes,
 int bm_umajor_algo_bytes(bm_ctx* ctx, uint64_t seed, int64_t k, int64_t* bytes, int64_t* sum_degree);
 
 /* Launch-shape knobs (autotuner).  waves_per_block in {1,2,4,8},
- * lds_slots per wave (table slots of 4 bytes for graphs with n < 2^17 and
- * female weights in 0..32767, else 8 bytes; a multiple of 4), blocks_per_cu
- * >= 1 (capped at launch by the occupancy the kernel reaches). */
+ * blocks_per_cu >= 1 (capped at launch by the occupancy the kernel reaches).
+ * lds_slots (a positive multiple of 4) is still checked and returned, but no
+ * kernel builds tables in LDS any more. */
 typedef struct bm_tuning {
     int32_t waves_per_block;
     int32_t lds_slots;
@@ -618,7 +621,8 @@ int bm_climb(bm_ctx* ctx, const bm_climb_opts* opts, int64_t* trace_score, doubl
  * five permutations of a uniform vertex triple, the random streams are
  * counter-based per chain, and exp is a deterministic function with the same
  * bits on the host and the device, so that any chain can be replayed exactly
- * on the CPU.  One chain per wavefront; all chains of all instances advance
+ * on the CPU.  One chain per wavefront (per block of four waves up to 1,024
+ * chains); all chains of all instances advance
  * in one kernel launch, replayed from a captured HIP graph. */
 typedef struct bm_anneal bm_anneal;
 
