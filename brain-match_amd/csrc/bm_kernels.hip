@@ -454,6 +454,7 @@ __global__ void __launch_bounds__(kAccThreads) k_accept_greedy(BmDevGraph g, int
     }
     __syncthreads();
     for (int64_t base = 0; base < npos; base += kAccThreads) {
+        if (s_nacc >= max_accept) break;   /* or every later tile is loaded and scanned for nothing */
         const int64_t i = base + t;
         const bool valid = i < npos;
         int64_t ci = -1, di = 0;

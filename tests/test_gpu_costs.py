@@ -1,0 +1,43 @@
+"""Calls whose time must follow the work they are asked for, compared with a
+second call on the same device rather than with a clock: factors of several
+lie between the two sides of every comparison."""
+import time
+
+import numpy as np
+import pytest
+from conftest import make_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def _best(prepare, call, reps=3):
+    t = []
+    for _ in range(reps):
+        prepare()
+        a = time.perf_counter()
+        call()
+        t.append(time.perf_counter() - a)
+    return min(t)
+
+
+def test_acceptance_ends_at_its_limit(bm, orc):
+    """One accepted swap of 2^22 positive candidates does not walk the other
+    4,095 tiles of 1,024 candidates."""
+    n, k = 3000, 1 << 22
+    male, female, _, pi = make_pair(bm, n=n, deg=3.0, seed=21)
+    uv = orc.uniform_pairs(5, 50000, n)
+    up = uv[orc.Oracle(n, male, female).swap_deltas(pi, uv) > 0]
+    with bm.Context(n, male, female) as ctx:
+        b = ctx.batch(k)
+        b.set_pairs(np.resize(up, (k, 2)))
+
+        def prepare():
+            ctx.set_mapping(pi)
+            b.eval_swaps()
+            assert b.stats()["n_pos"] == k
+
+        one = _best(prepare, lambda: b.accept_disjoint(1))
+        many = _best(prepare, lambda: b.accept_disjoint(0))
+        b.close()
+    print(f"[costs] one {1e3 * one:.2f} ms, all {1e3 * many:.2f} ms", flush=True)
+    assert one < 0.5 * many
