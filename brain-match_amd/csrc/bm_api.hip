@@ -82,6 +82,7 @@ struct bm_ctx {
     int4* d_moves;
     int64_t moves_cap;
     int64_t* d_nmoves;
+    int64_t* d_patch_plan;  /* 4 moves_cap + 1 work-item offsets of a table patch */
     int32_t* d_patch_rows;  /* rows touched by a table patch (bm_gain_update_rows) */
     int64_t gain_version;   /* bumped by every build and patch of the table */
     /* u-major evaluation (bm_batch_eval_swaps_umajor) */
@@ -281,6 +282,7 @@ static void free_ctx(bm_ctx* c) {
     (void)hipFree(c->d_f_self);
     (void)hipFree(c->d_moves);
     (void)hipFree(c->d_nmoves);
+    (void)hipFree(c->d_patch_plan);
     (void)hipFree(c->d_patch_rows);
     (void)hipFree(c->d_um_counts);
     (void)hipFree(c->d_um_off);
@@ -354,9 +356,12 @@ static int gain_moves_cap(bm_ctx* c, int64_t need) {
     if (c->moves_cap >= need) return BM_OK;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     (void)hipFree(c->d_moves);
+    (void)hipFree(c->d_patch_plan);
     c->d_moves = nullptr;
+    c->d_patch_plan = nullptr;
     c->moves_cap = 0;
     HIPCHK(c, hipMalloc((void**)&c->d_moves, (size_t)need * sizeof(int4)));
+    HIPCHK(c, hipMalloc((void**)&c->d_patch_plan, (size_t)(4 * need + 1) * sizeof(int64_t)));
     c->moves_cap = need;
     return BM_OK;
 }
@@ -366,20 +371,36 @@ static int64_t male_degree(const bm_ctx* c, int32_t x) {
     return (c->male.out.ptr[x + 1] - c->male.out.ptr[x]) + (c->male.in.ptr[x + 1] - c->male.in.ptr[x]);
 }
 
-/* Whether a patch of moves of the vertices xs (k of them) should also patch
- * the transposed copy: its additions land in as many rows as the moved
+/* Whether a patch of moves of vertices with `deg` male edges together should
+ * also patch the transposed copy: its additions land in as many rows as the moved
  * vertices have male edges, one 4-byte add per row and female entry, so it
  * pays against a 0.54 ms transpose (n = 18,524) only for moves of vertices of
  * ordinary degree (together at most 8x the mean); hub moves leave the copy to
  * be rebuilt. */
-static bool gt_patch_pays(const bm_ctx* c, const int32_t* xs, int k) {
-    int64_t deg = 0;
-    for (int i = 0; i < k; i++) deg += male_degree(c, xs[i]);
+static bool gt_patch_pays(const bm_ctx* c, int64_t deg) {
     const int64_t mean2 = c->n > 0 ? 2 * c->male.m / c->n : 0;
     return deg <= 8 * (mean2 > 1 ? mean2 : 1);
 }
 
-static int gain_patch(bm_ctx* c, const int64_t* d_count, int64_t max_moves, bool gt_allowed) {
+/* Whether a patch of n_moves moves of vertices with `deg` male edges together
+ * goes by rows (bm_launch_gain_update).  With d = deg / n_moves edges a move,
+ * each of the deg edges brings about d additions; by rows every row touched (at
+ * most deg and at most n) also searches all moves, which is worth d * deg >= 4 *
+ * n_moves * rows additions in LDS instead of memory; below d = 64 the form's
+ * third launch is not earned back.  us by items / by rows, n = 18,524: a swap
+ * of d = 44 13 / 16, 90 20 / 16, 280 49 / 24, of hubs 4,643 / 1,312; 122 swaps
+ * at d = 40 36 / 208, 9 at d = 120 59 / 56, 33 at d = 120 74 / 102, 64 at d =
+ * 430 1,287 / 809; n = 36,000, 59 swaps at d = 200 521 / 647.  A row past the
+ * LDS would be one wave's work: n = 50,000, a swap of d = 40 46 / 161. */
+static bool patch_by_rows(const bm_ctx* c, int64_t n_moves, double deg) {
+    if (n_moves < 1 || bm_gain_stride(c->n) * (int64_t)sizeof(int32_t) > BM_PATCH_LDS) return false;
+    const double d = deg / (double)n_moves, rows = deg < c->n ? deg : c->n;
+    return d >= 64.0 && d * deg >= 4.0 * (double)n_moves * rows;
+}
+
+/* d_count: *d_count <= max_moves moves; deg: about how many male edges their
+ * vertices have. */
+static int gain_patch(bm_ctx* c, const int64_t* d_count, int64_t max_moves, double deg, bool gt_allowed) {
     KTiming t;
     timing_begin(c, BM_KERNEL_GAIN_UPDATE, &t);
     if (max_moves > c->moves_cap) return fail(c, BM_ERR_STATE, "gain patch: %lld moves exceed the move list",
@@ -389,7 +410,8 @@ static int gain_patch(bm_ctx* c, const int64_t* d_count, int64_t max_moves, bool
      * the caller found that cheaper (gt_patch_pays) */
     const bool gt = gt_allowed && c->d_GT && c->gt_version == c->gain_version;
     HIPCHK(c, bm_launch_gain_update(devgraph(c), devgain(c), gt ? c->d_GT : nullptr, c->d_moves, d_count, max_moves,
-                                    c->d_patch_rows, c->num_cus, c->stream));
+                                    c->d_patch_plan, patch_by_rows(c, max_moves, deg) ? c->d_patch_rows : nullptr,
+                                    c->num_cus, c->stream));
     timing_end(c, &t);
     c->gain_version++;
     if (gt) c->gt_version = c->gain_version;
@@ -1416,12 +1438,12 @@ static int accept_impl(bm_batch* b, int64_t max_accept, int32_t* accepted, int64
     HIPCHK(c, bm_launch_accept(devgraph(c), c->d_pi, c->d_pi + c->n + 1, (const int2*)b->d_cand, b->d_delta, b->k, max_accept,
                                b->d_acc_scratch, b->acc_scratch_bytes, b->d_acc_idx, b->d_out, c->h_pin,
                                c->gain_on ? c->d_moves : nullptr, c->stream));
-    if (c->gain_on && b->k > 0) {
-        int rc = gain_patch(c, b->d_out + 2, 2 * b->k, false);
-        if (rc != BM_OK) return rc;
-    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const int64_t meta[2] = {c->h_pin[0], c->h_pin[1]};
+    if (c->gain_on && meta[0] > 0) {   /* the form of the patch depends on the number of moves */
+        const int rc = gain_patch(c, b->d_out + 2, 2 * meta[0], 2.0 * (double)meta[0] * (2.0 * c->male.m / c->n), false);
+        if (rc != BM_OK) return rc;
+    }
     if (accepted && meta[0] > 0) {
         std::vector<int64_t> idx((size_t)meta[0]);
         HIPCHK(c, hipMemcpy(idx.data(), b->d_acc_idx, (size_t)meta[0] * sizeof(int64_t), hipMemcpyDeviceToHost));
@@ -1525,8 +1547,8 @@ extern "C" int bm_apply_swap(bm_ctx* c, int32_t u, int32_t v) {
     }
     HIPCHK(c, bm_launch_apply_swap(c->d_pi, c->d_pi + c->n + 1, u, v, c->stream));
     if (c->gain_on) {
-        const int32_t xs[2] = {u, v};
-        return gain_patch(c, c->d_nmoves, 2, gt_patch_pays(c, xs, 2));
+        const int64_t deg = male_degree(c, u) + male_degree(c, v);
+        return gain_patch(c, c->d_nmoves, 2, (double)deg, gt_patch_pays(c, deg));
     }
     return BM_OK;
 }
@@ -1624,8 +1646,8 @@ extern "C" int bm_apply_perm3(bm_ctx* c, int32_t a, int32_t b, int32_t d, int32_
     }
     HIPCHK(c, bm_launch_apply_perm3(c->d_pi, c->d_pi + c->n + 1, a, b, d, p, c->stream));
     if (c->gain_on) {
-        const int32_t xs[3] = {a, b, d};
-        return gain_patch(c, c->d_nmoves, 3, gt_patch_pays(c, xs, 3));
+        const int64_t deg = male_degree(c, a) + male_degree(c, b) + male_degree(c, d);
+        return gain_patch(c, c->d_nmoves, 3, (double)deg, gt_patch_pays(c, deg));
     }
     return BM_OK;
 }

@@ -122,12 +122,15 @@ hipError_t bm_launch_row_bounds(const int64_t* ptr, const int2* rows, int32_t n,
 /* Table build: per column chunk, the work list (k_gain_edge_desc) then the
  * rows.  G.edesc must hold 2 x male edges + 1 entries. */
 hipError_t bm_launch_gain_build(const BmDevGraph& g, const BmGain& G, int32_t num_cus, hipStream_t s);
-/* Table patch after moves (moves[0..*count), *count <= max_moves); rows is
- * scratch of bm_gain_update_rows(n) int32 for the rows touched; GT (may be
- * NULL) is a transposed copy patched alongside. */
+/* Table patch after moves (moves[0..*count), *count <= max_moves), by work
+ * items (rows NULL; plan: 4 max_moves + 1 int64 of scratch) or by rows (rows:
+ * bm_gain_update_rows(n) int32 of scratch; plan unused; a table row of at most
+ * BM_PATCH_LDS bytes).  GT (may be NULL) is a transposed copy patched
+ * alongside. */
+#define BM_PATCH_LDS (152 * 1024)   /* of the 160 KB, beside the list of a row's edges */
 int64_t bm_gain_update_rows(int32_t n);
 hipError_t bm_launch_gain_update(const BmDevGraph& g, const BmGain& G, int32_t* GT, const int4* moves, const int64_t* count,
-                                 int64_t max_moves, int32_t* rows, int32_t num_cus, hipStream_t s);
+                                 int64_t max_moves, int64_t* plan, int32_t* rows, int32_t num_cus, hipStream_t s);
 /* Per-pair table lookups; with pis (the per-vertex words, refreshed) the
  * diagonal entries and self-loops come from them. */
 hipError_t bm_launch_gain_swap(const BmDevGraph& g, const BmGain& G, int mode, const int2* cand, const int64_t* off,

@@ -55,7 +55,6 @@ constexpr int kTileThreads = 256;
 constexpr int kPatchWaves = kPatchThreads / BM_WAVE;
 constexpr int kPatchSpan = 4 * BM_WAVE;      /* female-row entries a wave has in flight */
 constexpr int32_t kPatchDense = 16;          /* columns per entry from which a row goes through LDS */
-constexpr size_t kPatchLds = 152 * 1024;      /* of the 160 KB, beside the list of a row's edges */
 constexpr int32_t kPatchMany = 2048;         /* entries that are always enough for it */
 
 /* Word of the dense adjacency bitmap holding the pair {a, b}: bit (max & 31)
@@ -693,16 +692,115 @@ __global__ void __launch_bounds__(256) k_dense_fill(const int64_t* __restrict__ 
  * female's terms are subtracted and the new one's added; self-loops are not
  * in the table.
  *
- * k_patch_rows takes the edges of all (move, direction) slots, sums for every
- * row y the entries that will be added into it and lists the rows touched.
+ * Two forms, chosen by the caller (patch_by_rows in bm_api.hip).
+ *
+ * By work items, (move, side = old / new female, direction, group of 64 of x's
+ * edges, chunk of 64 entries of the female row): k_patch_plan counts each
+ * (move, side, direction)'s items and scans them into offsets; the waves of
+ * k_patch_items take items from the whole index space, so the work is the
+ * additions alone, whatever the number of moves, and a long female row spreads
+ * over the device.  An item: lanes hold 64 edges and 64 row entries, and each
+ * entry is applied for every edge in turn (the edge's row y and weight read out
+ * of its lane as scalars), by atomic adds into the table. */
+constexpr int kPlanThreads = 1024;
+
+__device__ __forceinline__ int64_t patch_items(const BmDevGraph& g, int4 mv, int side, int dir) {
+    const int32_t gx = side ? mv.z : mv.y;
+    if (mv.y == mv.z || gx == 0 || mv.x == 0) return 0;
+    const int64_t* mptr = dir ? g.m_out_ptr : g.m_in_ptr;
+    const int64_t* fptr = dir ? g.f_out_ptr : g.f_in_ptr;
+    const int64_t deg = mptr[mv.x + 1] - mptr[mv.x], len = fptr[gx + 1] - fptr[gx];
+    return ((deg + BM_WAVE - 1) / BM_WAVE) * ((len + BM_WAVE - 1) / BM_WAVE);
+}
+
+/* One block: off[s] = items of the slots before s, s = 4 move + 2 side + dir,
+ * off[4 nm] = all items. */
+__global__ void __launch_bounds__(kPlanThreads) k_patch_plan(BmDevGraph g, const int4* __restrict__ moves,
+                                                                  const int64_t* __restrict__ count,
+                                                                  int64_t* __restrict__ off) {
+    __shared__ int64_t part[kPlanThreads];
+    const int64_t slots = 4 * *count;
+    const int t = threadIdx.x;
+    const int64_t per = (slots + kPlanThreads - 1) / kPlanThreads;
+    const int64_t s0 = t * per, s1 = s0 + per < slots ? s0 + per : slots;
+    int64_t mine = 0;
+    for (int64_t sl = s0; sl < s1; sl++) mine += patch_items(g, moves[sl >> 2], (int)((sl >> 1) & 1), (int)(sl & 1));
+    part[t] = mine;
+    __syncthreads();
+    for (int o = 1; o < kPlanThreads; o <<= 1) {
+        const int64_t add = t >= o ? part[t - o] : 0;
+        __syncthreads();
+        part[t] += add;
+        __syncthreads();
+    }
+    int64_t run = t ? part[t - 1] : 0;
+    for (int64_t sl = s0; sl < s1; sl++) {
+        off[sl] = run;
+        run += patch_items(g, moves[sl >> 2], (int)((sl >> 1) & 1), (int)(sl & 1));
+    }
+    if (t == kPlanThreads - 1) off[slots] = part[t];
+}
+
+__global__ void __launch_bounds__(kPatchThreads) k_patch_items(BmDevGraph g, BmGain G, const int4* __restrict__ moves,
+                                                               const int64_t* __restrict__ count,
+                                                               const int64_t* __restrict__ off,
+                                                               int32_t* __restrict__ GT) {
+    const int lane = threadIdx.x & (BM_WAVE - 1);
+    const int64_t slots = 4 * *count;
+    const int64_t total = off[slots];
+    const int64_t nw = (int64_t)gridDim.x * kPatchWaves;
+    for (int64_t item = (int64_t)blockIdx.x * kPatchWaves + threadIdx.x / BM_WAVE; item < total; item += nw) {
+        /* the slot holding the item: the last s with off[s] <= item */
+        int64_t lo = 0, hi = slots;   /* off[lo] <= item < off[hi] */
+        while (hi - lo > 1) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (off[mid] <= item) lo = mid;
+            else hi = mid;
+        }
+        const int4 mv = moves[lo >> 2];
+        const int side = (int)((lo >> 1) & 1), dir = (int)(lo & 1);
+        const int32_t x = mv.x, gx = side ? mv.z : mv.y;
+        const int32_t sign = side ? 1 : -1;
+        const int64_t* mptr = dir ? g.m_out_ptr : g.m_in_ptr;
+        const int2* madj = dir ? g.m_out : g.m_in;
+        const int64_t* fptr = dir ? g.f_out_ptr : g.f_in_ptr;
+        const int2* fadj = dir ? g.f_out : g.f_in;
+        const int64_t b = mptr[x], e = mptr[x + 1];
+        const int64_t rb = fptr[gx], re = fptr[gx + 1];
+        const int64_t nchunk = (re - rb + BM_WAVE - 1) / BM_WAVE;
+        const int64_t local = item - off[lo];
+        const int64_t e0 = b + (local / nchunk) * BM_WAVE;
+        const int64_t i = e0 + lane;
+        const int2 ed = i < e ? madj[i] : make_int2(0, 0);
+        const int32_t yl = ed.x != x ? ed.x : 0;   /* 0: past the list or a self-loop */
+        const int32_t nv = e - e0 < BM_WAVE ? (int32_t)(e - e0) : BM_WAVE;
+        const int64_t ri = rb + (local % nchunk) * BM_WAVE + lane;
+        const bool rin = ri < re;
+        const int2 ent = rin ? fadj[ri] : make_int2(0, 0);
+        for (int32_t k = 0; k < nv; k++) {
+            const int32_t y = __builtin_amdgcn_readlane(yl, k);
+            if (y == 0) continue;
+            const int32_t w = __builtin_amdgcn_readlane(ed.y, k);
+            if (rin) {
+                const int32_t d = sign * (w < ent.y ? w : ent.y);
+                atomicAdd(&G.G[(int64_t)y * G.stride + ent.x], d);
+                if (GT) atomicAdd(&GT[(int64_t)ent.x * G.stride + y], d);   /* the transposed copy, when kept */
+            }
+        }
+    }
+}
+
+/* By rows: k_patch_rows takes the edges of all (move, direction) slots, sums for
+ * every row y the entries that will be added into it and lists the rows touched.
  * In k_gain_update each listed row has one owner, which finds the slots with
- * an edge at y by binary search: a wave adds a few entries straight into the
+ * an edge at y by binary search in all of them, so this form is for few moves:
+ * a wave adds a few entries straight into the
  * table; many (one for every kPatchDense columns, as a hub's edges bring) a
  * block adds into a copy of the row in LDS, so that the row crosses memory
  * once each way instead of a sector per entry and side.  The best swaps of a
  * heavy-tailed graph move hubs: at n = 18,524 the patch of a vertex with
- * edges to all others adds 3.5e8 entries to 18,523 rows, 1.39 ms by atomic
- * adds into the table and 0.90 ms here (0.60 ms for the bytes alone); over
+ * edges to all others adds 3.5e8 entries to 18,523 rows, 1.39 ms by work items
+ * and 0.90 ms here (0.60 ms for the bytes alone); over
  * the first 32 best swaps 555 us -> 339 us.  Blocks of 1,024 threads: 393 us. */
 __global__ void __launch_bounds__(kPatchThreads) k_patch_rows(BmDevGraph g, const int4* __restrict__ moves,
                                                               const int64_t* __restrict__ count,
@@ -775,7 +873,7 @@ __global__ void __launch_bounds__(kPatchThreads) k_gain_update(BmDevGraph g, BmG
                                                                const int64_t* __restrict__ count,
                                                                const int32_t* __restrict__ rows, int32_t dense,
                                                                int32_t* __restrict__ GT) {
-    extern __shared__ int32_t row[];   /* one table row, if rows are taken through LDS */
+    extern __shared__ int32_t row[];   /* one table row */
     __shared__ int2 s_found[kPatchThreads];   /* {slot - first, weight} of the edges at the row */
     __shared__ int32_t s_n;
     const int t = threadIdx.x, lane = t & (BM_WAVE - 1), wave = t / BM_WAVE;
@@ -2000,27 +2098,27 @@ hipError_t bm_launch_gain_build(const BmDevGraph& g, const BmGain& G, int32_t nu
 int64_t bm_gain_update_rows(int32_t n) { return 2 * ((int64_t)n + 1) + 1; }
 
 hipError_t bm_launch_gain_update(const BmDevGraph& g, const BmGain& G, int32_t* GT, const int4* moves, const int64_t* count,
-                                 int64_t max_moves, int32_t* rows, int32_t num_cus, hipStream_t s) {
+                                 int64_t max_moves, int64_t* plan, int32_t* rows, int32_t num_cus, hipStream_t s) {
     if (max_moves <= 0) return hipSuccess;
     const int64_t cus = num_cus > 0 ? num_cus : 256;
+    if (!rows) {
+        hipLaunchKernelGGL(k_patch_plan, dim3(1), dim3(kPlanThreads), 0, s, g, moves, count, plan);
+        /* persistent grid: every wave walks the item space */
+        hipLaunchKernelGGL(k_patch_items, dim3((unsigned)(4 * cus)), dim3(kPatchThreads), 0, s, g, G, moves, count, plan, GT);
+        return hipGetLastError();
+    }
     const int64_t used = (int64_t)g.n + 2;   /* the counter and the loads */
     int64_t zb = (used + 255) / 256;
     if (zb > 4 * cus) zb = 4 * cus;
     hipLaunchKernelGGL(k_zero_words, dim3((unsigned)zb), dim3(256), 0, s, reinterpret_cast<uint32_t*>(rows), used);
     hipLaunchKernelGGL(k_patch_rows, dim3((unsigned)(2 * cus)), dim3(kPatchThreads), 0, s, g, moves, count, rows);
-    /* a row wider than LDS is patched in place, however many its entries */
-    size_t lds = (size_t)G.stride * sizeof(int32_t);
-    int32_t dense = INT32_MAX;
-    if (lds <= kPatchLds) {
-        dense = (int32_t)(G.stride / kPatchDense);
-        if (dense > kPatchMany) dense = kPatchMany;
-        hipError_t e = hipFuncSetAttribute((const void*)k_gain_update, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds);
-        if (e != hipSuccess) return e;
-    } else {
-        lds = 0;
-    }
-    int64_t per = lds ? (int64_t)(kPatchLds / lds) : 4;
+    const size_t lds = (size_t)G.stride * sizeof(int32_t);
+    if (lds > BM_PATCH_LDS) return hipErrorInvalidValue;
+    int32_t dense = (int32_t)(G.stride / kPatchDense);
+    if (dense > kPatchMany) dense = kPatchMany;
+    hipError_t e = hipFuncSetAttribute((const void*)k_gain_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    int64_t per = (int64_t)(BM_PATCH_LDS / lds);
     if (per > 4) per = 4;
     hipLaunchKernelGGL(k_gain_update, dim3((unsigned)(per * cus)), dim3(kPatchThreads), lds, s, g, G, moves, count, rows,
                        dense, GT);

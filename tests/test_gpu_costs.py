@@ -41,3 +41,29 @@ def test_acceptance_ends_at_its_limit(bm, orc):
         b.close()
     print(f"[costs] one {1e3 * one:.2f} ms, all {1e3 * many:.2f} ms", flush=True)
     assert one < 0.5 * many
+
+
+def test_patch_of_an_accepted_batch_costs_less_than_a_build(bm):
+    """Hundreds of accepted swaps of a sparse graph, a few thousand edges in
+    all, are added to the table in a fraction of the time that builds it."""
+    n, k = 36000, 1 << 18
+    male, female, _, pi = make_pair(bm, n=n, deg=20.0, weights=bm.WEIGHTS_LOGNORMAL, seed=4)
+    with bm.Context(n, male, female) as ctx:
+        ctx.set_mapping(pi)
+        ctx.gain_enable(True)
+        ctx.timing_enable(True)
+        b = ctx.batch(k)
+        patch, build = [], []
+        for seed in (1, 2, 3):
+            ctx.timing_reset()
+            ctx.set_mapping(pi)
+            b.gen_pairs(seed, k)
+            b.eval_swaps()
+            accepted, _ = b.accept_disjoint()
+            ctx.sync()
+            assert accepted > 300
+            patch.append(ctx.timing(bm.KERNEL_GAIN_UPDATE)[1])
+            build.append(ctx.timing(bm.KERNEL_GAIN_BUILD)[1])
+        b.close()
+    print(f"[costs] {accepted} swaps: patch {min(patch):.3f} ms, build {min(build):.3f} ms", flush=True)
+    assert min(patch) < 0.5 * min(build)
