@@ -760,8 +760,11 @@ class Anneal:
         self._chk(_lib.bm_anneal_get_tuning(self.h, C.byref(t)))
         return {k: getattr(t, k) for k, _ in _Tuning._fields_}
 
-    def set_tuning(self, waves_per_block, lds_slots, blocks_per_cu, unroll=4):
-        t = _Tuning(waves_per_block, lds_slots, blocks_per_cu, 64, unroll)
+    def set_tuning(self, waves_per_block, lds_slots, blocks_per_cu, unroll=4, group_lanes=0):
+        """group_lanes 64: one wave per chain in this shape; 256: a block's
+        four waves per chain; 0: the library's choice of the two (tuning()
+        reports it), this shape applying to one wave per chain."""
+        t = _Tuning(waves_per_block, lds_slots, blocks_per_cu, group_lanes, unroll)
         self._chk(_lib.bm_anneal_set_tuning(self.h, C.byref(t)))
 
     def autotune(self, steps=100):

@@ -31,9 +31,8 @@
 
 extern "C" const char* bm_global_error(void);
 
-/* Chains that leave wave slots idle (256 CUs x 16 waves) are bound by the
- * latency of a step, so each gets the four waves of a block. */
-static constexpr int64_t kCoopChains = 1024;
+/* bm_tuning.group_lanes of the chain kernel */
+static constexpr int kWaveLanes = 64, kBlockLanes = 256;
 
 struct bm_anneal {
     int device;
@@ -58,6 +57,7 @@ struct bm_anneal {
     std::vector<int2*> prop_buf;      /* per instance, capacity prop_cap */
     std::vector<int64_t> prop_cap;
     BmAnnealSched sc;
+    double mean_deg;                  /* male edges per vertex, mean over the instances */
     BmLaunch L;
     int compact;
     int packed;
@@ -120,6 +120,35 @@ extern "C" const char* bm_anneal_last_error(const bm_anneal* a) {
 
 extern "C" int64_t bm_anneal_num_chains(const bm_anneal* a) { return a ? a->n_chains : 0; }
 
+/* Launch shape L for the chains: one wave per chain (lanes 64), the four waves
+ * of a block (256), or (any other value) whichever suits them.  A chain's steps
+ * are a serial chain of dependent loads, so where the blocks of the wide form
+ * are all resident four waves are faster as soon as a step has entries for
+ * them; in two rounds only with longer lists.  200 steps, one instance, 10%
+ * 3-vertex moves, us with four waves / with one: 256 chains of 10 edges a
+ * vertex 899 / 843, of 20 977 / 1,015, of 50 1,285 / 2,062, of 200 2,068 /
+ * 6,472; 1,024 chains (two rounds: 768 blocks are resident) of 50 2,738 /
+ * 2,288, of 100 3,229 / 3,920. */
+static hipError_t chain_shape(bm_anneal* a, BmLaunch L, int lanes) {
+    const int rot = a->sc.p_rot3 != 0;
+    dim3 grid, block;
+    L.coop = 1;
+    hipError_t e = bm_anneal_grid(a->packed, rot, L, (int64_t)1 << 40, &grid, &block);
+    if (e != hipSuccess) return e;
+    const int64_t resident = grid.x;
+    if (lanes == kWaveLanes || lanes == kBlockLanes)
+        L.coop = lanes == kBlockLanes;
+    else
+        L.coop = a->mean_deg >= 20.0 &&
+                 (a->n_chains <= resident || (a->mean_deg >= 80.0 && a->n_chains <= 4 * (int64_t)L.num_cus));
+    e = bm_anneal_grid(a->packed, rot, L, a->n_chains, &grid, &block);
+    if (e != hipSuccess) return e;
+    a->L = L;
+    a->grid = grid;
+    a->block = block;
+    return hipSuccess;
+}
+
 extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_inst, const bm_anneal_params* p) {
     if (!out) return afail(nullptr, BM_ERR_ARG, "bm_anneal_create: out is NULL");
     *out = nullptr;
@@ -180,7 +209,8 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
     /* launch shape: the swap kernel's tuning of the first context */
     a->L = bm_ctx_launch(ctxs[0], BM_KERNEL_SWAP);
     if (!a->compact && a->graphs[0].compact) a->L.lds_slots /= 2;
-    a->L.coop = a->n_chains <= kCoopChains;
+    for (int32_t i = 0; i < n_inst; i++)
+        a->mean_deg += (double)bm_ctx_male(ctxs[i])->m / a->graphs[i].n / n_inst;
 
     int64_t pool = 0;
     a->pi_off.resize((size_t)a->n_chains);
@@ -236,7 +266,7 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
     a->sc.traj_cap = p->traj_cap;
     a->sc.pad = 0;
     a->sc.p_pool = (uint64_t)llround(p->p_pool * 4294967296.0);
-    ACHK(bm_anneal_grid(a->packed, a->sc.p_rot3 != 0, a->L, a->n_chains, &a->grid, &a->block));
+    ACHK(chain_shape(a, a->L, 0));
     ACHK(hipStreamSynchronize(a->stream));
 #undef ACHK
     *out = a;
@@ -503,11 +533,11 @@ extern "C" int bm_anneal_reset(bm_anneal* a) {
 
 extern "C" int bm_anneal_get_tuning(const bm_anneal* a, bm_tuning* t) {
     if (!a || !t) return BM_ERR_ARG;
-    t->waves_per_block = a->L.waves_per_block;
+    t->waves_per_block = a->L.coop ? 4 : a->L.waves_per_block;
     t->lds_slots = a->L.lds_slots;
     t->blocks_per_cu = a->L.blocks_per_cu;
-    t->group_lanes = 64;
-    t->unroll = a->L.unroll == 2 ? 2 : 4;
+    t->group_lanes = a->L.coop ? kBlockLanes : kWaveLanes;
+    t->unroll = a->L.coop || a->L.unroll != 2 ? 4 : 2;
     return BM_OK;
 }
 
@@ -525,12 +555,8 @@ extern "C" int bm_anneal_set_tuning(bm_anneal* a, const bm_tuning* t) {
     L.lds_slots = t->lds_slots;
     L.blocks_per_cu = t->blocks_per_cu;
     L.unroll = t->unroll;
-    dim3 grid, block;
     AHIP(a, hipSetDevice(a->device));
-    AHIP(a, bm_anneal_grid(a->packed, a->sc.p_rot3 != 0, L, a->n_chains, &grid, &block));
-    a->L = L;
-    a->grid = grid;
-    a->block = block;
+    AHIP(a, chain_shape(a, L, t->group_lanes));
     if (a->exec) (void)hipGraphExecDestroy(a->exec);
     if (a->graph) (void)hipGraphDestroy(a->graph);
     a->exec = nullptr;
@@ -539,16 +565,15 @@ extern "C" int bm_anneal_set_tuning(bm_anneal* a, const bm_tuning* t) {
 }
 
 /* Times one launch of `steps` steps for every launch shape in a small grid
- * (list entries per lane x waves per block x table slots per wave x blocks
- * per CU), keeps the fastest, and resets the chains.  trials (may be NULL)
- * gets up to max_trials records {waves, slots, blocks_per_cu, unroll, ms}. */
+ * (one wave per chain: list entries per lane x waves per block x blocks per
+ * CU; then the four waves of a block per chain), keeps the fastest, and resets
+ * the chains.  trials (may be NULL) gets up to max_trials records {waves,
+ * slots, blocks_per_cu, unroll, ms}, the four-wave form's the last. */
 extern "C" int bm_anneal_autotune(bm_anneal* a, int64_t steps, bm_tuning* best, double* trials, int32_t max_trials,
                                   int32_t* n_trials) {
     if (!a || steps < 1) return afail(a, BM_ERR_ARG, "bm_anneal_autotune: invalid argument");
-    const int waves[4] = {1, 2, 4, 8};
-    const int slots_c[3] = {640, 1280, 2560}, slots_w[3] = {320, 640, 1280};
-    const int bpc[2] = {4, 16};
-    const int unrolls[2] = {2, 4};
+    const int bpc[3] = {4, 8, 16};
+    constexpr int kShapes = 2 * 4 * 3 + 1;
     bm_tuning bt;
     memset(&bt, 0, sizeof bt);
     double best_ms = 1e300;
@@ -558,44 +583,41 @@ extern "C" int bm_anneal_autotune(bm_anneal* a, int64_t steps, bm_tuning* best, 
     AHIP(a, hipEventCreate(&e0));
     AHIP(a, hipEventCreate(&e1));
     int rc = BM_OK;
-    for (int ui = 0; ui < 2 && rc == BM_OK; ui++)
-    for (int wi = 0; wi < 4 && rc == BM_OK; wi++)
-        for (int si = 0; si < 3 && rc == BM_OK; si++)
-            for (int bi = 0; bi < 2 && rc == BM_OK; bi++) {
-                bm_tuning t;
-                t.waves_per_block = waves[wi];
-                t.lds_slots = a->compact ? slots_c[si] : slots_w[si];
-                t.blocks_per_cu = bpc[bi];
-                t.group_lanes = 64;
-                t.unroll = unrolls[ui];
-                if ((size_t)t.waves_per_block * t.lds_slots * (a->compact ? 4 : 8) > 160 * 1024) continue;
-                if ((rc = bm_anneal_set_tuning(a, &t)) != BM_OK) break;
-                if ((rc = reset_chains(a)) != BM_OK) break;
-                hipError_t e = hipEventRecord(e0, a->stream);
-                if (e == hipSuccess)
-                    e = bm_launch_anneal(a->d_insts, a->packed, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
-                                         nullptr, a->d_props, a->L, a->grid, a->block, a->stream);
-                if (e == hipSuccess) e = hipEventRecord(e1, a->stream);
-                if (e == hipSuccess) e = hipEventSynchronize(e1);
-                float ms = 0.f;
-                if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-                if (e != hipSuccess) {
-                    rc = afail(a, BM_ERR_HIP, "bm_anneal_autotune: trial launch failed: %s", hipGetErrorString(e));
-                    break;
-                }
-                if (trials && nt < max_trials) {
-                    trials[5 * nt] = t.waves_per_block;
-                    trials[5 * nt + 1] = t.lds_slots;
-                    trials[5 * nt + 2] = t.blocks_per_cu;
-                    trials[5 * nt + 3] = t.unroll;
-                    trials[5 * nt + 4] = ms;
-                }
-                nt++;
-                if (ms < best_ms) {
-                    best_ms = ms;
-                    bt = t;
-                }
-            }
+    for (int i = 0; i < kShapes; i++) {
+        const bool share = i == kShapes - 1;
+        bm_tuning t;
+        t.waves_per_block = share ? 4 : 1 << (i / 3 % 4);
+        t.lds_slots = a->compact ? 1280 : 640;
+        t.blocks_per_cu = share ? 16 : bpc[i % 3];
+        t.group_lanes = share ? kBlockLanes : kWaveLanes;
+        t.unroll = share || i >= 12 ? 4 : 2;
+        if ((rc = bm_anneal_set_tuning(a, &t)) != BM_OK) break;
+        if ((rc = reset_chains(a)) != BM_OK) break;
+        hipError_t e = hipEventRecord(e0, a->stream);
+        if (e == hipSuccess)
+            e = bm_launch_anneal(a->d_insts, a->packed, a->d_chains, a->n_chains, a->d_pool, steps, a->sc,
+                                 nullptr, a->d_props, a->L, a->grid, a->block, a->stream);
+        if (e == hipSuccess) e = hipEventRecord(e1, a->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(e1);
+        float ms = 0.f;
+        if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
+        if (e != hipSuccess) {
+            rc = afail(a, BM_ERR_HIP, "bm_anneal_autotune: trial launch failed: %s", hipGetErrorString(e));
+            break;
+        }
+        if (trials && nt < max_trials) {
+            trials[5 * nt] = t.waves_per_block;
+            trials[5 * nt + 1] = t.lds_slots;
+            trials[5 * nt + 2] = t.blocks_per_cu;
+            trials[5 * nt + 3] = t.unroll;
+            trials[5 * nt + 4] = ms;
+        }
+        nt++;
+        if (ms < best_ms) {
+            best_ms = ms;
+            bt = t;
+        }
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc != BM_OK) return rc;

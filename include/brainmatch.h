@@ -403,7 +403,7 @@ typedef struct bm_tuning {
     int32_t waves_per_block;
     int32_t lds_slots;
     int32_t blocks_per_cu;
-    int32_t group_lanes;  /* lanes cooperating on one candidate (64) */
+    int32_t group_lanes;  /* lanes cooperating on one candidate (64; annealing chains: 64 or 256) */
     int32_t unroll;       /* list entries per lane in flight: 2, 4 or 8 (swap kernel),
                              2 or 4 (3-vertex kernel, annealing chains);
                              female-row entries per lane, 4, 8, 16 or 32 (table build,
@@ -621,9 +621,10 @@ int bm_climb(bm_ctx* ctx, const bm_climb_opts* opts, int64_t* trace_score, doubl
  * five permutations of a uniform vertex triple, the random streams are
  * counter-based per chain, and exp is a deterministic function with the same
  * bits on the host and the device, so that any chain can be replayed exactly
- * on the CPU.  One chain per wavefront (per block of four waves up to 1,024
- * chains); all chains of all instances advance
- * in one kernel launch, replayed from a captured HIP graph. */
+ * on the CPU.  One chain per wavefront, or per block of four waves where few
+ * chains of longer lists would leave the device idle (bm_anneal_set_tuning);
+ * all chains of all instances advance in one kernel launch, replayed from a
+ * captured HIP graph. */
 typedef struct bm_anneal bm_anneal;
 
 typedef struct bm_anneal_params {
@@ -687,15 +688,20 @@ int bm_anneal_get_pool(bm_anneal* a, int32_t inst, int32_t* uv, int64_t* k);
 uint64_t bm_anneal_p_pool(const bm_anneal* a);
 /* Chains back to their state at creation. */
 int bm_anneal_reset(bm_anneal* a);
-/* Launch shape of the chain kernel (waves_per_block, lds_slots, blocks_per_cu
- * as in bm_set_tuning; the default is the first context's swap-kernel shape). */
+/* Launch shape of the chain kernel.  group_lanes 64: one wave per chain, with
+ * waves_per_block, blocks_per_cu (as in bm_set_tuning) and unroll 2 or 4; 256:
+ * the four waves of a block share a chain, 4 list entries per lane (only
+ * blocks_per_cu counts); any other value leaves the choice between the two to
+ * the library, from the number of chains and the mean degree, as at creation
+ * (the rest then is the first context's swap-kernel shape).
+ * bm_anneal_get_tuning reports the shape that runs. */
 int bm_anneal_get_tuning(const bm_anneal* a, bm_tuning* t);
 int bm_anneal_set_tuning(bm_anneal* a, const bm_tuning* t);
-/* Autotuner: times one launch of `steps` steps for each shape of a grid of
- * list entries per lane {2,4} x waves per block {1,2,4,8} x table slots per
- * wave x blocks per CU {4,16}, keeps the fastest and resets the chains.
- * trials (5 doubles per trial: waves, slots, blocks_per_cu, unroll, ms; up to
- * max_trials) may be NULL.  bm_anneal_set_tuning takes unroll 2 or 4. */
+/* Autotuner: times one launch of `steps` steps for each shape of a grid, one
+ * wave per chain with list entries per lane {2,4} x waves per block {1,2,4,8} x
+ * blocks per CU {4,8,16}, then the four waves of a block per chain; keeps the
+ * fastest and resets the chains.  trials (5 doubles per trial: waves, slots,
+ * blocks_per_cu, unroll, ms, in this order; up to max_trials) may be NULL. */
 int bm_anneal_autotune(bm_anneal* a, int64_t steps, bm_tuning* best, double* trials, int32_t max_trials,
                        int32_t* n_trials);
 /* Last error of an annealing object (or of the last failed create). */

@@ -67,3 +67,48 @@ def test_patch_of_an_accepted_batch_costs_less_than_a_build(bm):
         b.close()
     print(f"[costs] {accepted} swaps: patch {min(patch):.3f} ms, build {min(build):.3f} ms", flush=True)
     assert min(patch) < 0.5 * min(build)
+
+
+def test_chain_shapes_are_the_ones_asked_for(bm):
+    """Four waves per chain and one wave per chain can both be selected and are
+    reported as what runs: with few chains and long lists the first takes about
+    a third of the second's time; the chains are the same."""
+    n = 4000
+    male, female, _, pi = make_pair(bm, n=n, deg=200.0, weights=bm.WEIGHTS_LOGNORMAL, seed=9)
+    with bm.Context(n, male, female) as ctx:
+        ctx.set_mapping(pi)
+        with bm.Anneal([ctx], chains_per_instance=64, seed=3, t0=50.0, decay=0.9999, p_rot3=0.1) as ann:
+            took, state = {}, {}
+            for lanes, waves, unroll in ((64, 1, 4), (64, 8, 2), (256, 1, 2), (0, 1, 2)):
+                ann.set_tuning(waves, 640, 16, unroll=unroll, group_lanes=lanes)
+                t = ann.tuning()
+                if lanes == 64:
+                    assert (t["group_lanes"], t["waves_per_block"], t["unroll"]) == (64, waves, unroll)
+                else:
+                    assert (t["group_lanes"], t["waves_per_block"], t["unroll"]) == (256, 4, 4)
+
+                def run():
+                    ann.run(200, 1)
+                    ann.state()
+
+                took[lanes] = _best(ann.reset, run)
+                state[lanes, waves] = ann.state()
+            want = state[64, 1]
+            for got in state.values():
+                assert all(np.array_equal(got[k], want[k]) for k in want)
+            best, trials = ann.autotune(steps=100)
+            assert best == ann.tuning() and best["group_lanes"] == 256 and int(np.argmin(trials[:, 4])) == len(trials) - 1
+    print(f"[costs] 64 lanes {1e3 * took[64]:.2f} ms, 256 lanes {1e3 * took[256]:.2f} ms", flush=True)
+    assert took[256] < 0.67 * took[64]
+
+
+def test_chains_of_short_lists_keep_a_wave_each(bm):
+    """Unasked, chains whose steps have no entries for four waves, or that would
+    take several rounds of blocks, keep one wave each."""
+    n = 2000
+    male, female, _, pi = make_pair(bm, n=n, deg=5.0, seed=9)
+    with bm.Context(n, male, female) as ctx:
+        ctx.set_mapping(pi)
+        for chains in (1, 1024):
+            with bm.Anneal([ctx], chains_per_instance=chains, seed=3, t0=50.0, decay=0.9999, p_rot3=0.1) as ann:
+                assert ann.tuning()["group_lanes"] == 64
