@@ -684,7 +684,8 @@ __device__ __forceinline__ uint64_t rank_key(float x, int64_t p) {
 constexpr int kSelBits = 12, kSelBins = 1 << kSelBits, kSelThreads = 256;
 static_assert(kSelBins == kHistBins, "the scoring kernel fills the first digit's histogram");
 constexpr int kSelPer = 16;          /* consecutive keys per lane, loaded before any is used */
-constexpr int kSortMax = 8192;       /* largest top, and most keys ranked */
+constexpr int kSortMax = 8192;       /* largest top, and keys a ranking block holds in LDS at a time */
+constexpr int kSelCap = 2 * kSortMax;   /* most keys written out and ranked */
 
 /* 2^20 scores, 4,096 wanted: 27 us with the clearing (six 11-bit passes handed
  * from block to block, a compaction and a one-block bitonic sort: 125 us).
@@ -692,14 +693,32 @@ constexpr int kSortMax = 8192;       /* largest top, and most keys ranked */
  * scoring kernel, the second out of one pass over the scores; then every key
  * at or above the 24-bit threshold is written out and ranked by counting.
  * Those are the `top` and the few others that share the threshold's 24 bits.
- * Only when so many keys share them that the written set would pass kSortMax
- * (scores equal to 2^-15: a network with dead units) does k_select_rest fix
- * further digits. */
+ * Only when so many keys share them that the written set would pass kSelCap
+ * (scores equal to 2^-15: a network with dead units, graphs of few distinct
+ * degrees) are further digits taken, each a pass of all blocks again: the
+ * score's last 8 bits, then the place in the pool, coarse and, past 2^25 pairs,
+ * fine.  Their kernels are launched always and leave at once otherwise.  One
+ * block for these digits took 796 us for 2^20 equal scores and, with room for
+ * kSortMax keys, ran for any pool when 8,192 were wanted (423 us). */
+constexpr int kSelStages = 5;
 struct SelState {
     uint32_t count;       /* keys written */
-    uint32_t pad[63];
-    uint32_t hist[2][kSelBins];
+    uint32_t more;        /* the first two digits do not settle the select */
+    uint32_t pad[62];
+    uint32_t hist[kSelStages][kSelBins];
 };
+
+/* Digit of a key at a stage; sh: the pool has at most 2^(sh + 12) pairs.  A
+ * smaller place is a larger digit, as in the key. */
+template <int STAGE>
+__device__ __forceinline__ uint32_t sel_digit(uint64_t key, int sh) {
+    const uint32_t u = (uint32_t)(key >> 32), p = 0xFFFFFFFFu - (uint32_t)key;
+    if (STAGE == 0) return u >> 20;
+    if (STAGE == 1) return (u >> 8) & (kSelBins - 1);
+    if (STAGE == 2) return u & 255u;
+    if (STAGE == 3) return (kSelBins - 1) - (p >> sh);
+    return (kSelBins - 1) - ((p >> (sh - kSelBits)) & (kSelBins - 1));
+}
 
 __global__ void __launch_bounds__(256) k_select_init(SelState* st) {
     uint32_t* p = reinterpret_cast<uint32_t*>(st);
@@ -824,7 +843,7 @@ __global__ void __launch_bounds__(kSelThreads) k_select_second(const float* __re
         if (h[i]) atomicAdd(&st->hist[1][i], h[i]);
 }
 
-/* Keys >= thr appended to out (at most kSortMax) by one block's share of the
+/* Keys >= thr appended to out (at most kSelCap) by one block's share of the
  * pool: each wave counts its lanes' keys, the block scans its waves' counts,
  * and one global atomic per block and round reserves the slots. */
 __device__ __forceinline__ void append_keys(const float* __restrict__ sc, int64_t P, uint64_t thr, uint32_t* count,
@@ -862,22 +881,37 @@ __device__ __forceinline__ void append_keys(const float* __restrict__ sc, int64_
 #pragma unroll
         for (int j = 0; j < kSelPer; j++)
             if (inmask & (1u << j)) {
-                if (at < (uint32_t)kSortMax) out[at] = rank_key(v[j], p0 + j);
+                if (at < (uint32_t)kSelCap) out[at] = rank_key(v[j], p0 + j);
                 at++;
             }
         __syncthreads();
     }
 }
 
-/* Threshold of the two digits; returns whether the keys at or above it fit
- * kSortMax. */
-template <int NT>
-__device__ __forceinline__ bool select_threshold(const SelState* st, uint32_t top, uint64_t* thr, DigitShared& S) {
+/* The smallest key of the digits of stages 0 .. STAGES - 1 that hold the top-th
+ * key; returns whether the keys from it on fit kSelCap (then the later stages
+ * are not needed).  Stages end early once they fit. */
+template <int STAGES>
+__device__ __forceinline__ bool select_threshold(const SelState* st, uint32_t top, int sh, uint64_t* thr, DigitShared& S) {
     uint32_t r = top, in;
-    const uint32_t d0 = find_digit<NT>(st->hist[0], &r, &in, S);
-    const uint32_t d1 = find_digit<NT>(st->hist[1], &r, &in, S);
-    *thr = ((uint64_t)((d0 << 20) | (d1 << 8))) << 32;
-    return (top - r) + in <= (uint32_t)kSortMax;
+    uint32_t u = find_digit<kSelThreads>(st->hist[0], &r, &in, S) << 20;
+    u |= find_digit<kSelThreads>(st->hist[1], &r, &in, S) << 8;
+    *thr = (uint64_t)u << 32;
+    if ((top - r) + in <= (uint32_t)kSelCap) return true;
+    if (STAGES < 3) return false;
+    u |= find_digit<kSelThreads>(st->hist[2], &r, &in, S);
+    *thr = (uint64_t)u << 32;
+    if ((top - r) + in <= (uint32_t)kSelCap) return true;
+    if (STAGES < 4) return false;
+    /* the last place of the digit's range has the smallest key in it */
+    uint64_t place = (uint64_t)(kSelBins - 1 - find_digit<kSelThreads>(st->hist[3], &r, &in, S)) << sh;
+    *thr = ((uint64_t)u << 32) | (0xFFFFFFFFull - (place + (1ull << sh) - 1));
+    if ((top - r) + in <= (uint32_t)kSelCap) return true;
+    if (STAGES < 5) return false;
+    const int fine = sh - kSelBits;
+    place += (uint64_t)(kSelBins - 1 - find_digit<kSelThreads>(st->hist[4], &r, &in, S)) << fine;
+    *thr = ((uint64_t)u << 32) | (0xFFFFFFFFull - (place + (1ull << fine) - 1));
+    return true;
 }
 
 __global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __restrict__ sc, int64_t P, SelState* st,
@@ -886,78 +920,92 @@ __global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __r
     __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
     __shared__ uint32_t base;
     uint64_t thr;
-    if (!select_threshold<kSelThreads>(st, top, &thr, S)) return;
+    if (!select_threshold<2>(st, top, 0, &thr, S)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->more = 1;
+        return;
+    }
     append_keys(sc, P, thr, &st->count, out, wcount, &base, blockIdx.x, gridDim.x);
 }
 
-/* One block: nothing when the two digits settled the select; otherwise the
- * remaining 40 bits of the threshold, digit by digit, and the keys. */
-__global__ void __launch_bounds__(1024) k_select_rest(const float* __restrict__ sc, int64_t P, SelState* st,
-                                                      uint64_t* __restrict__ out, uint32_t top) {
+/* Histogram of a further digit over the keys that share the earlier ones. */
+template <int STAGE>
+__global__ void __launch_bounds__(kSelThreads) k_select_digit(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                              uint32_t top, int sh) {
     __shared__ alignas(16) uint32_t h[kSelBins];
     __shared__ DigitShared S;
-    __shared__ uint32_t wcount[1024 / BM_WAVE];
-    __shared__ uint32_t base;
-    uint32_t r = top, in;
-    const uint32_t d0 = find_digit<1024>(st->hist[0], &r, &in, S);
-    const uint32_t d1 = find_digit<1024>(st->hist[1], &r, &in, S);
-    uint64_t thr = ((uint64_t)((d0 << 20) | (d1 << 8))) << 32;
-    if ((top - r) + in <= (uint32_t)kSortMax) return;
+    if (!st->more) return;
+    uint64_t thr;
+    if (select_threshold<STAGE>(st, top, sh, &thr, S)) return;
+    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x) h[i] = 0;
+    __syncthreads();
     const int lane = threadIdx.x & (BM_WAVE - 1);
-    for (int shift = 28; shift >= 0; shift = shift == 4 ? 0 : (shift == 0 ? -1 : shift - 12)) {
-        const int width = shift == 0 ? 4 : 12;
-        const uint64_t fixed = ~0ull << (shift + width);
-        __syncthreads();
-        for (int i = threadIdx.x; i < kSelBins; i += blockDim.x) h[i] = 0;
-        __syncthreads();
-        for (int64_t w0 = (int64_t)(threadIdx.x / BM_WAVE) * BM_WAVE * kSelPer; w0 < P;
-             w0 += (int64_t)blockDim.x * kSelPer) {
-            const int64_t p0 = w0 + (int64_t)lane * kSelPer;
-            float v[kSelPer];
-            load_scores(sc, p0, P, v);
+    /* every lane of a wave runs the same iterations (the ballots need them all) */
+    const int64_t wstride = (int64_t)gridDim.x * blockDim.x * kSelPer;
+    for (int64_t w0 = ((int64_t)blockIdx.x * (blockDim.x / BM_WAVE) + threadIdx.x / BM_WAVE) * BM_WAVE * kSelPer;
+         w0 < P; w0 += wstride) {
+        const int64_t p0 = w0 + (int64_t)lane * kSelPer;
+        float v[kSelPer];
+        load_scores(sc, p0, P, v);
 #pragma unroll
-            for (int j = 0; j < kSelPer; j++) {
-                const uint64_t k = rank_key(v[j], p0 + j);
-                wave_hist_add(h, p0 + j < P && (k & fixed) == thr, (uint32_t)(k >> shift) & ((1u << width) - 1u), lane);
-            }
+        for (int j = 0; j < kSelPer; j++) {
+            const uint64_t k = rank_key(v[j], p0 + j);
+            bool same = p0 + j < P;
+            if (STAGE == 2) same = same && (k >> 40) == (thr >> 40);
+            if (STAGE > 2) same = same && (k >> 32) == (thr >> 32);
+            if (STAGE > 3) same = same && sel_digit<3>(k, sh) == sel_digit<3>(thr, sh);
+            wave_hist_add(h, same, sel_digit<STAGE>(k, sh), lane);
         }
-        __syncthreads();
-        const uint32_t d = find_digit<1024>(h, &r, &in, S);
-        thr |= (uint64_t)d << shift;
-        if ((top - r) + in <= (uint32_t)kSortMax) break;
     }
-    append_keys(sc, P, thr, &st->count, out, wcount, &base, 0, 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x)
+        if (h[i]) atomicAdd(&st->hist[STAGE][i], h[i]);
+}
+
+__global__ void __launch_bounds__(kSelThreads) k_select_rest(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                             uint64_t* __restrict__ out, uint32_t top, int sh) {
+    __shared__ DigitShared S;
+    __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
+    __shared__ uint32_t base;
+    if (!st->more) return;
+    uint64_t thr;
+    (void)select_threshold<kSelStages>(st, top, sh, &thr, S);
+    append_keys(sc, P, thr, &st->count, out, wcount, &base, blockIdx.x, gridDim.x);
 }
 
 /* The written keys ranked by counting: a key's place in descending order is
- * the number of larger ones (keys are distinct).  Every block holds all keys
- * in LDS and ranks kRankKeys of them, 16 lanes per key counting a sixteenth
- * each; the `top` first places get their stream pairs. */
+ * the number of larger ones (keys are distinct).  Every block goes through all
+ * keys, kSortMax in LDS at a time, and ranks kRankKeys of them, 16 lanes per
+ * key counting a sixteenth each; the `top` first places get their stream
+ * pairs. */
 constexpr int kRankLanes = 16, kRankKeys = kSelThreads / kRankLanes;
 
 __global__ void __launch_bounds__(kSelThreads) k_select_rank(const uint64_t* __restrict__ keys, const SelState* st,
                                                              uint32_t top, uint64_t seed, int32_t n,
                                                              int2* __restrict__ out) {
     extern __shared__ ulonglong2 sk[];
-    const uint32_t cnt = st->count < (uint32_t)kSortMax ? st->count : (uint32_t)kSortMax;
+    const uint32_t cnt = st->count < (uint32_t)kSelCap ? st->count : (uint32_t)kSelCap;
     if ((uint32_t)blockIdx.x * kRankKeys >= cnt) return;
-    uint64_t* s = reinterpret_cast<uint64_t*>(sk);
-    /* every lane counts the same whole number of 16-byte words; key 0 is below every key */
-    const uint32_t words = (cnt + 2 * kRankLanes - 1) / (2 * kRankLanes) * kRankLanes;
-    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) {
-        ulonglong2 x;
-        x.x = 2 * i < cnt ? keys[2 * i] : 0ull;
-        x.y = 2 * i + 1 < cnt ? keys[2 * i + 1] : 0ull;
-        sk[i] = x;
-    }
-    __syncthreads();
     const uint32_t i = blockIdx.x * kRankKeys + threadIdx.x / kRankLanes, part = threadIdx.x % kRankLanes;
-    const uint64_t me = i < cnt ? s[i] : 0ull;
+    const uint64_t me = i < cnt ? keys[i] : 0ull;
     uint32_t rank = 0;
+    for (uint32_t b = 0; b < cnt; b += (uint32_t)kSortMax) {
+        const uint64_t* from = keys + b;
+        const uint32_t left = cnt - b < (uint32_t)kSortMax ? cnt - b : (uint32_t)kSortMax;
+        /* every lane counts the same whole number of 16-byte words; key 0 is below every key */
+        const uint32_t words = (left + 2 * kRankLanes - 1) / (2 * kRankLanes) * kRankLanes;
+        if (b) __syncthreads();   /* the keys before have been read */
+        for (uint32_t q = threadIdx.x; q < words; q += blockDim.x) {
+            ulonglong2 x;
+            x.x = 2 * q < left ? from[2 * q] : 0ull;
+            x.y = 2 * q + 1 < left ? from[2 * q + 1] : 0ull;
+            sk[q] = x;
+        }
+        __syncthreads();
 #pragma unroll 8
-    for (uint32_t q = part; q < words; q += kRankLanes) {
-        const ulonglong2 x = sk[q];
-        rank += (x.x > me ? 1u : 0u) + (x.y > me ? 1u : 0u);
+        for (uint32_t q = part; q < words; q += kRankLanes) {
+            const ulonglong2 x = sk[q];
+            rank += (x.x > me ? 1u : 0u) + (x.y > me ? 1u : 0u);
+        }
     }
 #pragma unroll
     for (int o = 1; o < kRankLanes; o <<= 1) rank += (uint32_t)__shfl_xor((int)rank, o, BM_WAVE);
@@ -1106,7 +1154,7 @@ hipError_t bm_launch_mlp_adam(const BmMlpDev& d, float lr, int64_t step, void* a
 }
 
 size_t bm_mlp_select_bytes(int64_t pool) {
-    return (size_t)pool * sizeof(float) + 512 + sizeof(SelState) + kSortMax * sizeof(uint64_t);
+    return (size_t)pool * sizeof(float) + 512 + sizeof(SelState) + kSelCap * sizeof(uint64_t);
 }
 
 int64_t bm_mlp_select_max_top(void) { return kSortMax; }
@@ -1127,17 +1175,25 @@ hipError_t bm_launch_mlp_rank_select(const BmMlpDev& d, const float* vf, uint64_
     q += (256 - (reinterpret_cast<uintptr_t>(q) & 255)) & 255;
     SelState* st = reinterpret_cast<SelState*>(q);
     uint64_t* keys = reinterpret_cast<uint64_t*>(st + 1);
-    hipLaunchKernelGGL(k_select_init, dim3(8), dim3(256), 0, s, st);
+    hipLaunchKernelGGL(k_select_init, dim3(16), dim3(256), 0, s, st);
     hipError_t e = launch_forward<true>(d, vf, nullptr, seed, n, pool, sc, st->hist[0], num_cus, s);
     if (e != hipSuccess) return e;
     const int blocks = grid_of(pool, kSelThreads * kSelPer, (int64_t)(num_cus > 0 ? num_cus : 256) * 4);
     hipLaunchKernelGGL(k_select_second, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top);
     hipLaunchKernelGGL(k_select_compact, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top);
-    hipLaunchKernelGGL(k_select_rest, dim3(1), dim3(1024), 0, s, sc, pool, st, keys, (uint32_t)top);
+    int sh = 0;
+    while (((int64_t)kSelBins << sh) < pool) sh++;
+    const int rest = grid_of(pool, kSelThreads * kSelPer, num_cus > 0 ? num_cus : 256);
+    hipLaunchKernelGGL(k_select_digit<2>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
+    hipLaunchKernelGGL(k_select_digit<3>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
+    /* a coarse digit's 2^sh places and the keys above it fit kSelCap */
+    if (sh > kSelBits + 1)
+        hipLaunchKernelGGL(k_select_digit<4>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
+    hipLaunchKernelGGL(k_select_rest, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top, sh);
     const size_t lds = kSortMax * sizeof(uint64_t);
     e = hipFuncSetAttribute((const void*)k_select_rank, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_select_rank, dim3(kSortMax / kRankKeys), dim3(kSelThreads), lds, s, keys, st, (uint32_t)top,
+    hipLaunchKernelGGL(k_select_rank, dim3(kSelCap / kRankKeys), dim3(kSelThreads), lds, s, keys, st, (uint32_t)top,
                        seed, n, out);
     return hipGetLastError();
 }
@@ -1162,7 +1218,7 @@ hipError_t bm_launch_mlp_rank(const BmMlpDev& d, const float* vf, uint64_t seed,
     char* temp = reinterpret_cast<char*>(idx_sorted + pool);
     temp += (256 - (reinterpret_cast<uintptr_t>(temp) & 255)) & 255;
     size_t temp_bytes = scratch_bytes - (size_t)(temp - p);
-    /* radix select of the top keys, then one block sorts them */
+    /* select of the top keys, then their ranking */
     if (top <= kSortMax && pool < (1LL << 32))
         return bm_launch_mlp_rank_select(d, vf, seed, n, pool, top, scratch, scratch_bytes, out, num_cus, s);
     hipError_t e = bm_launch_mlp_forward(d, vf, nullptr, seed, n, pool, sc, num_cus, s);

@@ -112,3 +112,31 @@ def test_chains_of_short_lists_keep_a_wave_each(bm):
         for chains in (1, 1024):
             with bm.Anneal([ctx], chains_per_instance=chains, seed=3, t0=50.0, decay=0.9999, p_rot3=0.1) as ann:
                 assert ann.tuning()["group_lanes"] == 64
+
+
+def test_ranking_ties_and_its_largest_top(bm):
+    """2^22 equal scores take all blocks' passes, not one block's, and 8,192
+    pairs wanted cost little more than 4,096."""
+    n = 2000
+    male, female, _, pi = make_pair(bm, n=n, deg=20.0, seed=2)
+    with bm.Context(n, male, female) as ctx:
+        ctx.set_mapping(pi)
+        with bm.Mlp(ctx, seed=1) as m:
+            m.refresh_features()
+            b = ctx.batch(8192)
+
+            def took(pool, top):
+                def call():
+                    b.gen_learned(m, 5, pool, top)
+                    ctx.sync()
+                call()
+                return _best(lambda: None, call, reps=5)
+
+            half, full, plain = took(1 << 20, 4096), took(1 << 20, 8192), took(1 << 22, 4096)
+            m.set_params(np.zeros(bm.Mlp.N_PARAMS, np.float32))
+            ties = took(1 << 22, 4096)
+            b.close()
+    print(f"[costs] 4096 {1e6 * half:.0f} us, 8192 {1e6 * full:.0f} us; 2^22 {1e6 * plain:.0f} us, equal {1e6 * ties:.0f} us",
+          flush=True)
+    assert full < 2.5 * half
+    assert ties < 4.0 * plain
