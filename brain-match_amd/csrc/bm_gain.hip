@@ -1241,10 +1241,13 @@ __global__ void __launch_bounds__(kBestThreads) k_best_tiles(BmDevGraph g, BmGai
         if (t == 0) s_thr = *reinterpret_cast<volatile int32_t*>(thr);
         __syncthreads();
         int4 a[4], m[4];   /* rows of tile (I, J) and of its mirror (J, I) */
+        /* a row ends in the middle of the last tile when the stride is an odd multiple of 32 */
+        const bool in_j = J * kTile + c4 < G.stride, in_i = I * kTile + c4 < G.stride;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            a[k] = *reinterpret_cast<const int4*>(&G.G[(int64_t)s_i[r0 + 16 * k].x * G.stride + J * kTile + c4]);
-            m[k] = *reinterpret_cast<const int4*>(&G.G[(int64_t)s_j[r0 + 16 * k].x * G.stride + I * kTile + c4]);
+            const int32_t *ra = &G.G[(int64_t)s_i[r0 + 16 * k].x * G.stride], *rm = &G.G[(int64_t)s_j[r0 + 16 * k].x * G.stride];
+            a[k] = in_j ? *reinterpret_cast<const int4*>(ra + J * kTile + c4) : make_int4(0, 0, 0, 0);
+            m[k] = in_i ? *reinterpret_cast<const int4*>(rm + I * kTile + c4) : make_int4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int k = 0; k < 4; k++) {
