@@ -506,17 +506,17 @@ static int scan_diag(bm_ctx* c, int64_t k, const int64_t** diag) {
 /* Launch shape of the scan kernels for a batch of k candidates.  Unless the
  * caller set one (bm_set_tuning), a batch too small to fill the device's wave
  * slots (k < 32,768: at most four candidates per slot) is bound by its longest
- * lists, so the swap kernel gives each candidate the four waves of a block
- * (n = 18,524: 4,096 pairs 111 us against 255 us with one wave each, 32,768
- * pairs 314 against 353 us, 65,536 pairs 527 against 476 us), the 3-vertex
- * kernel 4-wave blocks with more list entries per lane; a larger one runs in
- * the default throughput shape. */
+ * lists, so both kernels give each candidate the four waves of a block, 4 list
+ * entries per lane (n = 18,524, 4M edges: 4,096 pairs 111 us against 255 us
+ * with one wave each, 32,768 pairs 314 against 353 us, 65,536 pairs 527 against
+ * 476 us); a larger one runs in the default throughput shape.  Lists of 20
+ * entries leave three of the four waves idle: there 16,384 pairs take 120 us,
+ * 65,536 by one wave each 87 us. */
 static BmLaunch scan_launch(const bm_ctx* c, int kernel, int64_t k);
 
 static void default_tuning(bm_ctx* c) {
     const int cus = c->num_cus > 0 ? c->num_cus : 256;
-    /* slots per wave; 32 waves per CU fit 160 KiB when slots * slot bytes <= 5 KiB */
-    const int s = c->compact ? 1280 : 640;
+    const int s = c->compact ? 1280 : 640;   /* lds_slots: reported only */
     /* swap and 3-vertex kernels: the shape for large batches (see
      * scan_launch for small ones) -- 8-wave blocks, 2 list entries per lane:
      * occupancy over per-lane depth (2^20 pairs at n = 18,524: 4.5 against
@@ -533,12 +533,7 @@ static void default_tuning(bm_ctx* c) {
 
 static BmLaunch scan_launch(const bm_ctx* c, int kernel, int64_t k) {
     BmLaunch L = c->tune[kernel];
-    if (c->user_tuned[kernel] || k >= 32768) return L;
-    L.waves_per_block = 4;
-    L.lds_slots = c->compact ? 1280 : 640;
-    L.blocks_per_cu = 8;
-    L.unroll = kernel == BM_KERNEL_ROT3 ? 4 : 8;
-    L.coop = 1;
+    if (!c->user_tuned[kernel] && k < 32768) L.coop = 1;
     return L;
 }
 

@@ -165,7 +165,7 @@ swap_lists(const BmDevGraph& g, const int32_t* pi, const int32_t* inv, int32_t u
  * W = 1: one wave per candidate, any number of waves per
  * block; W = 4: the four waves of a block share a candidate (batches too
  * small to fill the device, where the longest list sets the time).  DIAG:
- * the current contributions of u and v come from diag (k_diag), so only the
+ * the current contributions of u and v come from diag (bm_launch_diag), so only the
  * lists of the new images are walked; their edges u <-> v, counted by both,
  * are looked up. */
 template <int MODE, bool PACKED, int U, int W, bool DIAG>
@@ -769,6 +769,7 @@ static hipError_t launch_swap_u(const BmDevGraph& g, const BmLaunch& L, const in
                                 uint64_t seed, int64_t k, int64_t* delta, const int64_t* diag, hipStream_t s) {
     if (L.coop) return launch_swap_one<M, P, 4, 4, D>(g, L, cand, off, seed, k, delta, diag, s);
     if (L.unroll == 2) return launch_swap_one<M, P, 2, 1, D>(g, L, cand, off, seed, k, delta, diag, s);
+    if (L.unroll == 8) return launch_swap_one<M, P, 8, 1, D>(g, L, cand, off, seed, k, delta, diag, s);
     return launch_swap_one<M, P, 4, 1, D>(g, L, cand, off, seed, k, delta, diag, s);
 }
 

@@ -409,10 +409,12 @@ typedef struct bm_tuning {
                              female-row entries per lane, 4, 8, 16 or 32 (table build,
                              which uses only this field) */
 } bm_tuning;
-/* Until bm_set_tuning is called for it, the swap (3-vertex) kernel runs a
- * batch of fewer than 32,768 candidates in 4-wave blocks with 8 (4) list
- * entries per lane, where one candidate's latency sets the time, and a larger
- * batch in the shape bm_get_tuning reports. */
+/* Until bm_set_tuning is called for it, the swap or 3-vertex kernel gives every
+ * candidate of a batch of fewer than 32,768 the four waves of a block (4 list
+ * entries per lane), since there one candidate's latency sets the time, and
+ * runs a larger batch in the shape bm_get_tuning reports.  BM_KERNEL_SCORE's
+ * shape is checked and returned, but the score has one form (fixed chunks of
+ * the male lists). */
 int bm_get_tuning(const bm_ctx* ctx, int32_t kernel, bm_tuning* t);
 int bm_set_tuning(bm_ctx* ctx, int32_t kernel, const bm_tuning* t);
 
