@@ -844,28 +844,32 @@ hipError_t bm_launch_anneal(const BmDevGraph* insts, int packed, BmChain* chains
     });
 }
 
-/* Chains back to their start: one block per chain copies its instance's
- * matching (n+1, then its inverse) to the chain's current and best matchings
- * and inverse. */
+/* Chains back to their start: a block per chain at a time copies its
+ * instance's matching (n+1, then its inverse) to the chain's current and best
+ * matchings and inverse. */
 __global__ void __launch_bounds__(256) k_anneal_reset(const BmDevGraph* __restrict__ insts,
-                                                      const BmChain* __restrict__ chains,
+                                                      const BmChain* __restrict__ chains, int64_t n_chains,
                                                       const int32_t* __restrict__ init,
                                                       const int64_t* __restrict__ init_off, int32_t* __restrict__ pool) {
-    const BmChain& ch = chains[blockIdx.x];
-    const int64_t len = (int64_t)insts[ch.inst].n + 1;
-    const int32_t* from = init + init_off[ch.inst];
-    int32_t* to = pool + ch.pi_off;
-    for (int64_t i = threadIdx.x; i < len; i += blockDim.x) {
-        const int32_t f = from[i];
-        to[i] = f;
-        to[len + i] = f;
-        to[2 * len + i] = from[len + i];
+    for (int64_t c = blockIdx.x; c < n_chains; c += gridDim.x) {
+        const BmChain& ch = chains[c];
+        const int64_t len = (int64_t)insts[ch.inst].n + 1;
+        const int32_t* from = init + init_off[ch.inst];
+        int32_t* to = pool + ch.pi_off;
+        for (int64_t i = threadIdx.x; i < len; i += blockDim.x) {
+            const int32_t f = from[i];
+            to[i] = f;
+            to[len + i] = f;
+            to[2 * len + i] = from[len + i];
+        }
     }
 }
 
 hipError_t bm_launch_anneal_reset(const BmDevGraph* insts, const BmChain* chains, int64_t n_chains,
                                   const int32_t* init, const int64_t* init_off, int32_t* pool, hipStream_t s) {
-    hipLaunchKernelGGL(k_anneal_reset, dim3((unsigned)n_chains), dim3(256), 0, s, insts, chains, init, init_off, pool);
+    /* fewer than 2^32 threads, whatever the number of chains */
+    const int64_t blocks = n_chains < (1 << 20) ? n_chains : 1 << 20;
+    hipLaunchKernelGGL(k_anneal_reset, dim3((unsigned)blocks), dim3(256), 0, s, insts, chains, n_chains, init, init_off, pool);
     return hipGetLastError();
 }
 

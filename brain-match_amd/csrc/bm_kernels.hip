@@ -670,28 +670,30 @@ __global__ void k_gen_amajor(int32_t n, uint64_t seed, const int64_t* __restrict
     }
 }
 
-/* One block per row: every entry takes the first empty slot from its home
- * bucket on (compare-and-swap; keys are unique in a row).  Within a bucket
+/* A block per row at a time: every entry takes the first empty slot from its
+ * home bucket on (compare-and-swap; keys are unique in a row).  Within a bucket
  * slots fill in order, which the lookups rely on. */
 template <bool PACKED>
 __global__ void __launch_bounds__(256) k_rowtab_fill(const int64_t* __restrict__ ptr, const int2* __restrict__ adj,
-                                                     const uint64_t* __restrict__ desc, uint4* __restrict__ tab) {
-    const int32_t row = blockIdx.x;
-    const int64_t b = ptr[row], e = ptr[row + 1];
-    const uint64_t d = desc[row];
-    const uint32_t lb = (uint32_t)(d & 63u);
-    const uint32_t per = RowSlots<PACKED>::kPerBucket, smask = (per << lb) - 1u;
-    for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
-        const int2 x = adj[i];
-        uint32_t s = row_home(x.x, lb) * per;
-        if (PACKED) {
-            uint32_t* T = reinterpret_cast<uint32_t*>(tab + (d >> 6));
-            const uint32_t v = ((uint32_t)x.x << 15) | (uint32_t)x.y;
-            while (atomicCAS(&T[s], 0u, v) != 0u) s = (s + 1u) & smask;
-        } else {
-            unsigned long long* T = reinterpret_cast<unsigned long long*>(tab + (d >> 6));
-            const unsigned long long v = ((unsigned long long)(uint32_t)x.y << 32) | (uint32_t)x.x;
-            while (atomicCAS(&T[s], 0ull, v) != 0ull) s = (s + 1u) & smask;
+                                                     int32_t n, const uint64_t* __restrict__ desc,
+                                                     uint4* __restrict__ tab) {
+    for (int64_t row = blockIdx.x; row <= n; row += gridDim.x) {
+        const int64_t b = ptr[row], e = ptr[row + 1];
+        const uint64_t d = desc[row];
+        const uint32_t lb = (uint32_t)(d & 63u);
+        const uint32_t per = RowSlots<PACKED>::kPerBucket, smask = (per << lb) - 1u;
+        for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
+            const int2 x = adj[i];
+            uint32_t s = row_home(x.x, lb) * per;
+            if (PACKED) {
+                uint32_t* T = reinterpret_cast<uint32_t*>(tab + (d >> 6));
+                const uint32_t v = ((uint32_t)x.x << 15) | (uint32_t)x.y;
+                while (atomicCAS(&T[s], 0u, v) != 0u) s = (s + 1u) & smask;
+            } else {
+                unsigned long long* T = reinterpret_cast<unsigned long long*>(tab + (d >> 6));
+                const unsigned long long v = ((unsigned long long)(uint32_t)x.y << 32) | (uint32_t)x.x;
+                while (atomicCAS(&T[s], 0ull, v) != 0ull) s = (s + 1u) & smask;
+            }
         }
     }
 }
@@ -716,7 +718,9 @@ static hipError_t set_lds(const void* fn, size_t bytes) {
 hipError_t bm_launch_rowtab_fill(int packed, const int64_t* ptr, const int2* adj, int32_t n, const uint64_t* desc,
                                  uint4* tab, hipStream_t s) {
     auto k = packed ? k_rowtab_fill<true> : k_rowtab_fill<false>;
-    hipLaunchKernelGGL(k, dim3((unsigned)n + 1u), dim3(256), 0, s, ptr, adj, desc, tab);
+    /* a launch of 2^32 threads or more is cut short without an error */
+    const int64_t rows = (int64_t)n + 1, blocks = rows < (1 << 20) ? rows : 1 << 20;
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, s, ptr, adj, n, desc, tab);
     return hipGetLastError();
 }
 
