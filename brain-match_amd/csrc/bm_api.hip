@@ -872,21 +872,26 @@ static int build_reorder(bm_ctx* c, const int32_t* changed, int32_t cnum, std::v
 }
 
 /* The changed vertices of an enumeration (the head of d_reorder) kept with
- * the batch: d_reorder belongs to the context's next enumeration. */
-static int keep_changed(bm_batch* b, int32_t cnum) {
+ * the batch: d_reorder belongs to the context's next enumeration.  *enum_c = 0
+ * where the device has no room for them: the candidates then go one by one. */
+static int keep_changed(bm_batch* b, int32_t cnum, int32_t* enum_c) {
     bm_ctx* c = b->ctx;
+    *enum_c = 0;
     if (b->changed_cap < cnum) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
         (void)hipFree(b->d_changed);
         b->d_changed = nullptr;
         b->changed_cap = 0;
-        int rc = dalloc(c, &b->d_changed, (size_t)cnum);
-        if (rc != BM_OK) return rc;
+        if (dalloc(c, &b->d_changed, (size_t)cnum) != BM_OK) {
+            (void)hipGetLastError();   /* a launch's status is read from it */
+            return BM_OK;
+        }
         b->changed_cap = cnum;
     }
     if (cnum > 0)
         HIPCHK(c, hipMemcpyAsync(b->d_changed, c->d_reorder, (size_t)cnum * sizeof(int32_t), hipMemcpyDeviceToDevice,
                                  c->stream));
+    *enum_c = cnum;
     return BM_OK;
 }
 
@@ -901,13 +906,14 @@ extern "C" int bm_batch_gen_changed_pairs(bm_batch* b, const int32_t* changed, i
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipMemcpyAsync(c->d_reorder, re.data(), re.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, bm_launch_gen_changed_pairs(c->n, cnum, c->d_reorder, P, (int2*)b->d_cand, c->stream));
-    if ((rc = keep_changed(b, cnum)) != BM_OK) return rc;
+    int32_t enum_c = 0;
+    if ((rc = keep_changed(b, cnum, &enum_c)) != BM_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));  /* re goes out of scope */
     b->k = P;
     b->kind = 1;
     b->generated = 1;
     b->evaluated = 0;
-    b->enum_c = cnum;
+    b->enum_c = enum_c;
     return BM_OK;
 }
 
@@ -983,13 +989,14 @@ extern "C" int bm_batch_gen_changed_triples(bm_batch* b, const int32_t* changed,
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipMemcpyAsync(c->d_reorder, re.data(), re.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, bm_launch_gen_changed_triples(c->n, cnum, c->d_reorder, T, (int4*)b->d_cand, c->stream));
-    if ((rc = keep_changed(b, cnum)) != BM_OK) return rc;
+    int32_t enum_c = 0;
+    if ((rc = keep_changed(b, cnum, &enum_c)) != BM_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     b->k = T;
     b->kind = 2;
     b->generated = 1;
     b->evaluated = 0;
-    b->enum_c = cnum;
+    b->enum_c = enum_c;
     return BM_OK;
 }
 
@@ -1020,20 +1027,39 @@ static bool by_place_rows(const bm_ctx* c, int32_t cnum, double lookups) {
     return lookups > 0.5 * (double)cnum * c->row_adds + 5e6;
 }
 
-/* Placement rows of changed vertices [i0, i0 + ng) of the batch. */
-static int place_group(bm_batch* b, int32_t i0, int32_t ng, BmPlace* p) {
-    bm_ctx* c = b->ctx;
-    const int64_t stride = bm_gain_stride(c->n);
-    const int64_t need = 2 * (int64_t)ng * bm_place_splits(ng) * stride;
+/* Scratch for the placement rows of an enumeration of cnum changed vertices
+ * (its largest group) and, for triples, the third section's terms.  false: the
+ * device has no room for it, and the candidates go one by one. */
+static bool place_scratch(bm_ctx* c, int32_t cnum, bool triples) {
+    const auto words = [&](int32_t ng) {
+        return ng > 0 ? 2 * (int64_t)ng * bm_place_splits(ng) * bm_gain_stride(c->n) : 0;
+    };
+    /* the whole groups and the last one, whose rows may be split further */
+    const int64_t whole = words(cnum >= BM_PLACE_GROUP ? BM_PLACE_GROUP : 0), last = words(cnum % BM_PLACE_GROUP);
+    const int64_t need = whole > last ? whole : last;
     if (c->place_cap < need) {
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
         (void)hipFree(c->d_place);
         c->d_place = nullptr;
         c->place_cap = 0;
-        int rc = dalloc(c, &c->d_place, (size_t)need);
-        if (rc != BM_OK) return rc;
+        if (dalloc(c, &c->d_place, (size_t)need) != BM_OK) {
+            (void)hipGetLastError();   /* a launch's status is read from it */
+            return false;
+        }
         c->place_cap = need;
     }
+    if (triples && !c->d_cross && dalloc(c, &c->d_cross, 2 * ((size_t)c->n + 1)) != BM_OK) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+/* Placement rows of changed vertices [i0, i0 + ng) of the batch (place_scratch
+ * has made room). */
+static int place_group(bm_batch* b, int32_t i0, int32_t ng, BmPlace* p) {
+    bm_ctx* c = b->ctx;
+    const int64_t stride = bm_gain_stride(c->n);
     p->rows = c->d_place;
     p->changed = b->d_changed + i0;
     p->ng = ng;
@@ -1067,10 +1093,6 @@ static int eval_changed_triples(bm_batch* b) {
     const int64_t cc = b->enum_c, nn = c->n;
     const int64_t s2 = cc * (cc - 1) * (cc - 2) / 6 + cc * (cc - 1) / 2 * (nn - cc);
     const int64_t rest = nn - cc - 1;
-    if (!c->d_cross) {
-        int rc = dalloc(c, &c->d_cross, 2 * ((size_t)c->n + 1));
-        if (rc != BM_OK) return rc;
-    }
     HIPCHK(c, bm_launch_diag(devgraph(c), c->d_chunks, c->n_chunks, c->d_diag, c->num_cus, c->stream));
     BmPlace p;
     int rc = place_group(b, 0, b->enum_c, &p);
@@ -1098,7 +1120,7 @@ extern "C" int bm_batch_eval_swaps(bm_batch* b) {
                                       b->d_delta, pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_SWAP, &t);
-        if (by_place_rows(c, b->enum_c, (double)b->k * 2.6 * c->male.m / c->n)) {
+        if (by_place_rows(c, b->enum_c, (double)b->k * 2.6 * c->male.m / c->n) && place_scratch(c, b->enum_c, false)) {
             const int rc = eval_changed_pairs(b);
             timing_end(c, &t);
             if (rc == BM_OK) b->evaluated = 1;
@@ -1283,7 +1305,8 @@ extern "C" int bm_batch_eval_rot3(bm_batch* b) {
                                       (int4*)b->d_cand, pis, c->stream));
     } else {
         timing_begin(c, BM_KERNEL_ROT3, &t);
-        if (b->enum_c <= BM_PLACE_GROUP && by_place_rows(c, b->enum_c, (double)b->k * 13.0 * c->male.m / c->n)) {
+        if (b->enum_c <= BM_PLACE_GROUP && by_place_rows(c, b->enum_c, (double)b->k * 13.0 * c->male.m / c->n) &&
+            place_scratch(c, b->enum_c, true)) {
             const int rc = eval_changed_triples(b);
             timing_end(c, &t);
             if (rc == BM_OK) b->evaluated = 1;
