@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(kScoreThreads) k_mlp_forward(const float4* __r
     const float b3 = M.b3[0];
     const int64_t groups = (k + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
     const int64_t step = (int64_t)gridDim.x * kScoreWaves;
-    int64_t gr = (int64_t)blockIdx.x * kScoreWaves + wave;
+    int64_t gr = (int64_t)wave * gridDim.x + blockIdx.x;   /* few groups go to as many blocks */
     v4s xn[kFwdTiles];
 #pragma unroll
     for (int z = 0; z < kFwdTiles; z++) {
@@ -1059,8 +1059,7 @@ template <bool HIST>
 static hipError_t launch_forward(const BmMlpDev& d, const float* vf, const int2* list, uint64_t seed, int32_t n,
                                  int64_t k, float* score, uint32_t* hist, int32_t num_cus, hipStream_t s) {
     PairSrc ps{list, seed, n};
-    const int64_t groups = (k + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
-    int64_t blocks = (groups + kScoreWaves - 1) / kScoreWaves;
+    int64_t blocks = (k + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
     const int64_t cap = num_cus > 0 ? num_cus : 256;
     if (blocks > cap) blocks = cap;
     const size_t lds = sizeof(ScoreShared) + (HIST ? kHistBins * sizeof(uint32_t) : 0);
