@@ -696,8 +696,8 @@ constexpr int kSelCap = 2 * kSortMax;   /* most keys written out and ranked */
  * Only when so many keys share them that the written set would pass kSelCap
  * (scores equal to 2^-15: a network with dead units, graphs of few distinct
  * degrees) are further digits taken, each a pass of all blocks again: the
- * score's last 8 bits, then the place in the pool, coarse and, past 2^25 pairs,
- * fine.  Their kernels are launched always and leave at once otherwise.  One
+ * score's last 8 bits (in the compaction's place), then the place in the pool,
+ * coarse and, past 2^25 pairs, fine.  Their kernels leave at once otherwise.  One
  * block for these digits took 796 us for 2^20 equal scores and, with room for
  * kSortMax keys, ran for any pool when 8,192 were wanted (423 us). */
 constexpr int kSelStages = 5;
@@ -914,29 +914,12 @@ __device__ __forceinline__ bool select_threshold(const SelState* st, uint32_t to
     return true;
 }
 
-__global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __restrict__ sc, int64_t P, SelState* st,
-                                                                uint64_t* __restrict__ out, uint32_t top) {
-    __shared__ DigitShared S;
-    __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
-    __shared__ uint32_t base;
-    uint64_t thr;
-    if (!select_threshold<2>(st, top, 0, &thr, S)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) st->more = 1;
-        return;
-    }
-    append_keys(sc, P, thr, &st->count, out, wcount, &base, blockIdx.x, gridDim.x);
-}
-
-/* Histogram of a further digit over the keys that share the earlier ones. */
+/* Histogram of a further digit over the keys that share thr's earlier ones. */
 template <int STAGE>
-__global__ void __launch_bounds__(kSelThreads) k_select_digit(const float* __restrict__ sc, int64_t P, SelState* st,
-                                                              uint32_t top, int sh) {
-    __shared__ alignas(16) uint32_t h[kSelBins];
-    __shared__ DigitShared S;
-    if (!st->more) return;
-    uint64_t thr;
-    if (select_threshold<STAGE>(st, top, sh, &thr, S)) return;
-    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x) h[i] = 0;
+__device__ __forceinline__ void digit_pass(const float* __restrict__ sc, int64_t P, SelState* st, uint64_t thr, int sh,
+                                           uint32_t* h) {
+    constexpr int bins = STAGE == 2 ? 256 : kSelBins;
+    for (int i = threadIdx.x; i < bins; i += blockDim.x) h[i] = 0;
     __syncthreads();
     const int lane = threadIdx.x & (BM_WAVE - 1);
     /* every lane of a wave runs the same iterations (the ballots need them all) */
@@ -957,8 +940,35 @@ __global__ void __launch_bounds__(kSelThreads) k_select_digit(const float* __res
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kSelBins; i += blockDim.x)
+    for (int i = threadIdx.x; i < bins; i += blockDim.x)
         if (h[i]) atomicAdd(&st->hist[STAGE][i], h[i]);
+}
+
+/* The keys, where two digits settle the select; else the third digit. */
+__global__ void __launch_bounds__(kSelThreads) k_select_compact(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                                uint64_t* __restrict__ out, uint32_t top) {
+    __shared__ uint32_t h[256];
+    __shared__ DigitShared S;
+    __shared__ uint32_t wcount[kSelThreads / BM_WAVE];
+    __shared__ uint32_t base;
+    uint64_t thr;
+    if (select_threshold<2>(st, top, 0, &thr, S)) {
+        append_keys(sc, P, thr, &st->count, out, wcount, &base, blockIdx.x, gridDim.x);
+        return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->more = 1;
+    digit_pass<2>(sc, P, st, thr, 0, h);
+}
+
+template <int STAGE>
+__global__ void __launch_bounds__(kSelThreads) k_select_digit(const float* __restrict__ sc, int64_t P, SelState* st,
+                                                              uint32_t top, int sh) {
+    __shared__ alignas(16) uint32_t h[kSelBins];
+    __shared__ DigitShared S;
+    if (!st->more) return;
+    uint64_t thr;
+    if (select_threshold<STAGE>(st, top, sh, &thr, S)) return;
+    digit_pass<STAGE>(sc, P, st, thr, sh, h);
 }
 
 __global__ void __launch_bounds__(kSelThreads) k_select_rest(const float* __restrict__ sc, int64_t P, SelState* st,
@@ -1180,15 +1190,16 @@ hipError_t bm_launch_mlp_rank_select(const BmMlpDev& d, const float* vf, uint64_
     const int blocks = grid_of(pool, kSelThreads * kSelPer, (int64_t)(num_cus > 0 ? num_cus : 256) * 4);
     hipLaunchKernelGGL(k_select_second, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top);
     hipLaunchKernelGGL(k_select_compact, dim3(blocks), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top);
-    int sh = 0;
-    while (((int64_t)kSelBins << sh) < pool) sh++;
-    const int rest = grid_of(pool, kSelThreads * kSelPer, num_cus > 0 ? num_cus : 256);
-    hipLaunchKernelGGL(k_select_digit<2>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
-    hipLaunchKernelGGL(k_select_digit<3>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
-    /* a coarse digit's 2^sh places and the keys above it fit kSelCap */
-    if (sh > kSelBits + 1)
-        hipLaunchKernelGGL(k_select_digit<4>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
-    hipLaunchKernelGGL(k_select_rest, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top, sh);
+    if (pool > kSelCap) {   /* else every key fits */
+        int sh = 0;
+        while (((int64_t)kSelBins << sh) < pool) sh++;
+        const int rest = grid_of(pool, kSelThreads * kSelPer, num_cus > 0 ? num_cus : 256);
+        hipLaunchKernelGGL(k_select_digit<3>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
+        /* a coarse digit's 2^sh places and the keys above it fit kSelCap */
+        if (sh > kSelBits + 1)
+            hipLaunchKernelGGL(k_select_digit<4>, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, (uint32_t)top, sh);
+        hipLaunchKernelGGL(k_select_rest, dim3(rest), dim3(kSelThreads), 0, s, sc, pool, st, keys, (uint32_t)top, sh);
+    }
     const size_t lds = kSortMax * sizeof(uint64_t);
     e = hipFuncSetAttribute((const void*)k_select_rank, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
