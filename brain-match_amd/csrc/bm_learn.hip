@@ -294,6 +294,8 @@ extern "C" int bm_mlp_gradient(bm_mlp* m, const int32_t* uv, const float* target
     return BM_OK;
 }
 
+static constexpr int64_t kTraceSteps = 4096;
+
 extern "C" int bm_mlp_train(bm_mlp* m, uint64_t seed, int64_t steps, int32_t batch, float lr, float* mse_trace) {
     if (!m || steps < 0 || batch < 16 || !(lr > 0.f)) return mfail(m, BM_ERR_ARG, "bm_mlp_train: invalid argument");
     MHIP(m, hipSetDevice(m->device));
@@ -308,7 +310,9 @@ extern "C" int bm_mlp_train(bm_mlp* m, uint64_t seed, int64_t steps, int32_t bat
         if (rc != BM_OK) return rc;
         m->train_cap = batch;
     }
-    int rc = grow(m, &m->d_trace, &m->trace_cap, steps);
+    /* the errors stay on the device for kTraceSteps steps at a time */
+    const int64_t slots = steps < kTraceSteps ? steps : kTraceSteps;
+    int rc = grow(m, &m->d_trace, &m->trace_cap, slots);
     if (rc != BM_OK) return rc;
     for (int64_t s = 0; s < steps; s++) {
         const uint64_t sd = bm_rand_at(seed, (uint64_t)s);
@@ -318,12 +322,14 @@ extern "C" int bm_mlp_train(bm_mlp* m, uint64_t seed, int64_t steps, int32_t bat
         rc = batch_gradient(m, nullptr, sd, batch, nullptr, bm_batch_deltas_dev(m->train_batch));
         if (rc != BM_OK) return rc;
         m->adam_step++;
-        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_act, batch, m->d_trace + s, m->num_cus, m->stream));
-    }
-    if (mse_trace && steps > 0) {
-        MHIP(m, hipMemcpyAsync(mse_trace, m->d_trace, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-        MHIP(m, hipStreamSynchronize(m->stream));
-        for (int64_t s = 0; s < steps; s++) mse_trace[s] /= (float)batch;
+        const int64_t slot = s % slots;
+        MHIP(m, bm_launch_mlp_adam(m->d, lr, m->adam_step, m->d_act, batch, m->d_trace + slot, m->num_cus, m->stream));
+        if (mse_trace && (slot == slots - 1 || s == steps - 1)) {
+            float* out = mse_trace + (s - slot);
+            MHIP(m, hipMemcpyAsync(out, m->d_trace, (size_t)(slot + 1) * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+            MHIP(m, hipStreamSynchronize(m->stream));
+            for (int64_t i = 0; i <= slot; i++) out[i] /= (float)batch;
+        }
     }
     MHIP(m, hipStreamSynchronize(m->stream));
     return BM_OK;
