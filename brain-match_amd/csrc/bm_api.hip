@@ -1590,10 +1590,11 @@ extern "C" int bm_best_swap(bm_ctx* c, int64_t* delta, int32_t* u, int32_t* v) {
     int4* out = reinterpret_cast<int4*>(c->h_pin);
     KTiming t;
     timing_begin(c, BM_KERNEL_GAIN_SWAP, &t);
-    HIPCHK(c, bm_launch_gain_pis(devgraph(c), devgain(c), c->d_pis, c->stream));
+    int32_t* thr = reinterpret_cast<int32_t*>(c->d_best);
+    HIPCHK(c, bm_launch_gain_pis(devgraph(c), devgain(c), c->d_pis, c->stream, tiles ? thr : nullptr));
     if (tiles)
         HIPCHK(c, bm_launch_gain_best_tiles(devgraph(c), devgain(c), c->d_pis, c->d_chunks, c->n_out_chunks, c->max_mw,
-                                            reinterpret_cast<int32_t*>(c->d_best), c->d_best + 1, kBestSwapParts, out,
+                                            thr, c->d_best + 1, kBestSwapParts, out,
                                             c->num_cus, c->stream));
     else
         HIPCHK(c, bm_launch_gain_best_swap(devgraph(c), devgain(c), c->d_GT, c->d_pis, c->d_best + 1, kBestSwapParts,

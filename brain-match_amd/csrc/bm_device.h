@@ -144,9 +144,10 @@ size_t bm_gain_umajor_lds(int32_t n);
 size_t bm_gain_umajor_bitmap_lds(int32_t n);
 hipError_t bm_launch_gain_transpose(const BmGain& G, int32_t nrows, int32_t* GT, int32_t num_cus, hipStream_t s);
 /* The per-vertex words {pi(v), G(v, pi(v)), self-loops}: bm_gain_pis_words(n)
- * int4, the diagonal alone behind them. */
+ * int4, the diagonal alone behind them.  thr (may be NULL) is reset for a
+ * bm_launch_gain_best_tiles that follows. */
 int64_t bm_gain_pis_words(int32_t n);
-hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, hipStream_t s);
+hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, hipStream_t s, int32_t* thr = nullptr);
 /* a-major 3-vertex lookups (best delta and permutation per stream entry);
  * needs bm_gain_rot3_amajor_lds(n) bytes of LDS.  Triples with an edge are
  * queued (queue_entries entries of 3 x int4, split into one region per

@@ -1208,8 +1208,6 @@ __device__ __forceinline__ void best_to_part(const BestPair& b, int4* part) {
         *part = make_int4((int32_t)(uint32_t)(uint64_t)d, (int32_t)(uint32_t)((uint64_t)d >> 32), u, v);
 }
 
-__global__ void k_best_init(int32_t* thr) { *thr = INT32_MIN; }
-
 __global__ void __launch_bounds__(kBestThreads) k_best_tiles(BmDevGraph g, BmGain G, const int4* __restrict__ pis,
                                                              int32_t tiles, int32_t* __restrict__ thr,
                                                              int4* __restrict__ part) {
@@ -1394,7 +1392,8 @@ __device__ __forceinline__ const int32_t* pis_diag(const int4* pis, int32_t n) {
 
 /* Per vertex v: {pi(v), G(v, pi(v)), male self-loop weight of v, female
  * self-loop weight of pi(v)} (BM_ABSENT for a missing loop). */
-__global__ void k_gain_pis(BmDevGraph g, BmGain G, int4* __restrict__ pis) {
+__global__ void k_gain_pis(BmDevGraph g, BmGain G, int4* __restrict__ pis, int32_t* __restrict__ thr) {
+    if (thr && blockIdx.x == 0 && threadIdx.x == 0) *thr = INT32_MIN;   /* k_best_tiles' best value */
     int32_t* diag = pis_diag(pis, g.n);
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= g.n; v += stride) {
@@ -2176,10 +2175,10 @@ hipError_t bm_launch_gain_transpose(const BmGain& G, int32_t nrows, int32_t* GT,
     return hipGetLastError();
 }
 
-hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, hipStream_t s) {
+hipError_t bm_launch_gain_pis(const BmDevGraph& g, const BmGain& G, int4* pis, hipStream_t s, int32_t* thr) {
     int64_t blocks = ((int64_t)g.n + 256) / 256;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(k_gain_pis, dim3((unsigned)blocks), dim3(256), 0, s, g, G, pis);
+    hipLaunchKernelGGL(k_gain_pis, dim3((unsigned)blocks), dim3(256), 0, s, g, G, pis, thr);
     return hipGetLastError();
 }
 
@@ -2247,7 +2246,6 @@ hipError_t bm_launch_gain_best_tiles(const BmDevGraph& g, const BmGain& G, const
     if (tb > max_parts / 2) tb = max_parts / 2;
     if (eb > 6 * cus) eb = 6 * cus;
     if (eb > max_parts / 2) eb = max_parts / 2;
-    hipLaunchKernelGGL(k_best_init, dim3(1), dim3(1), 0, s, thr);
     hipLaunchKernelGGL(k_best_tiles, dim3((unsigned)tb), dim3(kBestThreads), 0, s, g, G, pis, tiles, thr, part);
     if (eb > 0) {
         auto kern = g.packed ? k_best_edges<true> : k_best_edges<false>;
