@@ -493,6 +493,24 @@ def main():
 PROPOSAL_SOURCES = ("uniform", "twohop", "learned")
 
 
+#: Rounds whose score a timed climb keeps: the uniform climb makes 7,000 a second.
+TRACE_CAP = 1 << 22
+
+
+def score_marks(tr, tt, whole, score0, seconds, fracs):
+    """Score at fractions of a climb's time from its rounds' scores tr and times
+    tt; None where a trace that is not whole has ended."""
+    marks = {}
+    for frac in fracs:
+        i = int(np.searchsorted(tt, frac * seconds))
+        if i >= len(tr) and not whole:
+            at = None
+        else:
+            at = int(tr[min(i, len(tr) - 1)]) if len(tr) else score0
+        marks[f"{frac * seconds:g}s"] = at
+    return marks
+
+
 def compare_proposals(bm, ctx, pi0, seconds, args, sources=PROPOSAL_SOURCES, planted=None):
     """The learned-proposal workload on the n = 18,524 pair, from the greedy
     matching.  The network is trained on train_samples (candidate, exact
@@ -540,16 +558,14 @@ def compare_proposals(bm, ctx, pi0, seconds, args, sources=PROPOSAL_SOURCES, pla
         if name == "learned":
             mlp.set_params(trained)
         ctx.set_mapping(pi0)
-        tr, tt, res = ctx.climb(prop, seed=21, time_limit_s=seconds, per_round=4096, **kw)
-        marks = {}
-        for frac in (0.1, 0.25, 0.5, 0.75, 1.0):
-            i = int(np.searchsorted(tt, frac * seconds))
-            marks[f"{frac * seconds:g}s"] = int(tr[min(i, len(tr) - 1)]) if len(tr) else score0
+        tr, tt, res = ctx.climb(prop, seed=21, time_limit_s=seconds, per_round=4096, trace_cap=TRACE_CAP, **kw)
+        whole = res["iterations"] <= len(tr)
+        marks = score_marks(tr, tt, whole, score0, seconds, (0.1, 0.25, 0.5, 0.75, 1.0))
         last = tt >= 0.9 * seconds
         out[name] = {"final_score": res["final_score"], "gain": res["final_score"] - score0,
                      "rounds": res["iterations"], "accepted": res["accepted"], "evaluated": res["evaluations"],
                      "verify_failures": res["verify_failures"], "seconds": res["seconds"], "score_at": marks,
-                     "gain_last_10pct": int(tr[-1] - tr[last][0]) if last.any() else 0}
+                     "gain_last_10pct": (int(tr[-1] - tr[last][0]) if last.any() else 0) if whole else None}
         if name == "learned":
             out[name]["uniform_fallback_rounds"] = res["fallback_rounds"]
         if s_planted is not None:
@@ -859,11 +875,8 @@ def bench_scale(args, bm):
                                 {"pool": 1 << 20, "mlp": mlp, "refresh_every": 1, "retrain_every": 1,
                                  "retrain_lr": args.retrain_lr, "fallback": True})):
             ctx.set_mapping(pi0)
-            tr, tt, res = ctx.climb(prop, seed=31, time_limit_s=args.scale, per_round=4096, **kw)
-            marks = {}
-            for frac in (0.1, 0.25, 0.5, 1.0):
-                i = int(np.searchsorted(tt, frac * args.scale))
-                marks[f"{frac * args.scale:g}s"] = int(tr[min(i, len(tr) - 1)]) if len(tr) else score0
+            tr, tt, res = ctx.climb(prop, seed=31, time_limit_s=args.scale, per_round=4096, trace_cap=TRACE_CAP, **kw)
+            marks = score_marks(tr, tt, res["iterations"] <= len(tr), score0, args.scale, (0.1, 0.25, 0.5, 1.0))
             out["climb_" + name] = {"final_score": res["final_score"], "rounds": res["iterations"],
                                     "accepted": res["accepted"], "verify_failures": res["verify_failures"],
                                     "score_at": marks}
