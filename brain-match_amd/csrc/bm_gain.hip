@@ -71,22 +71,45 @@ __device__ __forceinline__ bool male_maybe(const BmGain& G, int32_t a, int32_t b
     return !G.m_adj || ((adj_word(G, a, b) >> ((a < b ? b : a) & 31)) & 1u);
 }
 
-/* K row-table lookups at once: key[k] in the row of descriptor d[k] where
- * go[k], else BM_ABSENT without a load.  Every first bucket is loaded before
- * any later one, so the K lookups cost one memory latency unless a key sits
- * past its home bucket. */
-template <bool PACKED, int K>
-__device__ __forceinline__ void find_many(const uint4* tab, const uint64_t* d, const int32_t* key, const bool* go,
-                                          int32_t* out) {
-    uint4 e[K];
+/* K row-table lookups: key[k] in the row of descriptor d[k] where go[k], else
+ * BM_ABSENT without a load.  find_load requests every first bucket before
+ * find_finish looks at any, so the K lookups cost one memory latency unless a
+ * key sits past its home bucket; those go on with the next bucket.  Two slots
+ * a bucket (wide) leave more of them, so there they go on together (n = 18,524,
+ * 4M edges, us: best partners of 512 vertices 597 with a second look at the
+ * home bucket, 538 one after the other, 470 together); with four slots the
+ * extra state costs more than it gives (packed: 372, 305, 317). */
+template <int K>
+__device__ __forceinline__ void find_load(const uint4* tab, const uint64_t* d, const int32_t* key, const bool* go,
+                                          uint4* e) {
 #pragma unroll
     for (int k = 0; k < K; k++) {
         e[k] = make_uint4(0u, 0u, 0u, 0u);
         if (go[k] && key[k] != 0) e[k] = tab[(d[k] >> 6) + row_home(key[k], (uint32_t)(d[k] & 63u))];
     }
+}
+template <bool PACKED, int K>
+__device__ __forceinline__ void find_finish(const uint4* tab, const uint64_t* d, const int32_t* key, uint4* e,
+                                            int32_t* out) {
+    uint32_t pend = 0;
 #pragma unroll
-    for (int k = 0; k < K; k++)
-        if (!row_bucket<PACKED>(e[k], key[k] != 0 ? key[k] : -1, out[k])) out[k] = row_find<PACKED>(tab, d[k], key[k]);
+    for (int k = 0; k < K; k++) {
+        if (row_bucket<PACKED>(e[k], key[k] != 0 ? key[k] : -1, out[k])) continue;
+        if (PACKED) out[k] = row_find_from<PACKED>(tab, d[k], key[k], 1u);
+        else pend |= 1u << k;
+    }
+    if (PACKED) return;
+    for (uint32_t skip = 1; pend; skip++) {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if ((pend >> k) & 1u) {
+                const uint32_t lb = (uint32_t)(d[k] & 63u);
+                e[k] = tab[(d[k] >> 6) + ((row_home(key[k], lb) + skip) & ((1u << lb) - 1u))];
+            }
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (((pend >> k) & 1u) && row_bucket<PACKED>(e[k], key[k], out[k])) pend &= ~(1u << k);
+    }
 }
 
 /* Weights inside a triple of male vertices v[0..2] with images f[0..2]:
@@ -96,8 +119,9 @@ __device__ __forceinline__ void find_many(const uint4* tab, const uint64_t* d, c
  * self-loops fs[x]); BM_ABSENT elsewhere.  md / fd are the row-table
  * descriptors of the rows of v[i] in M and f[x] in F (loaded by the caller
  * with its other gathers), so the up to 12 lookups cost two memory latencies
- * (six 16-byte buckets in registers at a time).
- * v[2] = f[2] = 0 serves a pair. */
+ * (six 16-byte buckets in registers at a time).  PAIR: v[2] = f[2] = 0, and the
+ * four lookups that are left cost one. */
+template <bool PACKED, bool PAIR>
 __device__ __forceinline__ void triple_weights(const BmDevGraph& g, const int32_t* v,
                                                const uint64_t* md, const int32_t* f, const uint64_t* fd,
                                                const int32_t* fs, const bool (*have)[3], int32_t (*w)[3],
@@ -129,13 +153,12 @@ __device__ __forceinline__ void triple_weights(const BmDevGraph& g, const int32_
             fg[k] = f[i] != 0;
             k++;
         }
-    if (g.packed) {   /* uniform */
-        find_many<true, 6>(g.m_out_t.tab, mt, mk, mg, mw);
-        find_many<true, 6>(g.f_out_t.tab, ft, fk, fg, fw);
-    } else {
-        find_many<false, 6>(g.m_out_t.tab, mt, mk, mg, mw);
-        find_many<false, 6>(g.f_out_t.tab, ft, fk, fg, fw);
-    }
+    uint4 me[6], fe[6];
+    find_load<6>(g.m_out_t.tab, mt, mk, mg, me);
+    if (PAIR) find_load<6>(g.f_out_t.tab, ft, fk, fg, fe);
+    find_finish<PACKED, 6>(g.m_out_t.tab, mt, mk, me, mw);
+    if (!PAIR) find_load<6>(g.f_out_t.tab, ft, fk, fg, fe);
+    find_finish<PACKED, 6>(g.f_out_t.tab, ft, fk, fe, fw);
     k = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
@@ -969,6 +992,7 @@ __global__ void __launch_bounds__(kPatchThreads) k_gain_update(BmDevGraph g, BmG
  * guf1 = G(u, f1), gvf1 = G(v, f1), gvf2 = G(v, f2), with e_uv = "a male
  * edge between u and v may exist" (either direction): an edge's weight and
  * the female weights its correction needs are looked up only then. */
+template <bool PACKED>
 __device__ __forceinline__ int64_t gain_swap_delta_from(const BmDevGraph& g, const BmGain& G, int32_t u, int32_t v,
                                                         int32_t f1, int32_t f2, bool e_uv, int64_t guf2, int64_t guf1,
                                                         int64_t gvf1, int64_t gvf2, int32_t su, int32_t sv,
@@ -984,7 +1008,7 @@ __device__ __forceinline__ int64_t gain_swap_delta_from(const BmDevGraph& g, con
         const uint64_t fd[3] = {g.f_out_t.desc[f1], g.f_out_t.desc[f2], 0ull};
         const int32_t vtx[3] = {u, v, 0}, f[3] = {f1, f2, 0};
         int32_t w[3][3], F[3][3];
-        triple_weights(g, vtx, md, f, fd, fs, have, w, F);
+        triple_weights<PACKED, true>(g, vtx, md, f, fd, fs, have, w, F);
         const int32_t w1 = w[0][1], w2 = w[1][0];
         /* u -> v lands on f2 -> f1; v -> u on f1 -> f2 */
         if (w1 != BM_ABSENT)
@@ -997,27 +1021,29 @@ __device__ __forceinline__ int64_t gain_swap_delta_from(const BmDevGraph& g, con
     return d;
 }
 
+template <bool PACKED>
 __device__ __forceinline__ int64_t gain_swap_delta(const BmDevGraph& g, const BmGain& G, int32_t u, int32_t v) {
     if (u == v) return 0;
     const int32_t f1 = g.pi[u], f2 = g.pi[v];
     const int32_t* Gu = G.G + (int64_t)u * G.stride;
     const int32_t* Gv = G.G + (int64_t)v * G.stride;
-    return gain_swap_delta_from(g, G, u, v, f1, f2, male_maybe(G, u, v), Gu[f2], Gu[f1], Gv[f1], Gv[f2], G.m_self[u],
+    return gain_swap_delta_from<PACKED>(g, G, u, v, f1, f2, male_maybe(G, u, v), Gu[f2], Gu[f1], Gv[f1], Gv[f2], G.m_self[u],
                                 G.m_self[v], G.f_self[f1], G.f_self[f2]);
 }
 
 /* The same from the per-vertex words {pi, G(v, pi(v)), male self-loop,
  * female self-loop of pi(v)}: two random table reads per pair instead of
  * four. */
+template <bool PACKED>
 __device__ __forceinline__ int64_t gain_swap_delta_pis(const BmDevGraph& g, const BmGain& G, const int4* pis, int32_t u,
                                                        int32_t v) {
     if (u == v) return 0;
     const int4 pu = pis[u], pv = pis[v];
-    return gain_swap_delta_from(g, G, u, v, pu.x, pv.x, male_maybe(G, u, v), G.G[(int64_t)u * G.stride + pv.x], pu.y,
+    return gain_swap_delta_from<PACKED>(g, G, u, v, pu.x, pv.x, male_maybe(G, u, v), G.G[(int64_t)u * G.stride + pv.x], pu.y,
                                 G.G[(int64_t)v * G.stride + pu.x], pv.y, pu.z, pv.z, pu.w, pv.w);
 }
 
-template <int MODE, bool PIS>
+template <int MODE, bool PIS, bool PACKED>
 __global__ void __launch_bounds__(256) k_gain_swap(BmDevGraph g, BmGain G, const int2* __restrict__ cand,
                                                    const int64_t* __restrict__ off, uint64_t seed, int64_t k,
                                                    int64_t* __restrict__ delta, const int4* __restrict__ pis) {
@@ -1035,7 +1061,7 @@ __global__ void __launch_bounds__(256) k_gain_swap(BmDevGraph g, BmGain G, const
                 else u = umajor_owner(off, g.n, c);
             }
             const int32_t v = bm_umajor_partner(seed, (uint64_t)c, u, g.n);
-            delta[c] = PIS ? gain_swap_delta_pis(g, G, pis, u, v) : gain_swap_delta(g, G, u, v);
+            delta[c] = PIS ? gain_swap_delta_pis<PACKED>(g, G, pis, u, v) : gain_swap_delta<PACKED>(g, G, u, v);
         }
         return;
     }
@@ -1049,7 +1075,7 @@ __global__ void __launch_bounds__(256) k_gain_swap(BmDevGraph g, BmGain G, const
         } else {
             bm_uniform_pair(seed, (uint64_t)c, g.n, &u, &v);
         }
-        delta[c] = PIS ? gain_swap_delta_pis(g, G, pis, u, v) : gain_swap_delta(g, G, u, v);
+        delta[c] = PIS ? gain_swap_delta_pis<PACKED>(g, G, pis, u, v) : gain_swap_delta<PACKED>(g, G, u, v);
     }
 }
 
@@ -1091,6 +1117,7 @@ __device__ __forceinline__ void best_block_reduce(int64_t& d, int32_t& u, int32_
 
 /* The block's threads scan the partners v = u+1..n of u and keep their best
  * (d, u, v) under best_before. */
+template <bool PACKED>
 __device__ __forceinline__ void best_partner_scan(const BmDevGraph& g, const BmGain& G, const int32_t* __restrict__ GT,
                                                   const int4* __restrict__ pis, int32_t u, int64_t& bd, int32_t& bu,
                                                   int32_t& bv) {
@@ -1120,7 +1147,7 @@ __device__ __forceinline__ void best_partner_scan(const BmDevGraph& g, const BmG
             if (v > n) continue;
             int64_t d;
             if (mm[j]) {   /* a male edge between u and v may exist (rare): the full correction */
-                d = gain_swap_delta_from(g, G, u, v, f1, pv[j].x, true, gu[j], pu.y, tv[j], pv[j].y, pu.z, pv[j].z,
+                d = gain_swap_delta_from<PACKED>(g, G, u, v, f1, pv[j].x, true, gu[j], pu.y, tv[j], pv[j].y, pu.z, pv[j].z,
                                          pu.w, pv[j].w);
             } else {       /* only self-loops, whose weights the per-vertex words carry */
                 d = (int64_t)gu[j] - pu.y + tv[j] - pv[j].y;
@@ -1132,11 +1159,12 @@ __device__ __forceinline__ void best_partner_scan(const BmDevGraph& g, const BmG
     }
 }
 
+template <bool PACKED>
 __global__ void __launch_bounds__(kBestThreads) k_gain_best_swap(BmDevGraph g, BmGain G, const int32_t* __restrict__ GT,
                                                                  const int4* __restrict__ pis, int4* __restrict__ part) {
     int64_t bd = INT64_MIN;
     int32_t bu = INT32_MAX, bv = INT32_MAX;
-    for (int32_t u = blockIdx.x + 1; u < g.n; u += gridDim.x) best_partner_scan(g, G, GT, pis, u, bd, bu, bv);
+    for (int32_t u = blockIdx.x + 1; u < g.n; u += gridDim.x) best_partner_scan<PACKED>(g, G, GT, pis, u, bd, bu, bv);
     best_block_reduce(bd, bu, bv);
     if (threadIdx.x == 0)
         part[blockIdx.x] = make_int4((int32_t)(uint32_t)(uint64_t)bd, (int32_t)(uint32_t)((uint64_t)bd >> 32), bu, bv);
@@ -1145,6 +1173,7 @@ __global__ void __launch_bounds__(kBestThreads) k_gain_best_swap(BmDevGraph g, B
 /* Best partner of each u in u0 .. u0 + count - 1: block i takes u0 + i (and
  * every gridDim.x-th after it) and writes {delta lo, delta hi, u, v} for it
  * (delta INT64_MIN, v INT32_MAX when u has no partner v > u). */
+template <bool PACKED>
 __global__ void __launch_bounds__(kBestThreads) k_gain_best_partners(BmDevGraph g, BmGain G,
                                                                      const int32_t* __restrict__ GT,
                                                                      const int4* __restrict__ pis, int32_t u0,
@@ -1153,7 +1182,7 @@ __global__ void __launch_bounds__(kBestThreads) k_gain_best_partners(BmDevGraph 
         const int32_t u = u0 + i;
         int64_t bd = INT64_MIN;
         int32_t bu = u, bv = INT32_MAX;
-        best_partner_scan(g, G, GT, pis, u, bd, bu, bv);
+        best_partner_scan<PACKED>(g, G, GT, pis, u, bd, bu, bv);
         best_block_reduce(bd, bu, bv);
         if (threadIdx.x == 0)
             out[i] = make_int4((int32_t)(uint32_t)(uint64_t)bd, (int32_t)(uint32_t)((uint64_t)bd >> 32), u, bv);
@@ -1479,8 +1508,8 @@ __global__ void __launch_bounds__(kPrThreads, 8) k_gain_swap_rows(BmDevGraph g, 
         __syncthreads();
         if (ed.x != 0 && ed.x != u) {
             int32_t F12, F21;
-            if (!row_bucket<true>(b12, pv.x, F12)) F12 = row_find<true>(g.f_out_t.tab, d12, pv.x);
-            if (!row_bucket<true>(b21, pv.x, F21)) F21 = row_find<true>(g.f_in_t.tab, d21, pv.x);
+            if (!row_bucket<true>(b12, pv.x, F12)) F12 = row_find_from<true>(g.f_out_t.tab, d12, pv.x, 1u);
+            if (!row_bucket<true>(b21, pv.x, F21)) F21 = row_find_from<true>(g.f_in_t.tab, d21, pv.x, 1u);
             atomicAdd(&S[ed.x], pair_correction(ed.y, F12, F21, pu.w, pv.w));
         }
         for (int64_t e = tid + kPrThreads; e < oc + ic; e += kPrThreads) {
@@ -1705,7 +1734,7 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_swap_umajor(BmDevGraph g, B
     }
 }
 
-template <bool PIS>
+template <bool PIS, bool PACKED>
 __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4* __restrict__ cand, int64_t k,
                                                    int64_t* __restrict__ best, uint8_t* __restrict__ perm,
                                                    int write_perm_into_cand, const int4* __restrict__ pis) {
@@ -1755,7 +1784,7 @@ __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4*
                 fd[i] = g.f_out_t.desc[f[i]];
             }
             const bool have[3][3] = {{false, e01, e02}, {e01, false, e12}, {e02, e12, false}};
-            triple_weights(g, vtx, md, f, fd, fs, have, w, F);
+            triple_weights<PACKED, false>(g, vtx, md, f, fd, fs, have, w, F);
         }
         int64_t bd;
         int bp;
@@ -1784,6 +1813,7 @@ __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4*
 constexpr int kR3Triples = 2;     /* triples per thread in flight */
 constexpr int kR3EdgeSplit = 16;  /* k_gain_rot3_edges blocks per queue region */
 
+template <bool PACKED>
 __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, BmGain G, const int32_t* __restrict__ GT,
                                                                  const int4* __restrict__ pis,
                                                                  const int64_t* __restrict__ off, uint64_t seed,
@@ -1873,7 +1903,7 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, B
                 const bool have[3][3] = {{false, ab, ac}, {ba, false, bc}, {ca, bc, false}};
                 const uint64_t md[3] = {mda, g.m_out_t.desc[b], g.m_out_t.desc[c]};
                 const uint64_t fd[3] = {fda, g.f_out_t.desc[pb.x], g.f_out_t.desc[pc.x]};
-                triple_weights(g, vtx, md, f, fd, fs, have, w, F);
+                triple_weights<PACKED, false>(g, vtx, md, f, fd, fs, have, w, F);
             }
             int64_t bd;
             int bp;
@@ -1937,6 +1967,7 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, B
  * off-diagonal gains and its edge flags (a->b, b->a, a->c, c->a, b-c); the
  * per-vertex words give the images, diagonal gains and self-loops, and
  * triple_weights the edges' weights and the female weights around them. */
+template <bool PACKED>
 __global__ void __launch_bounds__(256) k_gain_rot3_edges(BmDevGraph g, BmGain G, const int4* __restrict__ pis,
                                                          const int4* __restrict__ queue, int64_t qper,
                                                          const int32_t* __restrict__ qcount, int64_t* __restrict__ best,
@@ -1960,7 +1991,7 @@ __global__ void __launch_bounds__(256) k_gain_rot3_edges(BmDevGraph g, BmGain G,
         const uint64_t md[3] = {g.m_out_t.desc[vtx[0]], g.m_out_t.desc[vtx[1]], g.m_out_t.desc[vtx[2]]};
         const uint64_t fd[3] = {g.f_out_t.desc[f[0]], g.f_out_t.desc[f[1]], g.f_out_t.desc[f[2]]};
         int32_t w[3][3], F[3][3];
-        triple_weights(g, vtx, md, f, fd, fs, have, w, F);
+        triple_weights<PACKED, false>(g, vtx, md, f, fd, fs, have, w, F);
         int64_t bd;
         int bp;
         rot3_from_gains(Gv, w, F, sv, fs, bd, bp);
@@ -2132,13 +2163,12 @@ hipError_t bm_launch_gain_swap(const BmDevGraph& g, const BmGain& G, int mode, c
     if (k <= 0) return hipSuccess;
     int64_t blocks = (k + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-#define BM_GAIN_SWAP_LAUNCH(M)                                                                                        \
-    if (pis)                                                                                                          \
-        hipLaunchKernelGGL((k_gain_swap<M, true>), dim3((unsigned)blocks), dim3(256), 0, s, g, G, cand, off, seed, k, \
-                           delta, pis);                                                                               \
-    else                                                                                                              \
-        hipLaunchKernelGGL((k_gain_swap<M, false>), dim3((unsigned)blocks), dim3(256), 0, s, g, G, cand, off, seed,  \
-                           k, delta, pis);
+#define BM_GAIN_SWAP_LAUNCH(M)                                                                           \
+    {                                                                                                    \
+        auto kern = pis ? (g.packed ? k_gain_swap<M, true, true> : k_gain_swap<M, true, false>)          \
+                        : (g.packed ? k_gain_swap<M, false, true> : k_gain_swap<M, false, false>);       \
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, g, G, cand, off, seed, k, delta, pis); \
+    }
     if (mode == BM_CAND_LIST) {
         BM_GAIN_SWAP_LAUNCH(BM_CAND_LIST)
     } else if (mode == BM_CAND_UMAJOR) {
@@ -2229,7 +2259,8 @@ hipError_t bm_launch_gain_best_swap(const BmDevGraph& g, const BmGain& G, const 
     if (blocks > max_parts) blocks = max_parts;
     if (blocks > (int64_t)g.n - 1) blocks = (int64_t)g.n - 1;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_gain_best_swap, dim3((unsigned)blocks), dim3(kBestThreads), 0, s, g, G, GT, pis, part);
+    auto kern = g.packed ? k_gain_best_swap<true> : k_gain_best_swap<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBestThreads), 0, s, g, G, GT, pis, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_best_swap_final, dim3(1), dim3(kBestThreads), 0, s, part, (int32_t)blocks, out);
@@ -2263,7 +2294,8 @@ hipError_t bm_launch_gain_best_partners(const BmDevGraph& g, const BmGain& G, co
     int64_t blocks = count;
     const int64_t cap = (int64_t)8 * (num_cus > 0 ? num_cus : 256);
     if (blocks > cap) blocks = cap;
-    hipLaunchKernelGGL(k_gain_best_partners, dim3((unsigned)blocks), dim3(kBestThreads), 0, s, g, G, GT, pis, u0, count,
+    auto kern = g.packed ? k_gain_best_partners<true> : k_gain_best_partners<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBestThreads), 0, s, g, G, GT, pis, u0, count,
                        out);
     return hipGetLastError();
 }
@@ -2274,7 +2306,8 @@ hipError_t bm_launch_gain_rot3_amajor(const BmDevGraph& g, const BmGain& G, cons
                                       int32_t num_cus, hipStream_t s) {
     const size_t lds = bm_gain_rot3_amajor_lds(g.n);
     if (lds > kLdsBytes) return hipErrorInvalidValue;
-    const void* kern = (const void*)k_gain_rot3_amajor;
+    auto amajor = g.packed ? k_gain_rot3_amajor<true> : k_gain_rot3_amajor<false>;
+    const void* kern = (const void*)amajor;
     hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     int occ = 0;
@@ -2286,10 +2319,11 @@ hipError_t bm_launch_gain_rot3_amajor(const BmDevGraph& g, const BmGain& G, cons
     if (blocks > queue_regions) blocks = queue_regions;
     if (blocks < 1 || !queue_counts) return hipErrorInvalidValue;
     const int64_t qper = queue ? queue_entries / blocks : 0;   /* entries per block region */
-    hipLaunchKernelGGL(k_gain_rot3_amajor, dim3((unsigned)blocks), dim3(kUmThreads), lds, s, g, G, GT, pis, off, seed,
+    hipLaunchKernelGGL(amajor, dim3((unsigned)blocks), dim3(kUmThreads), lds, s, g, G, GT, pis, off, seed,
                        best, perm, queue, qper, queue_counts);
+    auto edges = g.packed ? k_gain_rot3_edges<true> : k_gain_rot3_edges<false>;
     if (qper > 0)
-        hipLaunchKernelGGL(k_gain_rot3_edges, dim3((unsigned)(blocks * kR3EdgeSplit)), dim3(256), 0, s, g, G, pis,
+        hipLaunchKernelGGL(edges, dim3((unsigned)(blocks * kR3EdgeSplit)), dim3(256), 0, s, g, G, pis,
                            queue, qper, queue_counts, best, perm);
     return hipGetLastError();
 }
@@ -2299,12 +2333,10 @@ hipError_t bm_launch_gain_rot3(const BmDevGraph& g, const BmGain& G, const int4*
     if (k <= 0) return hipSuccess;
     int64_t blocks = (k + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    if (pis)
-        hipLaunchKernelGGL(k_gain_rot3<true>, dim3((unsigned)blocks), dim3(256), 0, s, g, G, const_cast<int4*>(cand), k,
-                           best, perm, cand_out_perm ? 1 : 0, pis);
-    else
-        hipLaunchKernelGGL(k_gain_rot3<false>, dim3((unsigned)blocks), dim3(256), 0, s, g, G, const_cast<int4*>(cand), k,
-                           best, perm, cand_out_perm ? 1 : 0, pis);
+    auto kern = pis ? (g.packed ? k_gain_rot3<true, true> : k_gain_rot3<true, false>)
+                    : (g.packed ? k_gain_rot3<false, true> : k_gain_rot3<false, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, g, G, const_cast<int4*>(cand), k, best, perm,
+                       cand_out_perm ? 1 : 0, pis);
     return hipGetLastError();
 }
 

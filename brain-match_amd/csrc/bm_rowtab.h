@@ -45,18 +45,24 @@ __device__ __forceinline__ bool row_bucket(const uint4& v, int32_t key, int32_t&
     return h0 || h1 || v.z == 0u;
 }
 
-/* Weight of key in the row with descriptor d, or BM_ABSENT (key 0: absent). */
+/* Weight of key (not 0) in the row with descriptor d, or BM_ABSENT, `skip`
+ * buckets past its home on. */
 template <bool PACKED>
-__device__ __forceinline__ int32_t row_find(const uint4* __restrict__ tab, uint64_t d, int32_t key) {
-    if (key == 0) return BM_ABSENT;
+__device__ __forceinline__ int32_t row_find_from(const uint4* __restrict__ tab, uint64_t d, int32_t key, uint32_t skip) {
     const uint32_t lb = (uint32_t)(d & 63u), mask = (1u << lb) - 1u;
     const uint4* T = tab + (d >> 6);
-    uint32_t b = row_home(key, lb);
+    uint32_t b = (row_home(key, lb) + skip) & mask;
     for (;;) {
         int32_t w;
         if (row_bucket<PACKED>(T[b], key, w)) return w;
         b = (b + 1u) & mask;
     }
+}
+
+/* Weight of key in the row with descriptor d, or BM_ABSENT (key 0: absent). */
+template <bool PACKED>
+__device__ __forceinline__ int32_t row_find(const uint4* __restrict__ tab, uint64_t d, int32_t key) {
+    return key == 0 ? BM_ABSENT : row_find_from<PACKED>(tab, d, key, 0u);
 }
 
 }  // namespace bmd
