@@ -57,7 +57,7 @@ struct bm_anneal {
     std::vector<int2*> prop_buf;      /* per instance, capacity prop_cap */
     std::vector<int64_t> prop_cap;
     BmAnnealSched sc;
-    double mean_deg;                  /* male edges per vertex, mean over the instances */
+    double mean_deg, mean_n;          /* male edges per vertex and vertices, means over the instances */
     BmLaunch L;
     int compact;
     int packed;
@@ -122,26 +122,36 @@ extern "C" int64_t bm_anneal_num_chains(const bm_anneal* a) { return a ? a->n_ch
 
 /* Launch shape L for the chains: one wave per chain (lanes 64), the four waves
  * of a block (256), or (any other value) whichever suits them.  A chain's steps
- * are a serial chain of dependent loads, so where the blocks of the wide form
+ * are a serial chain of dependent loads, so while the blocks of the wide form
  * are all resident four waves are faster as soon as a step has entries for
- * them; in two rounds only with longer lists.  200 steps, one instance, 10%
- * 3-vertex moves, us with four waves / with one: 256 chains of 10 edges a
- * vertex 899 / 843, of 20 977 / 1,015, of 50 1,285 / 2,062, of 200 2,068 /
- * 6,472; 1,024 chains (two rounds: 768 blocks are resident) of 50 2,738 /
- * 2,288, of 100 3,229 / 3,920. */
+ * them; in two rounds with 100 edges a vertex; in more only where the matchings
+ * of all one-wave chains (8 n bytes each) outgrow the caches, of which the
+ * four-wave form has a quarter in use at a time.  One instance, 10% 3-vertex
+ * moves, 100 steps, time with four waves over time with one: 256 chains of
+ * 5 / 20 / 50 / 200 edges a vertex at n = 2,000 1.01 / 0.90 / 0.68 / 0.38, 1,024
+ * 1.29 / 1.13 / 0.87 / 0.49; 2,048 of 50 / 100 / 200 1.44 / 1.01 / 0.79, at n =
+ * 12,000 1.34 / 0.90 / 0.70; 4,096 of 100 / 200 1.44 / 1.08 and 1.03 / 0.77.
+ * 64 instances of n = 1,562 to 19,819, 3,072 chains: 36.1 -> 32.2 ms per 500
+ * steps (by LDS tables built per candidate, before row tables: 35.5). */
 static hipError_t chain_shape(bm_anneal* a, BmLaunch L, int lanes) {
     const int rot = a->sc.p_rot3 != 0;
     dim3 grid, block;
-    L.coop = 1;
-    hipError_t e = bm_anneal_grid(a->packed, rot, L, (int64_t)1 << 40, &grid, &block);
-    if (e != hipSuccess) return e;
-    const int64_t resident = grid.x;
+    int64_t resident = 0, roomy = 0;   /* four-wave blocks on the device at once, in few and in as many registers as they like */
+    for (int c = 2; c >= 1; c--) {
+        L.coop = c;
+        const hipError_t e = bm_anneal_grid(a->packed, rot, L, (int64_t)1 << 40, &grid, &block);
+        if (e != hipSuccess) return e;
+        (c == 2 ? resident : roomy) = grid.x;
+    }
     if (lanes == kWaveLanes || lanes == kBlockLanes)
         L.coop = lanes == kBlockLanes;
+    else if (a->n_chains <= 2 * resident)
+        L.coop = a->mean_deg >= (a->n_chains <= resident / 2 ? 20.0 : (a->n_chains <= resident ? 40.0 : 100.0));
     else
-        L.coop = a->mean_deg >= 20.0 &&
-                 (a->n_chains <= resident || (a->mean_deg >= 80.0 && a->n_chains <= 4 * (int64_t)L.num_cus));
-    e = bm_anneal_grid(a->packed, rot, L, a->n_chains, &grid, &block);
+        L.coop = a->mean_deg >= 150.0 &&
+                 8.0 * a->mean_n * (double)(a->n_chains < 16 * (int64_t)L.num_cus ? a->n_chains : 16 * (int64_t)L.num_cus) >= 1.5e8;
+    if (L.coop && a->n_chains > roomy) L.coop = 2;
+    const hipError_t e = bm_anneal_grid(a->packed, rot, L, a->n_chains, &grid, &block);
     if (e != hipSuccess) return e;
     a->L = L;
     a->grid = grid;
@@ -209,8 +219,10 @@ extern "C" int bm_anneal_create(bm_anneal** out, bm_ctx* const* ctxs, int32_t n_
     /* launch shape: the swap kernel's tuning of the first context */
     a->L = bm_ctx_launch(ctxs[0], BM_KERNEL_SWAP);
     if (!a->compact && a->graphs[0].compact) a->L.lds_slots /= 2;
-    for (int32_t i = 0; i < n_inst; i++)
+    for (int32_t i = 0; i < n_inst; i++) {
         a->mean_deg += (double)bm_ctx_male(ctxs[i])->m / a->graphs[i].n / n_inst;
+        a->mean_n += (double)a->graphs[i].n / n_inst;
+    }
 
     int64_t pool = 0;
     a->pi_off.resize((size_t)a->n_chains);

@@ -572,10 +572,14 @@ __global__ void __launch_bounds__(256) k_zero64(int64_t* __restrict__ p, int64_t
  * simulated_annealing (src/best-swap/score-lookup.c:345-400); its delta
  * comes from a lookup table and its stream from xoshiro256**, here the
  * delta is recomputed exactly every step and the streams are counter-based.
+ * MIN = 4 holds the four-wave form to 128 registers, four blocks a CU instead
+ * of three (one instance of n = 12,000, 200 edges a vertex, 10% 3-vertex moves,
+ * 100 steps: 1,024 chains 2.71 -> 1.97 ms, 4,096 8.74 -> 7.50); its spills cost
+ * up to 3% where three blocks hold all chains.
  * Each chain also sums the male degrees of the vertices of its moves (the
  * byte model of the delta kernels) and counts its 3-vertex and pool moves. */
-template <bool PACKED, int U, bool ROT, int W>
-__global__ void __launch_bounds__(W == 1 ? 512 : 64 * W) k_anneal(const BmDevGraph* __restrict__ insts,
+template <bool PACKED, int U, bool ROT, int W, int MIN = 1>
+__global__ void __launch_bounds__(W == 1 ? 512 : 64 * W, MIN) k_anneal(const BmDevGraph* __restrict__ insts,
                                                                   BmChain* __restrict__ chains, int64_t n_chains,
                                                                   int32_t* pool, int64_t steps, BmAnnealSched sc,
                                                                   int64_t* __restrict__ traj,
@@ -817,11 +821,12 @@ hipError_t bm_launch_rot3(const BmDevGraph& g, const BmLaunch& L, const int4* ca
                          : launch_rot3_one<false, 4, 1>(g, L, cand, k, best, perm, cand_out_perm, s);
 }
 
-/* Annealing chains: 2 or 4 list entries per lane in flight (L.unroll). */
+/* Annealing chains: 2 or 4 list entries per lane in flight (L.unroll), or four
+ * waves a chain (L.coop; 2: in 128 registers). */
 template <typename F>
 static hipError_t with_anneal(int packed, int rot, const BmLaunch& L, F f) {
 #define BM_ANNEAL_W(P, R) \
-    (L.coop ? f(k_anneal<P, 4, R, 4>) : (L.unroll == 2 ? f(k_anneal<P, 2, R, 1>) : f(k_anneal<P, 4, R, 1>)))
+    (L.coop ? (R && L.coop == 2 ? f(k_anneal<P, 4, R, 4, R ? 4 : 1>) : f(k_anneal<P, 4, R, 4>)) : (L.unroll == 2 ? f(k_anneal<P, 2, R, 1>) : f(k_anneal<P, 4, R, 1>)))
     if (packed) return rot ? BM_ANNEAL_W(true, true) : BM_ANNEAL_W(true, false);
     return rot ? BM_ANNEAL_W(false, true) : BM_ANNEAL_W(false, false);
 #undef BM_ANNEAL_W

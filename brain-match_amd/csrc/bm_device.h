@@ -198,7 +198,7 @@ struct BmLaunch {
     int32_t blocks_per_cu;     /* persistent grid: blocks per CU (capped by occupancy) */
     int32_t num_cus;
     int32_t unroll;            /* list entries per lane in flight (2, 4 or 8) */
-    int32_t coop;              /* 1 = the four waves of a block share a candidate or chain */
+    int32_t coop;              /* 1 = the four waves of a block share a candidate or chain (2: chains, in 128 registers) */
 };
 
 /* Candidate sources. */
