@@ -29,9 +29,12 @@ under "rot3".
 
 value = candidates / second over the K timed steps of the headline strategy
 (graph, matching and output buffers resident in HBM; the table build is inside
-every step).  roofline = the step's dominant kernel: algorithmic bytes per
+every step).  roofline = the step's dominant kernel: compulsory bytes per
 launch / mean launch time from HIP events on the library stream; traffic = HBM
 bytes per launch measured with rocprofv3 (profiles/swap_n18524_traffic.json).
+per_candidate_model = the bytes a scan of every candidate's lists would read
+(48 + 28 per incident male edge of a pair, 69 + 36 of a triple); neither
+strategy reads them, and the rates it gives are equivalents.
 lds_roofline = the row build against the LDS atomic-add rate (one add per
 male edge x entry of a sparse female row; the hub rows kept dense are summed
 by the tile pass, gain_table.dense_rows).
@@ -159,6 +162,15 @@ def gain_lookup_bytes(ctx, k):
     fo, _ = ctx.degrees(female=True)
     n = ctx.n
     return n * 2 * gain_stride(n) * 4 + (n + 1) * 16 + 16 * int(mo.sum()) + 16 * int(fo.sum()) + (n + 2) * 8 + 8 * k
+
+
+def scan_bytes(ctx, k, out):
+    """Compulsory HBM bytes of one scan launch over k generated candidates: the
+    out- and in-lists of both graphs once (8 B an entry), the matching and its
+    inverse, the stream offsets, and `out` bytes per candidate."""
+    mo, _ = ctx.degrees(female=False)
+    fo, _ = ctx.degrees(female=True)
+    return 16 * int(mo.sum()) + 16 * int(fo.sum()) + 2 * 4 * (ctx.n + 1) + (ctx.n + 2) * 8 + out * k
 
 
 def measured_traffic(args):
@@ -371,8 +383,8 @@ def main():
         pcb, pcd = stream_bytes(seeds[-1], K)
         gain["per_candidate_model"] = {
             "applies_to_this_strategy": False,
-            "why": "the table strategy reads four table entries per pair, not the pair's male lists; the model "
-                   "prices a list scan and applies to the scan kernel (scan_kernel.roofline)",
+            "why": "the table strategy reads four table entries per pair, not the pair's male lists, which the "
+                   "model prices",
             "bytes_per_step": pcb, "mean_D": pcd / K,
             "deltas_per_s_at_hbm_peak": K * HBM_PEAK_GBS * 1e9 / pcb,
             "equivalent_GBps": pcb / (wall / args.steps) / 1e9,
@@ -401,17 +413,26 @@ def main():
         launch_s = per_launch_ms(kt, bm.KERNEL_SWAP) / 1000
         algo = [stream_bytes(s, K) for s in sseeds]
         bytes_per_launch = sum(b for b, _ in algo) / len(algo)
+        cb = scan_bytes(ctx, K, 8)
         mean_D = sum(d for _, d in algo) / len(algo) / K
         scan = {
             "value": K * steps / wall,
             "steps": steps,
             "ms_per_step": 1000 * wall / steps,
-            "roofline": {"bound": "hbm", "achieved": bytes_per_launch / launch_s / 1e9, "peak": HBM_PEAK_GBS,
-                         "unit": "GB/s", "frac": bytes_per_launch / launch_s / 1e9 / HBM_PEAK_GBS,
-                         "algo_bytes_per_launch": bytes_per_launch, "mean_D": mean_D, "launch_ms": 1000 * launch_s},
+            # compulsory: every list of both graphs once, the matching and its
+            # inverse, the stream offsets, a delta per pair
+            "roofline": {"bound": "hbm", "achieved": cb / launch_s / 1e9, "peak": HBM_PEAK_GBS,
+                         "unit": "GB/s", "frac": cb / launch_s / 1e9 / HBM_PEAK_GBS,
+                         "algo_bytes_per_launch": cb, "launch_ms": 1000 * launch_s},
+            "per_candidate_model": {
+                "applies_to_this_strategy": False,
+                "why": "the kernel walks the shorter list of every term and shares the current terms, and is bound by "
+                       "row-table lookups",
+                "bytes_per_launch": bytes_per_launch, "mean_D": mean_D,
+                "equivalent_GBps": bytes_per_launch / launch_s / 1e9},
         }
         log(f"scan ({args.stream}): {steps} x {K} pairs in {wall:.3f}s -> {scan['value']:.4g} deltas/s "
-            f"({scan['roofline']['achieved']:.0f} GB/s algorithmic)")
+            f"(a scan of every list would read {scan['per_candidate_model']['equivalent_GBps']:.0f} GB/s)")
         if gain is not None:
             same = bool((batch.deltas(0, 1 << 16) == gain_deltas_head).all())
             scan["matches_gain_path"] = same
@@ -430,7 +451,8 @@ def main():
         rf = dict(gain[dom + "_roofline"])
         if dom == "build":
             lds_rf = dict(gain["build_lds_roofline"], kernel="k_gain_build (sparse female rows)")
-        rf["kernel"] = ("k_gain_swap_umajor" if umajor else "k_gain_swap<uniform>") if dom == "lookup" \
+        rows = "k_gain_swap_rows" if 2 * K >= N_VERTICES * N_VERTICES else "k_gain_swap_umajor"
+        rf["kernel"] = (rows if umajor else "k_gain_swap<uniform>") if dom == "lookup" \
             else "k_gain_edge_desc+k_gain_dense_tile+k_gain_build"
     else:
         rf = dict(scan["roofline"])
@@ -665,8 +687,8 @@ def bench_anneal(args, bm):
     the true matching shuffled), chains_per_instance annealing chains each (T_s = 50 * 0.9999^s,
     swaps and 3-vertex moves), all advanced by one kernel launch replayed
     from a HIP graph; the launch shape comes from the autotuner.  Reports
-    chain steps/s (one exact delta per step), the algorithmic GB/s of the
-    steps, the device recount check and a CPU replay of one chain."""
+    chain steps/s (one exact delta per step), the GB/s a scan of every move's
+    lists would read at that rate, the device recount check and a CPU replay of one chain."""
     from concurrent.futures import ThreadPoolExecutor
 
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
@@ -727,7 +749,7 @@ def bench_anneal(args, bm):
                    "chains": chains, "steps_per_launch": steps, "launches": args.anneal, "p_rot3": 0.1},
         "autotuner": {"best": best, "trials": trials.tolist()},
         "ms_per_launch": timed_ms / max(1, timed_launches),
-        "algorithmic_GBps": algo / max(1, total_steps) * rate / 1e9,
+        "per_candidate_model_GBps": algo / max(1, total_steps) * rate / 1e9,
         "recount_mismatches": int(bad),
         "cpu_replay_identical": replay_ok,
         "best_gain_per_instance": {"min": int(gain.min()), "median": int(np.median(gain)), "max": int(gain.max())},
@@ -787,7 +809,7 @@ def anneal_for(bm, ctx, pi0, seconds, chains, p_pool, mlp=None, refresh_s=2.0, s
     out = {"chains": ann.chains, "seconds": el, "steps_per_chain": int(st["steps"][0]),
            "steps_per_s": int(steps) / el, "kernel_steps_per_s": int(steps) / (kernel_ms / 1000),
            "exact_deltas_per_s": (int(steps) + 4 * int(rot.sum())) / el,
-           "algorithmic_GBps_kernel": algo / (kernel_ms / 1000) / 1e9, "kernel_ms": kernel_ms,
+           "per_candidate_model_GBps": algo / (kernel_ms / 1000) / 1e9, "kernel_ms": kernel_ms,
            "best_score": int(st["best"].max()), "median_best": int(np.median(st["best"])),
            "three_vertex_fraction": float(rot.sum() / max(1, steps)),
            "pool_fraction": float(pooled.sum() / max(1, steps)), "recount_mismatches": mism,
@@ -827,7 +849,7 @@ def bench_scale(args, bm):
     wall, kt = timed(ctx, (bm.KERNEL_SWAP,), lambda i: b.eval_swaps_umajor(77, K), 1)
     algo, _ = ctx.umajor_algo_bytes(77, K)
     ms = per_launch_ms(kt, bm.KERNEL_SWAP)
-    out["scan"] = {"deltas_per_s": K / wall, "launch_ms": ms, "algorithmic_GBps": algo / ms / 1e6}
+    out["scan"] = {"deltas_per_s": K / wall, "launch_ms": ms, "per_candidate_model_GBps": algo / ms / 1e6}
     head = b.deltas(0, 1 << 16)
     ctx.gain_enable(True)
     ctx.gain_rebuild()
@@ -867,7 +889,7 @@ def bench_scale(args, bm):
         r = anneal_for(bm, ctx, pi0, args.scale, 2048, p_pool, mlp if p_pool > 0 else None)
         out[name] = r
         log(f"{name}: best {r['best_score']} after {r['seconds']:.0f}s, {r['steps_per_s']:.4g} steps/s, "
-            f"{r['algorithmic_GBps_kernel']:.0f} GB/s algorithmic, recount mismatches {r['recount_mismatches']}")
+            f"{r['per_candidate_model_GBps']:.0f} GB/s by the list-scan model, recount mismatches {r['recount_mismatches']}")
     if args.scale_climbs:
         ctx.gain_enable(args.evaluator == "gain")   # the climbs' exact deltas: table or scan
         for name, prop, kw in (("uniform", bm.PROPOSAL_UNIFORM, {}),
@@ -1034,12 +1056,16 @@ def bench_rot3(ctx, bm, args):
             ab3 = (n * 8 * gain_stride(n) + (n + 1) * 16 + 16 * int(mo.sum()) + (n + 2) * 8
                    + T * (2 * 4 + 2 * 4 + 9))
         else:
-            ab3, _ = b3.algo_bytes(generated=False)
+            ab3 = scan_bytes(ctx, T, 9) + 16 * T   # the triples are listed
+            model, _ = b3.algo_bytes(generated=False)
         kern = "k_gain_rot3_amajor+k_gain_rot3_edges" if mode == "gain" else "k_rot3"
         out[mode] = {"value": T * steps / wall, "ms_per_step": 1000 * wall / steps, "launch_ms": 1000 * l3,
                      "roofline": {"bound": "hbm", "achieved": ab3 / l3 / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                   "frac": ab3 / l3 / 1e9 / HBM_PEAK_GBS, "algo_bytes_per_launch": ab3,
                                   "kernel": kern, "traffic": measured_traffic(args).get(kern)}}
+        if mode == "scan":
+            out[mode]["per_candidate_model"] = {"applies_to_this_strategy": False, "bytes_per_launch": model,
+                                                "equivalent_GBps": model / l3 / 1e9}
         b3.eval_rot3_amajor(99, T)
         heads[mode] = (b3.deltas(0, 1 << 16), b3.perms(0, 1 << 16))
         log(f"rot3 {mode}: {T} a-major triples in {1000 * wall / steps:.1f} ms/step ({1000 * l3:.1f} ms kernel) "
