@@ -574,11 +574,11 @@ extern "C" int bm_create(bm_ctx** out, int32_t n, const bm_edges* male, const bm
         free_ctx(c);
         return fail(nullptr, BM_ERR_NOMEM, "bm_create: out of host memory");
     }
-    /* Compact LDS slots need keys below 2^17 and female weights in 0..32767;
-     * compact kernels also sum a lane's contributions in 32 bits, which needs
-     * male weights within +-32767 (every contribution is then within
-     * +-32767, and a lane takes at most 2^12 + 8 edges of a list shorter
-     * than 2^18). */
+    /* Compact: ids below 2^17, female weights in 0..32767, male weights within
+     * +-32767.  With male weights >= 0 too the row tables are packed, and their
+     * kernels sum a lane's contributions in 32 bits: each is at most 32767, and
+     * a lane takes a sixty-fourth of at most eight lists shorter than 2^17,
+     * 2^14 entries. */
     c->compact = n < (1 << 17);
     for (int64_t e = 0; e < c->male.m && c->compact; e++)
         if (c->male.out.adj[e].y < -32767 || c->male.out.adj[e].y > 32767) c->compact = 0;
@@ -1242,9 +1242,11 @@ extern "C" int bm_batch_eval_swaps_umajor(bm_batch* b, uint64_t seed, int64_t k)
         const bool bitmaps = !staged && bm_gain_umajor_bitmap_lds(c->n) <= 160 * 1024;
         /* one row of deltas per first vertex where 32-bit sums and the image
          * order hold and a row serves half as many pairs as it has entries: the
-         * row costs more than the two rows staged as they are, a pair less (n =
-         * 18,524, 2^26 pairs 1.08 ms by rows as they are, 1.22 by rows of
-         * deltas; 2^28 pairs 2.00 and 1.69) */
+         * row costs more than the two rows staged as they are, a pair less (us
+         * for n^2/4, n^2/2 and n^2 pairs, rows as they are / rows of deltas: n
+         * = 18,524, 4M edges 1,138 / 1,188, 1,539 / 1,385, 2,282 / 1,810; n =
+         * 8,000 317 / 346, 411 / 381, 582 / 452; n = 2,000 69 / 72, 74 / 74, 86
+         * / 77) */
         const bool delta_rows = staged && c->pi_full && c->packed && c->rows_small &&
                                 k >= (int64_t)c->n * c->n / 2;
         if (staged && (rc = gain_transposed(c)) != BM_OK) return rc;
@@ -1846,7 +1848,7 @@ extern "C" int bm_gain_enable(bm_ctx* c, int on) {
         if (!c->user_tuned[BM_KERNEL_GAIN_BUILD]) c->tune[BM_KERNEL_GAIN_BUILD].unroll = nwin > 1 ? 8 : 4;
     }
     /* dense male adjacency for the table lookups' edge tests, when it fits
-     * 2 GiB (43 MB at n = 18,524); otherwise they probe the hash tables */
+     * 2 GiB (43 MB at n = 18,524); otherwise they look in the row tables */
     if (!c->d_m_adj) {
         const int64_t words = ((int64_t)c->n + 1 + 31) / 32;
         const size_t abytes = (size_t)((int64_t)c->n + 1) * (size_t)words * sizeof(uint32_t);

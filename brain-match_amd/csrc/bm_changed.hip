@@ -38,7 +38,7 @@ constexpr int kRowUnit = 256;    /* target entries per wave and step: four per l
  * 256 at a time: a thread finds its edge's target list, a block scan numbers
  * the lists' 256-entry units, and the waves take units in turn (so a hub's
  * long list spreads over them), the next unit's entries loading while the
- * last one's are added to the LDS row.  Two blocks per CU up to n = 19,000. */
+ * last one's are added to the LDS row.  Two blocks per CU up to n = 18,911. */
 __global__ void __launch_bounds__(kRowThreads) k_place_rows(BmDevGraph g, const int32_t* __restrict__ changed,
                                                             int32_t ng, int32_t splits, int32_t stride,
                                                             int32_t* __restrict__ rows) {

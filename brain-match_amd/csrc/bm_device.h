@@ -31,7 +31,7 @@ struct BmDevGraph {
     const int32_t* inv;         /* inverse matching (female -> male, 0 = none), n+1; NULL when two males share a female */
     BmRowTab f_out_t, f_in_t, m_out_t, m_in_t;
     int32_t packed;             /* 1: row tables hold 4-byte slots (compact, and male weights >= 0) */
-    int32_t compact;            /* 1: LDS slots are (key << 15) | w (n < 2^17, weights 0..32767) */
+    int32_t compact;            /* 1: n < 2^17, female weights 0..32767, male within +-32767 (read on the host) */
 };
 
 /* Inserts the rows (ptr, adj) into the zeroed row tables described by desc. */

@@ -33,9 +33,9 @@
  * with atomic adds, its waves taking the row's edges one at a time with the
  * next edge's entry already loading, and writes the chunk out coalesced.  Lookups: one
  * thread per candidate, or one block per first vertex of a u-major stream.
- * Patches after moves: (male edge, female-row entry) pairs flattened per wave
- * (64 edges at a time, prefix sum of their female-row lengths), with global
- * integer atomic adds.
+ * Patches after moves: by work items of 64 male edges times 64 female-row
+ * entries with atomic adds, or, for few moves of vertices with many edges, by
+ * the rows they touch, through LDS.
  */
 #include "bm_device.h"
 #include "bm_devutil.h"
@@ -1212,7 +1212,7 @@ __global__ void __launch_bounds__(kBestThreads) k_best_swap_final(const int4* __
  *   H(f, f') + H(f', f) - diagonals (+ self-loops, + the u <-> v correction).
  * So the table is read once, as 64 x 64 tiles of H against their mirror tiles
  * transposed through LDS, and needs no transposed copy to be kept, patched or
- * rebuilt: its 1.37 GB at n = 18,524 are what bounds the search (299 us, 4.6
+ * rebuilt: its 1.37 GB at n = 18,524 are what bounds the search (336 us, 4.1
  * TB/s, and 146 us for 4M edges; by first vertex with a transposed copy 3.15
  * ms and 0.54 ms for the copy).  The
  * correction of adjacent pairs is left out here: a pair that would be the best
@@ -1776,7 +1776,7 @@ __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4*
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = 0; j < 3; j++) w[i][j] = F[i][j] = BM_ABSENT;
-        if (e01 || e02 || e12) {   /* the hash-row descriptors only for a triple with an edge */
+        if (e01 || e02 || e12) {   /* the row descriptors only for a triple with an edge */
             uint64_t md[3], fd[3];
 #pragma unroll
             for (int i = 0; i < 3; i++) {
@@ -1804,7 +1804,7 @@ __global__ void __launch_bounds__(256) k_gain_rot3(BmDevGraph g, BmGain G, int4*
  * and b or c are tested in the bitmaps, between b and c in the dense
  * adjacency bitmap.  A triple with such an edge (about 7% at n = 18,524)
  * needs the edge's weight and the female weights its correction uses from
- * the hash tables, a chain of dependent loads that nearly every wave's batch
+ * the row tables, a chain of dependent loads that nearly every wave's batch
  * would wait for: it is appended instead, with its four staged gains and two
  * gathered ones, to the block's region of a queue in device memory, and
  * k_gain_rot3_edges finishes the queue with full waves after the launch
@@ -1879,7 +1879,7 @@ __global__ void __launch_bounds__(kUmThreads) k_gain_rot3_amajor(BmDevGraph g, B
         }
         __syncthreads();
         /* the five permutations' best for entry i from its gathered values;
-         * the edge corrections (descriptor loads and hash probes) only when
+         * the edge corrections (descriptor loads and lookups) only when
          * edges says so */
         auto finish = [&](int64_t i, int32_t b, int32_t c, const int4& pb, const int4& pc, uint32_t wbc, int32_t gbc,
                           int32_t gcb, bool edges) {

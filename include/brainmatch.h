@@ -387,8 +387,9 @@ int bm_timing_get(bm_ctx* ctx, int32_t kernel, int64_t* launches, double* total_
 int bm_timing_reset(bm_ctx* ctx);
 int bm_sync(bm_ctx* ctx);
 
-/* Algorithmic bytes of a batch (per-candidate byte model, summed exactly from
- * the degree arrays): pairs 48 + 28*D(u,v) (+8 if read from memory), triples
+/* Bytes a scan of every candidate's male lists would read (per-candidate byte
+ * model, summed exactly from the degree arrays; the kernels intersect lists and
+ * read less): pairs 48 + 28*D(u,v) (+8 if read from memory), triples
  * 69 + 36*D3 (+12 if read from memory). */
 int bm_batch_algo_bytes(bm_batch* b, int32_t generated, int64_t* bytes, int64_t* sum_degree);
 int bm_uniform_algo_bytes(bm_ctx* ctx, uint64_t seed, int64_t k, int64_t* bytes, int64_t* sum_degree);
@@ -661,8 +662,7 @@ int bm_anneal_trajectory(bm_anneal* a, int64_t* traj, int32_t* count);
 int bm_anneal_verify(bm_anneal* a, int64_t* mismatches);
 /* Launches run and their summed duration (HIP events around each launch). */
 int bm_anneal_timing(bm_anneal* a, int64_t* launches, double* total_ms);
-/* Algorithmic bytes of the chain steps run so far, from the byte model of
- * the swap and triple kernels (48 + 28 D per swap step, 69 + 36 D3 per
+/* The same model's bytes of the chain steps run so far (48 + 28 D per swap step, 69 + 36 D3 per
  * 3-vertex step, D summed by the chains from the male degrees). */
 int bm_anneal_algo_bytes(bm_anneal* a, int64_t* bytes, int64_t* steps);
 /* Per chain: 3-vertex moves and moves built on a pool pair, taken so far
